@@ -1,0 +1,722 @@
+// fused_any_kernel: every operator on operands of any alignment, stride, size and element type - what the
+// direct-to-LDS kernels of fused_kernel.h do not take: rows that do not start on 16-byte boundaries (an odd N
+// or K), float32 data, A or B without a unit stride, an output row stride that is not a multiple of 8.
+//
+// Where it differs from those kernels is the way of the operands: 16-byte pieces travel HBM -> registers ->
+// LDS (global loads take any alignment; the direct-to-LDS load is used only where its pieces are
+// aligned), one K step ahead in registers and one in the second LDS buffer.  The LDS layouts, the MFMA
+// operand lanes and the order of the epilogue are the same.  What bounds it: the matrix pipes for
+// float32 (64 cycles per 32x32x2 block, 157 TFLOP/s at most), the LDS for the 16- and 8-bit types (the
+// fragment reads of a 64x64 wave block need its full rate), the epilogue's HBM streams with peers.
+//
+// Nothing on the hot path is predicated: rows past M (or N) repeat the last row, columns of B past N are
+// read as they lie in memory as long as the piece ends inside the operand - what they produce are output
+// rows and columns that do not exist and are not stored.  Only k beyond K has to be zero on both sides
+// (the other operand may hold NaN there); those pieces are loaded element by element in the last K step
+// of a source.
+#pragma once
+
+#include "fused_kernel.h"
+
+constexpr int IN_F32 = 3;  // next to IN_BF16, IN_F16, IN_FP8
+
+template <int IN> struct AnyIn;
+template <> struct AnyIn<IN_BF16> { static constexpr int ES = 2; };
+template <> struct AnyIn<IN_F16> { static constexpr int ES = 2; };
+template <> struct AnyIn<IN_FP8> { static constexpr int ES = 1; };
+template <> struct AnyIn<IN_F32> { static constexpr int ES = 4; };
+
+// [k][n] tile of B in LDS, n contiguous.  16- and 8-bit data use the transpose-read layout of ColTile; a
+// float32 fragment is four 4-byte reads per lane, row k for the first half-wave and row k + 4 for the second,
+// 32 consecutive columns (128 bytes) each: the 128-byte blocks of rows with bit 2 of k set change
+// places, so that the halves meet on different banks (rows of 256 bytes and more).
+template <int RB, int ES>
+struct AnyColTile : ColTile<RB, ES> {};
+template <int RB>
+struct AnyColTile<RB, 4> {
+  IRIS_HD static int lds_offset(int krow, int c) {
+    return krow * RB + ((RB >= 256 ? c ^ (((krow >> 2) & 1) * 8) : c) * kChunkBytes);
+  }
+};
+
+// A workgroup computes BM x BN outputs with WM x WN x WK waves: a wave owns a (BM/WM) x (BN/WN) block, and with
+// WK > 1 every WK-th 128-byte slice of K (the partial blocks meet in LDS at the end).
+template <int IN_, class Out_, int BM_, int BN_, int WM_, int WN_, int WK_, bool BKC_>
+struct AnyCfg {
+  static constexpr int IN = IN_;
+  using Out = Out_;
+  static constexpr int ES = AnyIn<IN>::ES;
+  static constexpr int CE = kChunkBytes / ES;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_;
+  static constexpr bool BKC = BKC_;  // B as [n][k] (K-contiguous, or no unit stride at all), else [k][n]
+  static constexpr int NW = WM * WN * WK, NT = 64 * NW;
+  static constexpr int TM = BM / WM, TN = BN / WN, MB = TM / 32, NB = TN / 32;
+  static constexpr int KB = 128;               // bytes of K per row and slice
+  static constexpr int KE = KB / ES;           // ... in elements
+  static constexpr int KSTEP = KE * WK;        // elements of K per step of the workgroup
+  static constexpr int KM = IN == IN_FP8 ? 64 : IN == IN_F32 ? 8 : 16;  // k per fragment
+  static constexpr int KS = KE / KM;
+  static constexpr int NFRAG = IN == IN_FP8 ? 2 : 1;
+  static constexpr int RBB = BKC ? KB : BN * ES;
+  static constexpr int A_SLICE = BM * KB, B_SLICE = BN * KB;
+  static constexpr int A_BYTES = A_SLICE * WK, B_BYTES = B_SLICE * WK;
+  static constexpr int BUF_BYTES = A_BYTES + B_BYTES;
+  static constexpr int LA = A_BYTES / kChunkBytes / NT, LB = B_BYTES / kChunkBytes / NT;
+  static constexpr int CPR = BN * ES / kChunkBytes;  // pieces per row of a [k][n] tile
+  // Staged output tile: rows padded by 16 bytes against bank conflicts of the accumulator layout.
+  static constexpr int OE = kChunkBytes / Out::size;  // output elements per piece
+  static constexpr int TROW = BN * Out::size + 16;
+  static constexpr int TILE_BYTES = BM * TROW;
+  // Partial blocks of the waves along K: fp32, one 36-float row per output row, next to each other.
+  static constexpr int PART_ROW = BN * 4 + 16;
+  static constexpr int PART_BYTES = WK > 1 ? WK * BM * PART_ROW : 0;
+  static constexpr int SMEM0 = 2 * BUF_BYTES > TILE_BYTES ? 2 * BUF_BYTES : TILE_BYTES;
+  static constexpr int SMEM_BYTES = SMEM0 > TILE_BYTES + PART_BYTES ? SMEM0 : TILE_BYTES + PART_BYTES;
+  static constexpr int WG_PER_CU = NW == 4 ? 2 : 1;
+  static_assert(SMEM_BYTES * WG_PER_CU <= 160 * 1024, "LDS budget of a gfx950 CU");
+  static_assert((BM * 8) % NT == 0 && (BN * 8) % NT == 0 && NT % CPR == 0, "whole pieces per thread");
+};
+
+typedef u32x4_t u32x4_any_t __attribute__((aligned(1)));  // 16 bytes at any address
+#define GLOBAL_AS __attribute__((address_space(1)))
+
+// (Addresses computed from heap bases are integers to the compiler: without the address space it emits flat
+// accesses, which also wait on, and are waited for with, the LDS counter.)
+__device__ __forceinline__ u32x4_t load16_any(const char* p) { return *(const GLOBAL_AS u32x4_any_t*)(GLOBAL_AS const char*)p; }
+__device__ __forceinline__ u32x4_t load16_any_nt(const char* p) {
+  return __builtin_nontemporal_load((const GLOBAL_AS u32x4_any_t*)(GLOBAL_AS const char*)p);
+}
+// Results: past the caches' keep policy when the rows are whole 16-byte pieces, through them otherwise, where the L2 puts
+// the pieces of a line together first (bf16 4096x4095x352 27.3 -> 25.0 us; the aligned 4096x4096x352 23.5 against 24.5).
+__device__ __forceinline__ void store16_result(char* p, u32x4_t v, bool aligned) {
+  if (aligned) __builtin_nontemporal_store(v, (GLOBAL_AS u32x4_t*)(GLOBAL_AS char*)p);
+  else *(GLOBAL_AS u32x4_any_t*)(GLOBAL_AS char*)p = v;
+}
+
+// One 16-byte piece of output elements as floats.
+template <class Out>
+struct OutPiece;
+template <class Out16>
+struct OutPiece16 {
+  static __device__ __forceinline__ void unpack(u32x4_t v, float (&f)[8]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[2 * e] = Out16::to_float((unsigned short)(v[e] & 0xFFFF));
+      f[2 * e + 1] = Out16::to_float((unsigned short)(v[e] >> 16));
+    }
+  }
+  static __device__ __forceinline__ u32x4_t pack(const float (&f)[8]) {
+    return (u32x4_t){Out16::pack(f[0], f[1]), Out16::pack(f[2], f[3]), Out16::pack(f[4], f[5]), Out16::pack(f[6], f[7])};
+  }
+};
+template <> struct OutPiece<ElemBF16> : OutPiece16<OutBF16> {};
+template <> struct OutPiece<ElemF16> : OutPiece16<OutF16> {};
+template <>
+struct OutPiece<ElemF32> {
+  static __device__ __forceinline__ void unpack(u32x4_t v, float (&f)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = __uint_as_float(v[e]);
+  }
+  static __device__ __forceinline__ u32x4_t pack(const float (&f)[4]) {
+    return (u32x4_t){__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
+  }
+};
+
+// Element stores that are written through to memory at system scope (see store16_system).
+template <class Out>
+__device__ __forceinline__ void store_element_system(char* p, const char* from) {
+  if constexpr (Out::size == 2)
+    __hip_atomic_store((unsigned short*)p, *(const LDS_AS unsigned short*)(LDS_AS const char*)from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else
+    __hip_atomic_store((unsigned*)p, *(const LDS_AS unsigned*)(LDS_AS const char*)from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+template <class CFG>
+__global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_any_kernel(const FusedParams p) {
+  using Out = typename CFG::Out;
+  constexpr int IN = CFG::IN, ES = CFG::ES, CE = CFG::CE, BM = CFG::BM, BN = CFG::BN, NT = CFG::NT, KE = CFG::KE, KS = CFG::KS;
+  constexpr int LA = CFG::LA, LB = CFG::LB, MB = CFG::MB, NB = CFG::NB, NFRAG = CFG::NFRAG, OE = CFG::OE;
+  using ATile = RowTile<CFG::KB>;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave / (CFG::WM * CFG::WN), wm = wave / CFG::WN % CFG::WM, wn = wave % CFG::WN;
+
+  const int tidx = xcd_tile_index(blockIdx.x, gridDim.x, 0, p.tiles_m * p.tiles_n, p.num_xcd);
+  if (tidx < 0) return;
+  int tm, tn;
+  grouped_tile(tidx, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  const int nsrc = (p.gather == GATHER_K) ? p.world : 1;
+  const int klocal = (p.gather == GATHER_K) ? p.K_local : p.K;
+  const int nkb = cdiv(klocal, CFG::KSTEP);
+  const int nsteps = nsrc * nkb;
+
+  // ---- loaders: which pieces this thread fetches, from where, and where they live in LDS ---------------
+  // Consecutive threads take consecutive pieces of a row; with a strided operand consecutive rows, so that
+  // a transposed A (rows one element apart) is still read in whole lines.
+  const bool a_vec = p.s_ak == 1;
+  const char* a_ptr[LA];
+  int a_k[LA], a_lds[LA];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const int id = tid + i * NT, sub = id / (BM * 8), in_sub = id - sub * (BM * 8);
+    const int row = a_vec ? in_sub >> 3 : in_sub % BM, c = a_vec ? in_sub & 7 : in_sub / BM;
+    a_k[i] = sub * KE + c * CE;
+    a_lds[i] = sub * CFG::A_SLICE + ATile::lds_offset(row, c);
+    long long gm = min(m0 + row, p.M - 1);
+    int slot = p.gather == GATHER_K ? 0 : p.rank;
+    if (p.gather == GATHER_M) {
+      slot = (int)(gm / p.M_local);
+      gm -= (long long)slot * p.M_local;
+    }
+    const char* base = p.gather == GATHER_NONE ? p.A : slot_ptr(p.heap_bases, p.A, p.rank, slot);
+    a_ptr[i] = base + (gm * p.s_am + (long long)a_k[i] * p.s_ak) * ES;
+  }
+  const bool b_vec = !CFG::BKC || p.s_bk == 1;
+  const char* b_ptr[LB];
+  int b_k[LB], b_lds[LB];
+  int b_cols = CE;  // [k][n] tile: columns of this thread's piece that exist
+#pragma unroll
+  for (int i = 0; i < LB; ++i) {
+    const int id = tid + i * NT;
+    if constexpr (CFG::BKC) {
+      const int sub = id / (BN * 8), in_sub = id - sub * (BN * 8);
+      const int row = b_vec ? in_sub >> 3 : in_sub % BN, c = b_vec ? in_sub & 7 : in_sub / BN;
+      b_k[i] = sub * KE + c * CE;
+      b_lds[i] = CFG::A_BYTES + sub * CFG::B_SLICE + ATile::lds_offset(row, c);
+      b_ptr[i] = p.B + ((long long)min(n0 + row, p.N - 1) * p.s_bn + (long long)b_k[i] * p.s_bk) * ES;
+    } else {
+      const int krow = id / CFG::CPR, c = id % CFG::CPR, sub = krow / KE;
+      b_k[i] = krow;
+      b_lds[i] = CFG::A_BYTES + sub * CFG::B_SLICE + AnyColTile<CFG::RBB, ES>::lds_offset(krow - sub * KE, c);
+      const int gn = n0 + c * CE;
+      b_cols = p.N - gn;
+      b_ptr[i] = p.B + ((long long)krow * p.s_bk + (gn < p.N ? gn : 0)) * ES;  // pieces past N: any columns do
+    }
+  }
+  if (b_cols <= 0 || b_cols > CE) b_cols = CE;
+  // One past the last byte of B ([k][n]); a piece that ends beyond it is loaded element by element.  With rows
+  // at least a piece apart only a piece of the last row can.
+  const char* const b_end = p.B + ((long long)(p.K - 1) * p.s_bk + p.N) * ES;
+  const bool b_edge = !CFG::BKC && (n0 + BN > p.N || p.N < CE);
+  const int b_safe_k = !b_edge ? p.K : p.s_bk >= CE ? p.K - 1 : 0;  // rows below this one can be read in whole pieces
+
+  // Elements [0, count) of a piece, `stride` bytes apart; the rest of it zero.
+  auto load_elements = [&](const char* ptr, long long stride, int count) {
+    u32x4_t v = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int e = 0; e < CE; ++e)
+      if (e < count) {
+        const char* q = ptr + e * stride;
+        unsigned x;
+        if constexpr (ES == 4) x = *(const GLOBAL_AS unsigned*)(GLOBAL_AS const char*)q;
+        else if constexpr (ES == 2) x = *(const GLOBAL_AS unsigned short*)(GLOBAL_AS const char*)q;
+        else x = *(const GLOBAL_AS unsigned char*)(GLOBAL_AS const char*)q;
+        v[e * ES / 4] |= x << (8 * (e * ES % 4));
+      }
+    return v;
+  };
+
+  const long long a_step = (long long)CFG::KSTEP * p.s_ak * ES, b_step = (long long)CFG::KSTEP * p.s_bk * ES;
+  int f_kb = 0, f_src = 0;  // K step the next fetch brings
+  u32x4_t ra[LA], rb[LB];
+  auto fetch = [&]() {
+    const int left = klocal - f_kb * CFG::KSTEP;  // elements of K from this step on
+    if (left >= CFG::KSTEP && a_vec) {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) ra[i] = load16_any(a_ptr[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < LA; ++i)
+        ra[i] = a_vec && a_k[i] + CE <= left ? load16_any(a_ptr[i]) : load_elements(a_ptr[i], p.s_ak * ES, left - a_k[i]);
+    }
+    if (left >= CFG::KSTEP && b_vec && f_src * klocal + (f_kb + 1) * CFG::KSTEP <= b_safe_k) {
+#pragma unroll
+      for (int i = 0; i < LB; ++i) rb[i] = load16_any(b_ptr[i]);
+    } else if constexpr (CFG::BKC) {
+#pragma unroll
+      for (int i = 0; i < LB; ++i)
+        rb[i] = b_vec && b_k[i] + CE <= left ? load16_any(b_ptr[i]) : load_elements(b_ptr[i], p.s_bk * ES, left - b_k[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        if (b_k[i] >= left) rb[i] = (u32x4_t){0u, 0u, 0u, 0u};
+        else if (b_ptr[i] + 16 <= b_end) rb[i] = load16_any(b_ptr[i]);
+        else rb[i] = load_elements(b_ptr[i], ES, min(b_cols, p.N));
+      }
+    }
+    long long da = a_step, db = b_step;
+    if (++f_kb == nkb) {  // on to the next source's columns
+      f_kb = 0;
+      ++f_src;
+      da -= nkb * a_step;
+      db += (long long)klocal * p.s_bk * ES - nkb * b_step;
+      if (f_src < nsrc) da += p.heap_bases[f_src] - p.heap_bases[f_src - 1];
+    }
+#pragma unroll
+    for (int i = 0; i < LA; ++i) a_ptr[i] += da;
+#pragma unroll
+    for (int i = 0; i < LB; ++i) b_ptr[i] += db;
+  };
+  auto put = [&](int buf) {
+    char* const s = smem + buf * CFG::BUF_BYTES;
+#pragma unroll
+    for (int i = 0; i < LA; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + a_lds[i]) = ra[i];
+#pragma unroll
+    for (int i = 0; i < LB; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + b_lds[i]) = rb[i];
+  };
+
+  // ---- fragments ------------------------------------------------------------------------------------------
+  struct Frag {
+    i32x4_t a[MB][NFRAG], b[NB][NFRAG];
+  };
+  auto load_frag = [&](Frag& f, int buf, int kk) {
+    const char* const sa = smem + buf * CFG::BUF_BYTES + wk * CFG::A_SLICE;
+    const char* const sb = smem + buf * CFG::BUF_BYTES + CFG::A_BYTES + wk * CFG::B_SLICE;
+#pragma unroll
+    for (int h = 0; h < NFRAG; ++h) {
+      const int c = IN == IN_FP8 ? frag8_chunk(lane, kk, h) : frag16_chunk(lane, kk);  // float32: 4 k per half-wave
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        f.a[mb][h] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sa + ATile::lds_offset(wm * CFG::TM + frag16_row(lane), c) + mb * 32 * CFG::KB);
+      if constexpr (CFG::BKC) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          f.b[nb][h] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sb + ATile::lds_offset(wn * CFG::TN + frag16_row(lane), c) + nb * 32 * CFG::KB);
+      }
+    }
+    if constexpr (!CFG::BKC) {
+      using BTile = AnyColTile<CFG::RBB, ES>;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const int col = wn * CFG::TN + nb * 32;
+        if constexpr (IN == IN_F32) {
+          const int n = col + (lane & 31), k = kk * 8 + 4 * (lane >> 5);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            f.b[nb][0][e] = *(const LDS_AS int*)(LDS_AS char*)(sb + BTile::lds_offset(k + e, n / CE) + (n % CE) * 4);
+        } else if constexpr (IN == IN_FP8) {
+          const int n = col + tr8_ncol(lane);
+          i32x2_t t[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            t[r] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                (LDS_AS i32x2_t*)(LDS_AS char*)(sb + BTile::lds_offset(tr8_krow(lane, kk, r), n / CE) + n % CE));
+          f.b[nb][0] = (i32x4_t){t[0].x, t[0].y, t[1].x, t[1].y};
+          f.b[nb][NFRAG - 1] = (i32x4_t){t[2].x, t[2].y, t[3].x, t[3].y};
+        } else {
+          const int n = col + tr16_ncol(lane);
+          i32x2_t t[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            t[j] = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (LDS_AS i16x4_t*)(LDS_AS char*)(sb + BTile::lds_offset(tr16_krow(lane, kk, j), n / CE) + (n % CE) * 2)));
+          f.b[nb][0] = (i32x4_t){t[0].x, t[0].y, t[1].x, t[1].y};
+        }
+      }
+    }
+  };
+  f32x16_t acc[MB][NB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+  auto multiply = [&](const Frag& f) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        if constexpr (IN == IN_F32) {
+          // (element by element through a copy: bit_cast of a vector element lvalue reads element 0)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int a = f.a[mb][0][e], b = f.b[nb][0][e];
+            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(__int_as_float(b), __int_as_float(a), acc[mb][nb], 0, 0, 0);
+          }
+        } else {
+          acc[mb][nb] = mfma_block<IN, NFRAG>(f.a[mb], f.b[nb], acc[mb][nb]);
+        }
+      }
+  };
+  // Every wave's LDS accesses done, then everybody's; loads to registers stay in flight.
+  auto lds_barrier = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((0xF) | (0x3 << 14) | (0x7 << 4));  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // ---- K loop ---------------------------------------------------------------------------------------------
+  // Step s reads LDS buffer s & 1; meanwhile step s+1 arrives in registers, is put into the other buffer half
+  // way through the step's products, and the loads of step s+2 go out.
+  fetch();
+  put(0);
+  if (nsteps > 1) fetch();
+  lds_barrier();
+  for (int s = 0; s < nsteps; ++s) {
+    const int buf = s & 1;
+    Frag f[2];
+    load_frag(f[0], buf, 0);
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+      if (kk + 1 < KS) load_frag(f[(kk + 1) & 1], buf, kk + 1);
+      multiply(f[kk & 1]);
+      if (kk == KS / 2 - 1 && s + 1 < nsteps) {
+        put(buf ^ 1);
+        if (s + 2 < nsteps) fetch();
+      }
+    }
+    lds_barrier();
+  }
+
+  // ---- the tile in the output type, in LDS ------------------------------------------------------------------
+  if constexpr (CFG::WK > 1) {
+    // The waves along K leave their partial blocks behind the staged tile; wave 0 of each block adds them.
+    char* const part = smem + CFG::TILE_BYTES + wk * (BM * CFG::PART_ROW);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x4_t v = {__float_as_uint(acc[mb][nb][4 * q]), __float_as_uint(acc[mb][nb][4 * q + 1]),
+                             __float_as_uint(acc[mb][nb][4 * q + 2]), __float_as_uint(acc[mb][nb][4 * q + 3])};
+          *(LDS_AS u32x4_t*)(LDS_AS char*)(part + (wm * CFG::TM + mb * 32 + acc_col(lane)) * CFG::PART_ROW +
+                                           (wn * CFG::TN + nb * 32 + acc_row(lane, 4 * q)) * 4) = v;
+        }
+    lds_barrier();
+  }
+  auto stage4 = [&](int row, int col, const float (&sum)[4], float badd) {
+    char* const dst = smem + row * CFG::TROW + col * Out::size;
+    float h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = sum[e] * p.scale + badd;
+    if constexpr (Out::size == 4) {
+      *(LDS_AS u32x4_t*)(LDS_AS char*)dst = (u32x4_t){__float_as_uint(h[0]), __float_as_uint(h[1]), __float_as_uint(h[2]), __float_as_uint(h[3])};
+    } else {
+      using Out16 = typename std::conditional<Out::kFp32SumInReference, OutF16, OutBF16>::type;
+      *(LDS_AS u32x2_t*)(LDS_AS char*)dst = (u32x2_t){Out16::pack(h[0], h[1]), Out16::pack(h[2], h[3])};
+    }
+  };
+  auto bias_of = [&](int row) -> float {
+    return p.bias && m0 + row < p.M ? load_scalar_as_float(p.bias, (long long)(m0 + row) * p.s_bias, p.bias_dtype) : 0.f;
+  };
+  if constexpr (CFG::WK > 1) {
+    for (int q = tid; q < BM * BN / 4; q += NT) {
+      const int row = q / (BN / 4), col = q % (BN / 4) * 4;
+      float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < CFG::WK; ++w) {
+        const u32x4_t v = *(const LDS_AS u32x4_t*)(LDS_AS char*)(smem + CFG::TILE_BYTES + (w * BM + row) * CFG::PART_ROW + col * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += __uint_as_float(v[e]);
+      }
+      stage4(row, col, sum, bias_of(row));
+    }
+  } else {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int row = wm * CFG::TM + mb * 32 + acc_col(lane);
+      const float badd = bias_of(row);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float sum[4] = {acc[mb][nb][4 * q], acc[mb][nb][4 * q + 1], acc[mb][nb][4 * q + 2], acc[mb][nb][4 * q + 3]};
+          stage4(row, wn * CFG::TN + nb * 32 + acc_row(lane, 4 * q), sum, badd);
+        }
+    }
+  }
+  lds_barrier();
+
+  // ---- epilogue: pieces of OE consecutive columns, handed out row by row ---------------------------------------
+  constexpr int PPR = BN / OE;             // pieces per tile row
+  constexpr int RPP = NT / PPR;            // tile rows per pass of the workgroup
+  constexpr int PASSES = BM > RPP ? BM / RPP : 1;
+  static_assert(NT % PPR == 0 && (BM % RPP == 0 || BM < RPP), "epilogue pass shape");
+  const int m_end = min(m0 + BM, p.M);  // one past the tile's last row (threads may have no row in a 32x32 tile)
+  // A piece that would reach past the last column starts further left (both its threads then write the same
+  // values twice), as long as the tile has that many columns.
+  const int t_row = tid / PPR, tile_cols = min(BN, p.N - n0);
+  int t_col = tid % PPR * OE;
+  if (t_col < tile_cols && t_col + OE > tile_cols && tile_cols >= OE) t_col = tile_cols - OE;
+  const int gn = n0 + t_col;
+  const int cols = min(p.N - gn, OE);           // columns of this thread's pieces that exist (may be <= 0)
+  const bool whole = cols == OE && p.s_cn == 1;  // moved as 16 bytes, else element by element
+  const int ftn = cdiv(p.N, p.flag_bn);
+  const int ftotal = cdiv(p.M, p.flag_bm) * ftn;
+  auto staged = [&](int row) { return smem + row * CFG::TROW + t_col * Out::size; };
+  auto staged_piece = [&](int row) { return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)staged(row); };
+  auto staged_element = [&](int row, int e) -> float {
+    if constexpr (Out::size == 4) {
+      return *(const LDS_AS float*)(LDS_AS char*)(staged(row) + e * 4);
+    } else {
+      const unsigned short b = *(const LDS_AS unsigned short*)(LDS_AS char*)(staged(row) + e * 2);
+      return Out::kFp32SumInReference ? f16_bits_to_float(b) : bf16_bits_to_float(b);
+    }
+  };
+  auto offset = [&](int row, int e) {  // bytes into C (or aux) of element e of this thread's piece
+    return ((long long)(m0 + row + p.row_offset) * p.s_cm + (long long)(gn + e) * p.s_cn) * Out::size;
+  };
+  auto owner_at = [&](int gm, int g) { return owner_of(p.epi, (gm / p.flag_bm) * ftn + g / p.flag_bn, ftotal, p.world, p.rank); };
+
+  if (p.epi == EPI_ATOMIC) {
+    if constexpr (Out::size == 4) {
+      for (int d = tid; d < BM * BN; d += NT) {
+        const int row = d / BN, col = d % BN;
+        if (m0 + row >= p.M || n0 + col >= p.N) continue;
+        const float v = *(const LDS_AS float*)(LDS_AS char*)(smem + row * CFG::TROW + col * 4);
+        const long long eoff = ((long long)(m0 + row) * p.s_cm + (long long)(n0 + col) * p.s_cn) * 4;
+        for (int pr = 0; pr < p.world; ++pr) atomicAdd((float*)(slot_ptr(p.heap_bases, p.C, p.rank, pr) + eoff), v);
+      }
+    } else if (p.s_cn == 1) {
+      // Packed adds of aligned dwords, one per thread.  A row that starts in the middle of a dword is shifted by
+      // one element against them; the half of a dword that is not this tile's gets -0 added, which leaves
+      // every value as it is.
+      using Out16 = typename std::conditional<Out::kFp32SumInReference, OutF16, OutBF16>::type;
+      constexpr int DPR = BN / 2 + 1;
+      for (int d = tid; d < BM * DPR; d += NT) {
+        const int row = d / DPR;
+        if (m0 + row >= p.M) continue;
+        char* const at = p.C + ((long long)(m0 + row) * p.s_cm + n0) * 2;
+        const int e = 2 * (d - row * DPR) - (int)(((unsigned long long)at >> 1) & 1);
+        const bool lo = e >= 0 && e < BN && n0 + e < p.N, hi = e + 1 < BN && n0 + e + 1 < p.N;
+        if (!lo && !hi) continue;
+        const char* const s = smem + row * CFG::TROW;
+        const unsigned w = (lo ? *(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2) : 0x8000u) |
+                           (hi ? (unsigned)*(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2 + 2) : 0x8000u) << 16;
+        for (int pr = 0; pr < p.world; ++pr) atomic_add_packed<Out16>(slot_ptr(p.heap_bases, at, p.rank, pr) + e * 2, w);
+      }
+    } else {
+      for (int ps = 0; ps < PASSES; ++ps) {
+        const int row = ps * RPP + t_row;
+        if (m0 + row >= m_end) continue;
+        for (int e = 0; e < cols; ++e)
+          for (int pr = 0; pr < p.world; ++pr)
+            Out::atomic_add(slot_ptr(p.heap_bases, p.C, p.rank, pr) + offset(row, e), staged_element(row, e));
+      }
+    }
+    return;
+  }
+
+  const bool flags = epi_has_flags(p.epi);
+  const bool solo = flags && (!p.sum_peers || p.world == 1);  // no peer contributes: the sum is the own tile
+  // Stores of a result piece (or its elements) to wherever the operator wants it.
+  auto each_destination = [&](int gm, int g, auto&& store) {
+    if (p.epi == EPI_STORE) {
+      store(p.C);
+    } else if (p.epi == EPI_ALL_GATHER) {
+      for (int pr = 0; pr < p.world; ++pr) store(slot_ptr(p.heap_bases, p.C, p.rank, pr));
+    } else if (p.epi == EPI_ONE_SHOT) {
+      store(p.C);
+    } else {
+      const int owner = owner_at(gm, g);
+      if (!p.all_owners && owner != p.rank) return;
+      if (p.epi == EPI_TWO_SHOT) {
+        for (int pr = 0; pr < p.world; ++pr) store(slot_ptr(p.heap_bases, p.C, p.rank, pr));
+      } else {
+        store(slot_ptr(p.heap_bases, p.C, p.rank, p.all_owners ? owner : p.rank));
+      }
+    }
+  };
+  const bool aligned = (((unsigned long long)p.C | (unsigned long long)(p.s_cm * Out::size)) & 15) == 0 && p.N % OE == 0;
+  const bool owners = flags && p.epi != EPI_ONE_SHOT;
+  // A piece may be moved whole when all of it has one owner.
+  const bool piece_ok = whole && (!owners || gn / p.flag_bn == (gn + OE - 1) / p.flag_bn);
+
+#pragma unroll 2
+  for (int ps = 0; ps < PASSES; ++ps) {
+    const int row = ps * RPP + t_row, gm = m0 + row;
+    if (gm >= m_end) break;
+    if (flags) {
+      if (whole) {
+        store16_system_of_valu_data(p.aux + offset(row, 0), staged_piece(row));
+      } else {
+        for (int e = 0; e < cols; ++e) store_element_system<Out>(p.aux + offset(row, e), staged(row) + e * Out::size);
+      }
+      if (!solo) continue;
+    }
+    if (piece_ok) {
+      const u32x4_t v = staged_piece(row);
+      each_destination(gm, gn, [&](char* base) { store16_result(base + offset(row, 0), v, aligned); });
+    } else {
+      for (int e = 0; e < cols; ++e)
+        each_destination(gm, gn + e, [&](char* base) { Out::store(base + offset(row, e), staged_element(row, e)); });
+    }
+  }
+  if (!flags) return;
+
+  // Publish and wait, as in the tiled kernel: aux is written through, so relaxed flag stores behind the
+  // acknowledgement are enough.
+  const bool up_already = solo ? true : probe_peer_flags<BM, BN, NT>(p, m0, n0, tid);
+  wait_vmcnt<0>();
+  __syncthreads();
+  raise_flags<BM, BN, NT, true>(p, m0, n0, tid);
+  if (solo) return;
+  if (!up_already) wait_peer_flags<BM, BN, NT>(p, m0, n0, tid);
+  __syncthreads();
+
+  // Slot sum in ascending rank order from the own (already rounded) value, in fp32 or by the reference's rule.
+  const bool ref_chain = (p.acc_mode == IRIS_HIP_ACC_REFERENCE) && !Out::kFp32SumInReference;
+  auto add = [&](float sum, float x) {
+    sum += x;
+    return ref_chain ? Out::round(sum) : sum;
+  };
+  auto reduce = [&](auto np_tag) {
+    constexpr int NP = decltype(np_tag)::value;  // peers, all of whose loads go out together; 0: any number
+    constexpr int NPV = NP > 0 ? NP : 1;
+    constexpr int G = PASSES % 2 == 0 ? 2 : 1;  // passes whose loads are in flight together
+    for (int pg = 0; pg < PASSES; pg += G) {
+      if (m0 + pg * RPP >= p.M) break;
+      bool act[G];
+      u32x4_t pv[G][NPV];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const int row = (pg + g) * RPP + t_row;
+        act[g] = m0 + row < m_end && cols > 0;
+        if (act[g] && owners && !p.all_owners && piece_ok) act[g] = owner_at(m0 + row, gn) == p.rank;
+        if constexpr (NP > 0) {
+          if (act[g] && piece_ok) {
+#pragma unroll
+            for (int i = 0; i < NP; ++i) pv[g][i] = load16_any_nt(slot_ptr(p.heap_bases, p.aux, p.rank, i < p.rank ? i : i + 1) + offset(row, 0));
+          }
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const int row = (pg + g) * RPP + t_row, gm = m0 + row;
+        if (!act[g]) continue;
+        if (piece_ok) {
+          float sum[OE], x[OE];
+          OutPiece<Out>::unpack(staged_piece(row), sum);
+          if constexpr (NP > 0) {
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+              OutPiece<Out>::unpack(pv[g][i], x);
+#pragma unroll
+              for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
+            }
+          } else {
+            for (int pr = 0; pr < p.world; ++pr) {
+              if (pr == p.rank) continue;
+              OutPiece<Out>::unpack(load16_any_nt(slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row, 0)), x);
+#pragma unroll
+              for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
+            }
+          }
+          const u32x4_t v = OutPiece<Out>::pack(sum);
+          each_destination(gm, gn, [&](char* base) { store16_result(base + offset(row, 0), v, aligned); });
+        } else {
+          // Fewer columns than a piece, strided columns or several owners: all elements of a peer in one go.
+          float sum[OE];
+#pragma unroll
+          for (int e = 0; e < OE; ++e) sum[e] = e < cols ? staged_element(row, e) : 0.f;
+          for (int pr = 0; pr < p.world; ++pr) {
+            if (pr == p.rank) continue;
+            const char* const src = slot_ptr(p.heap_bases, p.aux, p.rank, pr);
+            float x[OE];
+#pragma unroll
+            for (int e = 0; e < OE; ++e) x[e] = e < cols ? Out::load(src + offset(row, e)) : 0.f;
+#pragma unroll
+            for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
+          }
+#pragma unroll
+          for (int e = 0; e < OE; ++e)
+            if (e < cols) each_destination(gm, gn + e, [&](char* base) { Out::store(base + offset(row, e), sum[e]); });
+        }
+      }
+    }
+  };
+  switch (p.world - 1) {
+    case 1: reduce(std::integral_constant<int, 1>{}); break;
+    case 3: reduce(std::integral_constant<int, 3>{}); break;
+    case 7: reduce(std::integral_constant<int, 7>{}); break;
+    default: reduce(std::integral_constant<int, 0>{}); break;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Launch
+// ------------------------------------------------------------------------------------------------
+template <class CFG>
+int launch_any(FusedParams p, int device, int cu_count, hipStream_t stream, const char* types) {
+  static std::atomic<bool> attr_set[64];  // see launch_mfma_grid
+  if (device < 0 || device >= 64) return iris_host::fail("device index %d out of range", device);
+  if (!attr_set[device].load(std::memory_order_acquire)) {
+    hipError_t e = hipFuncSetAttribute((const void*)fused_any_kernel<CFG>, hipFuncAttributeMaxDynamicSharedMemorySize, CFG::SMEM_BYTES);
+    if (e != hipSuccess) return (int)e;
+    attr_set[device].store(true, std::memory_order_release);
+  }
+  p.tiles_m = cdiv(p.M, CFG::BM);
+  p.tiles_n = cdiv(p.N, CFG::BN);
+  const long long total = (long long)p.tiles_m * p.tiles_n;
+  if (total > (1ll << 30)) return iris_host::fail("output of %d x %d has too many tiles", p.M, p.N);
+  // Close to square groups of the tiles an XCD works on at one time, as in dispatch_mfma_in.
+  const int resident = cu_count / p.num_xcd * CFG::WG_PER_CU, span = cdiv((int)total, p.num_xcd);
+  const int at_once = span < resident ? span : resident;
+  int g = 1;
+  while (g * g * 2 <= at_once && g * 2 <= p.tiles_m) g *= 2;
+  p.group_m = g;
+  const int grid = cdiv((int)total, p.num_xcd) * p.num_xcd;
+  char name[96];
+  snprintf(name, sizeof(name), "generic_%s_%dx%d_%s", types, CFG::BM, CFG::BN, CFG::BKC ? "nt" : "nn");
+  iris_host::set_last_kernel(name);
+  hipLaunchKernelGGL((fused_any_kernel<CFG>), dim3(grid), dim3(CFG::NT), CFG::SMEM_BYTES, stream, p);
+  return (int)hipGetLastError();
+}
+
+// Tile choice: the tile with the least expected time, area x (tiles the busiest CU gets) / rate.  The rates (TFLOP/s, plain
+// GEMM 4095x4095x4095 bf16 and 4096x4096x4096 float32, every CU busy) fall with the tile because LDS reads and
+// operand bytes per flop rise; for float32 they hardly do, the matrix pipes are the bound.  A CU with a single
+// workgroup of four waves has nothing to run while it waits (bf16 1024x4095x2049 on 256 tiles of 128x128: 40 us, where
+// the full rate would give 26).  Checked against forced tiles, us for 256x256 / 128x128 / 64x128 / 64x64 / 32x32, the
+// choice first: bf16 1999x2877x1371 64x128 41 (53 / 40 / - / 51 / 119), 1024x4095x2049 64x128 38 (68 / 40 / - / 48 / 105),
+// one-shot with seven peers 500x2877x1371 64x64 30 (92 / 46 / 32 / - / 51), 33x2877x1371 32x32 13 (49 / 31 / 25 / 20 / -); float32
+// 2048x2880x1024 64x128 106 (- / 133 / - / 109 / 159), 511x2880x1024 32x32 43 (- / 77 / 45 / 40 / -).
+struct AnyTile {
+  int bm, bn;
+  float rate16, rate32;
+};
+constexpr AnyTile kAnyTiles[] = {{256, 256, 855.f, 0.f}, {128, 128, 654.f, 137.f}, {64, 128, 508.f, 131.f}, {64, 64, 395.f, 127.f}, {32, 32, 195.f, 98.f}};
+
+inline int choose_any_tile(int M, int N, int cu, bool f32_in, bool f32_out) {
+  int best = 1;
+  float best_time = 0.f;
+  for (int i = f32_in || f32_out ? 1 : 0; i < 5; ++i) {
+    const AnyTile& t = kAnyTiles[i];
+    const long long per_cu = ((long long)cdiv(M, t.bm) * cdiv(N, t.bn) + cu - 1) / cu;
+    const float alone = i == 0 || per_cu > 1 ? 1.f : f32_in ? 1.15f : 1.5f;
+    const float time = (float)t.bm * t.bn * per_cu * alone / (f32_in ? t.rate32 : t.rate16);
+    if (best_time == 0.f || time < best_time) {
+      best = i;
+      best_time = time;
+    }
+  }
+  return best;
+}
+
+template <int IN, class Out, bool BKC>
+int dispatch_any_layout(const FusedParams& p, int device, int cu, hipStream_t s, const char* types) {
+  constexpr bool F32_IN = AnyIn<IN>::ES == 4, F32_OUT = Out::size == 4;
+  switch (choose_any_tile(p.M, p.N, cu, F32_IN, F32_OUT)) {
+    case 0:  // (a staged 256x256 tile of float32 would not fit the LDS)
+      if constexpr (!F32_OUT) return launch_any<AnyCfg<IN, Out, 256, 256, 2, 4, 1, BKC>>(p, device, cu, s, types);
+      break;
+    case 2: return launch_any<AnyCfg<IN, Out, 64, 128, 2, 2, 1, BKC>>(p, device, cu, s, types);
+    case 3: return launch_any<AnyCfg<IN, Out, 64, 64, 2, 2, 1, BKC>>(p, device, cu, s, types);
+    case 4: return launch_any<AnyCfg<IN, Out, 32, 32, 1, 1, 4, BKC>>(p, device, cu, s, types);
+  }
+  return launch_any<AnyCfg<IN, Out, 128, 128, 2, 2, 1, BKC>>(p, device, cu, s, types);
+}
+
+// The layout of B in LDS follows its unit stride: [k][n] when N is contiguous, else [n][k].
+template <int IN, class Out>
+int dispatch_any(const FusedParams& p, int device, int cu, hipStream_t s, const char* types) {
+  return p.s_bn == 1 ? dispatch_any_layout<IN, Out, false>(p, device, cu, s, types)
+                     : dispatch_any_layout<IN, Out, true>(p, device, cu, s, types);
+}

@@ -115,10 +115,3 @@ struct ElemF32 {
   static __device__ __forceinline__ void atomic_add(char* p, float f) { atomicAdd((float*)p, f); }
   static constexpr bool kFp32SumInReference = false;  // fp32 data sums in fp32 either way
 };
-struct ElemFP8 {
-  static constexpr int size = 1;
-  static __device__ __forceinline__ float load(const char* p) {
-    return __builtin_amdgcn_cvt_f32_fp8((int)*(const unsigned char*)p, 0);
-  }
-};
-

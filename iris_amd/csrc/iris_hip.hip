@@ -2,7 +2,7 @@
 // operators, and the C ABI declared in include/iris_hip.h.
 //
 // Two kernels implement every operator (the first lives in fused_kernel.h and is compiled in the
-// iris_hip_mfma_<type>.hip translation units, the second and the entry points are in this file):
+// iris_hip_mfma_<type>.hip translation units; the entry points are in this file):
 //
 //  * fused_mfma_kernel  - persistent tiled GEMM on the 32x32 MFMA blocks of CDNA4.  Operand tiles
 //    travel HBM -> LDS with 16-byte direct-to-LDS buffer loads into a ring of STAGES buffers
@@ -11,16 +11,17 @@
 //    a workgroup (8 as 2x4 for the 256x256 tile, 4 as 2x2 for the smaller ones) each own a block of
 //    fp32 accumulators that stays in the accumulation registers.  Requires 16-byte aligned,
 //    unit-stride rows (see mfma_ineligible()).
-//  * fused_generic_kernel - a plain 64x64 LDS-tiled kernel on fp32 MFMA for everything else (fp32 data,
-//    odd strides, sizes that are not multiples of 8 elements).
+//  * fused_any_kernel (any_kernel.h, compiled in the iris_hip_any_<type>.hip translation units) - any alignment,
+//    stride, size and element type, operands through registers: everything the first does not take (fp32
+//    data, odd strides, sizes that are not multiples of 8 elements).
 //
 // The flag-less operators (all_gather_matmul, matmul_all_gather, the atomic all-reduce) store or add
 // the tile directly.  The others end in the same epilogue protocol, which follows the reference kernels
 // (iris/ops/matmul_all_reduce.py:111-144, iris/ops/matmul_reduce_scatter.py:98-118,
 //  iris/mem/triton/context.py:733-764, 801-839, 953-997):
 //    1. cast the fp32 tile to the output type and store it to aux in the own slot,
-//    2. make those stores visible, then raise the flag of every finished flag tile (the MFMA
-//       kernel writes aux through to memory and raises relaxed; the generic kernel raises with release),
+//    2. make those stores visible (aux is written through to memory), then raise the flag of every finished
+//       flag tile,
 //    3. for the flag tiles this rank reduces: wait for the peers' flags, add the peers' aux tiles
 //       in ascending rank order, cast once, store to C (own slot; two-shot: every slot).
 
@@ -35,168 +36,8 @@
 #include <type_traits>
 #include <vector>
 
+#include "any_kernel.h"
 #include "fused_kernel.h"
-
-// ------------------------------------------------------------------------------------------------
-// Generic kernel: 64x64 tile, 256 threads, 4x4 outputs per thread, fp32 FMA.
-// ------------------------------------------------------------------------------------------------
-constexpr int GT = 64;   // generic tile edge
-constexpr int GK = 16;   // generic k step
-
-template <class In, class Out>
-__global__ void __launch_bounds__(256) fused_generic_kernel(const FusedParams p) {
-  __shared__ float As[GK][GT + 1];
-  __shared__ float Bs[GK][GT + 1];
-  __shared__ float Cs[GT][GT + 1];
-  const int tid = threadIdx.x;
-  const int tx = tid % 16, ty = tid / 16;
-  // Each of the four waves multiplies one 32x32 quadrant of the tile with fp32 MFMA
-  // (v_mfma_f32_32x32x2_f32: lane l supplies A[l % 32][l / 32] and B[l / 32][l % 32] of a 32x2 by 2x32
-  // product); inputs of every type are widened to fp32 in LDS first, so products are exact for 16-bit
-  // and fp8 data and accumulation is fp32 throughout.
-  const int lane = tid & 63, wave = tid >> 6;
-  const int qm = (wave >> 1) * 32, qn = (wave & 1) * 32;
-  const int total_tiles = p.tiles_m * p.tiles_n;
-  const int ftn = cdiv(p.N, p.flag_bn);
-  const int ftotal = cdiv(p.M, p.flag_bm) * ftn;
-  const int nsrc = (p.gather == GATHER_K) ? p.world : 1;
-  const int klocal = (p.gather == GATHER_K) ? p.K_local : p.K;
-
-  for (int tile = blockIdx.x; tile < total_tiles; tile += gridDim.x) {
-    const int tm = tile / p.tiles_n, tn = tile % p.tiles_n;
-    const int m0 = tm * GT, n0 = tn * GT;
-    f32x16_t quad;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) quad[r] = 0.f;
-
-    // One K step = GK columns of A and rows of B.  The operands of step t+1 are fetched into
-    // registers while the MFMAs of step t run, and stored to LDS after them.
-    const int ksteps = cdiv(klocal, GK);
-    const int nsteps = nsrc * ksteps;
-    auto fetch = [&](int step, float (&va)[4], float (&vb)[4]) {
-      const int src = step / ksteps, k0 = (step - src * ksteps) * GK;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {  // A tile: GT rows x GK k
-        const int idx = tid + e * 256;
-        const int r = idx / GK, kk = idx % GK;
-        const int gm = m0 + r, kl = k0 + kk;
-        va[e] = 0.f;
-        if (gm < p.M && kl < klocal) {
-          int slot = p.rank;
-          long long row = gm;
-          if (p.gather == GATHER_K) slot = src;
-          if (p.gather == GATHER_M) { slot = gm / p.M_local; row = gm - (long long)slot * p.M_local; }
-          const char* base = p.gather == GATHER_NONE ? p.A : slot_ptr(p.heap_bases, p.A, p.rank, slot);
-          va[e] = In::load(base + (row * p.s_am + (long long)kl * p.s_ak) * In::size);
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {  // B tile: GK k x GT columns
-        const int idx = tid + e * 256;
-        const int kk = idx / GT, c = idx % GT;
-        const int gn = n0 + c, kl = k0 + kk;
-        vb[e] = 0.f;
-        if (gn < p.N && kl < klocal) {
-          const long long kg = (long long)src * klocal + kl;
-          vb[e] = In::load(p.B + (kg * p.s_bk + (long long)gn * p.s_bn) * In::size);
-        }
-      }
-    };
-    float va[4], vb[4];
-    fetch(0, va, vb);
-    for (int step = 0; step < nsteps; ++step) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int idx = tid + e * 256;
-        As[idx % GK][idx / GK] = va[e];
-        Bs[idx / GT][idx % GT] = vb[e];
-      }
-      __syncthreads();
-      if (step + 1 < nsteps) fetch(step + 1, va, vb);
-#pragma unroll
-      for (int kk = 0; kk < GK; kk += 2) {
-        const float a = As[kk + (lane >> 5)][qm + (lane & 31)];
-        const float b = Bs[kk + (lane >> 5)][qn + (lane & 31)];
-        quad = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, quad, 0, 0, 0);
-      }
-      __syncthreads();
-    }
-    // Accumulator register r of lane l is element (8*(r/4) + 4*(l/32) + r%4, l%32) of the quadrant;
-    // the tile goes through LDS so that the epilogue below can work on 4x4 blocks per thread.
-#pragma unroll
-    for (int r = 0; r < 16; ++r) Cs[qm + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4)][qn + (lane & 31)] = quad[r];
-    __syncthreads();
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = Cs[ty * 4 + i][tx * 4 + j];
-
-    // Own tile, rounded to the output type.
-    float own[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int gm = m0 + ty * 4 + i;
-      float badd = 0.f;
-      if (p.bias && gm < p.M) badd = load_scalar_as_float(p.bias, (long long)gm * p.s_bias, p.bias_dtype);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) own[i][j] = Out::round(acc[i][j] * p.scale + badd);
-    }
-    const bool flags = epi_has_flags(p.epi);
-    char* const out1 = flags ? p.aux : p.C;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int gm = m0 + ty * 4 + i, gn = n0 + tx * 4 + j;
-        if (!(gm < p.M && gn < p.N)) continue;
-        const long long eoff = ((long long)(gm + p.row_offset) * p.s_cm + (long long)gn * p.s_cn) * Out::size;
-        if (p.epi == EPI_ALL_GATHER) {
-          for (int pr = 0; pr < p.world; ++pr) Out::store(slot_ptr(p.heap_bases, p.C, p.rank, pr) + eoff, own[i][j]);
-        } else if (p.epi == EPI_ATOMIC) {
-          for (int pr = 0; pr < p.world; ++pr) Out::atomic_add(slot_ptr(p.heap_bases, p.C, p.rank, pr) + eoff, own[i][j]);
-        } else {
-          Out::store(out1 + eoff, own[i][j]);
-        }
-      }
-    if (!flags) continue;
-
-    __atomic_thread_fence(__ATOMIC_RELEASE);
-    __syncthreads();
-    raise_flags<GT, GT, 256, false>(p, m0, n0, tid);
-    if (p.sum_peers && p.world > 1) {
-      wait_peer_flags<GT, GT, 256>(p, m0, n0, tid);
-      __syncthreads();
-    }
-    const bool ref_chain = (p.acc_mode == IRIS_HIP_ACC_REFERENCE) && !Out::kFp32SumInReference;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int gm = m0 + ty * 4 + i, gn = n0 + tx * 4 + j;
-        if (!(gm < p.M && gn < p.N)) continue;
-        const int t = (gm / p.flag_bm) * ftn + gn / p.flag_bn;
-        const int owner = owner_of(p.epi, t, ftotal, p.world, p.rank);
-        if (!p.all_owners && owner != p.rank) continue;
-        const long long eoff = ((long long)gm * p.s_cm + (long long)gn * p.s_cn) * Out::size;
-        float sum = own[i][j];
-        if (p.sum_peers)
-          for (int pr = 0; pr < p.world; ++pr) {
-            if (pr == p.rank) continue;
-            sum += Out::load(slot_ptr(p.heap_bases, p.aux, p.rank, pr) + eoff);
-            if (ref_chain) sum = Out::round(sum);
-          }
-        if (p.epi == EPI_TWO_SHOT) {
-          Out::store(p.C + eoff, sum);
-          for (int pr = 0; pr < p.world; ++pr)
-            if (pr != p.rank) Out::store(slot_ptr(p.heap_bases, p.C, p.rank, pr) + eoff, sum);
-        } else {
-          const int dst = p.all_owners ? owner : p.rank;
-          Out::store(slot_ptr(p.heap_bases, p.C, p.rank, dst) + eoff, sum);
-        }
-      }
-  }
-}
 
 // ------------------------------------------------------------------------------------------------
 // Host side
@@ -284,19 +125,7 @@ const char* mfma_ineligible(const FusedParams& p, int in_dtype, int out_dtype, i
   return nullptr;
 }
 
-template <class In, class Out>
-int launch_generic(FusedParams p, int cu_count, hipStream_t stream, const char* name) {
-  p.tiles_m = cdiv(p.M, GT);
-  p.tiles_n = cdiv(p.N, GT);
-  const long long total = (long long)p.tiles_m * p.tiles_n;
-  const long long cap = (long long)cu_count * 8;
-  const int grid = (int)(total < cap ? total : cap);
-  hipLaunchKernelGGL((fused_generic_kernel<In, Out>), dim3(grid < 1 ? 1 : grid), dim3(256), 0, stream, p);
-  snprintf(g_last_kernel, sizeof(g_last_kernel), "%s", name);
-  return (int)hipGetLastError();
-}
-
-// Type pairs the generic kernel is built for (the list of dispatch_generic below).
+// Type pairs the any-shape kernel is built for (the list of dispatch_generic below).
 bool generic_supported(int in_dtype, int out_dtype) {
   switch (in_dtype) {
     case IRIS_HIP_BF16: return out_dtype == IRIS_HIP_BF16 || out_dtype == IRIS_HIP_FP32;
@@ -307,27 +136,36 @@ bool generic_supported(int in_dtype, int out_dtype) {
   return false;
 }
 
-int dispatch_generic(const FusedParams& p, int in_dtype, int out_dtype, int cu, hipStream_t s) {
-#define GEN(I, O, name) return launch_generic<I, O>(p, cu, s, name)
-  if (in_dtype == IRIS_HIP_BF16 && out_dtype == IRIS_HIP_BF16) GEN(ElemBF16, ElemBF16, "generic_bf16");
-  if (in_dtype == IRIS_HIP_FP16 && out_dtype == IRIS_HIP_FP16) GEN(ElemF16, ElemF16, "generic_f16");
-  if (in_dtype == IRIS_HIP_FP32 && out_dtype == IRIS_HIP_FP32) GEN(ElemF32, ElemF32, "generic_f32");
-  if (in_dtype == IRIS_HIP_FP8_E4M3 && out_dtype == IRIS_HIP_BF16) GEN(ElemFP8, ElemBF16, "generic_fp8_bf16");
-  if (in_dtype == IRIS_HIP_FP8_E4M3 && out_dtype == IRIS_HIP_FP16) GEN(ElemFP8, ElemF16, "generic_fp8_f16");
-  if (in_dtype == IRIS_HIP_BF16 && out_dtype == IRIS_HIP_FP32) GEN(ElemBF16, ElemF32, "generic_bf16_f32");
-  if (in_dtype == IRIS_HIP_FP16 && out_dtype == IRIS_HIP_FP32) GEN(ElemF16, ElemF32, "generic_f16_f32");
-#undef GEN
-  return fail("unsupported element types in=%d out=%d", in_dtype, out_dtype);
-}
-
 }  // namespace
 
 // Instantiated in iris_hip_mfma_bf16.hip, iris_hip_mfma_f16.hip and iris_hip_mfma_fp8.hip.
 extern template int dispatch_mfma_in<IN_BF16>(FusedParams&, int, bool, int, int, hipStream_t);
 extern template int dispatch_mfma_in<IN_F16>(FusedParams&, int, bool, int, int, hipStream_t);
 extern template int dispatch_mfma_in<IN_FP8>(FusedParams&, int, bool, int, int, hipStream_t);
+// Instantiated in iris_hip_any_<type>.hip.
+extern template int dispatch_any<IN_BF16, ElemBF16>(const FusedParams&, int, int, hipStream_t, const char*);
+extern template int dispatch_any<IN_BF16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
+extern template int dispatch_any<IN_F16, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*);
+extern template int dispatch_any<IN_F16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
+extern template int dispatch_any<IN_F32, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
+extern template int dispatch_any<IN_FP8, ElemBF16>(const FusedParams&, int, int, hipStream_t, const char*);
+extern template int dispatch_any<IN_FP8, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*);
 
 namespace {
+
+int dispatch_generic(const FusedParams& p, int in_dtype, int out_dtype, int device, int cu, hipStream_t s) {
+  const bool out_f32 = out_dtype == IRIS_HIP_FP32;
+  switch (in_dtype) {
+    case IRIS_HIP_BF16:
+      return out_f32 ? dispatch_any<IN_BF16, ElemF32>(p, device, cu, s, "bf16_f32") : dispatch_any<IN_BF16, ElemBF16>(p, device, cu, s, "bf16");
+    case IRIS_HIP_FP16:
+      return out_f32 ? dispatch_any<IN_F16, ElemF32>(p, device, cu, s, "f16_f32") : dispatch_any<IN_F16, ElemF16>(p, device, cu, s, "f16");
+    case IRIS_HIP_FP32: return dispatch_any<IN_F32, ElemF32>(p, device, cu, s, "f32");
+    default:
+      return out_dtype == IRIS_HIP_BF16 ? dispatch_any<IN_FP8, ElemBF16>(p, device, cu, s, "fp8_bf16")
+                                        : dispatch_any<IN_FP8, ElemF16>(p, device, cu, s, "fp8_f16");
+  }
+}
 
 // ------------------------------------------------------------------------------------------------
 // Library-owned workspace of iris_hip_matmul_all_reduce_noalloc
@@ -490,7 +328,7 @@ int run_fused(FusedParams p, int in_dtype, int out_dtype, int path, void* stream
   if (path == IRIS_HIP_PATH_MFMA && why) return fail("MFMA kernel not applicable: %s", why);
   if (path == IRIS_HIP_PATH_GENERIC || why) {
     if (!generic_supported(in_dtype, out_dtype)) return fail("unsupported element types in=%d out=%d", in_dtype, out_dtype);
-    return check_only ? 0 : dispatch_generic(p, in_dtype, out_dtype, facts->cu_count, s);
+    return check_only ? 0 : dispatch_generic(p, in_dtype, out_dtype, device, facts->cu_count, s);
   }
   if (check_only) return 0;
 
