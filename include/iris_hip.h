@@ -60,6 +60,11 @@ enum {
   IRIS_HIP_ACC_REFERENCE = 1 /* the reference rule: fp32 only for fp16 data, else the data type
                                 (bf16 sums are re-rounded after every add; context.py:752) */
 };
+/* May be added (|) to acc_mode: the launch leaves the own slot's C as if it had been zeroed first.  Tiles that
+ * another rank owns (two_shot, reduce-scatter) are stored as zeros, and the atomic variant stores its product to
+ * the own slot instead of adding it to what is there.  Only for launches that no other rank's launch runs
+ * beside: a peer's result could already be in C. */
+enum { IRIS_HIP_CLEAR_C = 0x100 };
 
 /* Which A rows/columns come from which slot in iris_hip_all_gather_matmul (gather_dim). */
 enum {

@@ -17,6 +17,7 @@ ABI_VERSION = 5
 BF16, FP16, FP32, FP8_E4M3 = 0, 1, 2, 3
 VARIANT_ATOMIC, VARIANT_ONE_SHOT, VARIANT_TWO_SHOT = 0, 2, 3
 ACC_FP32, ACC_REFERENCE = 0, 1
+CLEAR_C = 0x100  # added to the acc_mode argument
 GATHER_K, GATHER_M = 1, 2
 PATH_AUTO, PATH_MFMA, PATH_GENERIC = 0, 1, 2
 STATUS_SPIN_TIMEOUT = 1

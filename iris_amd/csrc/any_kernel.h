@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   // values twice), as long as the tile has that many columns.
   const int t_row = tid / PPR, tile_cols = min(BN, p.N - n0);
   int t_col = tid % PPR * OE;
-  if (t_col < tile_cols && t_col + OE > tile_cols && tile_cols >= OE) t_col = tile_cols - OE;
+  if (p.s_cn == 1 && t_col < tile_cols && t_col + OE > tile_cols && tile_cols >= OE) t_col = tile_cols - OE;
   const int gn = n0 + t_col;
   const int cols = min(p.N - gn, OE);           // columns of this thread's pieces that exist (may be <= 0)
   const bool whole = cols == OE && p.s_cn == 1;  // moved as 16 bytes, else element by element
@@ -472,7 +472,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         if (m0 + row >= p.M || n0 + col >= p.N) continue;
         const float v = *(const LDS_AS float*)(LDS_AS char*)(smem + row * CFG::TROW + col * 4);
         const long long eoff = ((long long)(m0 + row) * p.s_cm + (long long)(n0 + col) * p.s_cn) * 4;
-        for (int pr = 0; pr < p.world; ++pr) atomicAdd((float*)(slot_ptr(p.heap_bases, p.C, p.rank, pr) + eoff), v);
+        for (int pr = 0; pr < p.world; ++pr) {
+          if (p.clear_c && pr == p.rank) *(float*)(p.C + eoff) = 0.f + v;
+          else atomicAdd((float*)(slot_ptr(p.heap_bases, p.C, p.rank, pr) + eoff), v);
+        }
       }
     } else if (p.s_cn == 1) {
       // Packed adds of aligned dwords, one per thread.  A row that starts in the middle of a dword is shifted by
@@ -490,15 +493,25 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         const char* const s = smem + row * CFG::TROW;
         const unsigned w = (lo ? *(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2) : 0x8000u) |
                            (hi ? (unsigned)*(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2 + 2) : 0x8000u) << 16;
-        for (int pr = 0; pr < p.world; ++pr) atomic_add_packed<Out16>(slot_ptr(p.heap_bases, at, p.rank, pr) + e * 2, w);
+        for (int pr = 0; pr < p.world; ++pr) {
+          if (p.clear_c && pr == p.rank) {
+            const unsigned z = added_to_zero(w);
+            if (lo) *(unsigned short*)(at + e * 2) = (unsigned short)z;
+            if (hi) *(unsigned short*)(at + e * 2 + 2) = (unsigned short)(z >> 16);
+          } else {
+            atomic_add_packed<Out16>(slot_ptr(p.heap_bases, at, p.rank, pr) + e * 2, w);
+          }
+        }
       }
     } else {
       for (int ps = 0; ps < PASSES; ++ps) {
         const int row = ps * RPP + t_row;
         if (m0 + row >= m_end) continue;
         for (int e = 0; e < cols; ++e)
-          for (int pr = 0; pr < p.world; ++pr)
-            Out::atomic_add(slot_ptr(p.heap_bases, p.C, p.rank, pr) + offset(row, e), staged_element(row, e));
+          for (int pr = 0; pr < p.world; ++pr) {
+            if (p.clear_c && pr == p.rank) Out::store(p.C + offset(row, e), 0.f + staged_element(row, e));
+            else Out::atomic_add(slot_ptr(p.heap_bases, p.C, p.rank, pr) + offset(row, e), staged_element(row, e));
+          }
       }
     }
     return;
@@ -538,6 +551,14 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         store16_system_of_valu_data(p.aux + offset(row, 0), staged_piece(row));
       } else {
         for (int e = 0; e < cols; ++e) store_element_system<Out>(p.aux + offset(row, e), staged(row) + e * Out::size);
+      }
+      if (p.clear_c && owners) {  // other ranks' tiles: zeros
+        if (piece_ok) {
+          if (owner_at(gm, gn) != p.rank) store16_result(p.C + offset(row, 0), (u32x4_t){0u, 0u, 0u, 0u}, aligned);
+        } else {
+          for (int e = 0; e < cols; ++e)
+            if (owner_at(gm, gn + e) != p.rank) Out::store(p.C + offset(row, e), 0.f);
+        }
       }
       if (!solo) continue;
     }

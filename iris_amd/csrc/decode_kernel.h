@@ -388,6 +388,10 @@ __global__ void __launch_bounds__(320) fused_decode_kernel(const FusedParams p_i
       if (p.epi == EPI_ATOMIC) {
         for (int pr = 0; pr < p.world; ++pr) {
           char* dst = (char*)(in_slot(c_own, pr) + goff);
+          if (p.clear_c && pr == p.rank) {
+            *(u32x2_t*)dst = (u32x2_t){added_to_zero(own.x), added_to_zero(own.y)};
+            continue;
+          }
           atomic_add_packed<Out>(dst, own.x);
           atomic_add_packed<Out>(dst + 4, own.y);
         }
@@ -451,6 +455,7 @@ __global__ void __launch_bounds__(320) fused_decode_kernel(const FusedParams p_i
   };
 
   if (valid) store8_system(p.aux + eoff, own);  // read by the peers as soon as the flag is up
+  if (p.clear_c && valid && owner != p.rank) __builtin_nontemporal_store((u32x2_t){0u, 0u}, (u32x2_t*)(c_own + eoff));
   if (solo && reduces) store_result(own);
   PHASE_STAMP(4);
   // When the helper found every flag up, the peers' tiles are in LDS by now (it waited for them before

@@ -68,6 +68,13 @@ __device__ __forceinline__ void atomic_add_packed(char* addr, unsigned word) {
                                                __builtin_bit_cast(s16x2_t, word));
 }
 
+// What two packed 16-bit floats leave behind when they are added to zeros: themselves, but +0 for -0.
+__device__ __forceinline__ unsigned added_to_zero(unsigned word) {
+  if ((word & 0xFFFFu) == 0x8000u) word &= 0xFFFF0000u;
+  if ((word >> 16) == 0x8000u) word &= 0xFFFFu;
+  return word;
+}
+
 __device__ __forceinline__ float load_scalar_as_float(const char* base, long long idx, int dtype) {
   if (dtype == IRIS_HIP_FP32) return ((const float*)base)[idx];
   unsigned short b = ((const unsigned short*)base)[idx];

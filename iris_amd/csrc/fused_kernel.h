@@ -60,6 +60,7 @@ struct FusedParams {
   int flag_bm, flag_bn;
   int epi;
   int acc_mode;
+  int clear_c;  // IRIS_HIP_CLEAR_C: the own slot's C ends up as if it had been zeroed before the launch
   int all_owners;
   int sum_peers;
   int bias_dtype;
@@ -397,7 +398,7 @@ __device__ __forceinline__ FusedParams pin_kernel_arguments(const FusedParams& a
                "+s"(q.status), "+s"(q.spin_limit));
   asm volatile("" : "+s"(q.s_am), "+s"(q.s_ak), "+s"(q.s_bk), "+s"(q.s_bn), "+s"(q.s_cm), "+s"(q.s_cn), "+s"(q.s_bias));
   asm volatile("" : "+s"(q.M), "+s"(q.N), "+s"(q.K), "+s"(q.K_local), "+s"(q.M_local), "+s"(q.gather), "+s"(q.rank),
-               "+s"(q.world), "+s"(q.flag_bm), "+s"(q.flag_bn), "+s"(q.epi), "+s"(q.acc_mode), "+s"(q.all_owners),
+               "+s"(q.world), "+s"(q.flag_bm), "+s"(q.flag_bn), "+s"(q.epi), "+s"(q.acc_mode), "+s"(q.clear_c), "+s"(q.all_owners),
                "+s"(q.sum_peers), "+s"(q.bias_dtype), "+s"(q.scale));
   asm volatile("" : "+s"(q.tiles_m), "+s"(q.tiles_n), "+s"(q.group_m), "+s"(q.num_xcd), "+s"(q.row_offset),
                "+s"(q.hb_in_args));
@@ -1106,7 +1107,6 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     const bool flags = epi_has_flags(p.epi);
     const bool solo = flags && (!p.sum_peers || p.world == 1);
     {
-      char* const out1 = flags ? p.aux : p.C;
       const int ftn1 = cdiv(p.N, p.flag_bn);
       const int ftotal1 = cdiv(p.M, p.flag_bm) * ftn1;
       const unsigned long long c_base = (unsigned long long)p.C;
@@ -1127,28 +1127,43 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
             if (gm >= p.M || gc >= p.N) continue;
             const unsigned w = *(const LDS_AS unsigned*)(LDS_AS char*)(smem + CFG::stage_offset(row, dc * 4));
             const long long eoff = ((long long)(gm + p.row_offset) * p.s_cm + gc) * 2;
-            for (int pr = 0; pr < p.world; ++pr) atomic_add_packed<Out>((char*)(in_slot(c_base, pr) + eoff), w);
+            for (int pr = 0; pr < p.world; ++pr) {
+              if (p.clear_c && pr == p.rank) *(unsigned*)(p.C + eoff) = added_to_zero(w);
+              else atomic_add_packed<Out>((char*)(in_slot(c_base, pr) + eoff), w);
+            }
           }
         }
-      } else
+      } else if (!flags) {
 #pragma unroll 4
-      for (int ps = 0; ps < PASSES; ++ps) {
-        const int gm = m0 + ps * RPP + t_row;
-        const u32x4_t v = *(const LDS_AS u32x4_t*)(LDS_AS char*)(smem + t_pass[ps & 1] + ps * RPP * CFG::TROW);
-        if (gm < p.M && col_ok) {
-          const long long eoff = ((long long)(gm + p.row_offset) * p.s_cm + gn) * 2;
-          if (p.epi == EPI_ALL_GATHER) {
-            // the tile goes to every rank's gathered output (iris/mem/triton/context.py:841-864)
-            for (int pr = 0; pr < p.world; ++pr) __builtin_nontemporal_store(v, (u32x4_t*)(in_slot(c_base, pr) + eoff));
-          } else if (flags) {
-            store16_system(out1 + eoff, v);  // aux: read by the peers as soon as the flag is up
-          } else {
-            __builtin_nontemporal_store(v, (u32x4_t*)(out1 + eoff));
+        for (int ps = 0; ps < PASSES; ++ps) {
+          const int gm = m0 + ps * RPP + t_row;
+          const u32x4_t v = *(const LDS_AS u32x4_t*)(LDS_AS char*)(smem + t_pass[ps & 1] + ps * RPP * CFG::TROW);
+          if (gm < p.M && col_ok) {
+            const long long eoff = ((long long)(gm + p.row_offset) * p.s_cm + gn) * 2;
+            if (p.epi == EPI_ALL_GATHER) {
+              // the tile goes to every rank's gathered output (iris/mem/triton/context.py:841-864)
+              for (int pr = 0; pr < p.world; ++pr) __builtin_nontemporal_store(v, (u32x4_t*)(in_slot(c_base, pr) + eoff));
+            } else {
+              __builtin_nontemporal_store(v, (u32x4_t*)(p.C + eoff));
+            }
           }
-          if (solo) {
+        }
+      } else {
+        const bool by_owner = p.epi != EPI_ONE_SHOT && (solo || p.clear_c);
+#pragma unroll 4
+        for (int ps = 0; ps < PASSES; ++ps) {
+          const int gm = m0 + ps * RPP + t_row;
+          const u32x4_t v = *(const LDS_AS u32x4_t*)(LDS_AS char*)(smem + t_pass[ps & 1] + ps * RPP * CFG::TROW);
+          if (gm < p.M && col_ok) {
+            const long long eoff = ((long long)gm * p.s_cm + gn) * 2;
+            store16_system(p.aux + eoff, v);  // aux: read by the peers as soon as the flag is up
             int owner = p.rank;
-            if (p.epi != EPI_ONE_SHOT) owner = owner_of(p.epi, (gm / p.flag_bm) * ftn1 + gn / p.flag_bn, ftotal1, p.world, p.rank);
-            if (p.all_owners || owner == p.rank) {
+            if (by_owner) {
+              owner = owner_of(p.epi, (gm / p.flag_bm) * ftn1 + gn / p.flag_bn, ftotal1, p.world, p.rank);
+              // Another rank's tile: zeros, behind the aux stores (8192 x 4096 reduce-scatter: a fill of its own took 10 us).
+              if (p.clear_c && owner != p.rank) __builtin_nontemporal_store((u32x4_t){0u, 0u, 0u, 0u}, (u32x4_t*)(p.C + eoff));
+            }
+            if (solo && (p.all_owners || owner == p.rank)) {
               if (p.epi == EPI_TWO_SHOT) {
                 for (int pr = 0; pr < p.world; ++pr) __builtin_nontemporal_store(v, (u32x4_t*)(in_slot(c_base, pr) + eoff));
               } else {

@@ -368,7 +368,7 @@ int matmul_all_reduce_impl(const void* A, const void* B, void* C, void* aux_buff
   p.rank = cur_rank; p.world = world_size;
   p.flag_bm = block_size_m; p.flag_bn = block_size_n;
   p.epi = variant == IRIS_HIP_VARIANT_ATOMIC ? EPI_ATOMIC : variant == IRIS_HIP_VARIANT_ONE_SHOT ? EPI_ONE_SHOT : EPI_TWO_SHOT;
-  p.acc_mode = acc_mode; p.all_owners = 0; p.sum_peers = 1;
+  p.acc_mode = acc_mode & ~IRIS_HIP_CLEAR_C; p.clear_c = (acc_mode & IRIS_HIP_CLEAR_C) != 0; p.all_owners = 0; p.sum_peers = 1;
   p.scale = scale; p.spin_limit = spin_limit; p.status = status;
   p.no_workspace_alloc = no_alloc ? 1 : 0;
   return run_fused(p, in_dtype, out_dtype, path, stream, check_only);
@@ -550,7 +550,7 @@ int iris_hip_matmul_reduce_scatter(const void* A, const void* B, void* C, void* 
   p.rank = cur_rank; p.world = world_size;
   p.flag_bm = block_size_m; p.flag_bn = block_size_n;
   p.epi = EPI_REDUCE_SCATTER;
-  p.acc_mode = acc_mode; p.all_owners = all_owners ? 1 : 0; p.sum_peers = sum_peers ? 1 : 0;
+  p.acc_mode = acc_mode & ~IRIS_HIP_CLEAR_C; p.clear_c = (acc_mode & IRIS_HIP_CLEAR_C) != 0; p.all_owners = all_owners ? 1 : 0; p.sum_peers = sum_peers ? 1 : 0;
   p.scale = scale; p.spin_limit = spin_limit; p.status = status;
   return run_fused(p, in_dtype, out_dtype, path, stream);
 }

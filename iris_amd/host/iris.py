@@ -302,6 +302,11 @@ class Iris:
             _dist.barrier(group=group)
         self.check_status()
 
+    def runs_alone(self):
+        """True when this process plays every rank itself: no process group, and the peers' flags and buffers are
+        whatever the program staged (stand_in_peers has the preambles restage them)."""
+        return not self.stand_in_peers and not (_dist.is_available() and _dist.is_initialized())
+
     def check_status(self):
         """Raise RuntimeError if a kernel set a status bit since the last check (needs a sync first)."""
         status = int(self._status_view[0]) if self._status_view is not None else int(self._status[0])

@@ -13,7 +13,7 @@ import torch
 from .. import _lib
 from ..host.logging import debug_on, log_rank
 from ._common import (acc_code, current_stream, dtype_code, iris_launch, is_fp8, path_code, ptr,
-                      require_gpu_tensors, stage_idle_peers)
+                      rearmed, require_gpu_tensors, stage_idle_peers)
 from .config import FusedConfig
 from .workspace import FusedWorkspace
 
@@ -140,14 +140,22 @@ def matmul_all_reduce(
         raise NotImplementedError(
             f"all_reduce_variant {config.all_reduce_variant!r} has no HIP kernel; use 'atomic', 'one_shot' or 'two_shot'"
         )
+    total_tiles = _tile_count(M, N, config)
+    stream = current_stream(shmem)
+    clear = 0
     needs_prepare = workspace is None or not workspace.matches(
         "matmul_all_reduce", (M, N, K), A.dtype, world_size, config.all_reduce_variant
     )
     if needs_prepare:
-        workspace = matmul_all_reduce_preamble(shmem, C, A, B, config=config, workspace=workspace)
+        if rearmed(shmem, workspace, C, "matmul_all_reduce", (M, N, K), A.dtype, world_size, config.all_reduce_variant,
+                   total_tiles, stream):
+            config.validate(world_size=world_size)
+            shmem.check_status()
+            clear = _lib.CLEAR_C
+        else:
+            workspace = matmul_all_reduce_preamble(shmem, C, A, B, config=config, workspace=workspace)
 
     device_context = shmem.get_device_context()
-    total_tiles = _tile_count(M, N, config)
     grid = (total_tiles,)
     if workspace.locks is not None and workspace.locks.numel() < total_tiles:
         raise ValueError(
@@ -183,15 +191,15 @@ def matmul_all_reduce(
         ptr(device_context), rank, world_size,
         config.block_size_m, config.block_size_n, config.block_size_k,
         _VARIANT_CODES[config.all_reduce_variant],
-        dtype_code(A.dtype), dtype_code(C.dtype), scale, acc,
-        shmem.spin_limit, ptr(shmem._status), path, current_stream(shmem),
+        dtype_code(A.dtype), dtype_code(C.dtype), scale, acc | clear,
+        shmem.spin_limit, ptr(shmem._status), path, stream,
         algorithm="matmul_all_reduce",
         rank=rank,
         dtype=A.dtype,
     )
 
-    if workspace is not None:
-        workspace.prepared = False
+    workspace.prepared = False
+    workspace.stream = stream
     if not async_op:
         shmem.barrier()
     return workspace

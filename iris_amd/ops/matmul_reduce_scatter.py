@@ -10,9 +10,10 @@ from typing import Optional
 
 import torch
 
+from .. import _lib
 from ..host.logging import debug_on, log_rank
 from ._common import (acc_code, current_stream, dtype_code, iris_launch, is_fp8, path_code, ptr,
-                      require_gpu_tensors, stage_idle_peers)
+                      rearmed, require_gpu_tensors, stage_idle_peers)
 from .config import FusedConfig
 from .workspace import FusedWorkspace
 
@@ -114,19 +115,27 @@ def matmul_reduce_scatter(
             raise ValueError(f"float8 inputs need a bfloat16/float16 output, got A:{A.dtype}, B:{B.dtype}, C:{C.dtype}")
     elif A.dtype != B.dtype or A.dtype != C.dtype:
         raise ValueError(f"All tensors must have same dtype, got A:{A.dtype}, B:{B.dtype}, C:{C.dtype}")
-    workspace = matmul_reduce_scatter_preamble(shmem, C, A, B, config, workspace)
-    if stage is not None:
-        stage(workspace)
-
     M, K = A.shape[:2]
     N = B.shape[1]
     rank = shmem.get_rank()
     world_size = shmem.get_num_ranks()
+    total_tiles = _tile_count(M, N, config)
+    stream = current_stream(shmem)
+    clear = 0
+    if stage is None and rearmed(shmem, workspace, C, "matmul_reduce_scatter", (M, N, K), A.dtype, world_size, "two_shot",
+                                 total_tiles, stream):
+        config.validate(world_size=world_size)
+        shmem.check_status()
+        clear = _lib.CLEAR_C
+    else:
+        workspace = matmul_reduce_scatter_preamble(shmem, C, A, B, config, workspace)
+        if stage is not None:
+            stage(workspace)
+
     if debug_on():
         log_rank(logging.DEBUG, "matmul_reduce_scatter: shape=(%d,%d,%d) dtype=%s rank=%d/%d", M, N, K, A.dtype, rank,
                  world_size, rank=rank, num_ranks=world_size)
 
-    total_tiles = _tile_count(M, N, config)
     if workspace.locks is not None and workspace.locks.numel() < total_tiles:
         raise _too_small(workspace.locks.numel(), total_tiles)
     grid = (total_tiles,)
@@ -150,13 +159,14 @@ def matmul_reduce_scatter(
         ptr(shmem.get_device_context()), rank, world_size,
         config.block_size_m, config.block_size_n, config.block_size_k,
         int(bool(all_owners)), int(bool(sum_peers)),
-        dtype_code(A.dtype), dtype_code(C.dtype), scale, acc,
-        shmem.spin_limit, ptr(shmem._status), path, current_stream(shmem),
+        dtype_code(A.dtype), dtype_code(C.dtype), scale, acc | clear,
+        shmem.spin_limit, ptr(shmem._status), path, stream,
         algorithm="matmul_reduce_scatter",
         rank=rank,
         dtype=A.dtype,
     )
 
+    workspace.stream = stream
     if not async_op:
         torch.cuda.synchronize()
         shmem.barrier()

@@ -19,6 +19,7 @@ class FusedWorkspace:
     aux_buffer: Optional[torch.Tensor] = None  # own GEMM tile results, read by the peers
     locks: Optional[torch.Tensor] = None  # int32 ready flag per flag tile
     prepared: bool = False
+    stream: Optional[int] = None  # raw HIP stream of the last launch that used the buffers
 
     def matches(self, operation, shape, dtype, world_size, variant="") -> bool:
         """True when the buffers were prepared for exactly this call and have not been used since."""

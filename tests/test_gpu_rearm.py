@@ -1,0 +1,69 @@
+"""A workspace handed back to the operator that used it: the second call runs no preamble and must still leave what a
+call with one leaves - own tiles reduced, every other tile of C zero - on each kernel family."""
+
+import pytest
+import torch
+
+import iris_amd as iris
+from iris_amd import _lib, ops
+from iris_amd.ccl import Config
+from helpers import assert_bits_equal, heap_tensor, oracle, randint_cpu, randn_cpu, stage_peers
+
+pytestmark = pytest.mark.gpu
+
+
+# 32x32 kernel, 64x64 and 256x256 tiles, the any-shape kernel with whole and with ragged pieces.
+@pytest.mark.parametrize("M,N,K,dtype,kernel", [
+    (96, 264, 72, torch.bfloat16, "mfma_bf16_32x32"), (640, 1024, 96, torch.float16, "mfma_f16_64x64"), (3072, 3080, 80, torch.bfloat16, "mfma_bf16_256x256"),
+    (130, 132, 40, torch.float32, "generic_f32"), (131, 267, 70, torch.float16, "generic_f16")])
+@pytest.mark.parametrize("op", ["one_shot", "two_shot", "atomic", "reduce_scatter"])
+def test_second_call_equals_first(op, M, N, K, dtype, kernel):
+    W, rank = 4, 2
+    ctx = iris.iris(1 << 27, num_ranks=W, rank=rank)
+    B = randint_cpu((K, N), 1, dtype)
+    peers = [randn_cpu((M, N), 20 + r, dtype) for r in range(W)]
+    dA, dB, dC = ctx.zeros((M, K), dtype=dtype), heap_tensor(ctx, B), ctx.zeros((M, N), dtype=dtype)
+    variant = "two_shot" if op == "reduce_scatter" else op
+    cfg = iris.FusedConfig(block_size_m=32, block_size_n=24, block_size_k=16, all_reduce_variant=variant)
+    preamble = ops.matmul_reduce_scatter_preamble if op == "reduce_scatter" else ops.matmul_all_reduce_preamble
+    call = ops.matmul_reduce_scatter if op == "reduce_scatter" else ops.matmul_all_reduce
+    ws = preamble(ctx, dC, dA, dB, cfg)
+    if op != "atomic":
+        stage_peers(ctx, ws, peers)
+    side = torch.cuda.Stream()
+    for turn in range(4):
+        A = randint_cpu((M, K), 40 + turn, dtype)
+        dA.copy_(A)
+        if turn:  # (the first call relies on the preamble's zeros)
+            dC.fill_(float("nan"))  # nothing of what C holds may survive
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side if turn == 2 else torch.cuda.current_stream()):  # turns 2 and 3: another stream than before
+            ws = call(ctx, dC, dA, dB, async_op=True, config=cfg, workspace=ws)
+        torch.cuda.synchronize()
+        assert _lib.last_kernel().startswith(kernel), _lib.last_kernel()
+        if op == "atomic":
+            exp = oracle.gemm(A, B)  # added to a zeroed C
+        elif op == "reduce_scatter":
+            exp = oracle.matmul_reduce_scatter(A, B, peers, rank, W, 32, 24)["C"][rank]
+        else:
+            exp = oracle.matmul_all_reduce(A, B, peers, rank, W, 32, 24, variant)["C"][rank]
+        assert_bits_equal(dC.cpu() + 0, exp + 0, f"{op} turn {turn}")  # (+ 0: zeros of one sign)
+        ctx.check_status()
+
+
+@pytest.mark.parametrize("variant", ["one_shot", "atomic"])
+def test_second_collective_equals_first(variant):
+    W, rank, M, N, dtype = 4, 1, 70, 264, torch.bfloat16
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=rank)
+    x, y = ctx.zeros((M, N), dtype=dtype), ctx.zeros((M, N), dtype=dtype)
+    cfg = Config(all_reduce_variant=variant)
+    ws = ctx.ccl.all_reduce_preamble(y, x, config=cfg)
+    for turn in range(3):
+        inputs = [randint_cpu((M, N), 10 * turn + r, dtype) for r in range(W)]
+        for r in range(W):
+            ctx.peer_view(x, r).copy_(inputs[r])
+        if turn:
+            y.fill_(float("nan"))
+        ws = ctx.ccl.all_reduce(y, x, async_op=True, config=cfg, workspace=ws)
+        exp = sum(i.float() for i in inputs).to(dtype) if variant == "one_shot" else inputs[rank]
+        assert_bits_equal(y.cpu() + 0, exp + 0, f"turn {turn}")
