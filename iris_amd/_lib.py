@@ -5,11 +5,13 @@ library has not been built, using an operator raises.
 """
 
 import ctypes
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # IRIS_HIP_LIBRARY names another build of the same library (e.g. one compiled with other tile shapes).
 LIBRARY_PATH = os.environ.get("IRIS_HIP_LIBRARY") or os.path.join(_HERE, "lib", "libiris_hip.so")
+LAUNCHER_PATH = os.path.join(_HERE, "lib", "_launch.so")
 
 ABI_VERSION = 5
 
@@ -93,6 +95,23 @@ PROTOTYPES = {
 }
 
 _lib = None
+_launch = None
+
+
+def launcher():
+    """The module iris_amd/lib/_launch.so: operator calls and the entry points behind them as built-in functions
+    (csrc/launcher.cpp).  Raises if it is not built."""
+    global _launch
+    if _launch is None:
+        library()  # checks the library and its version first
+        if not os.path.exists(LAUNCHER_PATH):
+            raise RuntimeError(f"{LAUNCHER_PATH} is missing: build it with `python -m iris_amd.csrc.build`")
+        spec = importlib.util.spec_from_file_location("_launch", LAUNCHER_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.load(LIBRARY_PATH)
+        _launch = module
+    return _launch
 
 
 def library():

@@ -1,4 +1,4 @@
-"""Build libiris_hip.so for gfx950 with hipcc.
+"""Build libiris_hip.so for gfx950 with hipcc, and the Python module that calls it with g++.
 
     python -m iris_amd.csrc.build [--force]
 
@@ -10,6 +10,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -23,6 +24,10 @@ HEADERS = [os.path.join(HERE, h) for h in ("fused_kernel.h", "decode_kernel.h", 
                                            "host_common.h")] + [
     os.path.join(ROOT, "include", "iris_hip.h")]
 OUTPUT = os.path.join(os.path.dirname(HERE), "lib", "libiris_hip.so")
+# The Python module through which the operators call the library's entry points (host code only; it reads torch's
+# tensors without going through their Python attributes).
+LAUNCHER_SOURCE = os.path.join(HERE, "launcher.cpp")
+LAUNCHER_OUTPUT = os.path.join(os.path.dirname(HERE), "lib", "_launch.so")
 
 FLAGS = [
     "--offload-arch=gfx950",
@@ -38,10 +43,23 @@ FLAGS = [
 
 
 def up_to_date():
-    if not os.path.exists(OUTPUT):
+    if not (os.path.exists(OUTPUT) and os.path.exists(LAUNCHER_OUTPUT)):
         return False
-    built = os.path.getmtime(OUTPUT)
-    return all(os.path.getmtime(f) <= built for f in SOURCES + HEADERS + [os.path.abspath(__file__)])
+    built = min(os.path.getmtime(OUTPUT), os.path.getmtime(LAUNCHER_OUTPUT))
+    return all(os.path.getmtime(f) <= built for f in SOURCES + HEADERS + [LAUNCHER_SOURCE, os.path.abspath(__file__)])
+
+
+def _build_launcher(verbose):
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    tmp = LAUNCHER_OUTPUT + ".tmp"
+    includes = [sysconfig.get_paths()["include"]] + include_paths()
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-I" + os.path.join(ROOT, "include")]
+         + [flag for path in includes for flag in ("-isystem", path)] + ["-o", tmp, LAUNCHER_SOURCE]
+         + ["-L" + path for path in library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"], verbose)
+    os.replace(tmp, LAUNCHER_OUTPUT)
 
 
 def _run(cmd, verbose):
@@ -77,8 +95,9 @@ def _build(output, flags, verbose):
     with tempfile.TemporaryDirectory(prefix="iris_hip_build_") as tmpdir:
         objects = [os.path.join(tmpdir, os.path.splitext(os.path.basename(src))[0] + ".o") for src in SOURCES]
         with concurrent.futures.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 1)) as pool:
-            jobs = [pool.submit(_run, [hipcc] + flags + ["-c", "-o", obj, src], verbose)
-                    for src, obj in zip(SOURCES, objects)]
+            jobs = [pool.submit(_build_launcher, verbose)]
+            jobs += [pool.submit(_run, [hipcc] + flags + ["-c", "-o", obj, src], verbose)
+                     for src, obj in zip(SOURCES, objects)]
             for job in jobs:
                 job.result()
         tmp = output + ".tmp"

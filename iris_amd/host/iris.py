@@ -92,6 +92,8 @@ class Iris:
         self.heap = SymmetricHeap(heap_size, self.gpu_id, self.cur_rank, self.num_ranks, backing=backing)
         self.device = str(self.heap.device) if backing == "host" else f"cuda:{self.gpu_id}"
         self.heap_bases = self.heap.get_heap_bases()
+        self._own_begin = self.heap.slot_base(self.cur_rank)  # addresses of the own slot (see is_symmetric)
+        self._own_end = self._own_begin + self.heap.heap_size
         self._ops = None
         self._ccl = None
         self._cu_count = None

@@ -17,7 +17,7 @@ _FP8 = getattr(torch, "float8_e4m3fn", None)
 if _FP8 is not None:
     _DTYPE_CODES[_FP8] = _lib.FP8_E4M3
 
-_ENTRY_POINTS = {}  # name -> bound foreign function (prototypes applied by _lib.library())
+_ENTRY_POINTS = {}  # name -> entry point of the kernel library (_lib.launcher())
 
 _PATHS = {"auto": _lib.PATH_AUTO, "mfma": _lib.PATH_MFMA, "generic": _lib.PATH_GENERIC}
 _ACC = {"fp32": _lib.ACC_FP32, "reference": _lib.ACC_REFERENCE}
@@ -59,9 +59,7 @@ def require_gpu_tensors(shmem, **tensors):
 
 
 def ptr(t):
-    """Device address of a tensor as the prototypes' void* takes it: a plain integer, None for no tensor
-    (the operators are called once per few microseconds for small shapes; a ctypes object per argument
-    was a tenth of the call)."""
+    """Device address of a tensor as the entry points take it: a plain integer, None for no tensor."""
     return t.data_ptr() if t is not None else None
 
 
@@ -70,6 +68,13 @@ def current_stream(shmem):
     `with torch.cuda.stream(...)` and graph capture); None for a host-backed context."""
     device = shmem.get_device_id()
     return torch._C._cuda_getCurrentRawStream(device) if device >= 0 else None
+
+
+def native(shmem):
+    """The module that takes whole operator calls (csrc/launcher.cpp), or None where the Python wrapper has to: on a
+    host-backed context and while DEBUG records are wanted.  Its try_<op> functions return False, with nothing done,
+    for every call that is not plainly in order; the wrapper then starts over and finds out why."""
+    return None if shmem.gpu_id < 0 or debug_on() else _lib.launcher()
 
 
 def rearmed(shmem, workspace, C, operation, shape, dtype, world_size, variant, tiles, stream):
@@ -101,7 +106,7 @@ def iris_launch(entry_name, grid, *args, algorithm, rank, dtype=None):
                  rank, rank=rank)
     entry = _ENTRY_POINTS.get(entry_name)
     if entry is None:
-        entry = _ENTRY_POINTS[entry_name] = getattr(_lib.library(), entry_name)
+        entry = _ENTRY_POINTS[entry_name] = getattr(_lib.launcher(), entry_name)
     err = entry(*args)
     if err != 0:
         detail = _lib.last_error()

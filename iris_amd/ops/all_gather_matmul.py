@@ -12,7 +12,7 @@ import torch
 
 from .. import _lib
 from ..host.logging import debug_on, log_rank
-from ._common import current_stream, dtype_code, iris_launch, is_fp8, path_code, ptr, require_gpu_tensors
+from ._common import current_stream, dtype_code, iris_launch, is_fp8, native, path_code, ptr, require_gpu_tensors
 from .config import FusedConfig
 from .workspace import FusedWorkspace
 
@@ -72,6 +72,15 @@ def all_gather_matmul(
     """
     if config is None:
         config = FusedConfig()
+    fast = native(shmem)
+    if fast is not None and fast.try_all_gather_matmul(shmem, output_tensor, A_sharded, B, bias, config, gather_dim, scale_a,
+                                                       scale_b, kernel_path, current_stream(shmem)):
+        if not async_op:
+            shmem.barrier()
+        if workspace is None:
+            workspace = FusedWorkspace("all_gather_matmul", (*output_tensor.shape, B.shape[0]), A_sharded.dtype,
+                                       shmem.num_ranks, prepared=True)
+        return workspace
     if gather_dim not in (0, 1):
         raise ValueError(f"gather_dim must be 0 (rows) or 1 (columns), got {gather_dim}")
     world_size = shmem.get_num_ranks()

@@ -67,3 +67,39 @@ def test_second_collective_equals_first(variant):
         ws = ctx.ccl.all_reduce(y, x, async_op=True, config=cfg, workspace=ws)
         exp = sum(i.float() for i in inputs).to(dtype) if variant == "one_shot" else inputs[rank]
         assert_bits_equal(y.cpu() + 0, exp + 0, f"turn {turn}")
+
+
+def test_calls_that_are_not_in_order_reach_the_python_checks():
+    """The native call path takes calls that are plainly in order and must leave every other one to the wrapper's
+    checks and messages, also on a workspace it has used."""
+    W, M, N, K, dtype = 2, 64, 128, 64, torch.bfloat16
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=0)
+    A, B, C = ctx.zeros((M, K), dtype=dtype), ctx.zeros((K, N), dtype=dtype), ctx.zeros((M, N), dtype=dtype)
+    cfg = iris.FusedConfig(block_size_m=32, block_size_n=32, block_size_k=32, all_reduce_variant="one_shot")
+    ws = ops.matmul_all_reduce_preamble(ctx, C, A, B, config=cfg)
+    stage_peers(ctx, ws, [C] * W)
+    for _ in range(2):
+        ws = ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws)
+    with pytest.raises(ValueError, match="Incompatible matrix dimensions"):
+        ctx.ops.matmul_all_reduce(C, A, B[:32], config=cfg, workspace=ws)
+    with pytest.raises(ValueError, match="same dtype"):
+        ctx.ops.matmul_all_reduce(C, A, B.half(), config=cfg, workspace=ws)
+    with pytest.raises(ValueError, match="scale_a"):
+        ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws, scale_a=1.0)
+    with pytest.raises(ValueError, match="kernel path"):
+        ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws, kernel_path="fast")
+    with pytest.raises(RuntimeError, match="is on cpu"):
+        ctx.ops.matmul_all_reduce(C, A, B.cpu(), config=cfg, workspace=ws)
+    with pytest.raises(AssertionError, match="too small for block_size_m"):
+        ctx.ops.matmul_all_reduce(C, A, B, config=iris.FusedConfig(all_reduce_variant="one_shot"), workspace=ws)
+    with pytest.raises(RuntimeError, match="symmetric heap"):
+        ctx.ops.all_gather_matmul(C, torch.zeros((M, K // W), dtype=dtype, device="cuda"), B, config=cfg)
+    with pytest.raises(RuntimeError, match="symmetric heap"):
+        ctx.ops.matmul_all_gather(torch.zeros((W * M, N), dtype=dtype, device="cuda"), A, B, config=cfg)
+    with pytest.raises(RuntimeError, match="symmetric heap"):
+        ctx.ccl.reduce_scatter(C, torch.zeros((M, N), dtype=dtype, device="cuda"))
+    ctx._status[0] = _lib.STATUS_SPIN_TIMEOUT  # as a kernel of an earlier call would leave it
+    with pytest.raises(RuntimeError, match="gave up waiting"):
+        ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws)
+    ws = ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws)
+    assert torch.all(C == 0)
