@@ -145,6 +145,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 
   const int tidx = xcd_tile_index(blockIdx.x, gridDim.x, 0, p.tiles_m * p.tiles_n, p.num_xcd);
   if (tidx < 0) return;
+#ifdef IRIS_HIP_PHASE_STAMPS
+  constexpr int it = 0;  // PHASE_STAMP records the first tile of a workgroup; there is only one here
+#endif
+  PHASE_STAMP(0);
   int tm, tn;
   grouped_tile(tidx, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
@@ -358,6 +362,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   put(0);
   if (nsteps > 1) fetch();
   lds_barrier();
+  PHASE_STAMP(1);
   for (int s = 0; s < nsteps; ++s) {
     const int buf = s & 1;
     Frag f[2];
@@ -373,6 +378,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     }
     lds_barrier();
   }
+
+  PHASE_STAMP(2);
 
   // ---- the tile in the output type, in LDS ------------------------------------------------------------------
   if constexpr (CFG::WK > 1) {
@@ -433,6 +440,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     }
   }
   lds_barrier();
+
+  PHASE_STAMP(3);
 
   // ---- epilogue: pieces of OE consecutive columns, handed out row by row ---------------------------------------
   constexpr int PPR = BN / OE;             // pieces per tile row
@@ -570,6 +579,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         each_destination(gm, gn + e, [&](char* base) { Out::store(base + offset(row, e), staged_element(row, e)); });
     }
   }
+  PHASE_STAMP(4);
   if (!flags) return;
 
   // Publish and wait, as in the tiled kernel: aux is written through, so relaxed flag stores behind the
@@ -577,10 +587,12 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const bool up_already = solo ? true : probe_peer_flags<BM, BN, NT>(p, m0, n0, tid);
   wait_vmcnt<0>();
   __syncthreads();
+  PHASE_STAMP(5);
   raise_flags<BM, BN, NT, true>(p, m0, n0, tid);
   if (solo) return;
   if (!up_already) wait_peer_flags<BM, BN, NT>(p, m0, n0, tid);
   __syncthreads();
+  PHASE_STAMP(6);
 
   // Slot sum in ascending rank order from the own (already rounded) value, in fp32 or by the reference's rule.
   const bool ref_chain = (p.acc_mode == IRIS_HIP_ACC_REFERENCE) && !Out::kFp32SumInReference;
@@ -659,6 +671,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     case 7: reduce(std::integral_constant<int, 7>{}); break;
     default: reduce(std::integral_constant<int, 0>{}); break;
   }
+  PHASE_STAMP(7);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -50,6 +50,12 @@ struct CclParams {
   // Work decomposition: a tile is cut into `upt` units (units per tile), `upr` of them per tile row.
   int upr, upt;
   long long total_units;
+  // A contiguous run of owned tiles as rectangles of tiles, each walked row by row over its whole width (ROWS builds).
+  struct Rect {
+    int pm0, pn0, width;  // first tile row and column, units per row
+    long long base;       // unit index of the rectangle's first unit
+  } rect[5];
+  int n_rects;
 };
 
 // Tile coordinates of tile id `t` in the grouped order (group_m tile-rows are walked column by
@@ -65,22 +71,31 @@ __device__ __forceinline__ void grouped_coords(int t, int tiles_m, int tiles_n, 
 }
 
 typedef __attribute__((ext_vector_type(4))) unsigned ccl_u32x4_t;
+typedef ccl_u32x4_t ccl_u32x4_any_t __attribute__((aligned(1)));  // rows may start anywhere (an odd N)
 
 // 16-byte accesses; NT marks data that is touched once (launches too large to stay in the
 // last-level cache), which keeps it from displacing other lines on its way through.
 template <bool NT>
 __device__ __forceinline__ ccl_u32x4_t load16(const char* p) {
-  if constexpr (NT) return __builtin_nontemporal_load((const ccl_u32x4_t*)p);
-  else return *(const ccl_u32x4_t*)p;
+  if constexpr (NT) return __builtin_nontemporal_load((const ccl_u32x4_any_t*)p);
+  else return *(const ccl_u32x4_any_t*)p;
 }
 template <bool NT>
 __device__ __forceinline__ void store16(char* p, ccl_u32x4_t v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, (ccl_u32x4_t*)p);
-  else *(ccl_u32x4_t*)p = v;
+  if constexpr (NT) __builtin_nontemporal_store(v, (ccl_u32x4_any_t*)p);
+  else *(ccl_u32x4_any_t*)p = v;
 }
 
 template <class E, int VEC>
 struct Chunk;  // VEC elements of type E, moved with one memory instruction
+
+// The elements of a chunk from `first` on.
+template <class E, int VEC>
+__device__ __forceinline__ void store_from(const Chunk<E, VEC>& c, char* p, int first) {
+#pragma unroll
+  for (int e = 0; e < VEC; ++e)
+    if (e >= first) E::store(p + e * E::size, c.v[e]);
+}
 
 template <class E>
 struct Chunk<E, 1> {
@@ -166,7 +181,8 @@ struct Chunk<ElemF32, 4> {
 
 // E: element traits.  VEC: elements per memory access (1 = any strides).  WCT: compile-time group
 // size (0 = run-time loop).  UPT: units (chunks) per thread and iteration.  NT: non-temporal accesses.
-template <class E, int VEC, int WCT, int UPT, bool NT>
+// ROWS: units walk the rectangles of CclParams::rect row by row (else tile by tile); stores go through the caches then.
+template <class E, int VEC, int WCT, int UPT, bool NT, bool ROWS>
 __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParams p) {
   // Byte offset of every group member's slot relative to the own slot.
   __shared__ long long slot_delta[kMaxGroup];
@@ -180,13 +196,17 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
     const int r = p.rank_start + i * p.rank_stride;
     return p.heap_bases[r] - p.heap_bases[p.iris_rank];
   };
+  auto put = [&](const Chunk<E, VEC>& c, char* dst, int from) {
+    if (VEC > 2 && from > 0) store_from(c, dst, from);
+    else c.template store<NT && !ROWS>(dst);
+  };
   const int W = WCT ? WCT : p.world;
   const bool tiled = (p.mode == CCL_TWO_SHOT || p.mode == CCL_REDUCE_SCATTER);
 
   const long long span = (long long)gridDim.x * kCclThreads * UPT;
   for (long long base = (long long)blockIdx.x * kCclThreads * UPT; base < p.total_units; base += span) {
     long long in_off[UPT], out_off[UPT];
-    int start[UPT];
+    int start[UPT], first[UPT];  // first: elements of the chunk that are its left neighbour's (see below)
     bool live[UPT];
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
@@ -194,7 +214,9 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
       live[u] = g < p.total_units;
       const long long gg = live[u] ? g : 0;
       int j, c;  // which owned tile, which unit inside it
-      if (p.total_units < (1ll << 31)) {
+      if (ROWS) {
+        j = c = 0;  // found below
+      } else if (p.total_units < (1ll << 31)) {
         j = (int)((unsigned)gg / (unsigned)p.upt);
         c = (int)((unsigned)gg - (unsigned)j * (unsigned)p.upt);
       } else {
@@ -202,7 +224,25 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
         c = (int)(gg - (long long)j * p.upt);
       }
       int pm, pn;
-      if (tiled) {
+      if constexpr (ROWS) {
+        int pm0 = p.rect[0].pm0, pn0 = p.rect[0].pn0, width = p.rect[0].width;
+        long long first_unit = 0;
+#pragma unroll
+        for (int i = 1; i < 5; ++i) {
+          if (i < p.n_rects && gg >= p.rect[i].base) {
+            pm0 = p.rect[i].pm0, pn0 = p.rect[i].pn0, width = p.rect[i].width;
+            first_unit = p.rect[i].base;
+          }
+        }
+        // (the host keeps launches of 2^31 units and more on the other path)
+        const unsigned in_rect = (unsigned)(gg - first_unit), r = in_rect / (unsigned)width, across = in_rect - r * (unsigned)width;
+        pm = pm0 + (int)(r / (unsigned)p.bm);
+        pn = pn0 + (int)(across / (unsigned)p.upr);
+        c = (int)(r % (unsigned)p.bm) * p.upr + (int)(across % (unsigned)p.upr);
+        const int first_m = pm / p.group_m * p.group_m;  // the inverse of grouped_coords
+        j = first_m * p.tiles_n + pn * min(p.tiles_m - first_m, p.group_m) + pm - first_m - p.first_tile;
+        start[u] = (j % p.comm_sms) % W;
+      } else if (tiled) {
         grouped_coords(p.first_tile + j * p.tile_stride, p.tiles_m, p.tiles_n, p.group_m, pm, pn);
         start[u] = (j % p.comm_sms) % W;
       } else {
@@ -211,8 +251,14 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
         start[u] = 0;
       }
       const int row = pm * p.bm + c / p.upr;
-      const int col = pn * p.bn + (c % p.upr) * VEC;
+      int col = pn * p.bn + (c % p.upr) * VEC;
       live[u] = live[u] && row < p.M && col < p.N;
+      // A chunk that would reach past the last column starts further left and stores its own elements only.
+      first[u] = 0;
+      if constexpr (VEC > 2) {
+        first[u] = max(col + VEC - p.N, 0);
+        col -= first[u];
+      }
       in_off[u] = ((long long)row * p.s_im + (long long)col * p.s_in) * E::size;
       out_off[u] = ((long long)row * p.s_om + (long long)col * p.s_on) * E::size;
     }
@@ -256,9 +302,9 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
         if (!live[u]) continue;
         if (p.mode == CCL_TWO_SHOT) {
 #pragma unroll
-          for (int i = 0; i < WCT; ++i) acc.template store<NT>(p.out + out_off[u] + delta(i));
+          for (int i = 0; i < WCT; ++i) put(acc, p.out + out_off[u] + delta(i), first[u]);
         } else {
-          acc.template store<NT>(p.out + out_off[u]);
+          put(acc, p.out + out_off[u], first[u]);
         }
       }
     } else {
@@ -275,18 +321,18 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
           for (int e = 0; e < VEC; ++e) acc.v[e] = (i == 0) ? (tiled ? x.v[e] : 0.0f + x.v[e]) : acc.v[e] + x.v[e];
         }
         if (p.mode == CCL_TWO_SHOT) {
-          for (int i = 0; i < W; ++i) acc.template store<NT>(p.out + out_off[u] + delta(i));
+          for (int i = 0; i < W; ++i) put(acc, p.out + out_off[u] + delta(i), first[u]);
         } else {
-          acc.template store<NT>(p.out + out_off[u]);
+          put(acc, p.out + out_off[u], first[u]);
         }
       }
     }
   }
 }
 
-template <class E, int VEC, int UPT, bool NT>
+template <class E, int VEC, int UPT, bool NT, bool ROWS>
 void launch_for_world(const CclParams& p, int grid, hipStream_t s) {
-#define CCL_KERNEL(W, U) hipLaunchKernelGGL((slot_reduce_kernel<E, VEC, W, U, NT>), dim3(grid), dim3(kCclThreads), 0, s, p)
+#define CCL_KERNEL(W, U) hipLaunchKernelGGL((slot_reduce_kernel<E, VEC, W, U, NT, ROWS>), dim3(grid), dim3(kCclThreads), 0, s, p)
   switch (p.mode == CCL_ATOMIC ? 0 : p.world) {
     case 1: CCL_KERNEL(1, UPT); break;
     case 2: CCL_KERNEL(2, UPT); break;
@@ -298,6 +344,45 @@ void launch_for_world(const CclParams& p, int grid, hipStream_t s) {
 }
 
 bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
+
+// The owned tiles of the block distribution are consecutive in the grouped order: the rest of a column, some columns of
+// a group, whole groups, and the mirror image at the end - at most five rectangles.  Walked row by row, a workgroup
+// moves kilobytes of every row instead of tiles' 128-byte rows (bf16 8192x2880 two-shot, eight ranks: 22.2 -> 19.8 us).
+void fill_rects(CclParams& p) {
+  long long base = 0;
+  auto add = [&](int pm0, int rows, int pn0, int cols) {
+    if (rows <= 0 || cols <= 0) return;
+    p.rect[p.n_rects++] = {pm0, pn0, cols * p.upr, base};
+    base += (long long)rows * p.bm * cols * p.upr;
+  };
+  const int per_group = p.group_m * p.tiles_n, total = p.tiles_m * p.tiles_n;
+  const int end = p.first_tile + p.n_owned;
+  int t = p.first_tile;
+  auto inside_group = [&](int stop) {  // tiles [t, stop) of one group
+    const int m0 = t / per_group * p.group_m, gs = p.tiles_m - m0 < p.group_m ? p.tiles_m - m0 : p.group_m;
+    const int a = t - m0 * p.tiles_n, b = stop - m0 * p.tiles_n;  // positions in the group, column by column
+    const int first_col = cdiv(a, gs), last_col = b / gs;          // whole columns [first_col, last_col)
+    if (first_col > last_col) {                                     // all in one column
+      add(m0 + a % gs, b - a, a / gs, 1);
+    } else {
+      if (a % gs) add(m0 + a % gs, gs - a % gs, a / gs, 1);
+      add(m0, gs, first_col, last_col - first_col);
+      if (b % gs) add(m0, b % gs, last_col, 1);
+    }
+    t = stop;
+  };
+  if (t % per_group) {
+    const int next = (t / per_group + 1) * per_group;
+    inside_group(next < end ? next : end);
+  }
+  const int whole_end = end == total ? end : end / per_group * per_group;
+  if (t < whole_end) {
+    const int m0 = t / per_group * p.group_m, m1 = whole_end == total ? p.tiles_m : whole_end / per_group * p.group_m;
+    add(m0, m1 - m0, 0, p.tiles_n);
+    t = whole_end;
+  }
+  if (t < end) inside_group(end);
+}
 
 int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   using iris_host::fail;
@@ -323,24 +408,13 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   if (rc) return rc;
 
   const bool tiled = (p.mode == CCL_TWO_SHOT || p.mode == CCL_REDUCE_SCATTER);
-  const int vec_full = 16 / es;
-  // 16-byte accesses need unit-stride rows that start on 16-byte boundaries in every slot (slots are
-  // 4 KiB aligned relative to each other) and tiles that are whole chunks wide.
-  bool vec_ok = p.s_in == 1 && p.s_on == 1 && aligned16(p.in) && aligned16(p.out) &&
-                (p.s_im * es) % 16 == 0 && (p.s_om * es) % 16 == 0 && p.N % vec_full == 0;
-  if (tiled && p.bn % vec_full) vec_ok = false;
-  int vec = vec_ok ? vec_full : 1;
-  // The atomic variant adds one dword at a time (packed 16-bit pairs, or one float): with a dword per
-  // thread a wave instruction covers 256 contiguous bytes, two whole lines for the L2's atomic units;
-  // with a 16-byte chunk per thread it touched eight lines with eight dwords each and the launch ran
-  // at a third of the rate.
-  if (p.mode == CCL_ATOMIC && vec_ok) vec = es == 4 ? 1 : 2;
-
   if (tiled) {
     p.tiles_m = cdiv(p.M, p.bm);
     p.tiles_n = cdiv(p.N, p.bn);
     const long long total = (long long)p.tiles_m * p.tiles_n;
     if (total >= (1ll << 31)) return fail("too many tiles");
+    if ((long long)p.bm * p.bn >= (1ll << 31)) return fail("block sizes %d x %d are too large", p.bm, p.bn);
+    if (p.group_m > p.tiles_m) p.group_m = p.tiles_m;  // the same order
     const int per_rank = (int)((total + p.world - 1) / p.world);
     if (distribution == IRIS_HIP_DISTRIBUTION_STRIDED) {
       p.first_tile = p.group_rank;
@@ -353,11 +427,38 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
       const long long remaining = total - p.first_tile;
       p.n_owned = remaining > 0 ? (int)(remaining < per_rank ? remaining : per_rank) : 0;
     }
-  } else {
+  }
+  // Bytes that the launch moves.
+  const long long moved = (tiled ? (long long)p.n_owned * p.bm * p.bn : (long long)p.M * p.N) * es *
+                          (p.mode == CCL_TWO_SHOT ? 2 * p.world : p.world + 1);
+  const bool large = moved > (32ll << 20);
+  // Large launches of the block distribution walk their tiles' rows instead of one tile after the other.
+  const bool rows = tiled && large && p.tile_stride == 1;
+
+  // 16-byte accesses need unit-stride rows and tiles that are whole chunks wide.  Rows may start anywhere and N need
+  // not be whole chunks (bf16 8192x2881, eight ranks: one-shot 145 -> 81 us against element accesses, reduce-scatter
+  // 20 -> 12), with two exceptions.  Outputs that overlap the inputs: a last chunk that starts inside its neighbour would
+  // read what that one has just written.  Two-shot launches that go tile by tile: they store 128-byte rows to every
+  // slot, and element accesses, of which a wave instruction is one such row, are the faster ones when those are
+  // misaligned (24 us against 28).
+  const int vec_full = 16 / es;
+  const bool whole = aligned16(p.in) && aligned16(p.out) && (p.s_im * es) % 16 == 0 && (p.s_om * es) % 16 == 0 && p.N % vec_full == 0;
+  const char* const in_end = p.in + ((long long)(p.M - 1) * p.s_im + p.N) * es;
+  const char* const out_end = p.out + ((long long)(p.M - 1) * p.s_om + p.N) * es;
+  const bool apart = p.s_im >= 0 && p.s_om >= 0 && (in_end <= p.out || out_end <= p.in);
+  const bool vec_ok = p.s_in == 1 && p.s_on == 1 && !(tiled && p.bn % vec_full) &&
+                      (whole || (p.mode != CCL_ATOMIC && (p.mode != CCL_TWO_SHOT || rows) && p.N >= vec_full && apart));
+  int vec = vec_ok ? vec_full : 1;
+  // The atomic variant adds one dword at a time (packed 16-bit pairs, or one float): with a dword per
+  // thread a wave instruction covers 256 contiguous bytes, two whole lines for the L2's atomic units;
+  // with a 16-byte chunk per thread it touched eight lines with eight dwords each and the launch ran
+  // at a third of the rate.
+  if (p.mode == CCL_ATOMIC && vec_ok) vec = es == 4 ? 1 : 2;
+
+  if (!tiled) {
     // No result depends on the tile grid: stream rows in runs of up to 2048 bytes.
     p.bm = 1;
-    p.bn = p.N < 2048 / es ? p.N : 2048 / es;
-    if (p.bn % vec) p.bn = vec;  // cannot happen with vec == 1; keeps runs whole chunks otherwise
+    p.bn = p.N < 2048 / es ? cdiv(p.N, vec) * vec : 2048 / es;
     p.tiles_m = p.M;
     p.tiles_n = cdiv(p.N, p.bn);
     p.first_tile = 0;
@@ -367,9 +468,10 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
     p.n_owned = (int)total;
   }
   p.upr = cdiv(p.bn, vec);
-  if ((long long)p.upr * p.bm >= (1ll << 31)) return fail("block sizes %d x %d are too large", p.bm, p.bn);
   p.upt = p.upr * p.bm;
   p.total_units = (long long)p.n_owned * p.upt;
+  const bool by_rows = rows && vec > 1 && p.total_units < (1ll << 31);
+  if (by_rows) fill_rects(p);
 
   hipStream_t s = (hipStream_t)stream;
   char name[96];
@@ -379,34 +481,37 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   iris_host::set_last_kernel(name);
   if (p.total_units == 0) return 0;  // this rank owns nothing
 
-  // Launches that move tens of megabytes stream with non-temporal accesses and four chunks per thread:
-  // their operands are read once, and lines taken into the last-level cache for them would first have to
-  // push out whatever dirty lines it holds (a rank's two-shot share of 8 x 128 MiB after a 256 MB buffer
-  // was zeroed: 74 instead of 92 us; reduce-scatter 42 instead of 62 us; 8 x 128 MiB one-shot 5.9
-  // instead of 5.1 TB/s).  Cacheable accesses win only when the same operands are still cached from a
-  // previous launch (43 against 63 us for the two-shot share), which a collective's inputs - other
-  // ranks' fresh results - are not.  Small launches keep cacheable accesses.
-  const long long moved = p.total_units * (long long)(vec * es) * (p.world + (p.mode == CCL_TWO_SHOT ? p.world : 1));
-  const bool stream_nt = vec > 1 && p.mode != CCL_ATOMIC && moved > (32ll << 20);
-  const int upt = stream_nt ? 4 : 2;
+  // Launches that move tens of megabytes read with non-temporal accesses: their operands are read once, and lines taken
+  // into the last-level cache for them would first have to push out whatever dirty lines it holds.  Tile by tile the
+  // stores are non-temporal too and a thread takes four chunks at a time (8 x 128 MiB one-shot 5.9 instead of 5.1 TB/s); by
+  // rows it takes two and stores through the caches.  One rank's share of 8192x8192 bf16 in us, eight ranks, right after a
+  // 256 MB buffer was zeroed / back to back: two-shot tile by tile 68 / 66, by rows 55 / 47 (58 / 54 with non-temporal stores,
+  // 78 / 44 with cached reads); reduce-scatter 36 / 34 and 30 / 28 (31 / 27, 53 / 26).  Small launches keep cacheable accesses, and
+  // so do misaligned rows of tiles, whose pieces of lines the L2 has to put together (8192x2881 reduce-scatter 12 against 18).
+  const bool stream_nt = vec > 1 && large && p.mode != CCL_ATOMIC && (whole || p.mode == CCL_ONE_SHOT);
+  const int upt = stream_nt && !by_rows ? 4 : 2;
   const long long per_wg = (long long)kCclThreads * upt;
   const long long want = (p.total_units + per_wg - 1) / per_wg;
   const long long cap = (long long)cu * 8;
   const int grid = (int)(want < cap ? want : cap);
 
-#define CCL_LAUNCH(E, V)                                       \
-  do {                                                         \
-    if (stream_nt) launch_for_world<E, V, 4, true>(p, grid, s); \
-    else launch_for_world<E, V, 2, false>(p, grid, s);          \
+#define CCL_LAUNCH(E, V)                                                           \
+  do {                                                                             \
+    if (by_rows && stream_nt) launch_for_world<E, V, 2, true, true>(p, grid, s);   \
+    else if (by_rows) launch_for_world<E, V, 2, false, true>(p, grid, s);          \
+    else if (stream_nt) launch_for_world<E, V, 4, true, false>(p, grid, s);        \
+    else launch_for_world<E, V, 2, false, false>(p, grid, s);                      \
   } while (0)
+#define CCL_ELEMENTS(E) launch_for_world<E, 1, 2, false, false>(p, grid, s)
   if (vec == 2) {  // atomic variant only
-    if (dtype == IRIS_HIP_BF16) launch_for_world<ElemBF16, 2, 2, false>(p, grid, s);
-    else launch_for_world<ElemF16, 2, 2, false>(p, grid, s);
+    if (dtype == IRIS_HIP_BF16) launch_for_world<ElemBF16, 2, 2, false, false>(p, grid, s);
+    else launch_for_world<ElemF16, 2, 2, false, false>(p, grid, s);
   }
-  else if (dtype == IRIS_HIP_BF16) { if (vec == 8) CCL_LAUNCH(ElemBF16, 8); else CCL_LAUNCH(ElemBF16, 1); }
-  else if (dtype == IRIS_HIP_FP16) { if (vec == 8) CCL_LAUNCH(ElemF16, 8); else CCL_LAUNCH(ElemF16, 1); }
-  else { if (vec == 4) CCL_LAUNCH(ElemF32, 4); else CCL_LAUNCH(ElemF32, 1); }
+  else if (dtype == IRIS_HIP_BF16) { if (vec == 8) CCL_LAUNCH(ElemBF16, 8); else CCL_ELEMENTS(ElemBF16); }
+  else if (dtype == IRIS_HIP_FP16) { if (vec == 8) CCL_LAUNCH(ElemF16, 8); else CCL_ELEMENTS(ElemF16); }
+  else { if (vec == 4) CCL_LAUNCH(ElemF32, 4); else CCL_ELEMENTS(ElemF32); }
 #undef CCL_LAUNCH
+#undef CCL_ELEMENTS
   return (int)hipGetLastError();
 }
 
