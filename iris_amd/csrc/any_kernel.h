@@ -6,8 +6,9 @@
 // LDS (global loads take any alignment; the direct-to-LDS load is used only where its pieces are
 // aligned), one K step ahead in registers and one in the second LDS buffer.  The LDS layouts, the MFMA
 // operand lanes and the order of the epilogue are the same.  What bounds it: the matrix pipes for
-// float32 (64 cycles per 32x32x2 block, 157 TFLOP/s at most), the LDS for the 16- and 8-bit types (the
-// fragment reads of a 64x64 wave block need its full rate), the epilogue's HBM streams with peers.
+// float32 (as three bf16 pieces per operand, see SPLIT; 157 TFLOP/s at most on its own MFMA), the LDS for the
+// 16- and 8-bit types (the fragment reads of a 64x64 wave block need its full rate), the epilogue's HBM streams
+// with peers.
 //
 // Nothing on the hot path is predicated: rows past M (or N) repeat the last row, columns of B past N are
 // read as they lie in memory as long as the piece ends inside the operand - what they produce are output
@@ -70,9 +71,18 @@ struct AnyCfg {
   // Partial blocks of the waves along K: fp32, one 36-float row per output row, next to each other.
   static constexpr int PART_ROW = BN * 4 + 16;
   static constexpr int PART_BYTES = WK > 1 ? WK * BM * PART_ROW : 0;
+  // float32 as three bf16 pieces (where the kernel says why): a step's tiles of A and of B, three planes each.
+  // Eight waves, alone on their CU, split one step while they multiply another and need two buffers; workgroups of
+  // four share a CU and take turns.
+  static constexpr bool SPLIT = IN == IN_F32 && WK == 1;
+  static constexpr int KB16 = KE * 2;  // bytes of K per row of a plane
+  static constexpr int A_PLANE = BM * KB16, B_PLANE = BN * KB16;
+  static constexpr int SPLIT_BUF = 3 * (A_PLANE + B_PLANE), SPLIT_BYTES = !SPLIT ? 0 : NW == 8 ? 2 * SPLIT_BUF : SPLIT_BUF;
   static constexpr int SMEM0 = 2 * BUF_BYTES > TILE_BYTES ? 2 * BUF_BYTES : TILE_BYTES;
-  static constexpr int SMEM_BYTES = SMEM0 > TILE_BYTES + PART_BYTES ? SMEM0 : TILE_BYTES + PART_BYTES;
-  static constexpr int WG_PER_CU = NW == 4 ? 2 : 1;
+  static constexpr int SMEM1 = SMEM0 > TILE_BYTES + PART_BYTES ? SMEM0 : TILE_BYTES + PART_BYTES;
+  static constexpr int FLAG_OFF = SMEM1 > SPLIT_BYTES ? SMEM1 : SPLIT_BYTES;  // SPLIT: the workgroup's vote
+  static constexpr int SMEM_BYTES = FLAG_OFF + (SPLIT ? kChunkBytes : 0);
+  static constexpr int WG_PER_CU = NW != 4 ? 1 : !SPLIT ? 2 : 160 * 1024 / SMEM_BYTES < 3 ? 160 * 1024 / SMEM_BYTES : 3;
   static_assert(SMEM_BYTES * WG_PER_CU <= 160 * 1024, "LDS budget of a gfx950 CU");
   static_assert((BM * 8) % NT == 0 && (BN * 8) % NT == 0 && NT % CPR == 0, "whole pieces per thread");
 };
@@ -162,46 +172,56 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   // Consecutive threads take consecutive pieces of a row; with a strided operand consecutive rows, so that
   // a transposed A (rows one element apart) is still read in whole lines.
   const bool a_vec = p.s_ak == 1;
-  const char* a_ptr[LA];
-  int a_k[LA], a_lds[LA];
+  const char* ptr[LA + LB];  // (A's pieces first, then B's)
+  int a_k[LA], lds_at[LA + LB];
+  int f_kb, f_src;  // K step the next fetch brings
+  auto point_at_a = [&](auto split_tag) {
 #pragma unroll
-  for (int i = 0; i < LA; ++i) {
-    const int id = tid + i * NT, sub = id / (BM * 8), in_sub = id - sub * (BM * 8);
-    const int row = a_vec ? in_sub >> 3 : in_sub % BM, c = a_vec ? in_sub & 7 : in_sub / BM;
-    a_k[i] = sub * KE + c * CE;
-    a_lds[i] = sub * CFG::A_SLICE + ATile::lds_offset(row, c);
-    long long gm = min(m0 + row, p.M - 1);
-    int slot = p.gather == GATHER_K ? 0 : p.rank;
-    if (p.gather == GATHER_M) {
-      slot = (int)(gm / p.M_local);
-      gm -= (long long)slot * p.M_local;
+    for (int i = 0; i < LA; ++i) {
+      const int id = tid + i * NT, sub = id / (BM * 8), in_sub = id - sub * (BM * 8);
+      const int row = a_vec ? in_sub >> 3 : in_sub % BM, c = a_vec ? in_sub & 7 : in_sub / BM;
+      a_k[i] = sub * KE + c * CE;
+      if constexpr (decltype(split_tag)::value) lds_at[i] = RowTile<CFG::KB16>::lds_offset(row, c >> 1) + (c & 1) * 8;
+      else lds_at[i] = sub * CFG::A_SLICE + ATile::lds_offset(row, c);
+      long long gm = min(m0 + row, p.M - 1);
+      int slot = p.gather == GATHER_K ? 0 : p.rank;
+      if (p.gather == GATHER_M) {
+        slot = (int)(gm / p.M_local);
+        gm -= (long long)slot * p.M_local;
+      }
+      const char* base = p.gather == GATHER_NONE ? p.A : slot_ptr(p.heap_bases, p.A, p.rank, slot);
+      ptr[i] = base + (gm * p.s_am + (long long)a_k[i] * p.s_ak) * ES;
     }
-    const char* base = p.gather == GATHER_NONE ? p.A : slot_ptr(p.heap_bases, p.A, p.rank, slot);
-    a_ptr[i] = base + (gm * p.s_am + (long long)a_k[i] * p.s_ak) * ES;
-  }
+    f_kb = f_src = 0;
+  };
   const bool b_vec = !CFG::BKC || p.s_bk == 1;
-  const char* b_ptr[LB];
-  int b_k[LB], b_lds[LB];
-  int b_cols = CE;  // [k][n] tile: columns of this thread's piece that exist
+  int b_k[LB];
+  int b_cols;  // [k][n] tile: columns of this thread's piece that exist
+  auto point_at_b = [&](auto split_tag) {
+    constexpr bool SPLIT = decltype(split_tag)::value;
+    b_cols = CE;
 #pragma unroll
-  for (int i = 0; i < LB; ++i) {
-    const int id = tid + i * NT;
-    if constexpr (CFG::BKC) {
-      const int sub = id / (BN * 8), in_sub = id - sub * (BN * 8);
-      const int row = b_vec ? in_sub >> 3 : in_sub % BN, c = b_vec ? in_sub & 7 : in_sub / BN;
-      b_k[i] = sub * KE + c * CE;
-      b_lds[i] = CFG::A_BYTES + sub * CFG::B_SLICE + ATile::lds_offset(row, c);
-      b_ptr[i] = p.B + ((long long)min(n0 + row, p.N - 1) * p.s_bn + (long long)b_k[i] * p.s_bk) * ES;
-    } else {
-      const int krow = id / CFG::CPR, c = id % CFG::CPR, sub = krow / KE;
-      b_k[i] = krow;
-      b_lds[i] = CFG::A_BYTES + sub * CFG::B_SLICE + AnyColTile<CFG::RBB, ES>::lds_offset(krow - sub * KE, c);
-      const int gn = n0 + c * CE;
-      b_cols = p.N - gn;
-      b_ptr[i] = p.B + ((long long)krow * p.s_bk + (gn < p.N ? gn : 0)) * ES;  // pieces past N: any columns do
+    for (int i = 0; i < LB; ++i) {
+      const int id = tid + i * NT;
+      if constexpr (CFG::BKC) {
+        const int sub = id / (BN * 8), in_sub = id - sub * (BN * 8);
+        const int row = b_vec ? in_sub >> 3 : in_sub % BN, c = b_vec ? in_sub & 7 : in_sub / BN;
+        b_k[i] = sub * KE + c * CE;
+        if constexpr (SPLIT) lds_at[LA + i] = 3 * CFG::A_PLANE + RowTile<CFG::KB16>::lds_offset(row, c >> 1) + (c & 1) * 8;
+        else lds_at[LA + i] = CFG::A_BYTES + sub * CFG::B_SLICE + ATile::lds_offset(row, c);
+        ptr[LA + i] = p.B + ((long long)min(n0 + row, p.N - 1) * p.s_bn + (long long)b_k[i] * p.s_bk) * ES;
+      } else {
+        const int krow = id / CFG::CPR, c = id % CFG::CPR, sub = krow / KE;
+        b_k[i] = krow;
+        if constexpr (SPLIT) lds_at[LA + i] = 3 * CFG::A_PLANE + ColTile<BN * 2, 2>::lds_offset(krow, c >> 1) + (c & 1) * 8;
+        else lds_at[LA + i] = CFG::A_BYTES + sub * CFG::B_SLICE + AnyColTile<CFG::RBB, ES>::lds_offset(krow - sub * KE, c);
+        const int gn = n0 + c * CE;
+        b_cols = p.N - gn;
+        ptr[LA + i] = p.B + ((long long)krow * p.s_bk + (gn < p.N ? gn : 0)) * ES;  // pieces past N: any columns do
+      }
     }
-  }
-  if (b_cols <= 0 || b_cols > CE) b_cols = CE;
+    if (b_cols <= 0 || b_cols > CE) b_cols = CE;
+  };
   // One past the last byte of B ([k][n]); a piece that ends beyond it is loaded element by element.  With rows
   // at least a piece apart only a piece of the last row can.
   const char* const b_end = p.B + ((long long)(p.K - 1) * p.s_bk + p.N) * ES;
@@ -225,33 +245,12 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   };
 
   const long long a_step = (long long)CFG::KSTEP * p.s_ak * ES, b_step = (long long)CFG::KSTEP * p.s_bk * ES;
-  int f_kb = 0, f_src = 0;  // K step the next fetch brings
-  u32x4_t ra[LA], rb[LB];
-  auto fetch = [&]() {
-    const int left = klocal - f_kb * CFG::KSTEP;  // elements of K from this step on
-    if (left >= CFG::KSTEP && a_vec) {
-#pragma unroll
-      for (int i = 0; i < LA; ++i) ra[i] = load16_any(a_ptr[i]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < LA; ++i)
-        ra[i] = a_vec && a_k[i] + CE <= left ? load16_any(a_ptr[i]) : load_elements(a_ptr[i], p.s_ak * ES, left - a_k[i]);
-    }
-    if (left >= CFG::KSTEP && b_vec && f_src * klocal + (f_kb + 1) * CFG::KSTEP <= b_safe_k) {
-#pragma unroll
-      for (int i = 0; i < LB; ++i) rb[i] = load16_any(b_ptr[i]);
-    } else if constexpr (CFG::BKC) {
-#pragma unroll
-      for (int i = 0; i < LB; ++i)
-        rb[i] = b_vec && b_k[i] + CE <= left ? load16_any(b_ptr[i]) : load_elements(b_ptr[i], p.s_bk * ES, left - b_k[i]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < LB; ++i) {
-        if (b_k[i] >= left) rb[i] = (u32x4_t){0u, 0u, 0u, 0u};
-        else if (b_ptr[i] + 16 <= b_end) rb[i] = load16_any(b_ptr[i]);
-        else rb[i] = load_elements(b_ptr[i], ES, min(b_cols, p.N));
-      }
-    }
+  u32x4_t raw[LA + LB];
+  // Whether the next fetch brings nothing but whole pieces.
+  auto plain = [&]() {
+    return a_vec && b_vec && klocal - f_kb * CFG::KSTEP >= CFG::KSTEP && f_src * klocal + (f_kb + 1) * CFG::KSTEP <= b_safe_k;
+  };
+  auto advance = [&]() {
     long long da = a_step, db = b_step;
     if (++f_kb == nkb) {  // on to the next source's columns
       f_kb = 0;
@@ -261,16 +260,43 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
       if (f_src < nsrc) da += p.heap_bases[f_src] - p.heap_bases[f_src - 1];
     }
 #pragma unroll
-    for (int i = 0; i < LA; ++i) a_ptr[i] += da;
+    for (int i = 0; i < LA; ++i) ptr[i] += da;
 #pragma unroll
-    for (int i = 0; i < LB; ++i) b_ptr[i] += db;
+    for (int i = 0; i < LB; ++i) ptr[LA + i] += db;
+  };
+  auto fetch = [&]() {
+    const int left = klocal - f_kb * CFG::KSTEP;  // elements of K from this step on
+    if (left >= CFG::KSTEP && a_vec) {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) raw[i] = load16_any(ptr[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < LA; ++i)
+        raw[i] = a_vec && a_k[i] + CE <= left ? load16_any(ptr[i]) : load_elements(ptr[i], p.s_ak * ES, left - a_k[i]);
+    }
+    if (left >= CFG::KSTEP && b_vec && f_src * klocal + (f_kb + 1) * CFG::KSTEP <= b_safe_k) {
+#pragma unroll
+      for (int i = 0; i < LB; ++i) raw[LA + i] = load16_any(ptr[LA + i]);
+    } else if constexpr (CFG::BKC) {
+#pragma unroll
+      for (int i = 0; i < LB; ++i)
+        raw[LA + i] = b_vec && b_k[i] + CE <= left ? load16_any(ptr[LA + i]) : load_elements(ptr[LA + i], p.s_bk * ES, left - b_k[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        if (b_k[i] >= left) raw[LA + i] = (u32x4_t){0u, 0u, 0u, 0u};
+        else if (ptr[LA + i] + 16 <= b_end) raw[LA + i] = load16_any(ptr[LA + i]);
+        else raw[LA + i] = load_elements(ptr[LA + i], ES, min(b_cols, p.N));
+      }
+    }
+    advance();
   };
   auto put = [&](int buf) {
     char* const s = smem + buf * CFG::BUF_BYTES;
 #pragma unroll
-    for (int i = 0; i < LA; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + a_lds[i]) = ra[i];
+    for (int i = 0; i < LA; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + lds_at[i]) = raw[i];
 #pragma unroll
-    for (int i = 0; i < LB; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + b_lds[i]) = rb[i];
+    for (int i = 0; i < LB; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + lds_at[LA + i]) = raw[LA + i];
   };
 
   // ---- fragments ------------------------------------------------------------------------------------------
@@ -324,12 +350,14 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     }
   };
   f32x16_t acc[MB][NB];
+  auto clear_sums = [&]() {
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+        for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+  };
   auto multiply = [&](const Frag& f) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -358,25 +386,203 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   // ---- K loop ---------------------------------------------------------------------------------------------
   // Step s reads LDS buffer s & 1; meanwhile step s+1 arrives in registers, is put into the other buffer half
   // way through the step's products, and the loads of step s+2 go out.
-  fetch();
-  put(0);
-  if (nsteps > 1) fetch();
-  lds_barrier();
-  PHASE_STAMP(1);
-  for (int s = 0; s < nsteps; ++s) {
-    const int buf = s & 1;
-    Frag f[2];
-    load_frag(f[0], buf, 0);
-#pragma unroll
-    for (int kk = 0; kk < KS; ++kk) {
-      if (kk + 1 < KS) load_frag(f[(kk + 1) & 1], buf, kk + 1);
-      multiply(f[kk & 1]);
-      if (kk == KS / 2 - 1 && s + 1 < nsteps) {
-        put(buf ^ 1);
-        if (s + 2 < nsteps) fetch();
-      }
-    }
+  auto k_loop = [&]() {
+    point_at_a(std::false_type{});
+    point_at_b(std::false_type{});
+    clear_sums();
+    fetch();
+    put(0);
+    if (nsteps > 1) fetch();
     lds_barrier();
+    PHASE_STAMP(1);
+    for (int s = 0; s < nsteps; ++s) {
+      const int buf = s & 1;
+      Frag f[2];
+      load_frag(f[0], buf, 0);
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+        if (kk + 1 < KS) load_frag(f[(kk + 1) & 1], buf, kk + 1);
+        multiply(f[kk & 1]);
+        if (kk == KS / 2 - 1 && s + 1 < nsteps) {
+          put(buf ^ 1);
+          if (s + 2 < nsteps) fetch();
+        }
+      }
+      lds_barrier();
+    }
+  };
+
+  if constexpr (!CFG::SPLIT) {
+    k_loop();
+  } else {
+    // float32 on the bf16 matrix pipes.  A float of at least 2^-110 (or zero) is the exact sum of three bf16
+    // numbers: the value rounded to eight bits, the remainder rounded, and the rest, which fits.  Six of the nine
+    // products of the pieces are added up (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the others are at
+    // most 2^-24 of the product and 2^-27 of it in the mean, below the rounding of one fp32 addition.  The sums are
+    // fp32, with six additions per 16 k instead of sixteen.  Error against 64 bits, 2-norm, normal operands,
+    // float32 MFMA -> three pieces: K = 512 4.1e-7 -> 3.5e-7, 1024 5.7e-7 -> 4.9e-7, 8192 1.62e-6 -> 1.44e-6.
+    // What the pieces cannot represent is left to the float32 MFMA, tile by tile: a nonzero operand below
+    // 2^-110 (found while splitting), and tiles with a sum that is not finite (infinities and NaN, and values
+    // that round to infinity in bf16), whose pieces need not add up to what the operands do.
+    // The pieces are formed once per workgroup on the way from registers to LDS, 7 VALU instructions per
+    // element.  What bounds it: the matrix pipes at the clock they hold under load (4096x4096x1536 in 282 us
+    // is 1.1 PFLOP/s of bf16 products, the bf16 tile kernel reaches 1.2-1.4); 137 -> 183 TFLOP/s of
+    // float32.  With the smaller tiles the LDS (6 bytes written per element, 9 KiB read per 12 products of a
+    // 32x64 wave block) and the splitting weigh as much: 2048x2880x1024 110 -> 98 us.
+    LDS_AS int* const vote = (LDS_AS int*)(LDS_AS char*)(smem + CFG::FLAG_OFF);
+    if (tid == 0) *vote = 0;
+    lds_barrier();
+    constexpr unsigned kSmallest = ((127u - 110u) << 24) - 1u;  // 2^-110, in the form of `low`
+    unsigned low = ~0u;  // smallest magnitude of a nonzero element: its bits without the sign, doubled, less one
+    // One of the six parts of the splitting of a 16-byte piece v, in which v is left as the remainder:
+    // elements 2 * (part & 1) and the next, plane part / 2.
+    auto split_part = [&](u32x4_t& v, u32x2_t (&w)[3], int part) {
+      const int e = 2 * (part & 1), i = part / 2;
+      if (i == 0) low = min(low, min((v[e] << 1) - 1u, (v[e + 1] << 1) - 1u));
+      const float x = __uint_as_float(v[e]), y = __uint_as_float(v[e + 1]);
+      const unsigned h = pack_bf16(x, y);
+      w[i][part & 1] = h;
+      if (i < 2) {
+        v[e] = __float_as_uint(x - __uint_as_float(h << 16));
+        v[e + 1] = __float_as_uint(y - __uint_as_float(h & 0xFFFF0000u));
+      }
+    };
+    auto put_plane = [&](const u32x2_t (&w)[3], int at, int plane, int i) {
+      *(LDS_AS u32x2_t*)(LDS_AS char*)(smem + at + i * plane) = w[i];
+    };
+    auto put_split = [&](u32x4_t& v, int at, int plane) {
+      u32x2_t w[3];
+#pragma unroll
+      for (int part = 0; part < 6; ++part) split_part(v, w, part);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) put_plane(w, at, plane, i);
+    };
+    struct Pieces {
+      i32x4_t a[MB][1], b[NB][1];
+    };
+    auto load_pieces = [&](Pieces& f, int buf, int kk, int i) {  // plane i of k-slice kk
+      const char* const sa = smem + buf * CFG::SPLIT_BUF + i * CFG::A_PLANE;
+      const char* const sb = smem + buf * CFG::SPLIT_BUF + 3 * CFG::A_PLANE + i * CFG::B_PLANE;
+      const int c = frag16_chunk(lane, kk);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        f.a[mb][0] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sa + RowTile<CFG::KB16>::lds_offset(wm * CFG::TM + frag16_row(lane), c) + mb * 32 * CFG::KB16);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        if constexpr (CFG::BKC) {
+          f.b[nb][0] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sb + RowTile<CFG::KB16>::lds_offset(wn * CFG::TN + frag16_row(lane), c) + nb * 32 * CFG::KB16);
+        } else {
+          const int n = wn * CFG::TN + nb * 32 + tr16_ncol(lane);
+          i32x2_t t[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            t[j] = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (LDS_AS i16x4_t*)(LDS_AS char*)(sb + ColTile<BN * 2, 2>::lds_offset(tr16_krow(lane, kk, j), n / 8) + (n % 8) * 2)));
+          f.b[nb][0] = (i32x4_t){t[0].x, t[0].y, t[1].x, t[1].y};
+        }
+      }
+    };
+    // Eight waves: the products of the step in buffer `buf`.  Between them, in parts of five to seven instructions that
+    // issue in the shadow of a product, the step that has arrived in registers is split and put into the
+    // other buffer, and the loads of the step after it go out.
+    constexpr int kPairs[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};  // the smallest products first
+    constexpr int KS16 = CFG::KE / 16, NMUL = KS16 * 6 * MB * NB, PARTS = 6 * (LA + LB);
+    auto step = [&](int buf, auto fetch_tag) {
+      const int to = (buf ^ 1) * CFG::SPLIT_BUF;
+      Pieces f[KS16][3];
+      u32x2_t w[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) load_pieces(f[0][i], buf, 0, i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < NMUL; ++m) {
+        const int kk = m / (6 * MB * NB), t = m / (MB * NB) % 6, mb = m / NB % MB, nb = m % NB;
+        acc[mb][nb] = mfma_block<IN_BF16, 1>(f[kk][kPairs[t][0]].a[mb], f[kk][kPairs[t][1]].b[nb], acc[mb][nb]);
+        if (kk + 1 < KS16 && m % (2 * MB * NB) == 0) load_pieces(f[kk + 1][t / 2], buf, kk + 1, t / 2);
+#pragma unroll
+        for (int j = 0; j <= PARTS / NMUL; ++j) {
+          const int q = (m * PARTS + NMUL - 1) / NMUL + j;
+          if (q * NMUL / PARTS != m || q >= PARTS) continue;
+          const int i = q / 6, part = q % 6;
+          split_part(raw[i], w, part);
+          if (part & 1) put_plane(w, to + lds_at[i], i < LA ? CFG::A_PLANE : CFG::B_PLANE, part / 2);
+          if (decltype(fetch_tag)::value && part == 5) raw[i] = load16_any(ptr[i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    bool redo = false;
+    point_at_a(std::true_type{});
+    point_at_b(std::true_type{});
+    clear_sums();
+    int s = 0;
+    bool stop = false;
+    auto close_step = [&]() {
+      if (s + 1 < nsteps && low < kSmallest) *vote = 1;
+      lds_barrier();
+      stop = (s & 7) == 7 && *vote != 0;  // (the same answer for everybody: nobody writes before the next barrier)
+      ++s;
+    };
+    fetch();
+    if constexpr (CFG::NW == 8) {
+#pragma unroll
+      for (int i = 0; i < LA + LB; ++i) put_split(raw[i], lds_at[i], i < LA ? CFG::A_PLANE : CFG::B_PLANE);
+      if (nsteps > 1) fetch();
+      lds_barrier();
+      PHASE_STAMP(1);
+      while (s < nsteps && !stop) {
+        // Steps that fetch whole pieces have a loop of their own: where a general fetch can reach the next step's
+        // splitting, the compiler waits there for every load at once.
+        while (!stop && s + 2 < nsteps && plain()) {
+          step(s & 1, std::true_type{});
+          advance();
+          close_step();
+        }
+        if (stop || s >= nsteps) break;
+        step(s & 1, std::false_type{});  // (behind the last step the pieces in registers are put down again, where nobody reads them)
+        if (s + 2 < nsteps) fetch();
+        close_step();
+      }
+    } else {
+      while (s < nsteps && !stop) {
+        if (s > 0) lds_barrier();
+#pragma unroll
+        for (int i = 0; i < LA + LB; ++i) put_split(raw[i], lds_at[i], i < LA ? CFG::A_PLANE : CFG::B_PLANE);
+        if (low < kSmallest) *vote = 1;
+        if (s + 1 < nsteps) fetch();
+        lds_barrier();
+        if (s == 0) PHASE_STAMP(1);
+        stop = (s & 7) == 7 && *vote != 0;
+#pragma unroll
+        for (int kk = 0; kk < KS16; ++kk) {
+          Pieces f[3];
+#pragma unroll
+          for (int i = 0; i < 3; ++i) load_pieces(f[i], 0, kk, i);
+#pragma unroll
+          for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+              for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mfma_block<IN_BF16, 1>(f[kPairs[t][0]].a[mb], f[kPairs[t][1]].b[nb], acc[mb][nb]);
+        }
+        ++s;
+      }
+      lds_barrier();
+    }
+    // The vote: sums of elements that exist, and what the splitting saw.
+    bool finite = true;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const bool there = n0 + wn * CFG::TN + nb * 32 + acc_row(lane, i) < p.N;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) finite = finite && (!there || __builtin_fabsf(acc[mb][nb][i]) <= 3.402823466e38f);
+      }
+    if (!finite) *vote = 1;
+    lds_barrier();
+    redo = *vote;
+    if (redo) k_loop();
   }
 
   PHASE_STAMP(2);
@@ -603,7 +809,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   auto reduce = [&](auto np_tag) {
     constexpr int NP = decltype(np_tag)::value;  // peers, all of whose loads go out together; 0: any number
     constexpr int NPV = NP > 0 ? NP : 1;
-    constexpr int G = PASSES % 2 == 0 ? 2 : 1;  // passes whose loads are in flight together
+    // Passes whose loads are in flight together: as many as the registers hold (the sums are staged and their
+    // accumulators free), every group of passes is a round trip to memory.
+    constexpr int kInFlight = CFG::NW == 8 ? 16 : 14;  // 16-byte pieces per thread; with more, fewer workgroups share a CU
+    constexpr int G = PASSES % 8 == 0 && 8 * NPV <= kInFlight ? 8 : PASSES % 4 == 0 && 4 * NPV <= kInFlight ? 4 : PASSES % 2 == 0 ? 2 : 1;
     for (int pg = 0; pg < PASSES; pg += G) {
       if (m0 + pg * RPP >= p.M) break;
       bool act[G];
@@ -705,27 +914,30 @@ int launch_any(FusedParams p, int device, int cu_count, hipStream_t stream, cons
 }
 
 // Tile choice: the tile with the least expected time, area x (tiles the busiest CU gets) / rate.  The rates (TFLOP/s, plain
-// GEMM 4095x4095x4095 bf16 and 4096x4096x4096 float32, every CU busy) fall with the tile because LDS reads and
-// operand bytes per flop rise; for float32 they hardly do, the matrix pipes are the bound.  A CU with a single
+// GEMM 4095x4095x4095 bf16 and 4096x4096x1536 float32, every CU busy) fall with the tile because LDS reads, operand
+// bytes and splitting per flop rise; the 32x32 tile of float32 multiplies on the float32 MFMA.  A CU with a single
 // workgroup of four waves has nothing to run while it waits (bf16 1024x4095x2049 on 256 tiles of 128x128: 40 us, where
 // the full rate would give 26).  Checked against forced tiles, us for 256x256 / 128x128 / 64x128 / 64x64 / 32x32, the
-// choice first: bf16 1999x2877x1371 64x128 41 (53 / 40 / - / 51 / 119), 1024x4095x2049 64x128 38 (68 / 40 / - / 48 / 105),
+// choice first (float32: 256x128 in the place of 256x256): bf16 1999x2877x1371 64x128 41 (53 / 40 / - / 51 / 119), 1024x4095x2049 64x128 38 (68 / 40 / - / 48 / 105),
 // one-shot with seven peers 500x2877x1371 64x64 30 (92 / 46 / 32 / - / 51), 33x2877x1371 32x32 13 (49 / 31 / 25 / 20 / -); float32
-// 2048x2880x1024 64x128 106 (- / 133 / - / 109 / 159), 511x2880x1024 32x32 43 (- / 77 / 45 / 40 / -).
+// 2048x2880x1024 64x128 98 (97 / 108 / - / 113 / 174), 4096x2048x1024 256x128 98 (- / 112 / 123 / 134 / 224), 2048x2048x4096
+// 128x128 199 (275 / - / 236 / 260 / 381), 512x2880x1024 64x64 40 (77 / 47 / 45 / - / 44), 300x4096x4096 32x32 129 (267 / 159 /
+// 153 / 138 / -), 1536x2880x1024 64x64 87 (79 / 100 / 80 / - / 121).
 struct AnyTile {
   int bm, bn;
-  float rate16, rate32;
+  float rate;
 };
-constexpr AnyTile kAnyTiles[] = {{256, 256, 855.f, 0.f}, {128, 128, 654.f, 137.f}, {64, 128, 508.f, 131.f}, {64, 64, 395.f, 127.f}, {32, 32, 195.f, 98.f}};
+constexpr AnyTile kAnyTiles[] = {{256, 256, 855.f}, {128, 128, 654.f}, {64, 128, 508.f}, {64, 64, 395.f}, {32, 32, 195.f}};
+constexpr AnyTile kAnyTilesF32[] = {{256, 128, 183.f}, {128, 128, 163.f}, {64, 128, 160.f}, {64, 64, 140.f}, {32, 32, 98.f}};  // the first two of eight waves
 
 inline int choose_any_tile(int M, int N, int cu, bool f32_in, bool f32_out) {
   int best = 1;
   float best_time = 0.f;
-  for (int i = f32_in || f32_out ? 1 : 0; i < 5; ++i) {
-    const AnyTile& t = kAnyTiles[i];
+  for (int i = f32_out && !f32_in ? 1 : 0; i < 5; ++i) {
+    const AnyTile& t = f32_in ? kAnyTilesF32[i] : kAnyTiles[i];
     const long long per_cu = ((long long)cdiv(M, t.bm) * cdiv(N, t.bn) + cu - 1) / cu;
-    const float alone = i == 0 || per_cu > 1 ? 1.f : f32_in ? 1.15f : 1.5f;
-    const float time = (float)t.bm * t.bn * per_cu * alone / (f32_in ? t.rate32 : t.rate16);
+    const float alone = i == 0 || per_cu > 1 || (f32_in && i == 1) ? 1.f : f32_in ? 1.15f : 1.5f;
+    const float time = (float)t.bm * t.bn * per_cu * alone / t.rate;
     if (best_time == 0.f || time < best_time) {
       best = i;
       best_time = time;
@@ -739,13 +951,14 @@ int dispatch_any_layout(const FusedParams& p, int device, int cu, hipStream_t s,
   constexpr bool F32_IN = AnyIn<IN>::ES == 4, F32_OUT = Out::size == 4;
   switch (choose_any_tile(p.M, p.N, cu, F32_IN, F32_OUT)) {
     case 0:  // (a staged 256x256 tile of float32 would not fit the LDS)
-      if constexpr (!F32_OUT) return launch_any<AnyCfg<IN, Out, 256, 256, 2, 4, 1, BKC>>(p, device, cu, s, types);
+      if constexpr (F32_IN) return launch_any<AnyCfg<IN, Out, 256, 128, 4, 2, 1, BKC>>(p, device, cu, s, types);
+      else if constexpr (!F32_OUT) return launch_any<AnyCfg<IN, Out, 256, 256, 2, 4, 1, BKC>>(p, device, cu, s, types);
       break;
     case 2: return launch_any<AnyCfg<IN, Out, 64, 128, 2, 2, 1, BKC>>(p, device, cu, s, types);
     case 3: return launch_any<AnyCfg<IN, Out, 64, 64, 2, 2, 1, BKC>>(p, device, cu, s, types);
     case 4: return launch_any<AnyCfg<IN, Out, 32, 32, 1, 1, 4, BKC>>(p, device, cu, s, types);
   }
-  return launch_any<AnyCfg<IN, Out, 128, 128, 2, 2, 1, BKC>>(p, device, cu, s, types);
+  return launch_any<AnyCfg<IN, Out, 128, 128, 2, F32_IN ? 4 : 2, 1, BKC>>(p, device, cu, s, types);
 }
 
 // The layout of B in LDS follows its unit stride: [k][n] when N is contiguous, else [n][k].
