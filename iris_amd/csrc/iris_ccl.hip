@@ -51,10 +51,7 @@ struct CclParams {
   int upr, upt;
   long long total_units;
   // A contiguous run of owned tiles as rectangles of tiles, each walked row by row over its whole width (ROWS builds).
-  struct Rect {
-    int pm0, pn0, width;  // first tile row and column, units per row
-    long long base;       // unit index of the rectangle's first unit
-  } rect[5];
+  RowRect rect[kMaxRowRects];
   int n_rects;
 };
 
@@ -225,22 +222,9 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
       }
       int pm, pn;
       if constexpr (ROWS) {
-        int pm0 = p.rect[0].pm0, pn0 = p.rect[0].pn0, width = p.rect[0].width;
-        long long first_unit = 0;
-#pragma unroll
-        for (int i = 1; i < 5; ++i) {
-          if (i < p.n_rects && gg >= p.rect[i].base) {
-            pm0 = p.rect[i].pm0, pn0 = p.rect[i].pn0, width = p.rect[i].width;
-            first_unit = p.rect[i].base;
-          }
-        }
         // (the host keeps launches of 2^31 units and more on the other path)
-        const unsigned in_rect = (unsigned)(gg - first_unit), r = in_rect / (unsigned)width, across = in_rect - r * (unsigned)width;
-        pm = pm0 + (int)(r / (unsigned)p.bm);
-        pn = pn0 + (int)(across / (unsigned)p.upr);
-        c = (int)(r % (unsigned)p.bm) * p.upr + (int)(across % (unsigned)p.upr);
-        const int first_m = pm / p.group_m * p.group_m;  // the inverse of grouped_coords
-        j = first_m * p.tiles_n + pn * min(p.tiles_m - first_m, p.group_m) + pm - first_m - p.first_tile;
+        row_rect_unit(p.rect, p.n_rects, gg, p.bm, p.upr, pm, pn, c);
+        j = grouped_tile_id(pm, pn, p.tiles_m, p.tiles_n, p.group_m) - p.first_tile;
         start[u] = (j % p.comm_sms) % W;
       } else if (tiled) {
         grouped_coords(p.first_tile + j * p.tile_stride, p.tiles_m, p.tiles_n, p.group_m, pm, pn);
@@ -345,45 +329,6 @@ void launch_for_world(const CclParams& p, int grid, hipStream_t s) {
 
 bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
-// The owned tiles of the block distribution are consecutive in the grouped order: the rest of a column, some columns of
-// a group, whole groups, and the mirror image at the end - at most five rectangles.  Walked row by row, a workgroup
-// moves kilobytes of every row instead of tiles' 128-byte rows (bf16 8192x2880 two-shot, eight ranks: 22.2 -> 19.8 us).
-void fill_rects(CclParams& p) {
-  long long base = 0;
-  auto add = [&](int pm0, int rows, int pn0, int cols) {
-    if (rows <= 0 || cols <= 0) return;
-    p.rect[p.n_rects++] = {pm0, pn0, cols * p.upr, base};
-    base += (long long)rows * p.bm * cols * p.upr;
-  };
-  const int per_group = p.group_m * p.tiles_n, total = p.tiles_m * p.tiles_n;
-  const int end = p.first_tile + p.n_owned;
-  int t = p.first_tile;
-  auto inside_group = [&](int stop) {  // tiles [t, stop) of one group
-    const int m0 = t / per_group * p.group_m, gs = p.tiles_m - m0 < p.group_m ? p.tiles_m - m0 : p.group_m;
-    const int a = t - m0 * p.tiles_n, b = stop - m0 * p.tiles_n;  // positions in the group, column by column
-    const int first_col = cdiv(a, gs), last_col = b / gs;          // whole columns [first_col, last_col)
-    if (first_col > last_col) {                                     // all in one column
-      add(m0 + a % gs, b - a, a / gs, 1);
-    } else {
-      if (a % gs) add(m0 + a % gs, gs - a % gs, a / gs, 1);
-      add(m0, gs, first_col, last_col - first_col);
-      if (b % gs) add(m0, b % gs, last_col, 1);
-    }
-    t = stop;
-  };
-  if (t % per_group) {
-    const int next = (t / per_group + 1) * per_group;
-    inside_group(next < end ? next : end);
-  }
-  const int whole_end = end == total ? end : end / per_group * per_group;
-  if (t < whole_end) {
-    const int m0 = t / per_group * p.group_m, m1 = whole_end == total ? p.tiles_m : whole_end / per_group * p.group_m;
-    add(m0, m1 - m0, 0, p.tiles_n);
-    t = whole_end;
-  }
-  if (t < end) inside_group(end);
-}
-
 int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   using iris_host::fail;
   iris_host::clear_last_error();
@@ -471,7 +416,7 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   p.upt = p.upr * p.bm;
   p.total_units = (long long)p.n_owned * p.upt;
   const bool by_rows = rows && vec > 1 && p.total_units < (1ll << 31);
-  if (by_rows) fill_rects(p);
+  if (by_rows) p.n_rects = row_rects(p.rect, p.first_tile, p.n_owned, p.tiles_m, p.tiles_n, p.group_m, p.bm, p.upr);
 
   hipStream_t s = (hipStream_t)stream;
   char name[96];

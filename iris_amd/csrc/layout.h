@@ -301,4 +301,79 @@ IRIS_HD bool decode_offsets_fit(long long a_rows, long long s_am, long long K, i
   return a_rows > 0 && s_am >= 0 && s_cm >= 0 && a_last < limit && c_last < limit;
 }
 
+// ---------------------------------------------------------------------------------------------
+// Stand-alone collectives: a consecutive run of tiles of the grouped order (groups of group_m tile rows walked column
+// by column) is the rest of a column, some columns of a group, whole groups, and the mirror image at the end - at most
+// five rectangles.  Walked row by row, a workgroup moves kilobytes of every row instead of tiles' 128-byte rows (bf16
+// 8192x2880 two-shot, eight ranks: 22.2 -> 19.8 us).
+// ---------------------------------------------------------------------------------------------
+struct RowRect {
+  int pm0, pn0, width;  // first tile row and column, units per row
+  long long base;       // index of the rectangle's first unit
+};
+constexpr int kMaxRowRects = 5;
+
+// The rectangles of tiles [first, first + n) of a tiles_m x tiles_n grid, group_m <= tiles_m; a tile has bm rows of upr
+// units.  Returns how many there are.
+inline int row_rects(RowRect (&rect)[kMaxRowRects], int first, int n, int tiles_m, int tiles_n, int group_m, int bm, int upr) {
+  int count = 0;
+  long long base = 0;
+  auto add = [&](int pm0, int rows, int pn0, int cols) {
+    if (rows <= 0 || cols <= 0) return;
+    rect[count++] = {pm0, pn0, cols * upr, base};
+    base += (long long)rows * bm * cols * upr;
+  };
+  const int per_group = group_m * tiles_n, total = tiles_m * tiles_n;
+  const int end = first + n;
+  int t = first;
+  auto inside_group = [&](int stop) {  // tiles [t, stop) of one group
+    const int m0 = t / per_group * group_m, gs = tiles_m - m0 < group_m ? tiles_m - m0 : group_m;
+    const int a = t - m0 * tiles_n, b = stop - m0 * tiles_n;  // positions in the group, column by column
+    const int first_col = (a + gs - 1) / gs, last_col = b / gs;  // whole columns [first_col, last_col)
+    if (first_col > last_col) {                                  // all in one column
+      add(m0 + a % gs, b - a, a / gs, 1);
+    } else {
+      if (a % gs) add(m0 + a % gs, gs - a % gs, a / gs, 1);
+      add(m0, gs, first_col, last_col - first_col);
+      if (b % gs) add(m0, b % gs, last_col, 1);
+    }
+    t = stop;
+  };
+  if (t % per_group) {
+    const long long next = ((long long)t / per_group + 1) * per_group;
+    inside_group(next < end ? (int)next : end);
+  }
+  const int whole_end = end == total ? end : end / per_group * per_group;
+  if (t < whole_end) {
+    const int m0 = t / per_group * group_m, m1 = whole_end == total ? tiles_m : whole_end / per_group * group_m;
+    add(m0, m1 - m0, 0, tiles_n);
+    t = whole_end;
+  }
+  if (t < end) inside_group(end);
+  return count;
+}
+
+// Tile (pm, pn) and unit inside it of unit g, for fewer than 2^31 units.
+IRIS_HD void row_rect_unit(const RowRect (&rect)[kMaxRowRects], int n_rects, long long g, int bm, int upr, int& pm, int& pn, int& unit) {
+  int pm0 = rect[0].pm0, pn0 = rect[0].pn0, width = rect[0].width;
+  long long first_unit = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxRowRects; ++i) {
+    if (i < n_rects && g >= rect[i].base) {
+      pm0 = rect[i].pm0, pn0 = rect[i].pn0, width = rect[i].width;
+      first_unit = rect[i].base;
+    }
+  }
+  const unsigned in_rect = (unsigned)(g - first_unit), r = in_rect / (unsigned)width, across = in_rect - r * (unsigned)width;
+  pm = pm0 + (int)(r / (unsigned)bm);
+  pn = pn0 + (int)(across / (unsigned)upr);
+  unit = (int)(r % (unsigned)bm) * upr + (int)(across % (unsigned)upr);
+}
+
+// Position of a tile in the grouped order.
+IRIS_HD int grouped_tile_id(int pm, int pn, int tiles_m, int tiles_n, int group_m) {
+  const int first_m = pm / group_m * group_m, gs = tiles_m - first_m < group_m ? tiles_m - first_m : group_m;
+  return first_m * tiles_n + pn * gs + pm - first_m;
+}
+
 }  // namespace iris_layout

@@ -336,6 +336,35 @@ void check_split_plan() {
   CHECK(split_plan(16, 32, 16).per_tile == 0, "16 K steps: the partial sum costs more than it saves");
 }
 
+// ---- row walk of the collectives -------------------------------------------------------------------
+// Units walked by rectangles are exactly the units of the owned tiles, each once, and lead back to their tile's id:
+// every grid of up to 7 x 6 tiles, every group height, every run of tiles.
+void check_row_rects() {
+  for (int tm = 1; tm <= 7; ++tm)
+    for (int tn = 1; tn <= 6; ++tn)
+      for (int g = 1; g <= tm; ++g) {
+        std::vector<std::pair<int, int>> tile;  // the grouped order, written down
+        for (int m0 = 0; m0 < tm; m0 += g)
+          for (int n = 0; n < tn; ++n)
+            for (int m = m0; m < tm && m < m0 + g; ++m) tile.push_back({m, n});
+        for (int first = 0; first < tm * tn; ++first)
+          for (int n = 1; first + n <= tm * tn; ++n) {
+            const int bm = 1 + (first + n) % 3, upr = 1 + n % 3, upt = bm * upr;
+            RowRect rect[kMaxRowRects];
+            const int count = row_rects(rect, first, n, tm, tn, g, bm, upr);
+            CHECK(count >= 1 && count <= kMaxRowRects, "%d rectangles (%d x %d, group %d, tiles %d + %d)", count, tm, tn, g, first, n);
+            std::vector<int> seen(n * upt);
+            for (long long u = 0; u < (long long)n * upt; ++u) {
+              int pm, pn, unit;
+              row_rect_unit(rect, count, u, bm, upr, pm, pn, unit);
+              const int j = grouped_tile_id(pm, pn, tm, tn, g) - first;
+              const bool owned = j >= 0 && j < n && unit >= 0 && unit < upt && tile[first + j] == std::make_pair(pm, pn);
+              CHECK(owned && seen[j * upt + unit]++ == 0, "unit %lld: tile %d unit %d (%d x %d, group %d, tiles %d + %d)", u, j, unit, tm, tn, g, first, n);
+            }
+          }
+      }
+}
+
 int main() {
   check_row_tile<64>(256);
   check_row_tile<128>(256);
@@ -357,6 +386,7 @@ int main() {
   check_flag_counts();
   check_decode_offsets();
   check_split_plan();
+  check_row_rects();
   if (failures) { printf("%d check(s) failed\n", failures); return 1; }
   printf("layout_sim: all checks passed\n");
   return 0;
