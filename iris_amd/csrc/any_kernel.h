@@ -419,16 +419,22 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     // numbers: the value rounded to eight bits, the remainder rounded, and the rest, which fits.  Six of the nine
     // products of the pieces are added up (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the others are at
     // most 2^-24 of the product and 2^-27 of it in the mean, below the rounding of one fp32 addition.  The sums are
-    // fp32, with six additions per 16 k instead of sixteen.  Error against 64 bits, 2-norm, normal operands,
-    // float32 MFMA -> three pieces: K = 512 4.1e-7 -> 3.5e-7, 1024 5.7e-7 -> 4.9e-7, 8192 1.62e-6 -> 1.44e-6.
+    // fp32; the five smaller products have sums of their own, 2^-8 of the others, so that one addition per 16 k rounds at
+    // the size of the result instead of sixteen.  Error against 64 bits, 2-norm, 1024x1024xK, float32 MFMA -> three
+    // pieces (with all six products in one sum):
+    //              normal operands               normal, A's negative half zero   uniform in [0, 1)
+    //   K =   64   1.44e-7 -> 0.50e-7 (1.10)     1.03e-7 -> 0.41e-7 (1.06)        1.15e-7 -> 0.49e-7 (0.84)
+    //       1024   5.7e-7  -> 1.9e-7  (4.9)      4.0e-7  -> 1.4e-7  (4.6)         4.3e-7  -> 1.6e-7  (2.9)
+    //       8192   1.62e-6 -> 0.57e-6 (1.44)     1.15e-6 -> 0.48e-6 (1.34)        1.19e-6 -> 0.42e-6 (0.75)
     // What the pieces cannot represent is left to the float32 MFMA, tile by tile: a nonzero operand below
     // 2^-110 (found while splitting), and tiles with a sum that is not finite (infinities and NaN, and values
     // that round to infinity in bf16), whose pieces need not add up to what the operands do.
     // The pieces are formed once per workgroup on the way from registers to LDS, 7 VALU instructions per
-    // element.  What bounds it: the matrix pipes at the clock they hold under load (4096x4096x1536 in 282 us
-    // is 1.1 PFLOP/s of bf16 products, the bf16 tile kernel reaches 1.2-1.4); 137 -> 183 TFLOP/s of
-    // float32.  With the smaller tiles the LDS (6 bytes written per element, 9 KiB read per 12 products of a
-    // 32x64 wave block) and the splitting weigh as much: 2048x2880x1024 110 -> 98 us.
+    // element.  What bounds it: the matrix pipes at the clock they hold under load, the LDS (6 bytes written per
+    // element, 9 KiB read per 12 products of a 32x64 wave block) and the splitting, about equally.  The second sums
+    // cost nothing (2048x2880x1024 two-shot 109.2 -> 108.1 us) but registers: a 256x128 tile, whose waves own 64x64, has none
+    // left (169 spilled) and would have to keep one sum; it is 12 % faster (4096x4096x1536 267 us, 128x128 298) with 2.6
+    // times the error, more than the float32 MFMA's where half of A is zero.
     LDS_AS int* const vote = (LDS_AS int*)(LDS_AS char*)(smem + CFG::FLAG_OFF);
     if (tid == 0) *vote = 0;
     lds_barrier();
@@ -485,6 +491,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     // Eight waves: the products of the step in buffer `buf`.  Between them, in parts of five to seven instructions that
     // issue in the shadow of a product, the step that has arrived in registers is split and put into the
     // other buffer, and the loads of the step after it go out.
+    f32x16_t small[MB][NB];  // sums of the five smaller products
     constexpr int kPairs[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};  // the smallest products first
     constexpr int KS16 = CFG::KE / 16, NMUL = KS16 * 6 * MB * NB, PARTS = 6 * (LA + LB);
     auto step = [&](int buf, auto fetch_tag) {
@@ -497,7 +504,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
       for (int m = 0; m < NMUL; ++m) {
         const int kk = m / (6 * MB * NB), t = m / (MB * NB) % 6, mb = m / NB % MB, nb = m % NB;
-        acc[mb][nb] = mfma_block<IN_BF16, 1>(f[kk][kPairs[t][0]].a[mb], f[kk][kPairs[t][1]].b[nb], acc[mb][nb]);
+        f32x16_t& sum = t < 5 ? small[mb][nb] : acc[mb][nb];
+        sum = mfma_block<IN_BF16, 1>(f[kk][kPairs[t][0]].a[mb], f[kk][kPairs[t][1]].b[nb], sum);
         if (kk + 1 < KS16 && m % (2 * MB * NB) == 0) load_pieces(f[kk + 1][t / 2], buf, kk + 1, t / 2);
 #pragma unroll
         for (int j = 0; j <= PARTS / NMUL; ++j) {
@@ -515,6 +523,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     point_at_a(std::true_type{});
     point_at_b(std::true_type{});
     clear_sums();
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) small[mb][nb] = acc[mb][nb];
     int s = 0;
     bool stop = false;
     auto close_step = [&]() {
@@ -563,12 +575,21 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-              for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mfma_block<IN_BF16, 1>(f[kPairs[t][0]].a[mb], f[kPairs[t][1]].b[nb], acc[mb][nb]);
+              for (int nb = 0; nb < NB; ++nb) {
+                f32x16_t& sum = t < 5 ? small[mb][nb] : acc[mb][nb];
+                sum = mfma_block<IN_BF16, 1>(f[kPairs[t][0]].a[mb], f[kPairs[t][1]].b[nb], sum);
+              }
         }
         ++s;
       }
       lds_barrier();
     }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[mb][nb][i] += small[mb][nb][i];
     // The vote: sums of elements that exist, and what the splitting saw.
     bool finite = true;
 #pragma unroll
@@ -918,22 +939,21 @@ int launch_any(FusedParams p, int device, int cu_count, hipStream_t stream, cons
 // bytes and splitting per flop rise; the 32x32 tile of float32 multiplies on the float32 MFMA.  A CU with a single
 // workgroup of four waves has nothing to run while it waits (bf16 1024x4095x2049 on 256 tiles of 128x128: 40 us, where
 // the full rate would give 26).  Checked against forced tiles, us for 256x256 / 128x128 / 64x128 / 64x64 / 32x32, the
-// choice first (float32: 256x128 in the place of 256x256): bf16 1999x2877x1371 64x128 41 (53 / 40 / - / 51 / 119), 1024x4095x2049 64x128 38 (68 / 40 / - / 48 / 105),
-// one-shot with seven peers 500x2877x1371 64x64 30 (92 / 46 / 32 / - / 51), 33x2877x1371 32x32 13 (49 / 31 / 25 / 20 / -); float32
-// 2048x2880x1024 64x128 98 (97 / 108 / - / 113 / 174), 4096x2048x1024 256x128 98 (- / 112 / 123 / 134 / 224), 2048x2048x4096
-// 128x128 199 (275 / - / 236 / 260 / 381), 512x2880x1024 64x64 40 (77 / 47 / 45 / - / 44), 300x4096x4096 32x32 129 (267 / 159 /
-// 153 / 138 / -), 1536x2880x1024 64x64 87 (79 / 100 / 80 / - / 121).
+// choice first (float32 without the largest): bf16 1999x2877x1371 64x128 41 (53 / 40 / - / 51 / 119), 1024x4095x2049 64x128 38 (68 / 40 /
+// - / 48 / 105), one-shot with seven peers 500x2877x1371 64x64 30 (92 / 46 / 32 / - / 51), 33x2877x1371 32x32 13 (49 / 31 / 25 / 20 / -);
+// float32 2048x2880x1024 64x128 98 (108 / - / 113 / 174), 2048x2048x4096 128x128 199 (- / 236 / 260 / 381), 512x2880x1024 64x64 40
+// (47 / 45 / - / 44), 300x4096x4096 32x32 129 (159 / 153 / 138 / -), 1536x2880x1024 64x64 87 (100 / 80 / - / 121).
 struct AnyTile {
   int bm, bn;
   float rate;
 };
 constexpr AnyTile kAnyTiles[] = {{256, 256, 855.f}, {128, 128, 654.f}, {64, 128, 508.f}, {64, 64, 395.f}, {32, 32, 195.f}};
-constexpr AnyTile kAnyTilesF32[] = {{256, 128, 183.f}, {128, 128, 163.f}, {64, 128, 160.f}, {64, 64, 140.f}, {32, 32, 98.f}};  // the first two of eight waves
+constexpr AnyTile kAnyTilesF32[] = {{0, 0, 0.f}, {128, 128, 163.f}, {64, 128, 160.f}, {64, 64, 140.f}, {32, 32, 98.f}};  // the largest of eight waves
 
 inline int choose_any_tile(int M, int N, int cu, bool f32_in, bool f32_out) {
   int best = 1;
   float best_time = 0.f;
-  for (int i = f32_out && !f32_in ? 1 : 0; i < 5; ++i) {
+  for (int i = f32_out ? 1 : 0; i < 5; ++i) {
     const AnyTile& t = f32_in ? kAnyTilesF32[i] : kAnyTiles[i];
     const long long per_cu = ((long long)cdiv(M, t.bm) * cdiv(N, t.bn) + cu - 1) / cu;
     const float alone = i == 0 || per_cu > 1 || (f32_in && i == 1) ? 1.f : f32_in ? 1.15f : 1.5f;
@@ -951,8 +971,7 @@ int dispatch_any_layout(const FusedParams& p, int device, int cu, hipStream_t s,
   constexpr bool F32_IN = AnyIn<IN>::ES == 4, F32_OUT = Out::size == 4;
   switch (choose_any_tile(p.M, p.N, cu, F32_IN, F32_OUT)) {
     case 0:  // (a staged 256x256 tile of float32 would not fit the LDS)
-      if constexpr (F32_IN) return launch_any<AnyCfg<IN, Out, 256, 128, 4, 2, 1, BKC>>(p, device, cu, s, types);
-      else if constexpr (!F32_OUT) return launch_any<AnyCfg<IN, Out, 256, 256, 2, 4, 1, BKC>>(p, device, cu, s, types);
+      if constexpr (!F32_OUT) return launch_any<AnyCfg<IN, Out, 256, 256, 2, 4, 1, BKC>>(p, device, cu, s, types);
       break;
     case 2: return launch_any<AnyCfg<IN, Out, 64, 128, 2, 2, 1, BKC>>(p, device, cu, s, types);
     case 3: return launch_any<AnyCfg<IN, Out, 64, 64, 2, 2, 1, BKC>>(p, device, cu, s, types);

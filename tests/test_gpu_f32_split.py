@@ -11,7 +11,7 @@ from iris_amd import _lib
 pytestmark = pytest.mark.gpu
 
 # Output sizes for every tile that splits (on 256 CUs), ragged, and the number of K steps from one to several.
-SHAPES = [(4093, 4095, 96, "256x128"), (1023, 3969, 333, "128x128"), (1999, 2877, 161, "64x128"), (511, 2879, 1025, "64x64"), (511, 2879, 31, "64x64")]
+SHAPES = [(4093, 4095, 96, "128x128"), (1023, 3969, 333, "128x128"), (1999, 2877, 161, "64x128"), (511, 2879, 1025, "64x64"), (511, 2879, 31, "64x64")]
 EPS = 2.0 ** -24
 
 
