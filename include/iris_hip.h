@@ -74,9 +74,9 @@ enum {
 
 /* Kernel selection (path). */
 enum {
-  IRIS_HIP_PATH_AUTO = 0,   /* MFMA kernel when the operands qualify, else the generic kernel */
+  IRIS_HIP_PATH_AUTO = 0,   /* MFMA kernel when the operands qualify, else the any-shape kernel */
   IRIS_HIP_PATH_MFMA = 1,   /* MFMA kernel or hipErrorInvalidValue */
-  IRIS_HIP_PATH_GENERIC = 2 /* generic kernel */
+  IRIS_HIP_PATH_GENERIC = 2 /* any-shape kernel */
 };
 
 /* Codes stored to *status by a kernel. */
