@@ -529,10 +529,14 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
       for (int nb = 0; nb < NB; ++nb) small[mb][nb] = acc[mb][nb];
     int s = 0;
     bool stop = false;
+    // Eight waves: one barrier per step.  What a wave reads of the vote behind the barrier of step s, another one may
+    // already be past: nobody writes ahead of the barrier of step s + 1 then (layout.h), `tiny` keeps the answer.
+    bool tiny = false;  // an operand of the steps put down so far is below 2^-110
     auto close_step = [&]() {
-      if (s + 1 < nsteps && low < kSmallest) *vote = 1;
+      if (s + 1 < nsteps) tiny = low < kSmallest;  // (the last step puts down leftovers)
+      if (tiny && vote_written_before_barrier(s)) *vote = 1;
       lds_barrier();
-      stop = (s & 7) == 7 && *vote != 0;  // (the same answer for everybody: nobody writes before the next barrier)
+      stop = vote_read_behind_barrier(s) && *vote != 0;
       ++s;
     };
     fetch();
@@ -564,7 +568,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         if (s + 1 < nsteps) fetch();
         lds_barrier();
         if (s == 0) PHASE_STAMP(1);
-        stop = (s & 7) == 7 && *vote != 0;
+        stop = vote_read_behind_barrier(s) && *vote != 0;  // (nobody writes before the barrier in front of the next step)
 #pragma unroll
         for (int kk = 0; kk < KS16; ++kk) {
           Pieces f[3];
@@ -600,7 +604,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) finite = finite && (!there || __builtin_fabsf(acc[mb][nb][i]) <= 3.402823466e38f);
       }
-    if (!finite) *vote = 1;
+    if (!finite || tiny) *vote = 1;
     lds_barrier();
     redo = *vote;
     if (redo) k_loop();

@@ -302,6 +302,15 @@ IRIS_HD bool decode_offsets_fit(long long a_rows, long long s_am, long long K, i
 }
 
 // ---------------------------------------------------------------------------------------------
+// The vote of a workgroup on a word in LDS, where the K loop has one barrier per step: in which steps the word is read
+// behind the barrier (to leave the loop early, the same step for every wave), and in which it may be written in front
+// of it.  Between two barriers there is either a read or a write: a wave that has read behind the barrier of step s may
+// run through step s + 1 while another one has yet to read.
+// ---------------------------------------------------------------------------------------------
+IRIS_HD bool vote_read_behind_barrier(int step) { return (step & 7) == 7; }
+IRIS_HD bool vote_written_before_barrier(int step) { return (step & 7) != 0; }
+
+// ---------------------------------------------------------------------------------------------
 // Stand-alone collectives: a consecutive run of tiles of the grouped order (groups of group_m tile rows walked column
 // by column) is the rest of a column, some columns of a group, whole groups, and the mirror image at the end - at most
 // five rectangles.  Walked row by row, a workgroup moves kilobytes of every row instead of tiles' 128-byte rows (bf16

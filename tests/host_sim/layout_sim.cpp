@@ -365,6 +365,26 @@ void check_row_rects() {
       }
 }
 
+// ---- vote of a workgroup in a loop with one barrier per step -----------------------------------------
+// A wave meets the first reason to leave in step `seen`.  Reads behind the barrier of step s may come as early as right
+// behind it or as late as right in front of the next one, when votes written in step s + 1 are there too: both have to
+// leave the loop in the same step, and before long.
+void check_vote() {
+  for (int nsteps = 1; nsteps <= 40; ++nsteps)
+    for (int seen = 0; seen < nsteps; ++seen) {
+      auto leaves = [&](bool late) {
+        for (int s = 0; s < nsteps; ++s) {
+          if (!vote_read_behind_barrier(s)) continue;
+          for (int w = seen; w <= s + (late && s + 1 < nsteps); ++w)
+            if (vote_written_before_barrier(w)) return s;
+        }
+        return nsteps;
+      };
+      CHECK(leaves(false) == leaves(true), "%d steps, reason met in step %d: early readers leave in step %d, late ones in step %d", nsteps, seen, leaves(false), leaves(true));
+      CHECK(leaves(false) <= seen + 8 || leaves(false) == nsteps, "%d steps, reason met in step %d: left in step %d", nsteps, seen, leaves(false));
+    }
+}
+
 int main() {
   check_row_tile<64>(256);
   check_row_tile<128>(256);
@@ -387,6 +407,7 @@ int main() {
   check_decode_offsets();
   check_split_plan();
   check_row_rects();
+  check_vote();
   if (failures) { printf("%d check(s) failed\n", failures); return 1; }
   printf("layout_sim: all checks passed\n");
   return 0;
