@@ -543,6 +543,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     if constexpr (CFG::NW == 8) {
 #pragma unroll
       for (int i = 0; i < LA + LB; ++i) put_split(raw[i], lds_at[i], i < LA ? CFG::A_PLANE : CFG::B_PLANE);
+      tiny = low < kSmallest;  // (with a single step the only look at it)
       if (nsteps > 1) fetch();
       lds_barrier();
       PHASE_STAMP(1);

@@ -10,8 +10,9 @@ from iris_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
-# Output sizes for every tile that splits (on 256 CUs), ragged, and the number of K steps from one to several.
-SHAPES = [(4093, 4095, 96, "128x128"), (1023, 3969, 333, "128x128"), (1999, 2877, 161, "64x128"), (511, 2879, 1025, "64x64"), (511, 2879, 31, "64x64")]
+# Output sizes for every tile that splits (on 256 CUs), ragged, and the number of K steps of 32 from one to several.
+SHAPES = [(4093, 4095, 31, "128x128"), (4093, 4095, 32, "128x128"), (4093, 4095, 33, "128x128"), (1999, 2877, 32, "64x128"),
+          (4093, 4095, 96, "128x128"), (1023, 3969, 333, "128x128"), (1999, 2877, 161, "64x128"), (511, 2879, 1025, "64x64"), (511, 2879, 31, "64x64")]
 EPS = 2.0 ** -24
 
 
