@@ -426,7 +426,11 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     //   K =   64   1.44e-7 -> 0.50e-7 (1.10)     1.03e-7 -> 0.41e-7 (1.06)        1.15e-7 -> 0.49e-7 (0.84)
     //       1024   5.7e-7  -> 1.9e-7  (4.9)      4.0e-7  -> 1.4e-7  (4.6)         4.3e-7  -> 1.6e-7  (2.9)
     //       8192   1.62e-6 -> 0.57e-6 (1.44)     1.15e-6 -> 0.48e-6 (1.34)        1.19e-6 -> 0.42e-6 (0.75)
-    // What the pieces cannot represent is left to the float32 MFMA, tile by tile: a nonzero operand below
+    // A sum with a single product in it is the exception: what is left out comes on top of the one rounding it has with
+    // the float32 MFMA (normal operands: largest error 0.5 -> 0.98 of a last place, 2-norm 2.48e-8 -> 2.52e-8; sums of two
+    // products 3.1e-8 -> 2.6e-8).  K = 1, where every sum is one, is left to the float32 MFMA.  The other products of
+    // pieces would bring it back for a longer K whose other products are zeros, at 2048x2880x1024 108 -> 119 us.
+    // What the pieces cannot represent is left to it too, tile by tile: a nonzero operand below
     // 2^-110 (found while splitting), and tiles with a sum that is not finite (infinities and NaN, and values
     // that round to infinity in bf16), whose pieces need not add up to what the operands do.
     // The pieces are formed once per workgroup on the way from registers to LDS, 7 VALU instructions per
@@ -605,7 +609,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) finite = finite && (!there || __builtin_fabsf(acc[mb][nb][i]) <= 3.402823466e38f);
       }
-    if (!finite || tiny) *vote = 1;
+    if (!finite || tiny || p.K == 1) *vote = 1;
     lds_barrier();
     redo = *vote;
     if (redo) k_loop();

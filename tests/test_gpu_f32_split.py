@@ -44,6 +44,16 @@ def test_error_is_that_of_fp32_sums(M, N, K, tile, b_transposed):
     assert ((got.double() - exact) / bound).abs().mean() < 1 / 8
 
 
+@pytest.mark.parametrize("b_transposed", [False, True], ids=["nn", "nt"])
+@pytest.mark.parametrize("M,N,tile", [(4093, 4095, "128x128"), (1999, 2877, "64x128"), (511, 2879, "64x64")])
+def test_a_single_product_is_rounded_once(M, N, tile, b_transposed):
+    g = torch.Generator().manual_seed(9)
+    a, b = torch.randn((M, 1), generator=g), torch.randn((1, N), generator=g)
+    got, kernel = _product(a, b, b_transposed)
+    assert kernel.startswith(f"generic_f32_{tile}")
+    assert torch.equal(got, a * b)
+
+
 @pytest.mark.parametrize("M,N,K,tile", SHAPES, ids=[f"{s[3]}_k{s[2]}" for s in SHAPES])
 def test_operands_that_three_pieces_do_not_hold(M, N, K, tile):
     """One row of A at a time picks single elements of B (powers of two elsewhere zero), so every product is exact in fp32."""
