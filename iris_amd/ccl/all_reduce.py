@@ -14,7 +14,7 @@ import torch
 
 from .. import _lib
 from ..host.logging import debug_on, log_rank
-from ..ops._common import current_stream, dtype_code, iris_launch, native, ptr, require_gpu_tensors
+from ..ops._common import check_launch, current_stream, dtype_code, iris_launch, native, ptr, require_gpu_tensors
 from .config import Config
 from .utils import ReduceOp, extract_group_info
 
@@ -111,7 +111,9 @@ def all_reduce(output_tensor, input_tensor, ctx, op=None, group=None, async_op=F
     if config is None:
         config = Config(block_size_m=32, block_size_n=64, all_reduce_distribution=1)
     fast = native(ctx) if workspace is not None and group is None else None
-    if fast is not None and fast.try_ccl_all_reduce(ctx, output_tensor, input_tensor, config, workspace, current_stream(ctx)):
+    done = fast.try_ccl_all_reduce(ctx, output_tensor, input_tensor, config, workspace, current_stream(ctx)) if fast is not None else None
+    if done is not None:
+        check_launch(done, ctx.get_rank())
         if not async_op:
             ctx.barrier()
         return workspace

@@ -7,7 +7,7 @@ iris/ccl/triton/reduce_scatter.py:143-192.
 import logging
 
 from ..host.logging import debug_on, log_rank
-from ..ops._common import current_stream, dtype_code, iris_launch, native, require_gpu_tensors
+from ..ops._common import check_launch, current_stream, dtype_code, iris_launch, native, require_gpu_tensors
 from .all_reduce import _check_tensors, _launch_head
 from .config import Config
 from .utils import ReduceOp
@@ -26,7 +26,9 @@ def reduce_scatter(output_tensor, input_tensor, ctx, op=None, group=None, async_
     if config is None:
         config = Config(block_size_m=32, block_size_n=64, all_reduce_distribution=1)
     fast = native(ctx) if group is None else None
-    if fast is not None and fast.try_ccl_reduce_scatter(ctx, output_tensor, input_tensor, config, current_stream(ctx)):
+    done = fast.try_ccl_reduce_scatter(ctx, output_tensor, input_tensor, config, current_stream(ctx)) if fast is not None else None
+    if done is not None:
+        check_launch(done, ctx.get_rank())
         if not async_op:
             ctx.barrier()
         return

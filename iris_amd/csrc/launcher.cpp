@@ -6,9 +6,11 @@
 //   <entry>(...)   one entry point with its C arguments (pointers as integers or None, the rest as int / float), returns
 //                  its int.  Types come from the declarations in iris_hip.h.
 //   try_<op>(...)  a whole operator call on its tensors: reads what the Python wrapper reads, and when every argument
-//                  is as it should be and the workspace can be used as it is, launches and returns True.
-//                  Anything else - an error to report, a preamble to run - returns False with nothing done, and the
+//                  is as it should be and the workspace can be used as it is, calls the entry point and returns its int.
+//                  Anything else - an argument to report, a preamble to run - returns None with nothing done, and the
 //                  Python wrapper takes the call from its start.  The wrapper is the authority on what is an error.
+//                  An entry point that fails is not called again: its error may be an earlier call's, found behind
+//                  a launch that went out.
 //
 //   load(path)     dlopen the library (once) and resolve the entry points; raises OSError
 #include <torch/csrc/Dtype.h>
@@ -251,11 +253,10 @@ PyObject* launch(F&& f) {
   Py_BEGIN_ALLOW_THREADS
   rc = f();
   Py_END_ALLOW_THREADS
-  require(rc == 0);  // the wrapper repeats the call and reports the error
-  Py_RETURN_TRUE;
+  return PyLong_FromLong(rc);
 }
 
-// Runs `body`; whatever it declines, or trips over, is the wrapper's.
+// Runs `body`; whatever it declines, or trips over in front of the launch, is the wrapper's.
 template <class F>
 PyObject* attempt(Py_ssize_t n, Py_ssize_t expected, F&& body) {
   if (n != expected) return PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", expected, n);
@@ -263,13 +264,15 @@ PyObject* attempt(Py_ssize_t n, Py_ssize_t expected, F&& body) {
     return body();
   } catch (...) {
     PyErr_Clear();
-    Py_RETURN_FALSE;
+    Py_RETURN_NONE;
   }
 }
 
-void used(PyObject* ws, PyObject* stream, bool unprepare) {
-  if (unprepare) require(PyObject_SetAttr(ws, at_prepared, Py_False) == 0);
-  require(PyObject_SetAttr(ws, at_stream, stream) == 0);
+// Notes in the workspace that a launch (whose result is `rc`) has used it; returns rc, or NULL with a Python error set.
+PyObject* used(PyObject* rc, PyObject* ws, PyObject* stream, bool unprepare) {
+  if (!rc || PyLong_AsLong(rc) != 0) return rc;
+  if ((unprepare && PyObject_SetAttr(ws, at_prepared, Py_False) != 0) || PyObject_SetAttr(ws, at_stream, stream) != 0) Py_CLEAR(rc);
+  return rc;
 }
 
 // try_matmul_all_reduce(shmem, C, A, B, config, workspace, scale_a, scale_b, slot_sum, kernel_path, stream)
@@ -292,13 +295,12 @@ PyObject* try_matmul_all_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const long long spin = int_of(a[0], at_spin_limit);
     int32_t* const status = shmem.status();
     void* const stream = PyLong_AsVoidPtr(a[10]);
-    PyObject* const done = launch([&] {
+    PyObject* const rc = launch([&] {
       return fn_iris_hip_matmul_all_reduce(A.ptr(), B.ptr(), C.ptr(), ws.aux, ws.locks, C.rows, C.cols, A.cols, A.s0, A.s1, B.s0, B.s1, C.s0, C.s1,
                                            context, shmem.rank, shmem.world, blocks.m, blocks.n, blocks.k, code, types.in, types.out,
                                            types.scale, acc, spin, status, path, stream);
     });
-    used(a[5], a[10], true);
-    return done;
+    return used(rc, a[5], a[10], true);
   });
 }
 
@@ -321,13 +323,12 @@ PyObject* try_matmul_reduce_scatter(PyObject*, PyObject* const* a, Py_ssize_t n)
     const long long spin = int_of(a[0], at_spin_limit);
     int32_t* const status = shmem.status();
     void* const stream = PyLong_AsVoidPtr(a[12]);
-    PyObject* const done = launch([&] {
+    PyObject* const rc = launch([&] {
       return fn_iris_hip_matmul_reduce_scatter(A.ptr(), B.ptr(), C.ptr(), ws.aux, ws.locks, C.rows, C.cols, A.cols, A.s0, A.s1, B.s0, B.s1, C.s0,
                                                C.s1, context, shmem.rank, shmem.world, blocks.m, blocks.n, blocks.k, all_owners, sum_peers,
                                                types.in, types.out, types.scale, acc, spin, status, path, stream);
     });
-    used(a[5], a[12], false);
-    return done;
+    return used(rc, a[5], a[12], false);
   });
 }
 
@@ -425,13 +426,12 @@ PyObject* try_ccl_all_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const int64_t* const bases = c.shmem.words(at_heap_bases);
     void* const stream = PyLong_AsVoidPtr(a[5]);
-    PyObject* const done = launch([&] {
+    PyObject* const rc = launch([&] {
       return fn_iris_hip_all_reduce(c.in.ptr(), c.out.ptr(), c.in.rows, c.in.cols, c.in.s0, c.in.s1, c.out.s0, c.out.s1, bases, c.shmem.rank,
                                     c.shmem.rank, c.shmem.world, 0, 1, c.bm, c.bn, c.swizzle, c.sms, c.xcds, c.chunk,
                                     one_shot ? IRIS_HIP_VARIANT_ONE_SHOT : IRIS_HIP_VARIANT_TWO_SHOT, c.distribution, c.type, stream);
     });
-    used(ws, a[5], true);
-    return done;
+    return used(rc, ws, a[5], true);
   });
 }
 

@@ -72,8 +72,9 @@ def current_stream(shmem):
 
 def native(shmem):
     """The module that takes whole operator calls (csrc/launcher.cpp), or None where the Python wrapper has to: on a
-    host-backed context and while DEBUG records are wanted.  Its try_<op> functions return False, with nothing done,
-    for every call that is not plainly in order; the wrapper then starts over and finds out why."""
+    host-backed context and while DEBUG records are wanted.  Its try_<op> functions return None, with nothing done,
+    for every call that is not plainly in order - the wrapper then starts over and finds out why - and the entry
+    point's result (for check_launch) for the others."""
     return None if shmem.gpu_id < 0 or debug_on() else _lib.launcher()
 
 
@@ -97,6 +98,15 @@ def rearmed(shmem, workspace, C, operation, shape, dtype, world_size, variant, t
     return shmem.runs_alone()
 
 
+def check_launch(err, rank):
+    """Raise RuntimeError for an entry point's non-zero result."""
+    if err != 0:
+        detail = _lib.last_error()
+        text = detail if detail else error_string(err)
+        log_rank(logging.ERROR, "HIP error code %d: %s", err, text, rank=rank)
+        raise RuntimeError(f"HIP error code {err}: {text}")
+
+
 def iris_launch(entry_name, grid, *args, algorithm, rank, dtype=None):
     """Launch seam: the reference launches `kernel_fn[grid](*args)` here
     (iris/host/tracing/kernel_artifacts.py:54-83); this calls the C entry point of the same operator
@@ -107,13 +117,7 @@ def iris_launch(entry_name, grid, *args, algorithm, rank, dtype=None):
     entry = _ENTRY_POINTS.get(entry_name)
     if entry is None:
         entry = _ENTRY_POINTS[entry_name] = getattr(_lib.launcher(), entry_name)
-    err = entry(*args)
-    if err != 0:
-        detail = _lib.last_error()
-        text = detail if detail else error_string(err)
-        log_rank(logging.ERROR, "HIP error code %d: %s", err, text, rank=rank)
-        raise RuntimeError(f"HIP error code {err}: {text}")
-    return None
+    check_launch(entry(*args), rank)
 
 
 def stage_idle_peers(shmem, workspace):

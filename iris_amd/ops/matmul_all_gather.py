@@ -12,7 +12,7 @@ import torch
 
 from .. import _lib
 from ..host.logging import debug_on, log_rank
-from ._common import current_stream, dtype_code, iris_launch, is_fp8, native, path_code, ptr, require_gpu_tensors
+from ._common import check_launch, current_stream, dtype_code, iris_launch, is_fp8, native, path_code, ptr, require_gpu_tensors
 from .config import FusedConfig
 from .workspace import FusedWorkspace
 
@@ -61,8 +61,10 @@ def matmul_all_gather(
     if config is None:
         config = FusedConfig()
     fast = native(shmem)
-    if fast is not None and fast.try_matmul_all_gather(shmem, output_tensor, A, B, bias, config, scale_a, scale_b, kernel_path,
-                                                       current_stream(shmem)):
+    done = fast.try_matmul_all_gather(shmem, output_tensor, A, B, bias, config, scale_a, scale_b, kernel_path,
+                                      current_stream(shmem)) if fast is not None else None
+    if done is not None:
+        check_launch(done, shmem.get_rank())
         if not async_op:
             shmem.barrier()
         if workspace is None:

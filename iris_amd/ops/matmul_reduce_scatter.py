@@ -12,7 +12,7 @@ import torch
 
 from .. import _lib
 from ..host.logging import debug_on, log_rank
-from ._common import (acc_code, current_stream, dtype_code, iris_launch, is_fp8, native, path_code, ptr,
+from ._common import (acc_code, check_launch, current_stream, dtype_code, iris_launch, is_fp8, native, path_code, ptr,
                       rearmed, require_gpu_tensors, stage_idle_peers)
 from .config import FusedConfig
 from .workspace import FusedWorkspace
@@ -105,8 +105,10 @@ def matmul_reduce_scatter(
     if config is None:
         config = FusedConfig()
     fast = native(shmem) if workspace is not None and stage is None else None
-    if fast is not None and fast.try_matmul_reduce_scatter(shmem, C, A, B, config, workspace, all_owners, sum_peers, scale_a,
-                                                           scale_b, slot_sum, kernel_path, current_stream(shmem)):
+    done = fast.try_matmul_reduce_scatter(shmem, C, A, B, config, workspace, all_owners, sum_peers, scale_a,
+                                          scale_b, slot_sum, kernel_path, current_stream(shmem)) if fast is not None else None
+    if done is not None:
+        check_launch(done, shmem.get_rank())
         if not async_op:
             shmem.barrier()
         return workspace

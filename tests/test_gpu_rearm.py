@@ -1,6 +1,9 @@
 """A workspace handed back to the operator that used it: the second call runs no preamble and must still leave what a
 call with one leaves - own tiles reduced, every other tile of C zero - on each kernel family."""
 
+import ctypes
+import subprocess
+
 import pytest
 import torch
 
@@ -103,3 +106,51 @@ def test_calls_that_are_not_in_order_reach_the_python_checks():
         ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws)
     ws = ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws)
     assert torch.all(C == 0)
+
+
+_FAILING = """
+int calls = 0;
+int iris_hip_matmul_all_reduce() { return ++calls, 98; }
+int iris_hip_matmul_reduce_scatter() { return ++calls, 98; }
+int iris_hip_all_gather_matmul() { return ++calls, 98; }
+int iris_hip_matmul_all_gather() { return ++calls, 98; }
+int iris_hip_all_reduce() { return ++calls, 98; }
+int iris_hip_reduce_scatter() { return ++calls, 98; }
+"""
+
+
+def test_a_failed_launch_is_reported_and_not_repeated(tmp_path):
+    """Entry points that return an error behind a launch that went out (as an earlier call's error does): one call, one
+    exception, and the workspace as it was."""
+    W, M, N, K, dtype = 2, 64, 128, 64, torch.bfloat16
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=0)
+    A, B, C = ctx.zeros((M, K), dtype=dtype), ctx.zeros((K, N), dtype=dtype), ctx.zeros((M, N), dtype=dtype)
+    wide = ctx.zeros((W * M, N), dtype=dtype)
+    cfg = iris.FusedConfig(block_size_m=32, block_size_n=32, block_size_k=32, all_reduce_variant="atomic")
+    one_shot = Config(all_reduce_variant="one_shot")
+    ws = ops.matmul_all_reduce_preamble(ctx, C, A, B, config=cfg)
+    rs = ctx.ops.matmul_reduce_scatter(C, A, B, config=cfg, sum_peers=False)
+    ccl = ctx.ccl.all_reduce_preamble(C, wide[:M], config=one_shot)
+    calls = [
+        lambda: ctx.ops.matmul_all_reduce(C, A, B, config=cfg, workspace=ws),
+        lambda: ctx.ops.matmul_reduce_scatter(C, A, B, config=cfg, workspace=rs, sum_peers=False),
+        lambda: ctx.ops.all_gather_matmul(wide, A, B, config=cfg, gather_dim=0),
+        lambda: ctx.ops.matmul_all_gather(wide, A, B, config=cfg),
+        lambda: ctx.ccl.all_reduce(C, wide[:M], config=one_shot, workspace=ccl),
+        lambda: ctx.ccl.reduce_scatter(C, wide[:M]),
+    ]
+    (tmp_path / "failing.c").write_text(_FAILING)
+    path = str(tmp_path / "failing.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", path, str(tmp_path / "failing.c")], check=True)
+    count = ctypes.c_int.in_dll(ctypes.CDLL(path), "calls")
+    _lib.launcher().load(path)
+    try:
+        for i, call in enumerate(calls):
+            with pytest.raises(RuntimeError, match="HIP error code 98"):
+                call()
+            assert count.value == i + 1, f"call {i}: entry points were called {count.value - i} times"
+    finally:
+        _lib.launcher().load(_lib.LIBRARY_PATH)
+    assert ws.prepared and ws.stream is None and ccl.prepared and ccl.stream is None
+    for call in calls:
+        call()
