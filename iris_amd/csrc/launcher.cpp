@@ -160,13 +160,15 @@ struct Shmem {
 struct Matrix {
   const at::Tensor& t;
   int64_t rows, cols, s0, s1;
+  void* data;
   Matrix(PyObject* o, const Shmem& shmem) : t(tensor(o)) {
     require(t.dim() == 2);
     shmem.on_device(t);
     rows = t.size(0), cols = t.size(1), s0 = t.stride(0), s1 = t.stride(1);
     require(rows > 0 && cols > 0);
+    data = t.mutable_data_ptr();  // (here, where it may throw: a tensor inside vmap has no memory to point at)
   }
-  void* ptr() const { return t.mutable_data_ptr(); }
+  void* ptr() const { return data; }
 };
 
 struct Blocks {
@@ -247,6 +249,7 @@ struct Workspace {
   }
 };
 
+// Calls `f`, which must not throw: the interpreter's lock is not held.
 template <class F>
 PyObject* launch(F&& f) {
   int rc;

@@ -108,6 +108,30 @@ def test_calls_that_are_not_in_order_reach_the_python_checks():
     assert torch.all(C == 0)
 
 
+def test_tensors_without_memory_are_refused():
+    """Inside vmap a batched operand has no address: an exception, raised where Python can take it."""
+    W, M, N, K, dtype = 2, 64, 128, 64, torch.bfloat16
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=0)
+    A, B, C = ctx.zeros((M, K), dtype=dtype), ctx.zeros((K, N), dtype=dtype), ctx.zeros((M, N), dtype=dtype)
+    wide, Bs = ctx.zeros((W * M, N), dtype=dtype), torch.zeros((3, K, N), dtype=dtype, device="cuda")
+    cfg = iris.FusedConfig(block_size_m=32, block_size_n=32, block_size_k=32, all_reduce_variant="one_shot")
+    ws = ops.matmul_all_reduce_preamble(ctx, C, A, B, config=cfg)
+    rs = ops.matmul_reduce_scatter_preamble(ctx, C, A, B, config=cfg)
+    rs.stream = torch.cuda.current_stream().cuda_stream
+    ccl = ctx.ccl.all_reduce_preamble(C, wide[:K], config=Config(all_reduce_variant="one_shot"))
+    calls = [
+        lambda b: ctx.ops.matmul_all_reduce(C, A, b, config=cfg, workspace=ws),
+        lambda b: ctx.ops.matmul_reduce_scatter(C, A, b, config=cfg, workspace=rs, sum_peers=False),
+        lambda b: ctx.ops.all_gather_matmul(wide, A, b, config=cfg, gather_dim=0),
+        lambda b: ctx.ops.matmul_all_gather(wide, A, b, config=cfg),
+        lambda b: ctx.ccl.all_reduce(b, wide[:K], config=Config(all_reduce_variant="one_shot"), workspace=ccl),
+        lambda b: ctx.ccl.reduce_scatter(b, wide[:K]),
+    ]
+    for call in calls:
+        with pytest.raises(RuntimeError, match="data pointer|storage"):
+            torch.vmap(lambda b: (call(b), b)[1])(Bs)
+
+
 _FAILING = """
 int calls = 0;
 int iris_hip_matmul_all_reduce() { return ++calls, 98; }
