@@ -725,7 +725,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     } else if (p.s_cn == 1) {
       // Packed adds of aligned dwords, one per thread.  A row that starts in the middle of a dword is shifted by
       // one element against them; the half of a dword that is not this tile's gets -0 added, which leaves
-      // every value as it is.
+      // every value of C as it is.  What lies next to C need not be a number (-0 makes a signalling NaN quiet): dwords
+      // that reach past the first or the last column are for the element of C alone.
       using Out16 = typename std::conditional<Out::kFp32SumInReference, OutF16, OutBF16>::type;
       constexpr int DPR = BN / 2 + 1;
       for (int d = tid; d < BM * DPR; d += NT) {
@@ -735,6 +736,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         const int e = 2 * (d - row * DPR) - (int)(((unsigned long long)at >> 1) & 1);
         const bool lo = e >= 0 && e < BN && n0 + e < p.N, hi = e + 1 < BN && n0 + e + 1 < p.N;
         if (!lo && !hi) continue;
+        const bool inside = n0 + e >= 0 && n0 + e + 1 < p.N;
         const char* const s = smem + row * CFG::TROW;
         const unsigned w = (lo ? *(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2) : 0x8000u) |
                            (hi ? (unsigned)*(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2 + 2) : 0x8000u) << 16;
@@ -744,7 +746,9 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
             if (lo) *(unsigned short*)(at + e * 2) = (unsigned short)z;
             if (hi) *(unsigned short*)(at + e * 2 + 2) = (unsigned short)(z >> 16);
           } else {
-            atomic_add_packed<Out16>(slot_ptr(p.heap_bases, at, p.rank, pr) + e * 2, w);
+            char* const to = slot_ptr(p.heap_bases, at, p.rank, pr) + e * 2;
+            if (inside) atomic_add_packed<Out16>(to, w);
+            else Out::atomic_add(lo ? to : to + 2, Out16::to_float((unsigned short)(lo ? w : w >> 16)));
           }
         }
       }

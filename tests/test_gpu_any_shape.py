@@ -115,3 +115,31 @@ def test_gathered_transposed_and_strided_operands(dtype, gather_dim, W, M, Kl, N
         kernel = _lib.last_kernel()
         assert kernel.startswith("generic"), kernel
         assert_bits_equal(out.cpu(), exp, f"{kernel} a_t={a_t} b_strided={b_strided} c_strided={c_strided}")
+
+
+# Bits that no arithmetic may pass over: signalling and quiet NaNs with a payload, subnormals, -0, infinity.
+PATTERNS = {torch.bfloat16: [0x7f81, 0xffa1, 0x7fc3, 0x0001, 0x807f, 0x8000, 0x7f80], torch.float16: [0x7c01, 0xfd01, 0x7e03, 0x0001, 0x83ff, 0x8000, 0x7c00]}
+
+
+# Columns that start and end in the middle of a dword, at either end, rows one after the other without a gap.
+@pytest.mark.parametrize("M,N,first,stride", [(67, 294, 1, 304), (67, 295, 1, 303), (67, 295, 0, 304), (5, 1, 3, 9), (641, 2370, 1, 2400), (67, 295, 0, 295)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_atomic_leaves_what_lies_next_to_c(dtype, M, N, first, stride):
+    W, rank, K = 3, 1, 24
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=rank)
+    A, B = _ints((M, K), 5, dtype), _ints((K, N), 6, dtype)
+    size, begin = M * stride + 8, 1  # (with a row stride of N the elements in front of and behind all of C)
+    flat = ctx.zeros((size,), dtype=dtype)
+    C = flat[begin:begin + M * stride].view(M, stride)[:, first:first + N]
+    bits = torch.tensor(PATTERNS[dtype], dtype=torch.int32).to(torch.int16)[torch.arange(size) % 7]
+    cfg = iris.FusedConfig(block_size_m=1, block_size_n=1, block_size_k=1, all_reduce_variant="atomic")
+    dA, dB = _view(ctx, A), _view(ctx, B)
+    ws = ops.matmul_all_reduce_preamble(ctx, C, dA, dB, config=cfg)
+    exp = bits.clone()
+    exp[begin:begin + M * stride].view(M, stride)[:, first:first + N] = (oracle.gemm(A, B).float() + 1).to(dtype).view(torch.int16)
+    for r in range(W):
+        ctx.peer_view(flat, r).view(torch.int16).copy_(bits)
+        ctx.peer_view(flat, r)[begin:begin + M * stride].view(M, stride)[:, first:first + N].fill_(1.0)
+    ops.matmul_all_reduce(ctx, C, dA, dB, config=cfg, workspace=ws, kernel_path="generic")
+    for r, got in enumerate(slot_copies(ctx, flat)):
+        assert torch.equal(got.view(torch.int16), exp), f"{_lib.last_kernel()} slot {r}"
