@@ -683,6 +683,6 @@ void iris_hip_set_split_tiles(int32_t mode) { iris_host::set_split_tile_mode(mod
 
 const char* iris_hip_last_error(void) { return g_last_error; }
 const char* iris_hip_last_kernel(void) { return g_last_kernel; }
-int iris_hip_abi_version(void) { return 5; }
+int iris_hip_abi_version(void) { return 6; }
 
 }  // extern "C"

@@ -281,6 +281,18 @@ def test_library_exports_every_declared_symbol():
     assert _lib.last_error() == ""
 
 
+def test_a_library_that_does_not_know_clear_c_is_refused(tmp_path):
+    """Version 5 has every symbol but reads IRIS_HIP_CLEAR_C in acc_mode as an unknown rule: reused workspaces would keep
+    what C held."""
+    source = "".join(f"int {name}() {{ return 5; }}\n" for name in _lib.PROTOTYPES)
+    (tmp_path / "old.c").write_text(source)
+    path = str(tmp_path / "old.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", path, str(tmp_path / "old.c")], check=True)
+    out = subprocess.run([sys.executable, "-c", "from iris_amd import _lib; _lib.library()"], cwd=ROOT, capture_output=True, text=True,
+                         env={**os.environ, "IRIS_HIP_LIBRARY": path})
+    assert out.returncode != 0 and "has ABI version 5" in out.stderr, out.stderr[-500:]
+
+
 def test_null_context_tensor_is_rejected_before_any_launch():
     """Every kernel translates addresses through the heap bases, so a NULL context tensor is an
     argument error for every fused entry point, whatever the world size; the check comes before the
