@@ -318,6 +318,9 @@ const char* iris_hip_last_error(void);
 /* Name of the kernel configuration the last successful launch on the calling thread used. */
 const char* iris_hip_last_kernel(void);
 
+/* 1 if launches on `stream` are being recorded into a graph, 0 if not (also when that cannot be found out). */
+int iris_hip_stream_capturing(void* stream);
+
 /* ABI version of this header.  6: IRIS_HIP_CLEAR_C (a version-5 library would take it for an accumulation rule it does not
  * know, and leave C as it is). */
 int iris_hip_abi_version(void);

@@ -91,6 +91,7 @@ PROTOTYPES = {
     "iris_hip_set_split_tiles": (None, [_i32]),
     "iris_hip_last_error": (ctypes.c_char_p, []),
     "iris_hip_last_kernel": (ctypes.c_char_p, []),
+    "iris_hip_stream_capturing": (_i32, [_ptr]),
     "iris_hip_abi_version": (_i32, []),
 }
 

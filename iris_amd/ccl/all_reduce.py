@@ -14,7 +14,7 @@ import torch
 
 from .. import _lib
 from ..host.logging import debug_on, log_rank
-from ..ops._common import check_launch, current_stream, dtype_code, iris_launch, native, ptr, require_gpu_tensors
+from ..ops._common import capturing, check_launch, current_stream, dtype_code, iris_launch, native, ptr, require_gpu_tensors
 from .config import Config
 from .utils import ReduceOp, extract_group_info
 
@@ -37,6 +37,7 @@ class AllReduceWorkspace:
     flags_per_tile: int = 0
     prepared: bool = False
     stream: Optional[int] = None  # raw HIP stream of the last launch
+    captured: bool = False  # a graph holds a launch of the workspace's
 
 
 def _check_variant(variant):
@@ -142,7 +143,7 @@ def all_reduce(output_tensor, input_tensor, ctx, op=None, group=None, async_op=F
     )
     stream = current_stream(ctx)
     if needs_prepare and workspace is not None and stream is not None and (workspace.stream, workspace.variant, workspace.shape, workspace.dtype) == (
-            stream, variant, (M, N), input_tensor.dtype) and ctx.runs_alone():
+            stream, variant, (M, N), input_tensor.dtype) and not workspace.captured and ctx.runs_alone() and not capturing(stream):
         # The same call again with no other process beside it: the preamble's barrier has nobody to wait for, work on one
         # stream is in order, and one_shot overwrites the whole output (64 x 2880 bf16: 25 us with it, 8 without).
         ctx.check_status()
@@ -163,6 +164,7 @@ def all_reduce(output_tensor, input_tensor, ctx, op=None, group=None, async_op=F
     )
     workspace.prepared = False
     workspace.stream = stream
+    workspace.captured = workspace.captured or capturing(stream)
     if not async_op:
         ctx.barrier()
     return workspace

@@ -683,6 +683,15 @@ void iris_hip_set_split_tiles(int32_t mode) { iris_host::set_split_tile_mode(mod
 
 const char* iris_hip_last_error(void) { return g_last_error; }
 const char* iris_hip_last_kernel(void) { return g_last_kernel; }
+int iris_hip_stream_capturing(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 int iris_hip_abi_version(void) { return 6; }
 
 }  // extern "C"

@@ -68,6 +68,8 @@ PyObject* call(int (*fn)(A...), const char* name, PyObject* const* args, Py_ssiz
   X(iris_hip_all_reduce)            \
   X(iris_hip_reduce_scatter)
 
+int (*fn_stream_capturing)(void*) = nullptr;
+
 #define DEFINE(name)                     \
   decltype(&::name) fn_##name = nullptr; \
   PyObject* py_##name(PyObject*, PyObject* const* args, Py_ssize_t n) { return call(fn_##name, #name, args, n); }
@@ -82,6 +84,8 @@ PyObject* load(PyObject*, PyObject* path_object) {
   fn_##name = (decltype(fn_##name))dlsym(lib, #name); \
   if (!fn_##name) return PyErr_Format(PyExc_OSError, "%s has no %s", path, #name);
   ENTRY_POINTS(RESOLVE)
+  fn_stream_capturing = (decltype(fn_stream_capturing))dlsym(lib, "iris_hip_stream_capturing");
+  if (!fn_stream_capturing) return PyErr_Format(PyExc_OSError, "%s has no iris_hip_stream_capturing", path);
   Py_RETURN_NONE;
 }
 
@@ -93,7 +97,7 @@ PyObject* load(PyObject*, PyObject* path_object) {
   X(runs_alone) X(block_size_m) X(block_size_n) X(block_size_k) X(group_size_m) X(num_sms) X(num_xcds) X(chunk_size)     \
   X(all_reduce_variant) X(all_reduce_num_rings) X(all_reduce_distribution) X(reduce_scatter_variant) X(swizzle_size)     \
   X(comm_sms) X(use_gluon) X(operation) X(shape) X(dtype) X(world_size) X(variant) X(aux_buffer) X(locks) X(prepared)    \
-  X(stream)
+  X(stream) X(captured)
 #define ATTRIBUTE_NAME(name) PyObject* at_##name = nullptr;
 ATTRIBUTES(ATTRIBUTE_NAME)
 
@@ -215,6 +219,15 @@ int acc_code(PyObject* rule) {
   return is_text(rule, "fp32") ? IRIS_HIP_ACC_FP32 : IRIS_HIP_ACC_REFERENCE;
 }
 
+// Whether a workspace that has been used may be used again by a call on `stream` as it is: the last launch was on the same
+// stream, and neither that nor an earlier one, nor this one, is part of a graph.
+void require_same_stream(PyObject* ws, const Shmem& shmem, PyObject* stream) {
+  const Ref last(PyObject_GetAttr(ws, at_stream));
+  require(last.o != Py_None && PyLong_AsUnsignedLongLong(last.o) == PyLong_AsUnsignedLongLong(stream) && !PyErr_Occurred());
+  require(Ref(PyObject_GetAttr(ws, at_captured)).o == Py_False && !fn_stream_capturing(PyLong_AsVoidPtr(stream)));
+  require(shmem.runs_alone() && *shmem.status() == 0);  // (a status to report is the wrapper's business)
+}
+
 // The buffers of a workspace that this very call used before (or, when `prepared` counts, has been prepared for).
 struct Workspace {
   void* aux = nullptr;
@@ -230,11 +243,7 @@ struct Workspace {
             as_int(PyTuple_GET_ITEM(shape.o, 1)) == C.cols && as_int(PyTuple_GET_ITEM(shape.o, 2)) == A.cols);
     require(THPDtype_Check(dtype.o) && ((THPDtype*)dtype.o)->scalar_type == A.t.scalar_type());
     clear = !(prepared_counts && Ref(PyObject_GetAttr(ws, at_prepared)).o == Py_True);
-    if (clear) {
-      const Ref last(PyObject_GetAttr(ws, at_stream));
-      require(last.o != Py_None && PyLong_AsUnsignedLongLong(last.o) == PyLong_AsUnsignedLongLong(stream) && !PyErr_Occurred());
-      require(shmem.runs_alone() && *shmem.status() == 0);  // (a status to report is the wrapper's business)
-    }
+    if (clear) require_same_stream(ws, shmem, stream);
     if (strcmp(variant, "atomic") == 0) {
       require(shmem.symmetric(C.t));
       return;
@@ -274,7 +283,9 @@ PyObject* attempt(Py_ssize_t n, Py_ssize_t expected, F&& body) {
 // Notes in the workspace that a launch (whose result is `rc`) has used it; returns rc, or NULL with a Python error set.
 PyObject* used(PyObject* rc, PyObject* ws, PyObject* stream, bool unprepare) {
   if (!rc || PyLong_AsLong(rc) != 0) return rc;
-  if ((unprepare && PyObject_SetAttr(ws, at_prepared, Py_False) != 0) || PyObject_SetAttr(ws, at_stream, stream) != 0) Py_CLEAR(rc);
+  if ((unprepare && PyObject_SetAttr(ws, at_prepared, Py_False) != 0) || PyObject_SetAttr(ws, at_stream, stream) != 0 ||
+      (fn_stream_capturing(PyLong_AsVoidPtr(stream)) && PyObject_SetAttr(ws, at_captured, Py_True) != 0))
+    Py_CLEAR(rc);
   return rc;
 }
 
@@ -422,11 +433,7 @@ PyObject* try_ccl_all_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
     require(PyTuple_CheckExact(shape.o) && PyTuple_GET_SIZE(shape.o) == 2 && as_int(PyTuple_GET_ITEM(shape.o, 0)) == c.in.rows &&
             as_int(PyTuple_GET_ITEM(shape.o, 1)) == c.in.cols);
     require(THPDtype_Check(dtype.o) && ((THPDtype*)dtype.o)->scalar_type == c.in.t.scalar_type());
-    if (Ref(PyObject_GetAttr(ws, at_prepared)).o != Py_True) {
-      const Ref last(PyObject_GetAttr(ws, at_stream));
-      require(last.o != Py_None && PyLong_AsUnsignedLongLong(last.o) == PyLong_AsUnsignedLongLong(a[5]) && !PyErr_Occurred());
-      require(c.shmem.runs_alone() && *c.shmem.status() == 0);
-    }
+    if (Ref(PyObject_GetAttr(ws, at_prepared)).o != Py_True) require_same_stream(ws, c.shmem, a[5]);
     const int64_t* const bases = c.shmem.words(at_heap_bases);
     void* const stream = PyLong_AsVoidPtr(a[5]);
     PyObject* const rc = launch([&] {

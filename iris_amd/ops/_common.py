@@ -70,6 +70,11 @@ def current_stream(shmem):
     return torch._C._cuda_getCurrentRawStream(device) if device >= 0 else None
 
 
+def capturing(stream):
+    """True while launches on a raw HIP stream are recorded into a graph."""
+    return stream is not None and _lib.library().iris_hip_stream_capturing(stream) != 0
+
+
 def native(shmem):
     """The module that takes whole operator calls (csrc/launcher.cpp), or None where the Python wrapper has to: on a
     host-backed context and while DEBUG records are wanted.  Its try_<op> functions return None, with nothing done,
@@ -86,16 +91,18 @@ def rearmed(shmem, workspace, C, operation, shape, dtype, world_size, variant, t
     tiles of C that this rank reduces are overwritten by the launch, the remaining tiles of C are zeroed by the
     launch itself (_lib.CLEAR_C), and work on one stream is ordered without the host waiting for the device
     (decode-sized calls: 32 us with the preamble's three fills and its barrier, 10 us without; 8192 x 4096 reduce-scatter
-    150 and 118 us).  Another stream than last time, other shapes or a process group: the preamble runs.
+    150 and 118 us).  Another stream than last time, other shapes or a process group: the preamble runs.  So it does under
+    graph capture, which its barrier does not allow, and once a graph holds a launch that uses the buffers: a
+    replay does not show here, and may run on any stream.
     """
-    if (workspace is None or stream is None or workspace.stream != stream or workspace.variant != variant or workspace.shape != shape
+    if (workspace is None or stream is None or workspace.captured or workspace.stream != stream or workspace.variant != variant or workspace.shape != shape
             or workspace.dtype != dtype or workspace.world_size != world_size or workspace.operation != operation):
         return False
     if variant != "atomic":
         locks, aux = workspace.locks, workspace.aux_buffer
         if locks is None or aux is None or locks.numel() != tiles or aux.shape != C.shape or aux.dtype != C.dtype:
             return False
-    return shmem.runs_alone()
+    return shmem.runs_alone() and not capturing(stream)
 
 
 def check_launch(err, rank):

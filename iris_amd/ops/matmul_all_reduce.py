@@ -12,7 +12,7 @@ import torch
 
 from .. import _lib
 from ..host.logging import debug_on, log_rank
-from ._common import (acc_code, check_launch, current_stream, dtype_code, iris_launch, is_fp8, native, path_code, ptr,
+from ._common import (acc_code, capturing, check_launch, current_stream, dtype_code, iris_launch, is_fp8, native, path_code, ptr,
                       rearmed, require_gpu_tensors, stage_idle_peers)
 from .config import FusedConfig
 from .workspace import FusedWorkspace
@@ -208,6 +208,7 @@ def matmul_all_reduce(
 
     workspace.prepared = False
     workspace.stream = stream
+    workspace.captured = workspace.captured or capturing(stream)
     if not async_op:
         shmem.barrier()
     return workspace

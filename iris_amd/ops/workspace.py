@@ -20,6 +20,7 @@ class FusedWorkspace:
     locks: Optional[torch.Tensor] = None  # int32 ready flag per flag tile
     prepared: bool = False
     stream: Optional[int] = None  # raw HIP stream of the last launch that used the buffers
+    captured: bool = False  # a graph holds a launch that uses the buffers, on whatever stream it is replayed
 
     def matches(self, operation, shape, dtype, world_size, variant="") -> bool:
         """True when the buffers were prepared for exactly this call and have not been used since."""

@@ -3,6 +3,7 @@ call with one leaves - own tiles reduced, every other tile of C zero - on each k
 
 import ctypes
 import subprocess
+import sys
 
 import pytest
 import torch
@@ -140,6 +141,7 @@ int iris_hip_all_gather_matmul() { return ++calls, 98; }
 int iris_hip_matmul_all_gather() { return ++calls, 98; }
 int iris_hip_all_reduce() { return ++calls, 98; }
 int iris_hip_reduce_scatter() { return ++calls, 98; }
+int iris_hip_stream_capturing() { return 0; }
 """
 
 
@@ -178,3 +180,73 @@ def test_a_failed_launch_is_reported_and_not_repeated(tmp_path):
     assert ws.prepared and ws.stream is None and ccl.prepared and ccl.stream is None
     for call in calls:
         call()
+
+
+class _Preamble(Exception):
+    pass
+
+
+@pytest.mark.parametrize("op", ["one_shot", "atomic", "reduce_scatter", "ccl"])
+@pytest.mark.parametrize("wrapper", [False, True], ids=["native", "wrapper"])
+def test_launches_in_graphs_and_the_preamble(op, wrapper, monkeypatch):
+    """A used workspace is not taken as it is while a graph is recorded (the preamble, which cannot be recorded, is asked
+    for), nor ever again once a launch that uses it is part of a graph, whose replays run on any stream."""
+    W, M, N, K, dtype = 2, 64, 128, 64, torch.bfloat16
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=0)
+    A, B, C, x = (ctx.zeros(s, dtype=dtype) for s in ((M, K), (K, N), (M, N), (M, N)))
+    cfg = iris.FusedConfig(block_size_m=32, block_size_n=32, block_size_k=32, all_reduce_variant="two_shot" if op == "reduce_scatter" else op)
+    ccl_cfg = Config(all_reduce_variant="one_shot")
+    if op == "ccl":
+        module, name = sys.modules["iris_amd.ccl.all_reduce"], "all_reduce_preamble"
+        ws = ctx.ccl.all_reduce_preamble(C, x, config=ccl_cfg)
+        call = lambda: ctx.ccl.all_reduce(C, x, async_op=True, config=ccl_cfg, workspace=ws)
+    elif op == "reduce_scatter":
+        module, name = sys.modules["iris_amd.ops.matmul_reduce_scatter"], "matmul_reduce_scatter_preamble"
+        ws = ops.matmul_reduce_scatter_preamble(ctx, C, A, B, config=cfg)
+        call = lambda: ctx.ops.matmul_reduce_scatter(C, A, B, async_op=True, config=cfg, workspace=ws, sum_peers=False)
+    else:
+        module, name = sys.modules["iris_amd.ops.matmul_all_reduce"], "matmul_all_reduce_preamble"
+        ws = ops.matmul_all_reduce_preamble(ctx, C, A, B, config=cfg)
+        call = lambda: ctx.ops.matmul_all_reduce(C, A, B, async_op=True, config=cfg, workspace=ws)
+        if op == "one_shot":
+            stage_peers(ctx, ws, [C] * W)
+    preamble, asked = getattr(module, name), []
+
+    def refuse(*args, **kwargs):
+        asked.append(1)
+        raise _Preamble
+
+    if wrapper:
+        monkeypatch.setattr(module, "native", lambda shmem: None)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+        call()
+        torch.cuda.synchronize()
+        monkeypatch.setattr(module, name, refuse)
+        call()  # as it is, without the preamble (the reduce-scatter's first call ran it)
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            with pytest.raises(_Preamble):
+                call()
+            if op != "reduce_scatter":  # (which has no launch without a preamble before it)
+                ws.prepared = True
+                call()
+        assert len(asked) == 1
+        if op == "reduce_scatter":
+            return
+        for _ in range(2):
+            graph.replay()
+            torch.cuda.synchronize()
+            ctx.check_status()
+            assert torch.all(C == 0)
+        with pytest.raises(_Preamble):
+            call()
+        monkeypatch.setattr(module, name, preamble)
+        call()  # with the preamble, and the next one too
+        monkeypatch.setattr(module, name, refuse)
+        with pytest.raises(_Preamble):
+            call()
+        torch.cuda.synchronize()
