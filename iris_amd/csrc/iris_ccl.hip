@@ -358,7 +358,6 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
     p.tiles_n = cdiv(p.N, p.bn);
     const long long total = (long long)p.tiles_m * p.tiles_n;
     if (total >= (1ll << 31)) return fail("too many tiles");
-    if ((long long)p.bm * p.bn >= (1ll << 31)) return fail("block sizes %d x %d are too large", p.bm, p.bn);
     if (p.group_m > p.tiles_m) p.group_m = p.tiles_m;  // the same order
     const int per_rank = (int)((total + p.world - 1) / p.world);
     if (distribution == IRIS_HIP_DISTRIBUTION_STRIDED) {
@@ -374,9 +373,9 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
     }
   }
   // Bytes that the launch moves.
-  const long long moved = (tiled ? (long long)p.n_owned * p.bm * p.bn : (long long)p.M * p.N) * es *
-                          (p.mode == CCL_TWO_SHOT ? 2 * p.world : p.world + 1);
-  const bool large = moved > (32ll << 20);
+  const double moved = (tiled ? (double)p.n_owned * p.bm * p.bn : (double)p.M * p.N) * es *
+                       (p.mode == CCL_TWO_SHOT ? 2 * p.world : p.world + 1);
+  const bool large = moved > (double)(32 << 20);
   // Large launches of the block distribution walk their tiles' rows instead of one tile after the other.
   const bool rows = tiled && large && p.tile_stride == 1;
 
@@ -391,8 +390,11 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   const char* const in_end = p.in + ((long long)(p.M - 1) * p.s_im + p.N) * es;
   const char* const out_end = p.out + ((long long)(p.M - 1) * p.s_om + p.N) * es;
   const bool apart = p.s_im >= 0 && p.s_om >= 0 && (in_end <= p.out || out_end <= p.in);
-  const bool vec_ok = p.s_in == 1 && p.s_on == 1 && !(tiled && p.bn % vec_full) &&
-                      (whole || (p.mode != CCL_ATOMIC && (p.mode != CCL_TWO_SHOT || rows) && p.N >= vec_full && apart));
+  const bool unit_stride = p.s_in == 1 && p.s_on == 1 && !(tiled && p.bn % vec_full);
+  // (A tile may have fewer than 2^31 units; the limit does not move with what misaligned rows are walked in.)
+  if (tiled && (long long)cdiv(p.bn, unit_stride && whole ? vec_full : 1) * p.bm >= (1ll << 31))
+    return fail("block sizes %d x %d are too large", p.bm, p.bn);
+  const bool vec_ok = unit_stride && (whole || (p.mode != CCL_ATOMIC && (p.mode != CCL_TWO_SHOT || rows) && p.N >= vec_full && apart));
   int vec = vec_ok ? vec_full : 1;
   // The atomic variant adds one dword at a time (packed 16-bit pairs, or one float): with a dword per
   // thread a wave instruction covers 256 contiguous bytes, two whole lines for the L2's atomic units;

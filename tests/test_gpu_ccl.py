@@ -232,3 +232,20 @@ def test_collectives_replay_in_a_hip_graph():
         for r, got in enumerate(slot_copies(ctx, d_ar)):
             assert_bits_equal(got, exp_ar[r], f"all_reduce slot {r}, replay {rep}")
         assert_bits_equal(d_rs.cpu(), exp_rs, f"reduce_scatter, replay {rep}")
+
+
+@pytest.mark.parametrize("distribution", [0, 1])
+def test_blocks_of_two_to_the_31_elements(distribution):
+    """The limit on block sizes counts 16-byte chunks where rows are whole chunks, elements elsewhere."""
+    W, M, N, dtype = 2, 64, 256, torch.bfloat16
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=0)
+    inputs = [randn_cpu((M, N), 60 + r, dtype) for r in range(W)]
+    d_in, d_out = _stage(ctx, inputs)
+    cfg = Config(block_size_m=1 << 16, block_size_n=1 << 15, all_reduce_distribution=distribution)
+    ctx.ccl.reduce_scatter(d_out, d_in, config=cfg)
+    assert_bits_equal(d_out.cpu(), (inputs[0].float() + inputs[1].float()).to(dtype), "one tile, rank 0's")
+    with pytest.raises(RuntimeError, match="block sizes"):
+        ctx.ccl.reduce_scatter(d_out[:, :250], d_in[:, :250], config=cfg)
+    cfg.block_size_n = 1 << 18
+    with pytest.raises(RuntimeError, match="block sizes"):
+        ctx.ccl.reduce_scatter(d_out, d_in, config=cfg)
