@@ -101,12 +101,16 @@ _launch = None
 
 def launcher():
     """The module iris_amd/lib/_launch.so: operator calls and the entry points behind them as built-in functions
-    (csrc/launcher.cpp).  Raises if it is not built."""
+    (csrc/launcher.cpp).  Raises if it is not built, or built for another torch or Python."""
     global _launch
     if _launch is None:
         library()  # checks the library and its version first
         if not os.path.exists(LAUNCHER_PATH):
             raise RuntimeError(f"{LAUNCHER_PATH} is missing: build it with `python -m iris_amd.csrc.build`")
+        from .csrc.build import launcher_fits, launcher_tag
+
+        if not launcher_fits(LAUNCHER_PATH):
+            raise RuntimeError(f"{LAUNCHER_PATH} is not an {launcher_tag()} build it again with `python -m iris_amd.csrc.build`")
         spec = importlib.util.spec_from_file_location("_launch", LAUNCHER_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)

@@ -42,8 +42,22 @@ FLAGS = [
 ]
 
 
+def launcher_tag():
+    """What _launch.so is tied to, as the text that its build puts into it: it reads the tensors of one torch for one
+    Python, and another one's differ without a symbol missing."""
+    import torch
+
+    return f"iris_amd launcher for torch {torch.__version__}, {sysconfig.get_config_var('SOABI')};"
+
+
+def launcher_fits(path):
+    """True when the module at `path` was built for the torch and the Python that run."""
+    with open(path, "rb") as f:
+        return launcher_tag().encode() in f.read()
+
+
 def up_to_date():
-    if not (os.path.exists(OUTPUT) and os.path.exists(LAUNCHER_OUTPUT)):
+    if not (os.path.exists(OUTPUT) and os.path.exists(LAUNCHER_OUTPUT) and launcher_fits(LAUNCHER_OUTPUT)):
         return False
     built = min(os.path.getmtime(OUTPUT), os.path.getmtime(LAUNCHER_OUTPUT))
     return all(os.path.getmtime(f) <= built for f in SOURCES + HEADERS + [LAUNCHER_SOURCE, os.path.abspath(__file__)])
@@ -56,7 +70,7 @@ def _build_launcher(verbose):
     tmp = LAUNCHER_OUTPUT + ".tmp"
     includes = [sysconfig.get_paths()["include"]] + include_paths()
     _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
-          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-I" + os.path.join(ROOT, "include")]
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f'-DIRIS_LAUNCHER_TAG="{launcher_tag()}"', "-I" + os.path.join(ROOT, "include")]
          + [flag for path in includes for flag in ("-isystem", path)] + ["-o", tmp, LAUNCHER_SOURCE]
          + ["-L" + path for path in library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"], verbose)
     os.replace(tmp, LAUNCHER_OUTPUT)

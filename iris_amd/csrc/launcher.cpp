@@ -478,5 +478,7 @@ PyMODINIT_FUNC PyInit__launch() {
 #define INTERN(name) \
   if (!(at_##name = PyUnicode_InternFromString(#name))) return nullptr;
   ATTRIBUTES(INTERN)
-  return PyModule_Create(&module_definition);
+  PyObject* const module = PyModule_Create(&module_definition);
+  if (module && PyModule_AddStringConstant(module, "BUILT_FOR", IRIS_LAUNCHER_TAG) != 0) return nullptr;
+  return module;
 }

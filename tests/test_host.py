@@ -293,6 +293,17 @@ def test_a_library_that_does_not_know_clear_c_is_refused(tmp_path):
     assert out.returncode != 0 and "has ABI version 5" in out.stderr, out.stderr[-500:]
 
 
+def test_a_launcher_of_another_torch_or_python_is_refused(monkeypatch):
+    from iris_amd.csrc import build
+
+    assert _lib.launcher().BUILT_FOR == build.launcher_tag() and build.launcher_fits(_lib.LAUNCHER_PATH)
+    monkeypatch.setattr(torch, "__version__", torch.__version__ + "1")
+    monkeypatch.setattr(_lib, "_launch", None)
+    assert not build.up_to_date()
+    with pytest.raises(RuntimeError, match="build it again"):
+        _lib.launcher()
+
+
 def test_null_context_tensor_is_rejected_before_any_launch():
     """Every kernel translates addresses through the heap bases, so a NULL context tensor is an
     argument error for every fused entry point, whatever the world size; the check comes before the
