@@ -250,3 +250,31 @@ def test_launches_in_graphs_and_the_preamble(op, wrapper, monkeypatch):
         with pytest.raises(_Preamble):
             call()
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("variant,W,rank", [("one_shot", 4, 1), ("two_shot", 1, 0)])
+def test_second_call_of_a_split_launch(variant, W, rank):
+    """The last round's tiles split between workgroups, flag tiles higher than the workgroups' (their arrivals are counted
+    in the flag): calls that find their own flags up give what the oracle gives."""
+    M, N, K, dtype = 5120, 3840, 200, torch.bfloat16
+    ctx = iris.iris(1 << 29, num_ranks=W, rank=rank)
+    B = randint_cpu((K, N), 6, dtype)
+    peers = [randn_cpu((M, N), 40 + r, dtype) for r in range(W)]
+    cfg = iris.FusedConfig(block_size_m=384, block_size_n=64, block_size_k=32, all_reduce_variant=variant)
+    dA, dB, dC = ctx.zeros((M, K), dtype=dtype), heap_tensor(ctx, B), ctx.zeros((M, N), dtype=dtype)
+    ws = ops.matmul_all_reduce_preamble(ctx, dC, dA, dB, config=cfg)
+    stage_peers(ctx, ws, peers)
+    _lib.library().iris_hip_set_split_tiles(1)
+    try:
+        for turn in range(3):
+            A = randint_cpu((M, K), 5 + turn, dtype)
+            dA.copy_(A)
+            if turn:
+                dC.fill_(float("nan"))
+            ws = ops.matmul_all_reduce(ctx, dC, dA, dB, config=cfg, workspace=ws)
+            assert _lib.last_kernel().endswith("_splitk"), _lib.last_kernel()
+            exp = oracle.matmul_all_reduce(A, B, peers, rank, W, 384, 64, variant, "fp32")
+            assert torch.equal(ws.locks.cpu(), torch.from_numpy(exp["locks"])), "flags"
+            assert_bits_equal(dC.cpu(), exp["C"][rank], f"turn {turn}")
+    finally:
+        _lib.library().iris_hip_set_split_tiles(-1)
