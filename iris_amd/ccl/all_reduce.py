@@ -100,7 +100,9 @@ def all_reduce(output_tensor, input_tensor, ctx, op=None, group=None, async_op=F
     must be on the symmetric heap, and so must the output for "two_shot" and "atomic", which write the
     peers' outputs.  op: only ReduceOp.SUM.  group: None, a ProcessGroup, or a list of ranks.
     async_op=False ends with ctx.barrier().  Returns the workspace with prepared=False, as the
-    reference does.
+    reference does.  A workspace that was last used by the same call on the same stream needs no preamble when this
+    process plays every rank alone and no graph holds a launch with it (see ops.matmul_all_reduce for what that leaves
+    to the caller); in place, one_shot then keeps the own input, which its preamble zeroes.
     """
     if op is None:
         op = ReduceOp.SUM

@@ -98,6 +98,13 @@ def matmul_all_reduce(
     aux buffers once their flags are up) into its own C; with "two_shot" it does so only for the
     tiles t with t % world_size == rank and writes the result into every rank's C.
 
+    The preamble runs when `workspace` is not freshly prepared.  A workspace that was last used by the same call (shapes,
+    variant) on the same stream, in a process that plays every rank alone (no process group, no
+    stand_in_peers), is used again without it, unless this launch or an earlier one with it is part of a graph: C
+    ends up as with the preamble, peers' C are left alone.  Nothing waits for the device then: what was written to A, B
+    or staged peers on other streams is for the caller to order, the own flags read 1 from the call before, and a
+    time-out of an asynchronous call is raised by the first call or barrier that finds it.
+
     Keyword-only additions to the reference signature:
         scale_a, scale_b: per-tensor dequantisation scales for float8_e4m3fn inputs (C is bfloat16
             or float16 then); the fp32 product is multiplied by scale_a * scale_b before the cast.

@@ -91,14 +91,17 @@ def matmul_reduce_scatter(
     kernel_path: str = "auto",
     stage=None,
 ) -> FusedWorkspace:
-    """C = reduce_scatter(A @ B) for this rank: C holds the reduced tiles this rank owns.
+    """C = reduce_scatter(A @ B) for this rank: C holds the reduced tiles this rank owns, zeros elsewhere.
+
+    The preamble runs on every call, except with `stage` None and a workspace that can be used as it is (conditions and
+    consequences: matmul_all_reduce).
 
     Keyword-only additions to the reference signature:
         all_owners: one GPU stands in for every rank's reduce step: each tile t is reduced and stored
             into C of slot owner(t) (with the default 256 x 64 tiles, contiguous row blocks per slot).
         sum_peers: if False, the peers contribute nothing (their flags and aux are not read).
-        stage: optional callable `stage(workspace)` run after the preamble (which zeroes the
-            workspace on every call) and before the launch - the place to write peers' partial
+        stage: optional callable `stage(workspace)` run after the preamble (which always runs then and
+            zeroes the workspace) and before the launch - the place to write peers' partial
             results and flags into the other slots when one GPU plays all ranks.
         scale_a, scale_b, slot_sum, kernel_path: as for matmul_all_reduce.
     """
