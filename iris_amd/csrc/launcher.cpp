@@ -219,12 +219,15 @@ int acc_code(PyObject* rule) {
   return is_text(rule, "fp32") ? IRIS_HIP_ACC_FP32 : IRIS_HIP_ACC_REFERENCE;
 }
 
+bool is_capturing(PyObject* stream) { return fn_stream_capturing(PyLong_AsVoidPtr(stream)) != 0; }
+
 // Whether a workspace that has been used may be used again by a call on `stream` as it is: the last launch was on the same
 // stream, and neither that nor an earlier one, nor this one, is part of a graph.
-void require_same_stream(PyObject* ws, const Shmem& shmem, PyObject* stream) {
+// (`capturing`: what is_capturing() says of the stream; asking HIP takes 0.15 us, so once per call.)
+void require_same_stream(PyObject* ws, const Shmem& shmem, PyObject* stream, bool capturing) {
   const Ref last(PyObject_GetAttr(ws, at_stream));
   require(last.o != Py_None && PyLong_AsUnsignedLongLong(last.o) == PyLong_AsUnsignedLongLong(stream) && !PyErr_Occurred());
-  require(Ref(PyObject_GetAttr(ws, at_captured)).o == Py_False && !fn_stream_capturing(PyLong_AsVoidPtr(stream)));
+  require(Ref(PyObject_GetAttr(ws, at_captured)).o == Py_False && !capturing);
   require(shmem.runs_alone() && *shmem.status() == 0);  // (a status to report is the wrapper's business)
 }
 
@@ -234,7 +237,7 @@ struct Workspace {
   int32_t* locks = nullptr;
   bool clear = false;  // reused without a preamble (rearmed() of the Python side states the conditions)
   Workspace(PyObject* ws, const Shmem& shmem, const char* operation, const char* variant, bool prepared_counts, const Matrix& A,
-            const Matrix& C, int64_t tiles, PyObject* stream) {
+            const Matrix& C, int64_t tiles, PyObject* stream, bool capturing) {
     require(ws != Py_None);
     require(is_text(Ref(PyObject_GetAttr(ws, at_operation)).o, operation) && is_text(Ref(PyObject_GetAttr(ws, at_variant)).o, variant));
     require(int_of(ws, at_world_size) == shmem.world);
@@ -243,7 +246,7 @@ struct Workspace {
             as_int(PyTuple_GET_ITEM(shape.o, 1)) == C.cols && as_int(PyTuple_GET_ITEM(shape.o, 2)) == A.cols);
     require(THPDtype_Check(dtype.o) && ((THPDtype*)dtype.o)->scalar_type == A.t.scalar_type());
     clear = !(prepared_counts && Ref(PyObject_GetAttr(ws, at_prepared)).o == Py_True);
-    if (clear) require_same_stream(ws, shmem, stream);
+    if (clear) require_same_stream(ws, shmem, stream, capturing);
     if (strcmp(variant, "atomic") == 0) {
       require(shmem.symmetric(C.t));
       return;
@@ -281,10 +284,10 @@ PyObject* attempt(Py_ssize_t n, Py_ssize_t expected, F&& body) {
 }
 
 // Notes in the workspace that a launch (whose result is `rc`) has used it; returns rc, or NULL with a Python error set.
-PyObject* used(PyObject* rc, PyObject* ws, PyObject* stream, bool unprepare) {
+PyObject* used(PyObject* rc, PyObject* ws, PyObject* stream, bool capturing, bool unprepare) {
   if (!rc || PyLong_AsLong(rc) != 0) return rc;
   if ((unprepare && PyObject_SetAttr(ws, at_prepared, Py_False) != 0) || PyObject_SetAttr(ws, at_stream, stream) != 0 ||
-      (fn_stream_capturing(PyLong_AsVoidPtr(stream)) && PyObject_SetAttr(ws, at_captured, Py_True) != 0))
+      (capturing && PyObject_SetAttr(ws, at_captured, Py_True) != 0))
     Py_CLEAR(rc);
   return rc;
 }
@@ -303,7 +306,8 @@ PyObject* try_matmul_all_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const char* const name = is_text(variant.o, "one_shot") ? "one_shot" : is_text(variant.o, "two_shot") ? "two_shot" : "atomic";
     require(is_text(variant.o, name));
     const int code = name[0] == 'o' ? IRIS_HIP_VARIANT_ONE_SHOT : name[0] == 't' ? IRIS_HIP_VARIANT_TWO_SHOT : IRIS_HIP_VARIANT_ATOMIC;
-    const Workspace ws(a[5], shmem, "matmul_all_reduce", name, true, A, C, blocks.tiles(C.rows, C.cols), a[10]);
+    const bool capturing = is_capturing(a[10]);
+    const Workspace ws(a[5], shmem, "matmul_all_reduce", name, true, A, C, blocks.tiles(C.rows, C.cols), a[10], capturing);
     const int acc = acc_code(a[8]) | (ws.clear ? IRIS_HIP_CLEAR_C : 0), path = path_code(a[9]);
     const int64_t* const context = shmem.words(at__device_context);
     const long long spin = int_of(a[0], at_spin_limit);
@@ -314,7 +318,7 @@ PyObject* try_matmul_all_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                            context, shmem.rank, shmem.world, blocks.m, blocks.n, blocks.k, code, types.in, types.out,
                                            types.scale, acc, spin, status, path, stream);
     });
-    return used(rc, a[5], a[10], true);
+    return used(rc, a[5], a[10], capturing, true);
   });
 }
 
@@ -329,7 +333,8 @@ PyObject* try_matmul_reduce_scatter(PyObject*, PyObject* const* a, Py_ssize_t n)
     Blocks::validate(a[4]);
     const Ref variant(PyObject_GetAttr(a[4], at_all_reduce_variant));
     require(is_text(variant.o, "two_shot") || is_text(variant.o, "one_shot") || is_text(variant.o, "atomic"));
-    const Workspace ws(a[5], shmem, "matmul_reduce_scatter", "two_shot", false, A, C, blocks.tiles(C.rows, C.cols), a[12]);
+    const bool capturing = is_capturing(a[12]);
+    const Workspace ws(a[5], shmem, "matmul_reduce_scatter", "two_shot", false, A, C, blocks.tiles(C.rows, C.cols), a[12], capturing);
     const int acc = acc_code(a[10]) | IRIS_HIP_CLEAR_C, path = path_code(a[11]);
     const int all_owners = PyObject_IsTrue(a[6]), sum_peers = PyObject_IsTrue(a[7]);
     require(all_owners >= 0 && sum_peers >= 0);
@@ -342,7 +347,7 @@ PyObject* try_matmul_reduce_scatter(PyObject*, PyObject* const* a, Py_ssize_t n)
                                                C.s1, context, shmem.rank, shmem.world, blocks.m, blocks.n, blocks.k, all_owners, sum_peers,
                                                types.in, types.out, types.scale, acc, spin, status, path, stream);
     });
-    return used(rc, a[5], a[12], false);
+    return used(rc, a[5], a[12], capturing, false);
   });
 }
 
@@ -433,7 +438,8 @@ PyObject* try_ccl_all_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
     require(PyTuple_CheckExact(shape.o) && PyTuple_GET_SIZE(shape.o) == 2 && as_int(PyTuple_GET_ITEM(shape.o, 0)) == c.in.rows &&
             as_int(PyTuple_GET_ITEM(shape.o, 1)) == c.in.cols);
     require(THPDtype_Check(dtype.o) && ((THPDtype*)dtype.o)->scalar_type == c.in.t.scalar_type());
-    if (Ref(PyObject_GetAttr(ws, at_prepared)).o != Py_True) require_same_stream(ws, c.shmem, a[5]);
+    const bool capturing = is_capturing(a[5]);
+    if (Ref(PyObject_GetAttr(ws, at_prepared)).o != Py_True) require_same_stream(ws, c.shmem, a[5], capturing);
     const int64_t* const bases = c.shmem.words(at_heap_bases);
     void* const stream = PyLong_AsVoidPtr(a[5]);
     PyObject* const rc = launch([&] {
@@ -441,7 +447,7 @@ PyObject* try_ccl_all_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     c.shmem.rank, c.shmem.world, 0, 1, c.bm, c.bn, c.swizzle, c.sms, c.xcds, c.chunk,
                                     one_shot ? IRIS_HIP_VARIANT_ONE_SHOT : IRIS_HIP_VARIANT_TWO_SHOT, c.distribution, c.type, stream);
     });
-    return used(rc, ws, a[5], true);
+    return used(rc, ws, a[5], capturing, true);
   });
 }
 
