@@ -1,13 +1,13 @@
 """Where the time of one fused launch goes: phase boundaries stamped inside the kernel.
 
     python -m iris_amd.csrc.build --stamps          # builds lib/libiris_hip_stamps.so
-    python -m iris_amd.bench.phase_stamps [--workload NAME] [--world W] [--flush zero|read|none] [--reps N]
+    python -m iris_amd.bench.phase_stamps [--workload NAME | --case NAME] [--world W] [--flush zero|read|none] [--reps N]
 
 The diagnostic build of the library records the device's constant-rate counter (s_memrealtime) in
 thread 0 of every workgroup at the phase boundaries of its first eight tiles.  This tool runs a workload of
-bench.py against that build and prints, per phase, the mean and the maximum over the workgroups, and
-the span from the first workgroup's entry to the last workgroup's last store.  Figures include the cost
-of the stamps themselves (one store per phase and workgroup).
+bench.py, or a listed case of perf/cases.py, against that build and prints, per phase, the mean and the
+maximum over the workgroups, and the span from the first workgroup's entry to the last workgroup's last
+store.  Figures include the cost of the stamps themselves (one store per phase and workgroup).
 """
 
 import argparse
@@ -28,6 +28,7 @@ PHASES = ["entry -> first operands in LDS", "K loop", "tile staged in LDS", "pha
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--workload", default=None)
+    ap.add_argument("--case", default=None, help="a listed case of perf/cases.py instead of a workload")
     ap.add_argument("--world", type=int, default=8)
     ap.add_argument("--flush", default="zero", choices=["zero", "read", "none"],
                     help="before every launch: zero a 256 MB buffer (the reference's do_bench), read it, or nothing")
@@ -63,8 +64,16 @@ def main():
 
     if args.split is not None:
         lib.iris_hip_set_split_tiles(args.split)
-    wl = bench.WORKLOADS[args.workload or bench.DEFAULT]()
-    wl.setup(iris, args.world)
+    if args.case:
+        from perf import cases
+
+        case = next(c for c in cases.listed() if c["name"] == args.case)
+        state, name, world = cases.prepare(case, 1), args.case, case["W"]
+        step = lambda: cases.run(state)
+    else:
+        wl = bench.WORKLOADS[args.workload or bench.DEFAULT]()
+        wl.setup(iris, args.world)
+        step, name, world = wl.step, wl.name, args.world
     max_wgs = 65536  # rows of the stamp buffer: tiles stamped per launch (eight per workgroup at most)
     stamps = torch.zeros((max_wgs, 16), dtype=torch.int64, device="cuda")
     cache = torch.empty(int(256e6) // 4, dtype=torch.int, device="cuda")
@@ -80,7 +89,7 @@ def main():
         stamps.zero_()
         torch.cuda.synchronize()
         lib.iris_hip_debug_set_stamps(ctypes.c_void_p(stamps.data_ptr()), stamps.shape[0])
-        wl.step()
+        step()
         torch.cuda.synchronize()
         lib.iris_hip_debug_set_stamps(ctypes.c_void_p(0), 0)
         if rep < 0:
@@ -106,7 +115,7 @@ def main():
             per_phase_max[i].append(float(d.max()) if d.numel() else 0.0)
             prev = torch.where(cur != 0, cur, prev)
         spans.append(float(t[:, last].max()) - t0)
-    print(f"workload {wl.name}  W={args.world}  kernel {_lib.last_kernel()}  tiles stamped {t.shape[0]}  flush={args.flush}  "
+    print(f"workload {name}  W={world}  kernel {_lib.last_kernel()}  tiles stamped {t.shape[0]}  flush={args.flush}  "
           f"{args.reps} launches; microseconds, mean over launches of (mean | max over tiles)")
     print(f"  {'workgroup entry after the first one':40s} {statistics.mean(entry_spread):8.2f}")
     for name, mean, mx in zip(PHASES, per_phase, per_phase_max):

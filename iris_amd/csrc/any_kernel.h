@@ -5,10 +5,10 @@
 // Where it differs from those kernels is the way of the operands: 16-byte pieces travel HBM -> registers ->
 // LDS (global loads take any alignment; the direct-to-LDS load is used only where its pieces are
 // aligned), one K step ahead in registers and one in the second LDS buffer.  The LDS layouts, the MFMA
-// operand lanes and the order of the epilogue are the same.  What bounds it: the matrix pipes for
-// float32 (as three bf16 pieces per operand, see SPLIT; 157 TFLOP/s at most on its own MFMA), the LDS for the
-// 16- and 8-bit types (the fragment reads of a 64x64 wave block need its full rate), the epilogue's HBM streams
-// with peers.
+// operand lanes and the order of the epilogue are the same.  What bounds it on the small tiles is no unit's rate but
+// the K step's chain - loads, LDS, barrier, fragments, products - which two or three workgroups per CU only partly hide
+// (over one launch of 64x128 tiles with its exchange: bf16 1999x2877x1371 MFMA 10 %, VALU 19 %, LDS 15 % busy; float32, as
+// three bf16 pieces per operand, 2048x2880x1024 27 %, 37 %, 23 %); with peers the epilogue's HBM streams come on top.
 //
 // Nothing on the hot path is predicated: rows past M (or N) repeat the last row, columns of B past N are
 // read as they lie in memory as long as the piece ends inside the operand - what they produce are output
@@ -434,8 +434,9 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     // 2^-110 (found while splitting), and tiles with a sum that is not finite (infinities and NaN, and values
     // that round to infinity in bf16), whose pieces need not add up to what the operands do.
     // The pieces are formed once per workgroup on the way from registers to LDS, 7 VALU instructions per
-    // element.  What bounds it: the matrix pipes at the clock they hold under load, the LDS (6 bytes written per
-    // element, 9 KiB read per 12 products of a 32x64 wave block) and the splitting, about equally.  The second sums
+    // element (15.6 of the 24.5 million of a 2048x2880x1024 launch).  What bounds it: splitting, products and LDS (6 bytes
+    // written per element, 9 KiB read per 12 products of a 32x64 wave block) one behind the other in a wave, 37, 27 and
+    // 23 % of the launch on the 64x128 tile.  The second sums
     // cost nothing (2048x2880x1024 two-shot 109.2 -> 108.1 us) but registers: a 256x128 tile, whose waves own 64x64, has none
     // left (169 spilled) and would have to keep one sum; it is 12 % faster (4096x4096x1536 267 us, 128x128 298) with 2.6
     // times the error, more than the float32 MFMA's where half of A is zero.
@@ -955,7 +956,7 @@ int launch_any(FusedParams p, int device, int cu_count, hipStream_t stream, cons
 // choice first (float32 without the largest): bf16 1999x2877x1371 64x128 41 (53 / 40 / - / 51 / 119), 1024x4095x2049 64x128 38 (68 / 40 /
 // - / 48 / 105), one-shot with seven peers 500x2877x1371 64x64 30 (92 / 46 / 32 / - / 51), 33x2877x1371 32x32 13 (49 / 31 / 25 / 20 / -);
 // float32 2048x2880x1024 64x128 98 (108 / - / 113 / 174), 2048x2048x4096 128x128 199 (- / 236 / 260 / 381), 512x2880x1024 64x64 40
-// (47 / 45 / - / 44), 300x4096x4096 32x32 129 (159 / 153 / 138 / -), 1536x2880x1024 64x64 87 (100 / 80 / - / 121).
+// (47 / 45 / - / 44), 300x4096x4096 32x32 129 (159 / 153 / 138 / -), and, the one miss, 1536x2880x1024 64x64 87 (100 / 80 / - / 121).
 struct AnyTile {
   int bm, bn;
   float rate;
