@@ -116,7 +116,8 @@ def all_reduce(output_tensor, input_tensor, ctx, op=None, group=None, async_op=F
     fast = native(ctx) if workspace is not None and group is None else None
     done = fast.try_ccl_all_reduce(ctx, output_tensor, input_tensor, config, workspace, current_stream(ctx)) if fast is not None else None
     if done is not None:
-        check_launch(done, ctx.get_rank())
+        if done:
+            check_launch(done, ctx.get_rank())
         if not async_op:
             ctx.barrier()
         return workspace

@@ -28,7 +28,8 @@ def reduce_scatter(output_tensor, input_tensor, ctx, op=None, group=None, async_
     fast = native(ctx) if group is None else None
     done = fast.try_ccl_reduce_scatter(ctx, output_tensor, input_tensor, config, current_stream(ctx)) if fast is not None else None
     if done is not None:
-        check_launch(done, ctx.get_rank())
+        if done:
+            check_launch(done, ctx.get_rank())
         if not async_op:
             ctx.barrier()
         return

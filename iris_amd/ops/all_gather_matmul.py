@@ -76,7 +76,8 @@ def all_gather_matmul(
     done = fast.try_all_gather_matmul(shmem, output_tensor, A_sharded, B, bias, config, gather_dim, scale_a,
                                       scale_b, kernel_path, current_stream(shmem)) if fast is not None else None
     if done is not None:
-        check_launch(done, shmem.get_rank())
+        if done:
+            check_launch(done, shmem.get_rank())
         if not async_op:
             shmem.barrier()
         if workspace is None:

@@ -64,7 +64,8 @@ def matmul_all_gather(
     done = fast.try_matmul_all_gather(shmem, output_tensor, A, B, bias, config, scale_a, scale_b, kernel_path,
                                       current_stream(shmem)) if fast is not None else None
     if done is not None:
-        check_launch(done, shmem.get_rank())
+        if done:
+            check_launch(done, shmem.get_rank())
         if not async_op:
             shmem.barrier()
         if workspace is None:

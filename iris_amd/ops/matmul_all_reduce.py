@@ -118,7 +118,8 @@ def matmul_all_reduce(
     done = fast.try_matmul_all_reduce(shmem, C, A, B, config, workspace, scale_a, scale_b, slot_sum,
                                       kernel_path, current_stream(shmem)) if fast is not None else None
     if done is not None:
-        check_launch(done, shmem.get_rank())
+        if done:
+            check_launch(done, shmem.get_rank())
         if not async_op:
             shmem.barrier()
         return workspace

@@ -111,7 +111,8 @@ def matmul_reduce_scatter(
     done = fast.try_matmul_reduce_scatter(shmem, C, A, B, config, workspace, all_owners, sum_peers, scale_a,
                                           scale_b, slot_sum, kernel_path, current_stream(shmem)) if fast is not None else None
     if done is not None:
-        check_launch(done, shmem.get_rank())
+        if done:
+            check_launch(done, shmem.get_rank())
         if not async_op:
             shmem.barrier()
         return workspace
