@@ -30,6 +30,7 @@ using namespace iris_layout;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(2))) int i32x2_t;
 typedef __attribute__((ext_vector_type(4))) int i32x4_t;
 typedef __attribute__((ext_vector_type(8))) int i32x8_t;
@@ -234,12 +235,15 @@ struct MfmaCfg {
   static constexpr int IN = IN_;
   static constexpr int ES = (IN_ == IN_FP8) ? 1 : 2;
   static constexpr int CE = kChunkBytes / ES;           // elements per 16-byte chunk
-  static constexpr int KM = (IN_ == IN_FP8) ? 64 : 16;  // k per MFMA
+  // MFMA block: 16x16x32 for 16-bit data on the eight-wave tile, else 32x32 (why: mfma_block16 below).
+  static constexpr int BLK = (IN_ != IN_FP8 && WM_ * WN_ == 8) ? 16 : 32;
+  static constexpr int KM = (IN_ == IN_FP8) ? 64 : BLK == 16 ? 32 : 16;  // k per MFMA
+  static constexpr int QUADS = BLK * BLK / 256;         // runs of four consecutive n that a lane owns of a block
   static constexpr int BM = BM_, BN = BN_, BK = BK_, STAGES = STAGES_;
   static constexpr bool B_KCONTIG = B_KCONTIG_;
   static constexpr int WM = WM_, WN = WN_, NW = WM_ * WN_, NT = 64 * NW;
   static constexpr int TM = BM / WM, TN = BN / WN;  // per-wave block
-  static constexpr int MB = TM / 32, NB = TN / 32;  // 32x32 MFMA blocks per wave
+  static constexpr int MB = TM / BLK, NB = TN / BLK;  // MFMA blocks per wave
   static constexpr int KSLICES = BK / KM;
   static constexpr int NFRAG = (IN_ == IN_FP8) ? 2 : 1;   // 16-byte pieces per operand fragment
   static constexpr int RBA = BK * ES;                        // bytes per A tile row
@@ -274,8 +278,8 @@ struct MfmaCfg {
   static constexpr int WAVES_PER_SIMD = WG_PER_CU * NW / 4;
   static_assert(NT % (BN / 8) == 0 && BM % (NT / (BN / 8)) == 0, "epilogue pass shape");
   static_assert(A_BYTES % (kDmaBytes * NW) == 0 && B_BYTES % (kDmaBytes * NW) == 0, "tile/loader mismatch");
-  static_assert(BK % KM == 0 && TM % 32 == 0 && TN % 32 == 0, "tile/MFMA mismatch");
-  static_assert(STAGES >= 3, "the ring needs at least three slots");
+  static_assert(BK % KM == 0 && TM % BLK == 0 && TN % BLK == 0, "tile/MFMA mismatch");
+  static_assert(STAGES >= (NW == 8 ? 5 : 3), "ring too short for the K loop");
   static_assert((STAGES - 2) * (LA + LB) <= 63, "vmcnt field too small for this prefetch depth");
 };
 
@@ -350,7 +354,7 @@ __device__ __forceinline__ unsigned lds_address(const void* p) {
 
 template <class CFG>
 struct MfmaAcc {
-  f32x16_t v[CFG::MB][CFG::NB];
+  typename std::conditional<CFG::BLK == 16, f32x4_t, f32x16_t>::type v[CFG::MB][CFG::NB];
 };
 
 // Operand fragments of one k-slice for a wave's block.
@@ -378,6 +382,26 @@ __device__ __forceinline__ f32x16_t mfma_block(const i32x4_t (&a)[NF], const i32
     // instruction (v_mfma_f32_32x32x64_f8f6f4).
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bv, av, c, 0, 0, 0, 0, 0, 0);
   }
+}
+
+// One 16x16 MFMA of 16-bit data, operands in the same order.  The tiled kernel multiplies with this shape: busy with
+// random data, the chip runs against its power limit, and a 16x16x32 product, which reads and writes its accumulators half
+// as often per flop as a 32x32x16 one, takes less of it (products from registers alone, eight waves of 128x64 per CU,
+// normal bf16 operands: 1750 against 2010 TFLOP/s, 2060 with the order of quad_block; both 2400 on zeros).  The
+// sums are the same, bit for bit: 32 k at a time in the same order.
+template <int IN>
+__device__ __forceinline__ f32x4_t mfma_block16(const i32x4_t (&a)[1], const i32x4_t (&b)[1], f32x4_t c) {
+  if constexpr (IN == IN_BF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b[0]), __builtin_bit_cast(bf16x8_t, a[0]), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, b[0]), __builtin_bit_cast(f16x8_t, a[0]), c, 0, 0, 0);
+}
+
+// The product a tile configuration is built on.
+template <class CFG, class ACC>
+__device__ __forceinline__ ACC mfma_of(const i32x4_t (&a)[CFG::NFRAG], const i32x4_t (&b)[CFG::NFRAG], ACC c) {
+  if constexpr (CFG::BLK == 16) return mfma_block16<CFG::IN>(a, b, c);
+  else return mfma_block<CFG::IN, CFG::NFRAG>(a, b, c);
 }
 
 constexpr int kMaxCachedSlots = 8;  // heap bases kept in registers; larger worlds re-load them
@@ -441,8 +465,10 @@ template <class CFG, bool ONE_ROUND, bool STREAMK = false>
 __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kernel(const FusedParams p_in) {
   static_assert(!STREAMK || (CFG::NW == 8 && !ONE_ROUND), "split tiles: eight-wave tile, looping build");
   using Out = typename OutOf<CFG::IN>::type;
-  using ATile = RowTile<CFG::RBA>;
-  constexpr int ES = CFG::ES, CE = CFG::CE, BM = CFG::BM, BN = CFG::BN, BK = CFG::BK;
+  // LDS layouts of A (and of B given K-contiguous, whose rows are as long), and of row-major B
+  using ATile = typename std::conditional<CFG::BLK == 16, RowTile16<CFG::RBA>, RowTile<CFG::RBA>>::type;
+  using BColTile = typename std::conditional<CFG::BLK == 16, ColTile16<CFG::RBB>, ColTile<CFG::RBB, CFG::ES>>::type;
+  constexpr int ES = CFG::ES, CE = CFG::CE, BM = CFG::BM, BN = CFG::BN, BK = CFG::BK, BLK = CFG::BLK;
   constexpr int MB = CFG::MB, NB = CFG::NB, TM = CFG::TM, TN = CFG::TN, NW = CFG::NW, NT = CFG::NT;
   constexpr bool PINGPONG = CFG::NW == 8;
   constexpr int STAGES = CFG::STAGES, LA = CFG::LA, LB = CFG::LB, NFRAG = CFG::NFRAG, KS = CFG::KSLICES;
@@ -510,10 +536,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     int row, c;
     const int off = (wave + i * NW) * kDmaBytes + lane * kChunkBytes;
     if constexpr (CFG::B_KCONTIG) {
-      RowTile<CFG::RBB>::from_lds(off, row, c);
+      ATile::from_lds(off, row, c);
       lb_off[i] = (unsigned)(row * p.s_bn * ES + c * kChunkBytes);
     } else {
-      ColTile<CFG::RBB, ES>::from_lds(off, row, c);
+      BColTile::from_lds(off, row, c);
       lb_off[i] = (unsigned)(row * p.s_bk * ES + c * kChunkBytes);
     }
     lb_row[i] = row;
@@ -521,79 +547,69 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
   }
 
   // ---- fragment read offsets (relative to the slot's A / B region) -------------------------------
+  auto frag_row = [&]() { return BLK == 16 ? mma16_row(lane) : frag16_row(lane); };
+  auto frag_chunk = [&](int kk, int h) {
+    return CFG::IN == IN_FP8 ? frag8_chunk(lane, kk, h) : BLK == 16 ? mma16_chunk(lane, kk) : frag16_chunk(lane, kk);
+  };
   int fa_off[KS][NFRAG];
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-    for (int h = 0; h < NFRAG; ++h) {
-      const int c = (CFG::IN == IN_FP8) ? frag8_chunk(lane, kk, h) : frag16_chunk(lane, kk);
-      fa_off[kk][h] = ATile::lds_offset(wm * TM + frag16_row(lane), c);
-    }
+    for (int h = 0; h < NFRAG; ++h) fa_off[kk][h] = ATile::lds_offset(wm * TM + frag_row(), frag_chunk(kk, h));
   // B operand: K-contiguous B reads exactly like A; row-major B uses transpose reads.
-  constexpr int NTR = (CFG::IN == IN_FP8) ? 1 : 2;  // distinct swizzles among the transpose reads
+  constexpr int NTR = (CFG::IN == IN_FP8 || BLK == 16) ? 1 : 2;  // distinct swizzles among the transpose reads
   int fb_off[CFG::B_KCONTIG ? KS : NB][CFG::B_KCONTIG ? NFRAG : NTR];
   if constexpr (CFG::B_KCONTIG) {
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-      for (int h = 0; h < NFRAG; ++h) {
-        const int c = (CFG::IN == IN_FP8) ? frag8_chunk(lane, kk, h) : frag16_chunk(lane, kk);
-        fb_off[kk][h] = RowTile<CFG::RBB>::lds_offset(wn * TN + frag16_row(lane), c);
-      }
+      for (int h = 0; h < NFRAG; ++h) fb_off[kk][h] = ATile::lds_offset(wn * TN + frag_row(), frag_chunk(kk, h));
   } else {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int j = 0; j < NTR; ++j) {
-        int krow, n;
-        if constexpr (CFG::IN == IN_FP8) {
-          krow = tr8_krow(lane, 0, 0);
-          n = wn * TN + nb * 32 + tr8_ncol(lane);
-        } else {
-          krow = tr16_krow(lane, 0, j);
-          n = wn * TN + nb * 32 + tr16_ncol(lane);
-        }
-        fb_off[nb][j] = ColTile<CFG::RBB, ES>::lds_offset(krow, n / CE) + (n % CE) * ES;
+        const int krow = CFG::IN == IN_FP8 ? tr8_krow(lane, 0, 0) : BLK == 16 ? mma16_tr_krow(lane, 0, 0) : tr16_krow(lane, 0, j);
+        const int n = wn * TN + nb * BLK + (CFG::IN == IN_FP8 ? tr8_ncol(lane) : BLK == 16 ? mma16_tr_ncol(lane) : tr16_ncol(lane));
+        fb_off[nb][j] = BColTile::lds_offset(krow, n / CE) + (n % CE) * ES;
       }
   }
 
   // Read the fragments of k-slice kk of ring slot `slot`.
-  auto load_frags_b = [&](Frags<CFG>& f, int slot_off, int kk) {  // slot_off: byte offset of the ring slot
+  auto load_frag_b = [&](i32x4_t (&dst)[NFRAG], int slot_off, int kk, int nb) {  // slot_off: byte offset of the ring slot
     const char* sb = smem + slot_off + CFG::A_BYTES;
+    if constexpr (CFG::B_KCONTIG) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      if constexpr (CFG::B_KCONTIG) {
+      for (int h = 0; h < NFRAG; ++h)
+        dst[h] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sb + fb_off[kk][h] + nb * BLK * CFG::RBB);
+    } else if constexpr (CFG::IN == IN_FP8) {
+      i32x2_t t[4];
 #pragma unroll
-        for (int h = 0; h < NFRAG; ++h)
-          f.b[nb][h] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sb + fb_off[kk][h] + nb * 32 * CFG::RBB);
-      } else if constexpr (CFG::IN == IN_FP8) {
-        i32x2_t t[4];
+      for (int r = 0; r < 4; ++r)
+        t[r] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+            (LDS_AS i32x2_t*)(LDS_AS char*)(sb + fb_off[nb][0] + (kk * 64 + 8 * r) * CFG::RBB));
+      dst[0] = (i32x4_t){t[0].x, t[0].y, t[1].x, t[1].y};
+      dst[NFRAG - 1] = (i32x4_t){t[2].x, t[2].y, t[3].x, t[3].y};
+    } else {
+      i32x2_t t[2];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          t[r] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-              (LDS_AS i32x2_t*)(LDS_AS char*)(sb + fb_off[nb][0] + (kk * 64 + 8 * r) * CFG::RBB));
-        f.b[nb][0] = (i32x4_t){t[0].x, t[0].y, t[1].x, t[1].y};
-        f.b[nb][NFRAG - 1] = (i32x4_t){t[2].x, t[2].y, t[3].x, t[3].y};
-      } else {
-        i16x4_t t0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (LDS_AS i16x4_t*)(LDS_AS char*)(sb + fb_off[nb][0] + kk * 16 * CFG::RBB));
-        i16x4_t t1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (LDS_AS i16x4_t*)(LDS_AS char*)(sb + fb_off[nb][NTR - 1] + kk * 16 * CFG::RBB));
-        i32x2_t u0 = __builtin_bit_cast(i32x2_t, t0), u1 = __builtin_bit_cast(i32x2_t, t1);
-        f.b[nb][0] = (i32x4_t){u0.x, u0.y, u1.x, u1.y};
-      }
+      for (int j = 0; j < 2; ++j)
+        t[j] = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (LDS_AS i16x4_t*)(LDS_AS char*)(sb + fb_off[nb][NTR == 2 ? j : 0] + (kk * CFG::KM + (NTR == 2 ? 0 : 4 * j)) * CFG::RBB)));
+      dst[0] = (i32x4_t){t[0].x, t[0].y, t[1].x, t[1].y};
     }
   };
-  auto load_frags_a = [&](Frags<CFG>& f, int slot_off, int kk, int mb) {
+  auto load_frag_a = [&](Frags<CFG>& f, int slot_off, int kk, int mb) {
     const char* sa = smem + slot_off;
 #pragma unroll
     for (int h = 0; h < NFRAG; ++h)
-      f.a[mb][h] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sa + fa_off[kk][h] + mb * 32 * CFG::RBA);
+      f.a[mb][h] = *(const LDS_AS i32x4_t*)(LDS_AS char*)(sa + fa_off[kk][h] + mb * BLK * CFG::RBA);
   };
   auto load_frags = [&](Frags<CFG>& f, int slot_off, int kk) {
-    load_frags_b(f, slot_off, kk);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) load_frags_a(f, slot_off, kk, mb);
+    for (int nb = 0; nb < NB; ++nb) load_frag_b(f.b[nb], slot_off, kk, nb);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) load_frag_a(f, slot_off, kk, mb);
   };
 
   const int total_tiles = p.tiles_m * p.tiles_n;
@@ -740,11 +756,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc.v[mb][nb][i] = 0.f;
+        for (int i = 0; i < 4 * CFG::QUADS; ++i) acc.v[mb][nb][i] = 0.f;
 
     // ---- prologue: fill STAGES-1 ring slots, wait for the first ----------------------------------
-    // The two-group loop reads a slot in both of its phases and refills it one step later than the
-    // single-group loop, so it keeps one step less in flight.
+    // The two-group loop reads a slot, and the next one's first fragments, while it refills: one step less is in flight.
     constexpr int AHEAD = PINGPONG ? STAGES - 2 : STAGES - 1;  // K steps issued before the loop starts
 #pragma unroll
     for (int s = 0; s < AHEAD; ++s) {
@@ -770,13 +785,26 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     constexpr int RING_UNROLL = (NW == 4) ? STAGES : 1;
     int s = k_begin, ring_pos = 0;
     if constexpr (PINGPONG) {
-      // Eight waves, two per SIMD: waves 0-3 and waves 4-7 run half a step apart.  A step is a
-      // memory phase (all fragment reads of the step, then the direct-to-LDS loads that refill the
-      // slot of the previous step) and a compute phase (nothing but MFMAs), each closed by a
-      // workgroup barrier, so that on every SIMD one wave feeds the matrix pipe while the other
-      // one has the LDS and memory ports to itself.
+      // Eight waves, two per SIMD: waves 0-3 and waves 4-7 run half a step apart.  A step is a memory phase (the
+      // direct-to-LDS loads of the step three further on) and a compute phase (the products, with the fragment reads
+      // in their shadow), each closed by a workgroup barrier, so that on every SIMD one wave feeds the matrix pipe
+      // while the other one has the memory port to itself.  A direct-to-LDS load does not issue in the shadow of an
+      // MFMA: a wave takes some 80 cycles to get one accepted.
+      //
+      // A memory phase also reads the left half of B's fragments of its step; a compute phase reads A's lower rows of its
+      // own step (quad_block needs them half way through) and of the next step A's upper rows, into the registers that
+      // the first half has done with, and the right half of B, into those free in the last quadrant.  The next step's
+      // slot has landed for all waves by then - the late group waits for it at the end of its previous memory phase -,
+      // which takes a ring of five: this step's slot, the next one's, one that is being waited for, one with loads in
+      // flight, and the one being refilled, which the other group may have left only half a step ago.
+      //
+      // What bounds it is power, with anything but zeros in the operands (bf16 4096x4096x8192 as a plain product, whole
+      // launch: 186 us on normal data, 138 on zeros).  Before - 32x32x16 products, half of the fragments read in the
+      // memory phase, a ring of four - it took 203 (zeros 130: one wave per SIMD issues a 16x16x32 product every 17
+      // cycles, not 16), 8192x1792x4096 98 -> 92; 16x16x32 products in that loop 197 and 98; every fragment of B read in the
+      // memory phase 189; the left half of B one step ahead as well, through a copy, 188.  e4m3, whose 32x32x64 products
+      // stay, runs as before (100 us).
       const bool late = wave >= 4;
-      if (late) __builtin_amdgcn_s_barrier();
       // The loader position of the common case - a whole K step inside one source - is carried in
       // scalar registers that advance by constants, and its loads need no per-lane k test; partial
       // steps, source changes and the empty steps past the end take the general path.
@@ -795,36 +823,24 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       unsigned rd = 0;                                    // byte offset of the slot this step reads
       unsigned wr = AHEAD * CFG::STAGE_BYTES;             // ... and of the slot it refills
       const unsigned wr_wave = smem_base + wave * kDmaBytes;
-      // The fragments of the first half of a step's MFMAs are read in the memory phase, those of the
-      // second half between the MFMAs of the first (LDS reads issue in the shadow of an MFMA;
-      // direct-to-LDS loads do not, a wave takes some 80 cycles to get one accepted).
-      constexpr int NMFMA = KS * MB * NB;
-      constexpr bool SPLIT_K = KS >= 2;                    // halves split by k-slice, else by row block
-      static_assert(KS == 1 || KS % 2 == 0, "k-slices split in two halves");
-      static_assert(MB % 2 == 0, "row blocks split in two halves");
-      // Late fragment reads, in pieces: per late k-slice the B fragments, then one row block of A each;
-      // with a single slice the upper row blocks of A.
-      constexpr int LATE_PIECES = SPLIT_K ? (KS / 2) * (1 + MB) : MB / 2;
-      auto late_piece = [&](int pc) {
-        if constexpr (SPLIT_K) {
-          const int kk = KS / 2 + pc / (1 + MB), q = pc % (1 + MB);
-          if (q == 0)
-            load_frags_b(fr[kk], rd, kk);
-          else
-            load_frags_a(fr[kk], rd, kk, q - 1);
-        } else {
-          load_frags_a(fr[0], rd, 0, MB / 2 + pc);
-        }
+      constexpr int NMFMA = MB * NB, HA = MB / 2, HB = NB / 2, Q = NMFMA / 4;
+      __builtin_amdgcn_sched_barrier(0);  // (no fragment read moves up past the prologue's barrier)
+#pragma unroll
+      for (int nb = HB; nb < NB; ++nb) load_frag_b(fr[0].b[nb], 0, 0, nb);
+#pragma unroll
+      for (int mb = 0; mb < HA; ++mb) load_frag_a(fr[0], 0, 0, mb);
+      if (late) {
+        wait_vmcnt<(AHEAD - 2) * (LA + LB)>();
+        __builtin_amdgcn_s_barrier();
+      }
+      auto product = [&](int i) {
+        int mb, nb;
+        quad_block<MB, NB>(i, mb, nb);
+        acc.v[mb][nb] = mfma_of<CFG>(fr[0].a[mb], fr[0].b[nb], acc.v[mb][nb]);
       };
       for (; s < k_end; ++s) {
-        if constexpr (SPLIT_K) {
 #pragma unroll
-          for (int kk = 0; kk < KS / 2; ++kk) load_frags(fr[kk], rd, kk);
-        } else {
-          load_frags_b(fr[0], rd, 0);
-#pragma unroll
-          for (int mb = 0; mb < MB / 2; ++mb) load_frags_a(fr[0], rd, 0, mb);
-        }
+        for (int nb = 0; nb < HB; ++nb) load_frag_b(fr[0].b[nb], rd, 0, nb);
         __builtin_amdgcn_sched_barrier(0);
         if (k_left >= BK) {
 #pragma unroll
@@ -845,30 +861,29 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
           b_so += b_inc;
           k_left -= BK;
         }
-        // Own early fragment reads done and own loads of step s+1 landed.
-        wait_vmcnt_lgkm0<(AHEAD - 1) * (LA + LB)>();
+        const unsigned rd_next = rd + CFG::STAGE_BYTES == CFG::RING_BYTES ? 0 : rd + CFG::STAGE_BYTES;
+        // Own fragment reads done and own loads of step s+2 landed.
+        wait_vmcnt_lgkm0<(LA + LB)>();
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        // First half of the MFMAs with the late fragment reads spread between them.
 #pragma unroll
-        for (int i = 0; i < NMFMA / 2; ++i) {
-          const int kk = i / (MB * NB), mb = (i / NB) % MB, nb = i % NB;  // one slice: mb < MB/2 here
-          acc.v[mb][nb] = mfma_block<CFG::IN, NFRAG>(fr[kk].a[mb], fr[kk].b[nb], acc.v[mb][nb]);
+        for (int i = 0; i < NMFMA; ++i) {
+          product(i);
 #pragma unroll
-          for (int pc = 0; pc < LATE_PIECES; ++pc)
-            if (pc * (NMFMA / 2) / LATE_PIECES == i) late_piece(pc);
+          for (int pc = 0; pc < HA; ++pc) {
+            if (pc * Q / HA == i) load_frag_a(fr[0], rd, 0, HA + pc);             // this step's lower rows
+            if (2 * Q + pc * Q / HA == i) load_frag_a(fr[0], rd_next, 0, pc);     // the next step's upper rows
+          }
+#pragma unroll
+          for (int pc = 0; pc < HB; ++pc) {
+            if (3 * Q + pc * Q / HB == i) load_frag_b(fr[0].b[HB + pc], rd_next, 0, HB + pc);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int i = NMFMA / 2; i < NMFMA; ++i) {
-          const int kk = i / (MB * NB), mb = (i / NB) % MB, nb = i % NB;
-          acc.v[mb][nb] = mfma_block<CFG::IN, NFRAG>(fr[kk].a[mb], fr[kk].b[nb], acc.v[mb][nb]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        rd = rd + CFG::STAGE_BYTES == CFG::RING_BYTES ? 0 : rd + CFG::STAGE_BYTES;
+        rd = rd_next;
         wr = wr + CFG::STAGE_BYTES == CFG::RING_BYTES ? 0 : wr + CFG::STAGE_BYTES;
       }
       if (!late) __builtin_amdgcn_s_barrier();
@@ -902,7 +917,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
           for (int j = 0; j < NLOAD; ++j)
             if (j * NSLOT / NLOAD == kk * MB + mb) issue_one(L, j);
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) acc.v[mb][nb] = mfma_block<CFG::IN, NFRAG>(f.a[mb], f.b[nb], acc.v[mb][nb]);
+          for (int i = 0; i < NB; ++i) {
+            const int nb = mb & 1 ? NB - 1 - i : i;  // (see quad_block)
+            acc.v[mb][nb] = mfma_of<CFG>(f.a[mb], f.b[nb], acc.v[mb][nb]);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -927,7 +945,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     if constexpr (STREAMK) {
       // Partial sums travel in the accumulators' own layout: 16-byte piece j of thread t at byte
       // (j * NT + t) * 16 of the piece's slot, so that every wave instruction moves 1 KiB.
-      constexpr int PIECES = MB * NB * 4;  // 16-byte pieces per thread
+      constexpr int PIECES = MB * NB * CFG::QUADS;  // 16-byte pieces per thread
       constexpr long long SLOT_BYTES = (long long)PIECES * NT * 16;
       if (item == ITEM_PART) {
         // (The base goes through an empty asm so that the compiler computes the pieces' addresses here, one
@@ -937,7 +955,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
         char* const dst = (char*)slot_base + tid * 16;
 #pragma unroll
         for (int j = 0; j < PIECES; ++j) {
-          const int mb = j / (NB * 4), nb = (j / 4) % NB, q = j % 4;
+          const int mb = j / (NB * CFG::QUADS), nb = j / CFG::QUADS % NB, q = j % CFG::QUADS;
           u32x4_t v;
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = __float_as_uint(acc_read(acc.v[mb][nb][4 * q + e]));
@@ -1009,14 +1027,14 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     // lane and BN*2 contiguous bytes per row, with many loads in flight per thread.
     {
       // Split tiles: 16-byte pieces of a partial sum, in the layout its workgroup stored them in.
-      constexpr int PIECES = MB * NB * 4, NBATCH = 4, BATCH = PIECES / NBATCH;
+      constexpr int PIECES = MB * NB * CFG::QUADS, NBATCH = 4, BATCH = PIECES / NBATCH;
       constexpr long long SLOT_BYTES = (long long)PIECES * NT * 16;
       float badd[MB];
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         badd[mb] = 0.f;
         if (p.bias) {
-          const int gm = m0 + wm * TM + mb * 32 + acc_col(lane);
+          const int gm = m0 + wm * TM + mb * BLK + (BLK == 16 ? mma16_acc_col(lane) : acc_col(lane));
           if (gm < p.M) badd[mb] = load_scalar_as_float(p.bias, (long long)gm * p.s_bias, p.bias_dtype);
         }
       }
@@ -1027,19 +1045,19 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       asm volatile("" : "+v"(lane_s));
       // Piece j of the thread: 4 consecutive n of one m, from their fp32 sums to the staged tile.
       auto stage_piece = [&](int j, const float (&sum)[4]) {
-        const int mb = j / (NB * 4), nb = (j / 4) % NB, q = j % 4;
+        const int mb = j / (NB * CFG::QUADS), nb = j / CFG::QUADS % NB, q = j % CFG::QUADS;
         float h[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) h[e] = sum[e] * p.scale + badd[mb];
         u32x2_t w;
         w.x = Out::pack(h[0], h[1]);
         w.y = Out::pack(h[2], h[3]);
-        const int trow = wm * TM + mb * 32 + acc_col(lane_s);
-        const int tcol = wn * TN + nb * 32 + acc_row(lane_s, 4 * q);
+        const int trow = wm * TM + mb * BLK + (BLK == 16 ? mma16_acc_col(lane_s) : acc_col(lane_s));
+        const int tcol = wn * TN + nb * BLK + (BLK == 16 ? mma16_acc_row(lane_s, 0) : acc_row(lane_s, 4 * q));
         *(LDS_AS u32x2_t*)(LDS_AS char*)(smem + CFG::stage_offset(trow, tcol * 2)) = w;
       };
       auto own_piece = [&](int j, float (&sum)[4]) {
-        const int mb = j / (NB * 4), nb = (j / 4) % NB, q = j % 4;
+        const int mb = j / (NB * CFG::QUADS), nb = j / CFG::QUADS % NB, q = j % CFG::QUADS;
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[e] = acc_read(acc.v[mb][nb][4 * q + e]);
       };
@@ -1459,7 +1477,7 @@ int launch_mfma(const FusedParams& p, int device, int cu_count, hipStream_t stre
       q.interleave = 0;  // the plan hands out the last round of every XCD's span
       q.tile_rotate = 0;
       q.group_m = q.group_m_spans;
-      constexpr long long slot_bytes = (long long)CFG::MB * CFG::NB * 4 * CFG::NT * 16;
+      constexpr long long slot_bytes = (long long)CFG::MB * CFG::NB * CFG::QUADS * CFG::NT * 16;
       // No workspace (the stream is being captured before its first split launch, or the device has
       // used up its workspaces): hand the tiles out whole.
       if (iris_host::split_tile_workspace(device, stream, sk_grid, slot_bytes, &q.sk_partials, &q.sk_flags, &q.sk_epoch) == 0) {
@@ -1487,7 +1505,7 @@ int launch_mfma(const FusedParams& p, int device, int cu_count, hipStream_t stre
 }
 
 // Tile shapes of the MFMA kernel (run_fused picks one per launch).
-//   big       256x256, 8 waves, 64-byte K steps, 4-slot ring: half the operand bytes per flop of the
+//   big       256x256, 8 waves, 64-byte K steps, 5-slot ring: half the operand bytes per flop of the
 //             128x128 tiles; from about half the CUs busy.
 //   small     128x128, 4 waves, 128-byte K steps, 4-slot ring: too few big tiles.
 //   small2    128x128, 4 waves, 64-byte K steps, 64 KiB ring, two workgroups per CU: more 128x128 tiles
@@ -1502,7 +1520,7 @@ constexpr int tile_bk(int kind, int in) {  // K elements per step
   return (kind == TILE_BIG || kind == TILE_SMALL2 ? 64 : 128) / (in == IN_FP8 ? 1 : 2);
 }
 template <int IN, bool BKC>
-using BigTile = MfmaCfg<IN, 256, 256, tile_bk(TILE_BIG, IN), 2, 4, 4, BKC>;
+using BigTile = MfmaCfg<IN, 256, 256, tile_bk(TILE_BIG, IN), 2, 4, 5, BKC>;
 template <int IN, bool BKC>
 using SmallTile = MfmaCfg<IN, 128, 128, tile_bk(TILE_SMALL, IN), 2, 2, 4, BKC>;
 template <int IN, bool BKC>

@@ -115,6 +115,67 @@ IRIS_HD int tr8_ncol(int lane) {
   return 16 * (g % 2) + 8 * (p % 2);
 }
 
+// ---------------------------------------------------------------------------------------------
+// MFMA 16x16 operand lanes, 16-bit (v_mfma_f32_16x16x32_{bf16,f16}): lane l supplies, for row (or column)
+// l%16, the 8 k-values 8*(l/16)..+7 of the 32-wide k-slice.
+// ---------------------------------------------------------------------------------------------
+IRIS_HD int mma16_row(int lane) { return lane % 16; }
+IRIS_HD int mma16_chunk(int lane, int kk) { return kk * 4 + lane / 16; }
+
+// The row tile those reads want.  LDS serves a 16-byte read 16 lanes at a time, and not 16 in a row: lanes {0-3, 12-15,
+// 20-27}, then {4-11, 16-19, 28-31}, then the same of the upper half-wave (measured with address patterns of an MI355X:
+// 4.2 cycles per read and CU where these meet on 16 distinct chunks of a 256-byte bank line, 8 with RowTile<64>, whose
+// rows 0-3 of one chunk and 4-7 of the next share theirs).
+template <int RB>
+struct RowTile16 : RowTile<RB> {};
+template <>
+struct RowTile16<64> {
+  static constexpr int kChunksPerRow = 4;
+  IRIS_HD static int swizzle(int row) { return (row >> 1) & 2; }
+  IRIS_HD static int lds_offset(int row, int c) { return row * 64 + ((c ^ swizzle(row)) * kChunkBytes); }
+  IRIS_HD static void from_lds(int off, int& row, int& c) {
+    row = off / 64;
+    c = ((off % 64) / kChunkBytes) ^ swizzle(row);
+  }
+};
+
+// Transpose read j (0,1) of k-slice kk of a 16-wide column block: as tr16_* above, but the 16-lane groups of a
+// wave all take the same 16 columns, 8 k-rows apart.
+IRIS_HD int mma16_tr_krow(int lane, int kk, int j) { return kk * 32 + 8 * (lane / 16) + 4 * j + lane % 16 / 4; }
+IRIS_HD int mma16_tr_ncol(int lane) { return 4 * (lane % 4); }
+
+// The column tile those reads want: a half-wave touches k-rows {0..3, 8..11} (plus a multiple of 4) x 32 contiguous
+// bytes, so 32-byte blocks are XORed with the k-row's bits 0, 1 and 3: eight blocks, one 256-byte bank line.  With two
+// tile rows to a bank line (RB = 128) the row parity already separates rows, and bits 1 and 3 are left.
+template <int RB>
+struct ColTile16 {
+  static constexpr int kChunksPerRow = RB / kChunkBytes;
+  static_assert(RB == 128 || RB >= 256, "tile row too short for the swizzle");
+  IRIS_HD static int swizzle(int krow) {
+    return RB >= 256 ? 2 * ((krow & 3) | ((krow >> 1) & 4)) : 2 * (((krow >> 1) & 1) | ((krow >> 2) & 2));
+  }
+  IRIS_HD static int lds_offset(int krow, int c) { return krow * RB + ((c ^ swizzle(krow)) * kChunkBytes); }
+  IRIS_HD static void from_lds(int off, int& krow, int& c) {
+    krow = off / RB;
+    c = ((off % RB) / kChunkBytes) ^ swizzle(krow);
+  }
+};
+
+// Accumulator of D = X * Y for the 16x16 MFMA: register i (0..3) of lane l holds D[4*(l/16) + i][l%16].
+IRIS_HD int mma16_acc_row(int lane, int i) { return 4 * (lane / 16) + i; }
+IRIS_HD int mma16_acc_col(int lane) { return lane % 16; }
+
+// Block i of a k-slice's products over MB x NB blocks: quadrant by quadrant (upper left, upper right, lower right, lower
+// left), row by row inside one, every other row backwards, so that consecutive products mostly share an operand (less
+// switching, a few percent of the power) and the first quadrant needs only half of the fragments.
+template <int MB, int NB>
+IRIS_HD constexpr void quad_block(int i, int& mb, int& nb) {
+  constexpr int QM = MB / 2, QN = NB / 2, Q = QM * QN;
+  const int q = i / Q, r = i % Q, row = r / QN, col = r % QN;
+  mb = (q >= 2 ? QM : 0) + row;
+  nb = (q == 1 || q == 2 ? QN : 0) + ((row & 1) ? QN - 1 - col : col);
+}
+
 // Accumulator of D = X * Y for the 32x32 MFMA: register i (0..15) of lane l holds
 //   D[row = 8*(i/4) + 4*(l/32) + i%4][col = l%32].
 // The kernels issue mfma(Bfrag, Afrag) so that D rows run along n and columns along m: every

@@ -152,6 +152,93 @@ void sim_col_operand(int BK) {
       }
 }
 
+// The 16x16x32 products of 16-bit data: fragments of 16 rows (mma16_*), [k][n] tiles in ColTile16.
+template <int RB>
+void check_col_tile16(int krows) {
+  using T = ColTile16<RB>;
+  std::set<int> seen;
+  for (int k = 0; k < krows; ++k)
+    for (int c = 0; c < T::kChunksPerRow; ++c) {
+      int off = T::lds_offset(k, c), k2, c2;
+      CHECK(off >= 0 && off < krows * RB && seen.insert(off).second, "col tile 16 offset out of range or reused");
+      T::from_lds(off, k2, c2);
+      CHECK(k2 == k && c2 == c, "col tile 16 inverse mismatch");
+    }
+}
+
+template <int RB>
+void sim_row_operand16(int rows) {
+  using T = RowTile16<RB>;
+  std::set<int> seen;
+  for (int off = 0; off < rows * RB; off += 16) {
+    int row, c;
+    T::from_lds(off, row, c);
+    CHECK(row < rows && T::lds_offset(row, c) == off && seen.insert(row * T::kChunksPerRow + c).second, "row tile 16 inverse mismatch RB=%d", RB);
+  }
+  for (int r0 = 0; r0 + 16 <= rows; r0 += 16)
+    for (int kk = 0; kk < RB / 64; ++kk) {
+      std::set<int> banks[4];  // the lanes that LDS serves together
+      for (int lane = 0; lane < 64; ++lane) {
+        // the kernel adds the block's first row to the address of row lane % 16: the swizzle must repeat every 16 rows
+        const int off = T::lds_offset(mma16_row(lane), mma16_chunk(lane, kk)) + r0 * RB;
+        int row, c;
+        T::from_lds(off, row, c);
+        CHECK(row == r0 + lane % 16 && c == kk * 4 + lane / 16, "row operand 16: RB=%d lane %d", RB, lane);
+        const int l = lane % 32, second = (l >= 4 && l < 12) || (l >= 16 && l < 20) || l >= 28;
+        banks[lane / 32 * 2 + second].insert(off % 256 / 16);
+      }
+      for (int g = 0; g < 4; ++g) CHECK(banks[g].size() == 16, "row operand 16: bank conflict RB=%d group %d (%zu)", RB, g, banks[g].size());
+    }
+}
+
+template <int RB>
+void sim_col_operand16(int BK) {
+  using T = ColTile16<RB>;
+  for (int n0 = 0; n0 + 16 <= RB / 2; n0 += 16)
+    for (int kk = 0; kk < BK / 32; ++kk)
+      for (int j = 0; j < 2; ++j) {
+        int addr[64];
+        std::set<int> banks[2];
+        for (int lane = 0; lane < 64; ++lane) {
+          // one address per column block, read j and slice kk at constant distances from it
+          const int n = n0 + mma16_tr_ncol(lane);
+          addr[lane] = T::lds_offset(mma16_tr_krow(lane, 0, 0), n / 8) + n % 8 * 2 + (kk * 32 + 4 * j) * RB;
+          CHECK(addr[lane] == T::lds_offset(mma16_tr_krow(lane, kk, j), n / 8) + n % 8 * 2, "col operand 16: swizzle of read %d", j);
+          for (int b = 0; b < 8; b += 4) banks[lane / 32].insert((addr[lane] + b) % 256 / 4);
+        }
+        for (int g = 0; g < 2; ++g) CHECK(banks[g].size() == 64, "col operand 16: bank conflict RB=%d half-wave %d (%zu)", RB, g, banks[g].size());
+        for (int lane = 0; lane < 64; ++lane)
+          for (int e = 0; e < 4; ++e) {
+            const int i = lane % 16, src = lane / 16 * 16 + 4 * e + i / 4;  // the transpose within 16 lanes
+            int k, c;
+            T::from_lds(addr[src] / 16 * 16, k, c);
+            const int n = c * 8 + addr[src] % 16 / 2 + i % 4;
+            CHECK(k == kk * 32 + 8 * (lane / 16) + 4 * j + e && n == n0 + i, "col operand 16: lane %d elem %d got (k%d,n%d)", lane, e, k, n);
+          }
+      }
+}
+
+// The order of a k-slice's products: every block once, the first quadrant from the first half of the fragments, the first
+// half of the products from half of A's.
+template <int MB, int NB>
+void check_quad_blocks() {
+  std::set<int> seen;
+  for (int i = 0; i < MB * NB; ++i) {
+    int mb, nb;
+    quad_block<MB, NB>(i, mb, nb);
+    CHECK(mb >= 0 && mb < MB && nb >= 0 && nb < NB && seen.insert(mb * NB + nb).second, "quad_block<%d,%d>(%d)", MB, NB, i);
+    if (i < MB * NB / 4) CHECK(mb < MB / 2 && nb < NB / 2, "quad_block: first quadrant");
+    if (i < MB * NB / 2) CHECK(mb < MB / 2, "quad_block: first half");
+  }
+}
+
+void check_acc_layout16() {
+  std::set<int> seen;
+  for (int lane = 0; lane < 64; ++lane)
+    for (int i = 0; i < 4; ++i) seen.insert(mma16_acc_row(lane, i) * 16 + mma16_acc_col(lane));
+  CHECK(seen.size() == 256 && *seen.rbegin() == 255, "acc layout 16 must cover the block");
+}
+
 // ---- accumulator layout: every (n, m) of a 32x32 block owned exactly once -----------------------------
 void check_acc_layout() {
   std::set<int> seen;
@@ -401,6 +488,17 @@ int main() {
   sim_col_operand<256, 1>(64);      // fp8 B tile 64 x 256
   sim_col_operand<128, 1>(64);      // fp8 B tile 64 x 128
   check_acc_layout();
+  check_col_tile16<512>(32);
+  check_col_tile16<256>(64);
+  check_col_tile16<128>(64);
+  sim_row_operand16<64>(256);
+  sim_row_operand16<128>(128);
+  sim_col_operand16<512>(32);
+  sim_col_operand16<256>(64);
+  sim_col_operand16<128>(64);
+  check_acc_layout16();
+  check_quad_blocks<8, 4>();
+  check_quad_blocks<4, 2>();
   check_tile_orders();
   check_dealt_order();
   check_flag_counts();
