@@ -314,6 +314,65 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
   }
 }
 
+// One-shot of dense tensors (rows one behind the other, whole 16-byte chunks): a chunk's place is its index, and ascending
+// rank order needs no table of the slots.  A small call is its chain of dependent round trips - arguments, heap
+// bases, chunks, stores - and what stands between them: the kernel above puts the bases through LDS and a barrier, works
+// out rows and columns with five divisions, and gives a thread two chunks, 45 workgroups for 64x2880.  In a loop, eight ranks,
+// bf16, kernel above -> this one: 512x2880 5.4 -> 4.8 us and 64x2880 4.87 -> 4.80 (the host makes a call every 4.6 us),
+// 1024x2880 10.5 -> 9.4, 8192x2880 70.6 -> 68.6; two ranks 1000x4096 5.7 -> 4.7, 4096x4096 16.9 -> 15.7.  Workgroups of 64
+// threads are no better than these of 128, nor are 256.
+template <class E, int W, int UPT, bool NT>
+__global__ void __launch_bounds__(kCclThreads) dense_sum_kernel(const CclParams p) {
+  constexpr int VEC = kChunkBytes / E::size;
+  long long delta[W];
+#pragma unroll
+  for (int i = 0; i < W; ++i) delta[i] = p.heap_bases[p.rank_start + i * p.rank_stride] - p.heap_bases[p.iris_rank];
+  const long long span = (long long)gridDim.x * blockDim.x * UPT;
+  for (long long base = (long long)blockIdx.x * blockDim.x * UPT + threadIdx.x; base < p.total_units; base += span) {
+    Chunk<E, VEC> x[UPT][W];
+    long long off[UPT];
+#pragma unroll
+    for (int u = 0; u < UPT; ++u) {
+      const long long g = base + (long long)u * blockDim.x;
+      off[u] = (g < p.total_units ? g : base) * kChunkBytes;  // (chunks past the end: the first one again)
+#pragma unroll
+      for (int i = 0; i < W; ++i) x[u][i].template load<NT>(p.in + off[u] + delta[i]);
+    }
+#pragma unroll
+    for (int u = 0; u < UPT; ++u) {
+      Chunk<E, VEC> acc;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        float a = 0.0f + x[u][0].v[e];  // from +0, as above
+#pragma unroll
+        for (int i = 1; i < W; ++i) a += x[u][i].v[e];
+        acc.v[e] = a;
+      }
+      if (base + (long long)u * blockDim.x < p.total_units) acc.template store<NT>(p.out + off[u]);
+    }
+  }
+}
+
+template <class E>
+void launch_dense(const CclParams& p, int cu, bool stream_nt, hipStream_t s) {
+  const int upt = stream_nt ? 4 : 1;
+  const int threads = stream_nt ? kCclThreads : kCclThreads / 2;
+  const long long want = (p.total_units + (long long)threads * upt - 1) / ((long long)threads * upt);
+  const long long cap = (long long)cu * 8 * (kCclThreads / threads);
+  const int grid = (int)(want < cap ? want : cap);
+#define DENSE_KERNEL(W)                                                                                           \
+  do {                                                                                                            \
+    if (stream_nt) hipLaunchKernelGGL((dense_sum_kernel<E, W, 4, true>), dim3(grid), dim3(threads), 0, s, p);     \
+    else hipLaunchKernelGGL((dense_sum_kernel<E, W, 1, false>), dim3(grid), dim3(threads), 0, s, p);              \
+  } while (0)
+  switch (p.world) {
+    case 2: DENSE_KERNEL(2); break;
+    case 4: DENSE_KERNEL(4); break;
+    default: DENSE_KERNEL(8); break;
+  }
+#undef DENSE_KERNEL
+}
+
 template <class E, int VEC, int UPT, bool NT, bool ROWS>
 void launch_for_world(const CclParams& p, int grid, hipStream_t s) {
 #define CCL_KERNEL(W, U) hipLaunchKernelGGL((slot_reduce_kernel<E, VEC, W, U, NT, ROWS>), dim3(grid), dim3(kCclThreads), 0, s, p)
@@ -436,6 +495,13 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   // 78 / 44 with cached reads); reduce-scatter 36 / 34 and 30 / 28 (31 / 27, 53 / 26).  Small launches keep cacheable accesses, and
   // so do misaligned rows of tiles, whose pieces of lines the L2 has to put together (8192x2881 reduce-scatter 12 against 18).
   const bool stream_nt = vec > 1 && large && p.mode != CCL_ATOMIC && (whole || p.mode == CCL_ONE_SHOT);
+  if (p.mode == CCL_ONE_SHOT && whole && unit_stride && p.s_im == p.N && p.s_om == p.N && (p.world == 2 || p.world == 4 || p.world == 8)) {
+    p.total_units = (long long)p.M * p.N / vec_full;
+    if (dtype == IRIS_HIP_BF16) launch_dense<ElemBF16>(p, cu, stream_nt, s);
+    else if (dtype == IRIS_HIP_FP16) launch_dense<ElemF16>(p, cu, stream_nt, s);
+    else launch_dense<ElemF32>(p, cu, stream_nt, s);
+    return (int)hipGetLastError();
+  }
   const int upt = stream_nt && !by_rows ? 4 : 2;
   const long long per_wg = (long long)kCclThreads * upt;
   const long long want = (p.total_units + per_wg - 1) / per_wg;
