@@ -4,7 +4,7 @@
 // The kernels move operand tiles from HBM into LDS with 16-byte direct-to-LDS buffer loads
 // (one wave instruction deposits 64 lanes x 16 B = 1 KiB of contiguous LDS), read the
 // K-contiguous operand with 16-byte LDS reads and the N-contiguous operand with the gfx950
-// LDS transpose reads, and feed 32x32 MFMA blocks.  The functions below say, for every lane,
+// LDS transpose reads, and feed 32x32 or 16x16 MFMA blocks.  The functions below say, for every lane,
 // which global 16-byte chunk it fetches, where that chunk lives in LDS, and which LDS address
 // a lane presents when it assembles an MFMA operand.
 //
