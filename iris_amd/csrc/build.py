@@ -15,11 +15,12 @@ import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
-# One translation unit per input type of the MFMA kernel and of the any-shape kernel (they hold most of the
-# compile time and are compiled side by side), the entry points, and the stand-alone collectives.
+# One translation unit per input type of the MFMA kernel, of the kernel for small outputs and of the any-shape kernel (they
+# hold most of the compile time and are compiled side by side), the entry points, and the stand-alone collectives.
 SOURCES = [os.path.join(HERE, f) for f in (
     "iris_hip_mfma_bf16.hip", "iris_hip_mfma_f16.hip", "iris_hip_mfma_fp8.hip", "iris_hip_any_bf16.hip",
-    "iris_hip_any_f16.hip", "iris_hip_any_fp8.hip", "iris_hip_any_f32.hip", "iris_hip.hip", "iris_ccl.hip")]
+    "iris_hip_any_f16.hip", "iris_hip_any_fp8.hip", "iris_hip_any_f32.hip", "iris_hip_decode_bf16.hip",
+    "iris_hip_decode_f16.hip", "iris_hip_decode_fp8.hip", "iris_hip.hip", "iris_ccl.hip")]
 HEADERS = [os.path.join(HERE, h) for h in ("fused_kernel.h", "decode_kernel.h", "any_kernel.h", "layout.h", "device_util.h",
                                            "host_common.h")] + [
     os.path.join(ROOT, "include", "iris_hip.h")]

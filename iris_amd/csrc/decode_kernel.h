@@ -31,7 +31,7 @@
 // fp32 rounding of each other otherwise (the K sum is split four ways here).
 #pragma once
 
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+#include "fused_kernel.h"
 
 template <int IN_, bool B_KCONTIG_, int QB_ = 256>
 struct DecodeCfg {
@@ -494,4 +494,20 @@ int launch_decode(FusedParams& p, int device, hipStream_t stream, const char* na
   iris_host::set_last_kernel(name);
   hipLaunchKernelGGL((fused_decode_kernel<IN, BKC, QB>), dim3(grid), dim3(CFG::NT), CFG::SMEM_BYTES, stream, p);
   return (int)hipGetLastError();
+}
+
+template <int IN>
+int dispatch_decode(FusedParams& p, bool bkc, int device, int cu, hipStream_t s) {
+  static const char* tnames[3] = {"bf16", "f16", "fp8"};
+  char dname[96];
+  // More tiles than CUs: half the K per chunk, so that a workgroup's LDS (80 KiB) lets two share a CU
+  // and the whole output is in flight at once instead of in two rounds (fp16, eight ranks, 64x8192x512
+  // 13.8 -> 9.3 us, 128x4096x4096 27.3 -> 24.5 us).  Also when K is at most two such chunks: every load
+  // is in flight from the start either way, and the first MFMA waits for half as many bytes (0.3 us).
+  const int kbytes = p.K * (IN == IN_FP8 ? 1 : 2);
+  const bool halves = (long long)cdiv(p.M, 32) * cdiv(p.N, 32) > cu || kbytes <= 1024;
+  const int chunk = halves ? DecodeCfg<IN, false, 128>::CHUNK : DecodeCfg<IN, false, 256>::CHUNK;
+  snprintf(dname, sizeof(dname), "mfma_%s_32x32x%d_%s", tnames[IN], chunk, bkc ? "nt" : "nn");
+  if (halves) return bkc ? launch_decode<IN, true, 128>(p, device, s, dname) : launch_decode<IN, false, 128>(p, device, s, dname);
+  return bkc ? launch_decode<IN, true, 256>(p, device, s, dname) : launch_decode<IN, false, 256>(p, device, s, dname);
 }

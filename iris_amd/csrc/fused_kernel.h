@@ -1,6 +1,6 @@
 // The MFMA kernel of libiris_hip (fused_mfma_kernel) with the types it shares with the generic
 // kernel (FusedParams, the flag helpers), its tile shapes and its launch code.  The kernel is
-// instantiated for 3 input types x 4 tile shapes x 2 operand layouts (plus the one-round builds);
+// instantiated for 3 input types x 5 tile shapes x 2 operand layouts (plus the one-round builds);
 // each input type is compiled in a translation unit of its own (iris_hip_mfma_<type>.hip), which
 // instantiates dispatch_mfma_in<IN> below, so that the build can compile them side by side.
 #pragma once
@@ -1535,25 +1535,16 @@ inline int tile_rows(int kind) {
 }
 inline int tile_cols(int kind) { return kind == TILE_BIG ? 256 : kind == TILE_DECODE ? 32 : kind == TILE_SKINNY64 ? 64 : 128; }
 
-#include "decode_kernel.h"
+// The 32x32 kernel (decode_kernel.h), in translation units of its own: what the compiler makes of a kernel depends on the other
+// kernels of its module (beside the tiles the fp16 builds changed with every edit here: 32x2880x512, eight ranks, 7.20 -> 7.30 us).
+// Instantiated in iris_hip_decode_<type>.hip.
+template <int IN>
+int dispatch_decode(FusedParams& p, bool bkc, int device, int cu, hipStream_t s);
 
 template <int IN>
 int dispatch_mfma_in(FusedParams& p, int kind, bool bkc, int device, int cu, hipStream_t s) {
   const int bm = tile_rows(kind), bn = tile_cols(kind);
-  if (kind == TILE_DECODE) {
-    static const char* tnames[3] = {"bf16", "f16", "fp8"};
-    char dname[96];
-    // More tiles than CUs: half the K per chunk, so that a workgroup's LDS (80 KiB) lets two share a CU
-    // and the whole output is in flight at once instead of in two rounds (fp16, eight ranks, 64x8192x512
-    // 13.8 -> 9.3 us, 128x4096x4096 27.3 -> 24.5 us).  Also when K is at most two such chunks: every load
-    // is in flight from the start either way, and the first MFMA waits for half as many bytes (0.3 us).
-    const int kbytes = p.K * (IN == IN_FP8 ? 1 : 2);
-    const bool halves = (long long)cdiv(p.M, 32) * cdiv(p.N, 32) > cu || kbytes <= 1024;
-    const int chunk = halves ? DecodeCfg<IN, false, 128>::CHUNK : DecodeCfg<IN, false, 256>::CHUNK;
-    snprintf(dname, sizeof(dname), "mfma_%s_32x32x%d_%s", tnames[IN], chunk, bkc ? "nt" : "nn");
-    if (halves) return bkc ? launch_decode<IN, true, 128>(p, device, s, dname) : launch_decode<IN, false, 128>(p, device, s, dname);
-    return bkc ? launch_decode<IN, true, 256>(p, device, s, dname) : launch_decode<IN, false, 256>(p, device, s, dname);
-  }
+  if (kind == TILE_DECODE) return dispatch_decode<IN>(p, bkc, device, cu, s);
   p.tiles_m = cdiv(p.M, bm);
   p.tiles_n = cdiv(p.N, bn);
   // Group height: tile-rows walked together so that the tiles an XCD works on at one time - its whole

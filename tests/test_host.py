@@ -394,6 +394,18 @@ def test_no_product_code_touches_the_oracle():
                 assert "oracle" not in text.replace("There is no fallback", ""), f"{f} mentions the oracle"
 
 
+def test_the_kernel_for_small_outputs_has_translation_units_of_its_own():
+    """What the compiler makes of the decode kernel depends on the other kernels of its module."""
+    csrc = os.path.join(ROOT, "iris_amd", "csrc")
+    includes = {f: re.findall(r'^#include "(.*)"', open(os.path.join(csrc, f)).read(), re.M)
+                for f in os.listdir(csrc) if f.endswith((".h", ".hip"))}
+    users = {f for f, names in includes.items() if "decode_kernel.h" in names}
+    assert users == {f"iris_hip_decode_{t}.hip" for t in ("bf16", "f16", "fp8")}
+    for f in users:
+        assert includes[f] == ["decode_kernel.h"]
+        assert re.findall(r"^template .*? (\w+)<", open(os.path.join(csrc, f)).read(), re.M) == ["dispatch_decode"]
+
+
 # -- index math of the kernels, replayed on the CPU ------------------------------------------------------------------
 def test_layout_simulation(tmp_path):
     exe = tmp_path / "layout_sim"
