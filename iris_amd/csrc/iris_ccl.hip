@@ -1,12 +1,13 @@
 // Stand-alone collectives over the symmetric heap (all-reduce, reduce-scatter): the rank-local part
-// of iris/ccl/triton/all_reduce.py and iris/ccl/triton/reduce_scatter.py as one streaming kernel.
+// of iris/ccl/triton/all_reduce.py and iris/ccl/triton/reduce_scatter.py as one streaming kernel
+// (slot_reduce_kernel), and a second one for the one-shot all-reduce of dense tensors (dense_sum_kernel).
 //
 // These are pure HBM kernels: every output element is the sum of W input elements that sit at the
-// same heap offset in W slots.  The kernel walks a flat index space of 16-byte chunks (or single
+// same heap offset in W slots.  The first kernel walks a flat index space of 16-byte chunks (or single
 // elements when the operands are not 16-byte friendly), W loads in flight per chunk and several
 // chunks per thread, fp32 sums, one cast, 16-byte stores.
 //
-// What the reference fixes, and this kernel reproduces element for element:
+// What the reference fixes, and these kernels reproduce element for element:
 //   * which tiles a rank reduces (two-shot distributions, iris/ccl/triton/all_reduce.py:620-633),
 //   * the grouped tile order that turns a tile id into tile coordinates (:639-644),
 //   * the order of the fp32 additions: ascending group index from zero for one-shot (:403-414),
@@ -479,11 +480,14 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   const bool by_rows = rows && vec > 1 && p.total_units < (1ll << 31);
   if (by_rows) p.n_rects = row_rects(p.rect, p.first_tile, p.n_owned, p.tiles_m, p.tiles_n, p.group_m, p.bm, p.upr);
 
+  const bool dense = p.mode == CCL_ONE_SHOT && whole && unit_stride && p.s_im == p.N && p.s_om == p.N &&
+                     (p.world == 2 || p.world == 4 || p.world == 8);
+
   hipStream_t s = (hipStream_t)stream;
   char name[96];
   static const char* modes[4] = {"one_shot", "two_shot", "reduce_scatter", "atomic"};
   static const char* types[3] = {"bf16", "f16", "f32"};
-  snprintf(name, sizeof(name), "slot_reduce_%s_%s_vec%d", modes[p.mode], types[dtype], vec);
+  snprintf(name, sizeof(name), "%s_%s_%s_vec%d", dense ? "dense_sum" : "slot_reduce", modes[p.mode], types[dtype], vec);
   iris_host::set_last_kernel(name);
   if (p.total_units == 0) return 0;  // this rank owns nothing
 
@@ -495,7 +499,7 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   // 78 / 44 with cached reads); reduce-scatter 36 / 34 and 30 / 28 (31 / 27, 53 / 26).  Small launches keep cacheable accesses, and
   // so do misaligned rows of tiles, whose pieces of lines the L2 has to put together (8192x2881 reduce-scatter 12 against 18).
   const bool stream_nt = vec > 1 && large && p.mode != CCL_ATOMIC && (whole || p.mode == CCL_ONE_SHOT);
-  if (p.mode == CCL_ONE_SHOT && whole && unit_stride && p.s_im == p.N && p.s_om == p.N && (p.world == 2 || p.world == 4 || p.world == 8)) {
+  if (dense) {
     p.total_units = (long long)p.M * p.N / vec_full;
     if (dtype == IRIS_HIP_BF16) launch_dense<ElemBF16>(p, cu, stream_nt, s);
     else if (dtype == IRIS_HIP_FP16) launch_dense<ElemF16>(p, cu, stream_nt, s);

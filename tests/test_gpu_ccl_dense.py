@@ -31,7 +31,7 @@ def test_dense_one_shot(W, rank, M, N, dtype):
         ctx.peer_view(x, r).copy_(inputs[r])
         ctx.peer_view(y, r).fill_(3.0)
     ctx.ccl.all_reduce(y, x, config=Config(all_reduce_variant="one_shot"))
-    assert "one_shot" in _lib.last_kernel() and "vec1" not in _lib.last_kernel(), _lib.last_kernel()
+    assert _lib.last_kernel().startswith("dense_sum_one_shot_"), _lib.last_kernel()
     exp = torch.zeros((M, N))
     for r in range(W):
         exp += inputs[r].float()
@@ -40,3 +40,34 @@ def test_dense_one_shot(W, rank, M, N, dtype):
         assert_bits_equal(ctx.peer_view(x, r).cpu(), inputs[r], f"input of slot {r}")
         if r != rank:
             assert bool((ctx.peer_view(y, r) == 3.0).all()), f"output of slot {r} was written"
+
+
+def _staged(W, rank, M, N, dtype, row=None):
+    """Inputs of all ranks in one heap, rows `row` elements apart; outputs filled with 3."""
+    row = row or N
+    ctx = iris.iris(1 << 24, num_ranks=W, rank=rank)
+    x, y = ctx.zeros((M, row), dtype=dtype), ctx.zeros((M, row), dtype=dtype)
+    inputs = [randn_cpu((M, N), 70 + r, dtype) for r in range(W)]
+    for r in range(W):
+        ctx.peer_view(x, r)[:, :N].copy_(inputs[r])
+        ctx.peer_view(y, r).fill_(3.0)
+    return ctx, x, y, inputs
+
+
+def _sum(inputs, dtype):
+    exp = torch.zeros(inputs[0].shape)
+    for t in inputs:
+        exp += t.float()
+    return exp.to(dtype)
+
+
+# What the dense kernel does not take: a group size it is not built for, rows with space between them, and rows that are not
+# whole chunks.
+@pytest.mark.parametrize("W,rank,N,row", [(3, 1, 256, 256), (1, 0, 256, 256), (4, 2, 256, 264), (4, 2, 250, 250)])
+def test_other_one_shots_run_the_general_kernel(W, rank, N, row):
+    dtype = torch.float16
+    ctx, x, y, inputs = _staged(W, rank, 21, N, dtype, row)
+    y = y[:, :N]
+    ctx.ccl.all_reduce(y, x[:, :N], config=Config(all_reduce_variant="one_shot"))
+    assert _lib.last_kernel().startswith("slot_reduce_one_shot_"), _lib.last_kernel()
+    assert_bits_equal(y.cpu(), _sum(inputs, dtype), f"{W} ranks, {N} columns, rows {row} apart")
