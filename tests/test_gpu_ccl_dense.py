@@ -61,6 +61,37 @@ def _sum(inputs, dtype):
     return exp.to(dtype)
 
 
+# Members between outsiders; two members that start past rank 0; four next to each other.
+@pytest.mark.parametrize("W,rank,group,dtype", [
+    (8, 5, [1, 3, 5, 7], torch.bfloat16), (8, 6, [2, 6], torch.float32), (8, 2, [2, 3, 4, 5], torch.float16)])
+def test_dense_one_shot_of_a_group(W, rank, group, dtype):
+    ctx, x, y, inputs = _staged(W, rank, 33, 264, dtype)
+    outsiders = [r for r in range(W) if r not in group]
+    for r in outsiders:
+        ctx.peer_view(x, r).fill_(float("nan"))
+    ctx.ccl.all_reduce(y, x, group=group, config=Config(all_reduce_variant="one_shot"))
+    assert _lib.last_kernel().startswith("dense_sum_one_shot_"), _lib.last_kernel()
+    assert_bits_equal(y.cpu(), _sum([inputs[r] for r in group], dtype), f"group {group}")
+    for r in range(W):
+        if r != rank:
+            assert bool((ctx.peer_view(y, r) == 3.0).all()), f"output of slot {r} was written"
+
+
+@pytest.mark.parametrize("M,N", [(5, 136), (2048, 4096)])  # the second one streams, four chunks to a thread
+def test_dense_one_shot_in_place(M, N):
+    W, rank, dtype = 8, 3, torch.bfloat16
+    ctx = iris.iris(2 * M * N * 2 + (1 << 21), num_ranks=W, rank=rank)
+    x, other = ctx.zeros((M, N), dtype=dtype), ctx.zeros((M, N), dtype=dtype)
+    inputs = [randn_cpu((M, N), 90 + r, dtype) for r in range(W)]
+    for r in range(W):
+        ctx.peer_view(x, r).copy_(inputs[r])
+    cfg = Config(all_reduce_variant="one_shot")
+    ws = ctx.ccl.all_reduce_preamble(other, x, config=cfg)  # (it zeroes the output it is given)
+    ctx.ccl.all_reduce(x, x, config=cfg, workspace=ws)
+    assert _lib.last_kernel().startswith("dense_sum_one_shot_"), _lib.last_kernel()
+    assert_bits_equal(x.cpu(), _sum(inputs, dtype), "in place")
+
+
 # What the dense kernel does not take: a group size it is not built for, rows with space between them, and rows that are not
 # whole chunks.
 @pytest.mark.parametrize("W,rank,N,row", [(3, 1, 256, 256), (1, 0, 256, 256), (4, 2, 256, 264), (4, 2, 250, 250)])
