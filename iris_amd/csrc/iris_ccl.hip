@@ -320,8 +320,8 @@ __global__ void __launch_bounds__(kCclThreads) slot_reduce_kernel(const CclParam
 // bases, chunks, stores - and what stands between them: the kernel above puts the bases through LDS and a barrier, works
 // out rows and columns with five divisions, and gives a thread two chunks, 45 workgroups for 64x2880.  In a loop, eight ranks,
 // bf16, kernel above -> this one: 512x2880 5.4 -> 4.8 us and 64x2880 4.87 -> 4.80 (the host makes a call every 4.6 us),
-// 1024x2880 10.5 -> 9.4, 8192x2880 70.6 -> 68.6; two ranks 1000x4096 5.7 -> 4.7, 4096x4096 16.9 -> 15.7.  Workgroups of 64
-// threads are no better than these of 128, nor are 256.
+// 1024x2880 10.5 -> 9.4, 4096x4096 51.2 -> 48.5, 8192x2880 the same (69.9 and 70.3); two ranks 1000x4096 5.7 -> 4.7, 4096x4096
+// 16.9 -> 15.7.  Workgroups of 64 threads are no better than these of 128, nor are 256.
 template <class E, int W, int UPT, bool NT>
 __global__ void __launch_bounds__(kCclThreads) dense_sum_kernel(const CclParams p) {
   constexpr int VEC = kChunkBytes / E::size;
@@ -480,14 +480,19 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
   const bool by_rows = rows && vec > 1 && p.total_units < (1ll << 31);
   if (by_rows) p.n_rects = row_rects(p.rect, p.first_tile, p.n_owned, p.tiles_m, p.tiles_n, p.group_m, p.bm, p.upr);
 
+  // Dense one-shot launches, except those of eight ranks and 16-bit data that move more than half a gigabyte: there
+  // dense_sum_kernel waits for a thread's first eight loads before it sends out the other twenty-four, and the general kernel
+  // has the memory busier (bf16, general / dense: 8192x4096 103.1 / 105.0 us, 8192x8192 205.5 / 210.3, 16384x8192 422 / 428;
+  // below the line 6144x4096 74.5 / 73.5, 4096x4096 51.2 / 48.5).  With every load sent out first it is the equal of the
+  // general one on these and 1 to 3 % slower on smaller ones (fp16 2048x4096 24.2 -> 25.0).
   const bool dense = p.mode == CCL_ONE_SHOT && whole && unit_stride && p.s_im == p.N && p.s_om == p.N &&
-                     (p.world == 2 || p.world == 4 || p.world == 8);
+                     (p.world == 2 || p.world == 4 || (p.world == 8 && (es == 4 || moved <= (double)(512 << 20))));
 
   hipStream_t s = (hipStream_t)stream;
   char name[96];
-  static const char* modes[4] = {"one_shot", "two_shot", "reduce_scatter", "atomic"};
+  static const char* modes[4] = {"slot_reduce_one_shot", "slot_reduce_two_shot", "slot_reduce_reduce_scatter", "slot_reduce_atomic"};
   static const char* types[3] = {"bf16", "f16", "f32"};
-  snprintf(name, sizeof(name), "%s_%s_%s_vec%d", dense ? "dense_sum" : "slot_reduce", modes[p.mode], types[dtype], vec);
+  snprintf(name, sizeof(name), "%s_%s_vec%d", dense ? "dense_sum_one_shot" : modes[p.mode], types[dtype], vec);
   iris_host::set_last_kernel(name);
   if (p.total_units == 0) return 0;  // this rank owns nothing
 

@@ -102,3 +102,23 @@ def test_other_one_shots_run_the_general_kernel(W, rank, N, row):
     ctx.ccl.all_reduce(y, x[:, :N], config=Config(all_reduce_variant="one_shot"))
     assert _lib.last_kernel().startswith("slot_reduce_one_shot_"), _lib.last_kernel()
     assert_bits_equal(y.cpu(), _sum(inputs, dtype), f"{W} ranks, {N} columns, rows {row} apart")
+
+
+# Eight ranks and 16-bit data on both sides of 512 MiB of traffic (nine tensors); float32 stays with the dense kernel.
+@pytest.mark.parametrize("M,dtype,kernel", [
+    (7281, torch.bfloat16, "dense_sum"), (7282, torch.bfloat16, "slot_reduce"), (7282, torch.float16, "slot_reduce"),
+    (3641, torch.float32, "dense_sum")])
+def test_large_dense_one_shots_of_eight_ranks(M, dtype, kernel):
+    W, rank, N = 8, 6, 4096
+    es = torch.empty((), dtype=dtype).element_size()
+    ctx = iris.iris(2 * M * N * es + (1 << 21), num_ranks=W, rank=rank)
+    x, y = ctx.zeros((M, N), dtype=dtype), ctx.zeros((M, N), dtype=dtype)
+    exp = torch.zeros((M, N), device="cuda")
+    for r in range(W):
+        g = torch.Generator(device="cuda").manual_seed(50 + r)
+        data = torch.randn((M, N), generator=g, device="cuda").to(dtype)
+        ctx.peer_view(x, r).copy_(data)
+        exp += data.float()
+    ctx.ccl.all_reduce(y, x, config=Config(all_reduce_variant="one_shot"))
+    assert _lib.last_kernel().startswith(kernel), _lib.last_kernel()
+    assert torch.equal(y, exp.to(dtype))
