@@ -785,6 +785,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     constexpr int RING_UNROLL = (NW == 4) ? STAGES : 1;
     int s = k_begin, ring_pos = 0;
     if constexpr (PINGPONG) {
+      static_assert(KS == 1 && MB % 2 == 0 && NB % 2 == 0, "eight-wave loop: one k-slice per step, blocks in quadrants");
       // Eight waves, two per SIMD: waves 0-3 and waves 4-7 run half a step apart.  A step is a memory phase (the
       // direct-to-LDS loads of the step three further on) and a compute phase (the products, with the fragment reads
       // in their shadow), each closed by a workgroup barrier, so that on every SIMD one wave feeds the matrix pipe
