@@ -272,6 +272,15 @@ struct MfmaCfg {
     if (STAGE_SWIZZLED) return STAGE_OFF + row * TROW + ((((b >> 4) ^ row) & (BN / 8 - 1)) << 4) + (b & 15);
     return row * TROW + b;
   }
+  // The same for a place `rows` further down and `bytes` further right, from the offset of a lane's first one.  Swizzled rows:
+  // the lane's row and chunk have none of the bits that rows (modulo a period of the swizzle) and bytes set, so the chunk's
+  // place changes by an XOR with a constant.  (The swizzle of each of a thread's 32 places anew: 4096x4096x64 fp16 as a
+  // plain product 12.3 us instead of 11.8, 16384x8192x128 102.4 instead of 96.7.)
+  __host__ __device__ static constexpr int stage_step(int first, int rows, int bytes) {
+    if (STAGE_SWIZZLED) return (first ^ (bytes ^ ((rows & (BN / 8 - 1)) << 4))) + rows * TROW;
+    return first + rows * TROW + bytes;
+  }
+  static_assert(!STAGE_SWIZZLED || (TM % (BN / 8) == 0 && STAGE_OFF % TROW == 0), "places of a lane an XOR apart");
   // Four-wave tiles whose ring fits twice into a CU's LDS run two workgroups per CU, so that the
   // memory round trips of one workgroup's epilogue hide behind the other's K loop.
   static constexpr int WG_PER_CU = (NW == 4 && SMEM_BYTES <= 80 * 1024) ? 2 : 1;
@@ -1030,20 +1039,34 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       // Split tiles: 16-byte pieces of a partial sum, in the layout its workgroup stored them in.
       constexpr int PIECES = MB * NB * CFG::QUADS, NBATCH = 4, BATCH = PIECES / NBATCH;
       constexpr long long SLOT_BYTES = (long long)PIECES * NT * 16;
-      float badd[MB];
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        badd[mb] = 0.f;
-        if (p.bias) {
+      float badd[MB] = {};
+      if (p.bias) {
+        // Every load is out before the first is used (a block at a time the blocks of sixteen rows made eight round trips of
+        // it, 6 of the 113 us of a plain fp16 16384x8192x128 with bias).  Rows past the end, which are never stored, take the last one's.
+        const bool wide = p.bias_dtype == IRIS_HIP_FP32;
+        unsigned raw[MB];
+        auto row_of = [&](int mb) -> long long {
           const int gm = m0 + wm * TM + mb * BLK + (BLK == 16 ? mma16_acc_col(lane) : acc_col(lane));
-          if (gm < p.M) badd[mb] = load_scalar_as_float(p.bias, (long long)gm * p.s_bias, p.bias_dtype);
+          return (long long)min(gm, p.M - 1) * p.s_bias;
+        };
+        if (wide) {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) raw[mb] = ((const unsigned*)p.bias)[row_of(mb)];
+        } else {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) raw[mb] = ((const unsigned short*)p.bias)[row_of(mb)];
         }
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          badd[mb] = wide ? __uint_as_float(raw[mb]) : p.bias_dtype == IRIS_HIP_BF16 ? bf16_bits_to_float((unsigned short)raw[mb]) : f16_bits_to_float((unsigned short)raw[mb]);
       }
-      // The lane index as the staging addresses see it goes through an empty asm: with the swizzled layout
-      // a lane has one address term per (column block, quarter), and the compiler would otherwise compute
-      // them once, ahead of the tile loop, and carry eight more registers through the K loop.
+      // The lane index as the staging addresses see it goes through an empty asm: the compiler would otherwise compute
+      // them once, ahead of the tile loop, and carry more registers through the K loop.  A lane has one address, of its
+      // first piece; the others are a constant away from it.
       int lane_s = lane;
       asm volatile("" : "+v"(lane_s));
+      const int stage_first = CFG::stage_offset(wm * TM + (BLK == 16 ? mma16_acc_col(lane_s) : acc_col(lane_s)),
+                                                (wn * TN + (BLK == 16 ? mma16_acc_row(lane_s, 0) : acc_row(lane_s, 0))) * 2);
       // Piece j of the thread: 4 consecutive n of one m, from their fp32 sums to the staged tile.
       auto stage_piece = [&](int j, const float (&sum)[4]) {
         const int mb = j / (NB * CFG::QUADS), nb = j / CFG::QUADS % NB, q = j % CFG::QUADS;
@@ -1053,9 +1076,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
         u32x2_t w;
         w.x = Out::pack(h[0], h[1]);
         w.y = Out::pack(h[2], h[3]);
-        const int trow = wm * TM + mb * BLK + (BLK == 16 ? mma16_acc_col(lane_s) : acc_col(lane_s));
-        const int tcol = wn * TN + nb * BLK + (BLK == 16 ? mma16_acc_row(lane_s, 0) : acc_row(lane_s, 4 * q));
-        *(LDS_AS u32x2_t*)(LDS_AS char*)(smem + CFG::stage_offset(trow, tcol * 2)) = w;
+        *(LDS_AS u32x2_t*)(LDS_AS char*)(smem + CFG::stage_step(stage_first, mb * BLK, (nb * BLK + 8 * q) * 2)) = w;
       };
       auto own_piece = [&](int j, float (&sum)[4]) {
         const int mb = j / (NB * CFG::QUADS), nb = j / CFG::QUADS % NB, q = j % CFG::QUADS;

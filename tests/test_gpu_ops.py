@@ -408,6 +408,27 @@ def test_matmul_all_gather_big_tile():
         assert_bits_equal(got, exp[r], f"slot {r}")
 
 
+# Rows that end inside a tile (the bias of rows past the end is not there to be read), on the 256x256, 128x128, 64x128 and 32x32 tiles.
+@pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M_local,N,dtype,tile", [
+    (2049, 4096, torch.float16, "f16_256x256"), (2070, 4096, torch.bfloat16, "bf16_256x256"), (1030, 3584, torch.float16, "f16_128x128"),
+    (890, 2880, torch.bfloat16, "bf16_64x128"), (33, 512, torch.float16, "f16_32x32")])
+def test_bias_of_any_type_and_stride(M_local, N, dtype, tile, bias_dtype):
+    W, rank, K = 2, 1, 2048 if tile == "f16_128x128" else 64
+    ctx = _ctx(W, rank, heap=1 << 27)
+    A, B = randint_cpu((M_local, K), 80, dtype, 0, 2), randint_cpu((K, N), 81, dtype, -1, 2)
+    bias = randint_cpu((M_local,), 82, bias_dtype, -8, 9)
+    dbias = torch.full((3 * M_local,), float("nan"), dtype=bias_dtype, device="cuda")[::3]  # whatever lies between is not added
+    dbias.copy_(bias)
+    dA, dB = heap_tensor(ctx, A), heap_tensor(ctx, B)
+    out = ctx.zeros((W * M_local, N), dtype=dtype)
+    ctx.ops.matmul_all_gather(out, dA, dB, bias=dbias, config=iris.FusedConfig(block_size_m=32, block_size_n=64, block_size_k=8))
+    assert _lib.last_kernel().startswith("mfma_" + tile), _lib.last_kernel()
+    exp = oracle.matmul_all_gather(A, B, rank, W, bias=bias)
+    for r, got in enumerate(slot_copies(ctx, out)):
+        assert_bits_equal(got, exp[r], f"{_lib.last_kernel()} slot {r}")
+
+
 @pytest.mark.parametrize("path", ["mfma", "generic"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_all_reduce_atomic(path, dtype):
