@@ -713,7 +713,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     // them between its MFMAs (a wave issues in order: a burst of loads right after the barrier would
     // hold back the MFMAs behind it while the memory pipeline absorbs the burst).  Steps past the end
     // load nothing (every lane is out of range and deposits zeros), which keeps the per-thread count
-    // of outstanding loads identical on every step.
+    // of outstanding loads identical on every step that has any.
     struct StepLoads {
       int klim;
       unsigned sa, sb, a_soff, b_soff;
@@ -746,7 +746,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     auto issue_one = [&](const StepLoads& L, int j) { issue_at(L, j, load_offset(L, j)); };  // j in [0, LA + LB)
     auto end_step = [&]() {
       ++i_step;
-      if (++i_kb == nkb) {  // next source slot (gather along K only)
+      if (__builtin_expect(++i_kb == nkb, 0)) {  // next source slot (gather along K only)
         i_kb = 0;
         ++i_src;
         if (p.gather == GATHER_K && i_src < nsrc) ra = make_rsrc_words(in_slot(a_own, i_src) + a_tile_off);
@@ -767,18 +767,29 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
 #pragma unroll
         for (int i = 0; i < 4 * CFG::QUADS; ++i) acc.v[mb][nb][i] = 0.f;
 
-    // ---- prologue: fill STAGES-1 ring slots, wait for the first ----------------------------------
-    // The two-group loop reads a slot, and the next one's first fragments, while it refills: one step less is in flight.
-    constexpr int AHEAD = PINGPONG ? STAGES - 2 : STAGES - 1;  // K steps issued before the loop starts
+    // ---- prologue: the first K steps, wait for the first of them ------------------------------------
+    // Four-wave loop: STAGES-1 steps.  Two-group loop: three (a slot, and the next one's first fragments, are read while a third
+    // one is refilled).  When the first step is there already, from its prefetch, what the first product waits for is the loads'
+    // acceptance, 0.3 us a step: the early waves then stay two steps ahead, and the late ones send their third step out after the barrier.
+    const bool late = PINGPONG && wave >= 4;
+    const bool there = PREFETCH_NEXT && first_step_prefetched;
+    const int ahead = late || !there ? 3 : 2;  // K steps in flight before the loop starts
+    if constexpr (PINGPONG) {
+      if (there) end_step();  // only the loader position moves on
+      else issue(0);
+      issue(1);
+      if (!there) {
+        issue(2);
+        wait_vmcnt<2 * (LA + LB)>();
+      } else {
+        wait_vmcnt<LA + LB>();
+      }
+    } else {
 #pragma unroll
-    for (int s = 0; s < AHEAD; ++s) {
-      if (PREFETCH_NEXT && s == 0 && first_step_prefetched)
-        end_step();  // already on its way (or there): only the loader position moves on
-      else
-        issue(s);
+      for (int s = 0; s < STAGES - 1; ++s) issue(s);
+      wait_vmcnt<(STAGES - 2) * (LA + LB)>();
     }
     first_step_prefetched = false;
-    wait_vmcnt<(AHEAD - 1) * (LA + LB)>();
     __builtin_amdgcn_s_barrier();
     PHASE_STAMP(1);
     Frags<CFG> fr[KS < 2 ? 2 : KS];  // one set per k-slice (two for the loops that double-buffer)
@@ -796,7 +807,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     if constexpr (PINGPONG) {
       static_assert(KS == 1 && MB % 2 == 0 && NB % 2 == 0, "eight-wave loop: one k-slice per step, blocks in quadrants");
       // Eight waves, two per SIMD: waves 0-3 and waves 4-7 run half a step apart.  A step is a memory phase (the
-      // direct-to-LDS loads of the step three further on) and a compute phase (the products, with the fragment reads
+      // direct-to-LDS loads of a later step) and a compute phase (the products, with the fragment reads
       // in their shadow), each closed by a workgroup barrier, so that on every SIMD one wave feeds the matrix pipe
       // while the other one has the memory port to itself.  A direct-to-LDS load does not issue in the shadow of an
       // MFMA: a wave takes some 80 cycles to get one accepted.
@@ -808,13 +819,16 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       // which takes a ring of five: this step's slot, the next one's, one that is being waited for, one with loads in
       // flight, and the one being refilled, which the other group may have left only half a step ago.
       //
+      // The last steps, which have nothing to load any more, are a loop of their own: to load nothing takes as long as to load.
+      // Memory phases are as long as compute phases, so what else stands in them counts: a test of whether there is anything
+      // to load cost 4 to 7 % with long K, and without the hints of which way a step usually goes the compiler kept
+      // the usual way's scalars in vector registers in the build for split tiles (1 to 3 %).
+      //
       // What bounds it is power, with anything but zeros in the operands (bf16 4096x4096x8192 as a plain product, whole
       // launch: 186 us on normal data, 138 on zeros).  Before - 32x32x16 products, half of the fragments read in the
       // memory phase, a ring of four - it took 203 (zeros 130: one wave per SIMD issues a 16x16x32 product every 17
       // cycles, not 16), 8192x1792x4096 98 -> 92; 16x16x32 products in that loop 197 and 98; every fragment of B read in the
-      // memory phase 189; the left half of B one step ahead as well, through a copy, 188.  e4m3, whose 32x32x64 products
-      // stay, runs as before (100 us).
-      const bool late = wave >= 4;
+      // memory phase 189; the left half of B one step ahead as well, through a copy, 188.
       // The loader position of the common case - a whole K step inside one source - is carried in
       // scalar registers that advance by constants, and its loads need no per-lane k test; partial
       // steps, source changes and the empty steps past the end take the general path.
@@ -829,9 +843,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
             CFG::B_KCONTIG ? (unsigned)(kglob * ES) : (unsigned)(kglob * p.s_bk * ES));
         k_left = i_step < k_end ? klocal - i_kb * BK : 0;
       };
-      resync();
       unsigned rd = 0;                                    // byte offset of the slot this step reads
-      unsigned wr = AHEAD * CFG::STAGE_BYTES;             // ... and of the slot it refills
+      unsigned wr = ahead * CFG::STAGE_BYTES;             // ... and of the slot it refills
       const unsigned wr_wave = smem_base + wave * kDmaBytes;
       constexpr int NMFMA = MB * NB, HA = MB / 2, HB = NB / 2, Q = NMFMA / 4;
       __builtin_amdgcn_sched_barrier(0);  // (no fragment read moves up past the prologue's barrier)
@@ -840,40 +853,44 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
 #pragma unroll
       for (int mb = 0; mb < HA; ++mb) load_frag_a(fr[0], 0, 0, mb);
       if (late) {
-        wait_vmcnt<(AHEAD - 2) * (LA + LB)>();
+        if (there) issue(2);
+        wait_vmcnt<LA + LB>();
         __builtin_amdgcn_s_barrier();
       }
+      resync();
       auto product = [&](int i) {
         int mb, nb;
         quad_block<MB, NB>(i, mb, nb);
         acc.v[mb][nb] = mfma_of<CFG>(fr[0].a[mb], fr[0].b[nb], acc.v[mb][nb]);
       };
-      for (; s < k_end; ++s) {
+      auto k_step = [&](auto loads) __attribute__((always_inline)) {
 #pragma unroll
         for (int nb = 0; nb < HB; ++nb) load_frag_b(fr[0].b[nb], rd, 0, nb);
         __builtin_amdgcn_sched_barrier(0);
-        if (k_left >= BK) {
+        if constexpr (decltype(loads)::value) {
+          if (__builtin_expect(k_left >= BK, 1)) {
 #pragma unroll
-          for (int j = 0; j < LA; ++j) dma16(ra, wr_wave + wr + j * NW * kDmaBytes, a_voff[j], a_so);
+            for (int j = 0; j < LA; ++j) dma16(ra, wr_wave + wr + j * NW * kDmaBytes, a_voff[j], a_so);
 #pragma unroll
-          for (int i = 0; i < LB; ++i)
-            dma16(rb, wr_wave + wr + CFG::A_BYTES + i * NW * kDmaBytes, b_voff[i], b_so);
-        } else {
-          const StepLoads L = begin_step(wr);
+            for (int i = 0; i < LB; ++i)
+              dma16(rb, wr_wave + wr + CFG::A_BYTES + i * NW * kDmaBytes, b_voff[i], b_so);
+          } else {
+            const StepLoads L = begin_step(wr);
 #pragma unroll
-          for (int j = 0; j < LA + LB; ++j) issue_one(L, j);
-        }
-        end_step();
-        if (i_kb == 0) {
-          resync();
-        } else {
-          a_so += BK * ES;
-          b_so += b_inc;
-          k_left -= BK;
+            for (int j = 0; j < LA + LB; ++j) issue_one(L, j);
+          }
+          end_step();
+          if (__builtin_expect(i_kb == 0, 0)) {
+            resync();
+          } else {
+            a_so += BK * ES;
+            b_so += b_inc;
+            k_left -= BK;
+          }
         }
         const unsigned rd_next = rd + CFG::STAGE_BYTES == CFG::RING_BYTES ? 0 : rd + CFG::STAGE_BYTES;
-        // Own fragment reads done and own loads of step s+2 landed.
-        wait_vmcnt_lgkm0<(LA + LB)>();
+        // Own fragment reads done, and own loads landed: of step s+2, of waves that are two steps ahead s+1, and at the end all.
+        wait_vmcnt_lgkm0<decltype(loads)::value ? LA + LB : 0>();
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
@@ -895,7 +912,9 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
         __builtin_amdgcn_sched_barrier(0);
         rd = rd_next;
         wr = wr + CFG::STAGE_BYTES == CFG::RING_BYTES ? 0 : wr + CFG::STAGE_BYTES;
-      }
+      };
+      for (const int last = k_end - ahead; s < last; ++s) k_step(std::true_type{});
+      for (; s < k_end; ++s) k_step(std::false_type{});
       if (!late) __builtin_amdgcn_s_barrier();
     } else
     while (s < k_end) {
