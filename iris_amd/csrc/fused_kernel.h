@@ -393,11 +393,11 @@ __device__ __forceinline__ f32x16_t mfma_block(const i32x4_t (&a)[NF], const i32
   }
 }
 
-// One 16x16 MFMA of 16-bit data, operands in the same order.  The tiled kernel multiplies with this shape: busy with
+// One 16x16 MFMA of 16-bit data, operands in the same order.  The eight-wave tile multiplies with this shape: busy with
 // random data, the chip runs against its power limit, and a 16x16x32 product, which reads and writes its accumulators half
 // as often per flop as a 32x32x16 one, takes less of it (products from registers alone, eight waves of 128x64 per CU,
 // normal bf16 operands: 1750 against 2010 TFLOP/s, 2060 with the order of quad_block; both 2400 on zeros).  The
-// sums are the same, bit for bit: 32 k at a time in the same order.
+// results are those of two 32x32x16 products, bit for bit (the same rows on both tiles, random data: tests/test_gpu_k_steps.py).
 template <int IN>
 __device__ __forceinline__ f32x4_t mfma_block16(const i32x4_t (&a)[1], const i32x4_t (&b)[1], f32x4_t c) {
   if constexpr (IN == IN_BF16)

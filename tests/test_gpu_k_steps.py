@@ -6,7 +6,7 @@ import torch
 
 import iris_amd as iris
 from iris_amd import _lib, ops
-from helpers import assert_bits_equal, heap_tensor, oracle, randint_cpu
+from helpers import assert_bits_equal, heap_tensor, oracle, randint_cpu, randn_cpu
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +49,16 @@ def test_few_k_steps_of_several_sources(M, N, W, K_local):
     got, kernel = _product(A, B, W, W - 1, gather_dim=1)
     assert "_256x256x" in kernel, kernel
     assert_bits_equal(got, oracle.gemm(A, B, torch.bfloat16), f"{kernel}, {W} sources of {K_local}")
+
+
+# 16x16x32 products (256x256 tile) and 32x32x16 ones (128x128) of the same rows: random data, no sum exact, 3.4 million results
+# rounded to 16 bits; sums that differed in their last bit would round differently in about one of 2^15.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_both_shapes_of_products_give_the_same_bits(dtype):
+    M, N, K = 3072, 3328, 2080
+    A, B = randn_cpu((M, K), 304, dtype, K ** -0.5), randn_cpu((K, N), 305, dtype)
+    big, kernel = _product(A, B)
+    assert "_256x256x" in kernel, kernel
+    rows, kernel = _product(A[:1024].contiguous(), B)
+    assert "_128x128x" in kernel, kernel
+    assert_bits_equal(rows, big[:1024], "the same rows on the other tile")
