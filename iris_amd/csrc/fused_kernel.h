@@ -946,10 +946,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
           for (int j = 0; j < NLOAD; ++j)
             if (j * NSLOT / NLOAD == kk * MB + mb) issue_one(L, j);
 #pragma unroll
-          for (int i = 0; i < NB; ++i) {
-            const int nb = mb & 1 ? NB - 1 - i : i;  // (see quad_block)
-            acc.v[mb][nb] = mfma_of<CFG>(f.a[mb], f.b[nb], acc.v[mb][nb]);
-          }
+          for (int nb = 0; nb < NB; ++nb) acc.v[mb][nb] = mfma_of<CFG>(f.a[mb], f.b[nb], acc.v[mb][nb]);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
