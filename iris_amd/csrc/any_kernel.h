@@ -92,7 +92,7 @@ typedef u32x4_t u32x4_any_t __attribute__((aligned(1)));  // 16 bytes at any add
 // For the lambdas that the K loop is made of.  They keep their arrays in the kernel's registers only where they are inlined,
 // which the compiler's cost limit did not allow where a piece has sixteen elements: e4m3 operands were worked on in
 // scratch memory (1999x2877x1371 as a plain GEMM 200 -> 31 us, 4095x4095x2047 223 -> 75, 200x1001x3001 56 -> 12.5).
-#define INLINED __attribute__((always_inline))
+#define KLOOP_INLINED __attribute__((always_inline))
 
 // (Addresses computed from heap bases are integers to the compiler: without the address space it emits flat
 // accesses, which also wait on, and are waited for with, the LDS counter.)
@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const int b_safe_k = !b_edge ? p.K : p.s_bk >= CE ? p.K - 1 : 0;  // rows below this one can be read in whole pieces
 
   // Elements [0, count) of a piece, `stride` bytes apart; the rest of it zero.
-  auto load_elements = [&](const char* ptr, long long stride, int count) INLINED {
+  auto load_elements = [&](const char* ptr, long long stride, int count) KLOOP_INLINED {
     u32x4_t v = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int e = 0; e < CE; ++e)
@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   auto plain = [&]() {
     return a_vec && b_vec && klocal - f_kb * CFG::KSTEP >= CFG::KSTEP && f_src * klocal + (f_kb + 1) * CFG::KSTEP <= b_safe_k;
   };
-  auto advance = [&]() INLINED {
+  auto advance = [&]() KLOOP_INLINED {
     long long da = a_step, db = b_step;
     if (++f_kb == nkb) {  // on to the next source's columns
       f_kb = 0;
@@ -268,7 +268,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
     for (int i = 0; i < LB; ++i) ptr[LA + i] += db;
   };
-  auto fetch = [&]() INLINED {
+  auto fetch = [&]() KLOOP_INLINED {
     const int left = klocal - f_kb * CFG::KSTEP;  // elements of K from this step on
     if (left >= CFG::KSTEP && a_vec) {
 #pragma unroll
@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     }
     advance();
   };
-  auto put = [&](int buf) INLINED {
+  auto put = [&](int buf) KLOOP_INLINED {
     char* const s = smem + buf * CFG::BUF_BYTES;
 #pragma unroll
     for (int i = 0; i < LA; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + lds_at[i]) = raw[i];
@@ -307,7 +307,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   struct Frag {
     i32x4_t a[MB][NFRAG], b[NB][NFRAG];
   };
-  auto load_frag = [&](Frag& f, int buf, int kk) INLINED {
+  auto load_frag = [&](Frag& f, int buf, int kk) KLOOP_INLINED {
     const char* const sa = smem + buf * CFG::BUF_BYTES + wk * CFG::A_SLICE;
     const char* const sb = smem + buf * CFG::BUF_BYTES + CFG::A_BYTES + wk * CFG::B_SLICE;
 #pragma unroll
@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
   };
-  auto multiply = [&](const Frag& f) INLINED {
+  auto multiply = [&](const Frag& f) KLOOP_INLINED {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   // ---- K loop ---------------------------------------------------------------------------------------------
   // Step s reads LDS buffer s & 1; meanwhile step s+1 arrives in registers, is put into the other buffer half
   // way through the step's products, and the loads of step s+2 go out.
-  auto k_loop = [&]() INLINED {
+  auto k_loop = [&]() KLOOP_INLINED {
     point_at_a(std::false_type{});
     point_at_b(std::false_type{});
     clear_sums();
