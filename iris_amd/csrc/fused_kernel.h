@@ -746,7 +746,9 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     auto issue_one = [&](const StepLoads& L, int j) { issue_at(L, j, load_offset(L, j)); };  // j in [0, LA + LB)
     auto end_step = [&]() {
       ++i_step;
-      if (__builtin_expect(++i_kb == nkb, 0)) {  // next source slot (gather along K only)
+      ++i_kb;
+      const bool source_done = PINGPONG ? __builtin_expect(i_kb == nkb, 0) : i_kb == nkb;  // (the four-wave loop is slower with the hint)
+      if (source_done) {  // next source slot (gather along K only)
         i_kb = 0;
         ++i_src;
         if (p.gather == GATHER_K && i_src < nsrc) ra = make_rsrc_words(in_slot(a_own, i_src) + a_tile_off);
@@ -1056,9 +1058,18 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       constexpr int PIECES = MB * NB * CFG::QUADS, NBATCH = 4, BATCH = PIECES / NBATCH;
       constexpr long long SLOT_BYTES = (long long)PIECES * NT * 16;
       float badd[MB] = {};
-      if (p.bias) {
+      if constexpr (MB <= 2) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          if (p.bias) {
+            const int gm = m0 + wm * TM + mb * BLK + acc_col(lane);
+            if (gm < p.M) badd[mb] = load_scalar_as_float(p.bias, (long long)gm * p.s_bias, p.bias_dtype);
+          }
+        }
+      } else if (p.bias) {
         // Every load is out before the first is used (a block at a time the blocks of sixteen rows made eight round trips of
         // it, 6 of the 113 us of a plain fp16 16384x8192x128 with bias).  Rows past the end, which are never stored, take the last one's.
+        // (The four-wave tiles, with one or two rows a lane, are 0.6 % slower in this form, bias or not: fp16 two-shot 896x2880x512.)
         const bool wide = p.bias_dtype == IRIS_HIP_FP32;
         unsigned raw[MB];
         auto row_of = [&](int mb) -> long long {
