@@ -387,6 +387,22 @@ void launch_for_world(const CclParams& p, int grid, hipStream_t s) {
 #undef CCL_KERNEL
 }
 
+// The names of all configurations, put together once (formatting one takes longer than the checks of a small call).
+const char* kernel_name(int mode, int dtype, int vec) {
+  struct Names {
+    char text[5][3][9][48];
+    Names() {
+      static const char* modes[5] = {"slot_reduce_one_shot", "slot_reduce_two_shot", "slot_reduce_reduce_scatter", "slot_reduce_atomic", "dense_sum_one_shot"};
+      static const char* types[3] = {"bf16", "f16", "f32"};
+      for (int m = 0; m < 5; ++m)
+        for (int t = 0; t < 3; ++t)
+          for (int v = 0; v < 9; ++v) snprintf(text[m][t][v], sizeof(text[m][t][v]), "%s_%s_vec%d", modes[m], types[t], v);
+    }
+  };
+  static const Names names;
+  return names.text[mode][dtype][vec];
+}
+
 bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
 int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
@@ -489,11 +505,7 @@ int run_ccl(CclParams p, int distribution, int dtype, void* stream) {
                      (p.world == 2 || p.world == 4 || (p.world == 8 && (es == 4 || moved <= (double)(512 << 20))));
 
   hipStream_t s = (hipStream_t)stream;
-  char name[96];
-  static const char* modes[4] = {"slot_reduce_one_shot", "slot_reduce_two_shot", "slot_reduce_reduce_scatter", "slot_reduce_atomic"};
-  static const char* types[3] = {"bf16", "f16", "f32"};
-  snprintf(name, sizeof(name), "%s_%s_vec%d", dense ? "dense_sum_one_shot" : modes[p.mode], types[dtype], vec);
-  iris_host::set_last_kernel(name);
+  iris_host::set_last_kernel(kernel_name(dense ? 4 : p.mode, dtype, vec));
   if (p.total_units == 0) return 0;  // this rank owns nothing
 
   // Launches that move tens of megabytes read with non-temporal accesses: their operands are read once, and lines taken
