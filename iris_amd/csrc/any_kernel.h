@@ -91,7 +91,8 @@ typedef u32x4_t u32x4_any_t __attribute__((aligned(1)));  // 16 bytes at any add
 #define GLOBAL_AS __attribute__((address_space(1)))
 // For the lambdas that the K loop is made of.  They keep their arrays in the kernel's registers only where they are inlined,
 // which the compiler's cost limit did not allow where a piece has sixteen elements: e4m3 operands were worked on in
-// scratch memory (1999x2877x1371 as a plain GEMM 200 -> 31 us, 4095x4095x2047 223 -> 75, 200x1001x3001 56 -> 12.5).
+// scratch memory (1999x2877x1371 as a plain GEMM 200 -> 31 us, 4095x4095x2047 223 -> 75, 200x1001x3001 56 -> 12.5).  On the
+// 256x256 tile (the 4095x4095x2047) 17 to 19 registers still do not fit and are spilled, 72 to 80 bytes a lane.
 #define KLOOP_INLINED __attribute__((always_inline))
 
 // (Addresses computed from heap bases are integers to the compiler: without the address space it emits flat
@@ -971,6 +972,7 @@ int launch_any(FusedParams p, int device, int cu_count, hipStream_t stream, cons
 // - / 48 / 105), one-shot with seven peers 500x2877x1371 64x64 30 (92 / 46 / 32 / - / 51), 33x2877x1371 32x32 13 (49 / 31 / 25 / 20 / -);
 // float32 2048x2880x1024 64x128 98 (108 / - / 113 / 174), 2048x2048x4096 128x128 199 (- / 236 / 260 / 381), 512x2880x1024 64x64 40
 // (47 / 45 / - / 44), 300x4096x4096 32x32 129 (159 / 153 / 138 / -), and, the one miss, 1536x2880x1024 64x64 87 (100 / 80 / - / 121).
+// (e4m3 goes by the rates of bf16; they have not been measured for it.)
 struct AnyTile {
   int bm, bn;
   float rate;

@@ -2,11 +2,12 @@
 // operators, and the C ABI declared in include/iris_hip.h.
 //
 // Two kernels implement every operator (the first lives in fused_kernel.h and is compiled in the
-// iris_hip_mfma_<type>.hip translation units; the entry points are in this file):
+// iris_hip_mfma_<type>.hip translation units; small outputs have one of their own, decode_kernel.h; the entry points are in this file):
 //
-//  * fused_mfma_kernel  - persistent tiled GEMM on the 32x32 MFMA blocks of CDNA4.  Operand tiles
-//    travel HBM -> LDS with 16-byte direct-to-LDS buffer loads into a ring of STAGES buffers
-//    (prefetch distance STAGES-1, one workgroup barrier per K step); the K-contiguous operand is
+//  * fused_mfma_kernel  - persistent tiled GEMM on the matrix cores of CDNA4 (16x16 products of 16-bit data on the
+//    256x256 tile, 32x32 products otherwise).  Operand tiles travel HBM -> LDS with 16-byte direct-to-LDS buffer
+//    loads into a ring of STAGES buffers (four-wave tiles: STAGES-1 K steps in flight, one workgroup barrier per
+//    step; the eight-wave tile, whose wave groups run half a step apart: two or three, and two barriers); the K-contiguous operand is
 //    read back with 16-byte LDS reads, the N-contiguous one with LDS transpose reads.  The waves of
 //    a workgroup (8 as 2x4 for the 256x256 tile, 4 as 2x2 for the smaller ones) each own a block of
 //    fp32 accumulators that stays in the accumulation registers.  Requires 16-byte aligned,
