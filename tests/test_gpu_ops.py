@@ -422,6 +422,8 @@ def test_bias_of_any_type_and_stride(M_local, N, dtype, tile, bias_dtype):
     dbias.copy_(bias)
     dA, dB = heap_tensor(ctx, A), heap_tensor(ctx, B)
     out = ctx.zeros((W * M_local, N), dtype=dtype)
+    for r in range(W):
+        ctx.peer_view(out, r).zero_()
     ctx.ops.matmul_all_gather(out, dA, dB, bias=dbias, config=iris.FusedConfig(block_size_m=32, block_size_n=64, block_size_k=8))
     assert _lib.last_kernel().startswith("mfma_" + tile), _lib.last_kernel()
     exp = oracle.matmul_all_gather(A, B, rank, W, bias=bias)

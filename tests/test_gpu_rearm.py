@@ -198,6 +198,7 @@ def test_launches_in_graphs_and_the_preamble(op, wrapper, monkeypatch):
     ccl_cfg = Config(all_reduce_variant="one_shot")
     if op == "ccl":
         module, name = sys.modules["iris_amd.ccl.all_reduce"], "all_reduce_preamble"
+        ctx.peer_view(x, 1).zero_()  # (a heap's memory is as it was found; zeros() clears the own slot)
         ws = ctx.ccl.all_reduce_preamble(C, x, config=ccl_cfg)
         call = lambda: ctx.ccl.all_reduce(C, x, async_op=True, config=ccl_cfg, workspace=ws)
     elif op == "reduce_scatter":
