@@ -89,11 +89,11 @@ struct AnyCfg {
 
 typedef u32x4_t u32x4_any_t __attribute__((aligned(1)));  // 16 bytes at any address
 #define GLOBAL_AS __attribute__((address_space(1)))
-// For the lambdas that the K loop is made of.  They keep their arrays in the kernel's registers only where they are inlined,
+// For the lambdas that the kernel is made of.  They keep their arrays in the kernel's registers only where they are inlined,
 // which the compiler's cost limit did not allow where a piece has sixteen elements: e4m3 operands were worked on in
 // scratch memory (1999x2877x1371 as a plain GEMM 200 -> 31 us, 4095x4095x2047 223 -> 75, 200x1001x3001 56 -> 12.5).  On the
 // 256x256 tile (the 4095x4095x2047) 17 to 19 registers still do not fit and are spilled, 72 to 80 bytes a lane.
-#define KLOOP_INLINED __attribute__((always_inline))
+#define INLINED __attribute__((always_inline))
 
 // (Addresses computed from heap bases are integers to the compiler: without the address space it emits flat
 // accesses, which also wait on, and are waited for with, the LDS counter.)
@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const char* ptr[LA + LB];  // (A's pieces first, then B's)
   int a_k[LA], lds_at[LA + LB];
   int f_kb, f_src;  // K step the next fetch brings
-  auto point_at_a = [&](auto split_tag) {
+  auto point_at_a = [&](auto split_tag) INLINED {
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
       const int id = tid + i * NT, sub = id / (BM * 8), in_sub = id - sub * (BM * 8);
@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const bool b_vec = !CFG::BKC || p.s_bk == 1;
   int b_k[LB];
   int b_cols;  // [k][n] tile: columns of this thread's piece that exist
-  auto point_at_b = [&](auto split_tag) {
+  auto point_at_b = [&](auto split_tag) INLINED {
     constexpr bool SPLIT = decltype(split_tag)::value;
     b_cols = CE;
 #pragma unroll
@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const int b_safe_k = !b_edge ? p.K : p.s_bk >= CE ? p.K - 1 : 0;  // rows below this one can be read in whole pieces
 
   // Elements [0, count) of a piece, `stride` bytes apart; the rest of it zero.
-  auto load_elements = [&](const char* ptr, long long stride, int count) KLOOP_INLINED {
+  auto load_elements = [&](const char* ptr, long long stride, int count) INLINED {
     u32x4_t v = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int e = 0; e < CE; ++e)
@@ -252,10 +252,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const long long a_step = (long long)CFG::KSTEP * p.s_ak * ES, b_step = (long long)CFG::KSTEP * p.s_bk * ES;
   u32x4_t raw[LA + LB];
   // Whether the next fetch brings nothing but whole pieces.
-  auto plain = [&]() {
+  auto plain = [&]() INLINED {
     return a_vec && b_vec && klocal - f_kb * CFG::KSTEP >= CFG::KSTEP && f_src * klocal + (f_kb + 1) * CFG::KSTEP <= b_safe_k;
   };
-  auto advance = [&]() KLOOP_INLINED {
+  auto advance = [&]() INLINED {
     long long da = a_step, db = b_step;
     if (++f_kb == nkb) {  // on to the next source's columns
       f_kb = 0;
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
     for (int i = 0; i < LB; ++i) ptr[LA + i] += db;
   };
-  auto fetch = [&]() KLOOP_INLINED {
+  auto fetch = [&]() INLINED {
     const int left = klocal - f_kb * CFG::KSTEP;  // elements of K from this step on
     if (left >= CFG::KSTEP && a_vec) {
 #pragma unroll
@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     }
     advance();
   };
-  auto put = [&](int buf) KLOOP_INLINED {
+  auto put = [&](int buf) INLINED {
     char* const s = smem + buf * CFG::BUF_BYTES;
 #pragma unroll
     for (int i = 0; i < LA; ++i) *(LDS_AS u32x4_t*)(LDS_AS char*)(s + lds_at[i]) = raw[i];
@@ -308,7 +308,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   struct Frag {
     i32x4_t a[MB][NFRAG], b[NB][NFRAG];
   };
-  auto load_frag = [&](Frag& f, int buf, int kk) KLOOP_INLINED {
+  auto load_frag = [&](Frag& f, int buf, int kk) INLINED {
     const char* const sa = smem + buf * CFG::BUF_BYTES + wk * CFG::A_SLICE;
     const char* const sb = smem + buf * CFG::BUF_BYTES + CFG::A_BYTES + wk * CFG::B_SLICE;
 #pragma unroll
@@ -355,7 +355,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     }
   };
   f32x16_t acc[MB][NB];
-  auto clear_sums = [&]() {
+  auto clear_sums = [&]() INLINED {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -363,7 +363,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
   };
-  auto multiply = [&](const Frag& f) KLOOP_INLINED {
+  auto multiply = [&](const Frag& f) INLINED {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -381,7 +381,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
       }
   };
   // Every wave's LDS accesses done, then everybody's; loads to registers stay in flight.
-  auto lds_barrier = [&]() {
+  auto lds_barrier = [&]() INLINED {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt((0xF) | (0x3 << 14) | (0x7 << 4));  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
@@ -391,7 +391,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   // ---- K loop ---------------------------------------------------------------------------------------------
   // Step s reads LDS buffer s & 1; meanwhile step s+1 arrives in registers, is put into the other buffer half
   // way through the step's products, and the loads of step s+2 go out.
-  auto k_loop = [&]() KLOOP_INLINED {
+  auto k_loop = [&]() INLINED {
     point_at_a(std::false_type{});
     point_at_b(std::false_type{});
     clear_sums();
@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     unsigned low = ~0u;  // smallest magnitude of a nonzero element: its bits without the sign, doubled, less one
     // One of the six parts of the splitting of a 16-byte piece v, in which v is left as the remainder:
     // elements 2 * (part & 1) and the next, plane part / 2.
-    auto split_part = [&](u32x4_t& v, u32x2_t (&w)[3], int part) {
+    auto split_part = [&](u32x4_t& v, u32x2_t (&w)[3], int part) INLINED {
       const int e = 2 * (part & 1), i = part / 2;
       if (i == 0) low = min(low, min((v[e] << 1) - 1u, (v[e + 1] << 1) - 1u));
       const float x = __uint_as_float(v[e]), y = __uint_as_float(v[e + 1]);
@@ -463,10 +463,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         v[e + 1] = __float_as_uint(y - __uint_as_float(h & 0xFFFF0000u));
       }
     };
-    auto put_plane = [&](const u32x2_t (&w)[3], int at, int plane, int i) {
+    auto put_plane = [&](const u32x2_t (&w)[3], int at, int plane, int i) INLINED {
       *(LDS_AS u32x2_t*)(LDS_AS char*)(smem + at + i * plane) = w[i];
     };
-    auto put_split = [&](u32x4_t& v, int at, int plane) {
+    auto put_split = [&](u32x4_t& v, int at, int plane) INLINED {
       u32x2_t w[3];
 #pragma unroll
       for (int part = 0; part < 6; ++part) split_part(v, w, part);
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     struct Pieces {
       i32x4_t a[MB][1], b[NB][1];
     };
-    auto load_pieces = [&](Pieces& f, int buf, int kk, int i) {  // plane i of k-slice kk
+    auto load_pieces = [&](Pieces& f, int buf, int kk, int i) INLINED {  // plane i of k-slice kk
       const char* const sa = smem + buf * CFG::SPLIT_BUF + i * CFG::A_PLANE;
       const char* const sb = smem + buf * CFG::SPLIT_BUF + 3 * CFG::A_PLANE + i * CFG::B_PLANE;
       const int c = frag16_chunk(lane, kk);
@@ -504,7 +504,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     f32x16_t small[MB][NB];  // sums of the five smaller products
     constexpr int kPairs[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};  // the smallest products first
     constexpr int KS16 = CFG::KE / 16, NMUL = KS16 * 6 * MB * NB, PARTS = 6 * (LA + LB);
-    auto step = [&](int buf, auto fetch_tag) {
+    auto step = [&](int buf, auto fetch_tag) INLINED {
       const int to = (buf ^ 1) * CFG::SPLIT_BUF;
       Pieces f[KS16][3];
       u32x2_t w[3];
@@ -542,7 +542,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
     // Eight waves: one barrier per step.  What a wave reads of the vote behind the barrier of step s, another one may
     // already be past: nobody writes ahead of the barrier of step s + 1 then (layout.h), `tiny` keeps the answer.
     bool tiny = false;  // an operand of the steps put down so far is below 2^-110
-    auto close_step = [&]() {
+    auto close_step = [&]() INLINED {
       if (s + 1 < nsteps) tiny = low < kSmallest;  // (the last step puts down leftovers)
       if (tiny && vote_written_before_barrier(s)) *vote = 1;
       lds_barrier();
@@ -640,7 +640,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         }
     lds_barrier();
   }
-  auto stage4 = [&](int row, int col, const float (&sum)[4], float badd) {
+  auto stage4 = [&](int row, int col, const float (&sum)[4], float badd) INLINED {
     char* const dst = smem + row * CFG::TROW + col * Out::size;
     float h[4];
 #pragma unroll
@@ -652,7 +652,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
       *(LDS_AS u32x2_t*)(LDS_AS char*)dst = (u32x2_t){Out16::pack(h[0], h[1]), Out16::pack(h[2], h[3])};
     }
   };
-  auto bias_of = [&](int row) -> float {
+  auto bias_of = [&](int row) INLINED -> float {
     return p.bias && m0 + row < p.M ? load_scalar_as_float(p.bias, (long long)(m0 + row) * p.s_bias, p.bias_dtype) : 0.f;
   };
   if constexpr (CFG::WK > 1) {
@@ -701,9 +701,9 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const bool whole = cols == OE && p.s_cn == 1;  // moved as 16 bytes, else element by element
   const int ftn = cdiv(p.N, p.flag_bn);
   const int ftotal = cdiv(p.M, p.flag_bm) * ftn;
-  auto staged = [&](int row) { return smem + row * CFG::TROW + t_col * Out::size; };
-  auto staged_piece = [&](int row) { return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)staged(row); };
-  auto staged_element = [&](int row, int e) -> float {
+  auto staged = [&](int row) INLINED { return smem + row * CFG::TROW + t_col * Out::size; };
+  auto staged_piece = [&](int row) INLINED { return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)staged(row); };
+  auto staged_element = [&](int row, int e) INLINED -> float {
     if constexpr (Out::size == 4) {
       return *(const LDS_AS float*)(LDS_AS char*)(staged(row) + e * 4);
     } else {
@@ -711,10 +711,10 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
       return Out::kFp32SumInReference ? f16_bits_to_float(b) : bf16_bits_to_float(b);
     }
   };
-  auto offset = [&](int row, int e) {  // bytes into C (or aux) of element e of this thread's piece
+  auto offset = [&](int row, int e) INLINED {  // bytes into C (or aux) of element e of this thread's piece
     return ((long long)(m0 + row + p.row_offset) * p.s_cm + (long long)(gn + e) * p.s_cn) * Out::size;
   };
-  auto owner_at = [&](int gm, int g) { return owner_of(p.epi, (gm / p.flag_bm) * ftn + g / p.flag_bn, ftotal, p.world, p.rank); };
+  auto owner_at = [&](int gm, int g) INLINED { return owner_of(p.epi, (gm / p.flag_bm) * ftn + g / p.flag_bn, ftotal, p.world, p.rank); };
 
   if (p.epi == EPI_ATOMIC) {
     if constexpr (Out::size == 4) {
@@ -785,7 +785,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const bool flags = epi_has_flags(p.epi);
   const bool solo = flags && (!p.sum_peers || p.world == 1);  // no peer contributes: the sum is the own tile
   // Stores of a result piece (or its elements) to wherever the operator wants it.
-  auto each_destination = [&](int gm, int g, auto&& store) {
+  auto each_destination = [&](int gm, int g, auto&& store) INLINED {
     if (p.epi == EPI_STORE) {
       store(p.C);
     } else if (p.epi == EPI_ALL_GATHER) {
@@ -852,11 +852,12 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 
   // Slot sum in ascending rank order from the own (already rounded) value, in fp32 or by the reference's rule.
   const bool ref_chain = (p.acc_mode == IRIS_HIP_ACC_REFERENCE) && !Out::kFp32SumInReference;
-  auto add = [&](float sum, float x) {
+  auto add = [&](float sum, float x) INLINED {
     sum += x;
     return ref_chain ? Out::round(sum) : sum;
   };
-  auto reduce = [&](auto np_tag) {
+  auto reduce = [&](auto np_tag, auto nt_tag) INLINED {
+    auto load_peer = [](const char* at) INLINED { return decltype(nt_tag)::value ? load16_any_nt(at) : load16_any(at); };
     constexpr int NP = decltype(np_tag)::value;  // peers, all of whose loads go out together; 0: any number
     constexpr int NPV = NP > 0 ? NP : 1;
     // Passes whose loads are in flight together: as many as the registers hold (the sums are staged and their
@@ -875,7 +876,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
         if constexpr (NP > 0) {
           if (act[g] && piece_ok) {
 #pragma unroll
-            for (int i = 0; i < NP; ++i) pv[g][i] = load16_any_nt(slot_ptr(p.heap_bases, p.aux, p.rank, i < p.rank ? i : i + 1) + offset(row, 0));
+            for (int i = 0; i < NP; ++i) pv[g][i] = load_peer(slot_ptr(p.heap_bases, p.aux, p.rank, i < p.rank ? i : i + 1) + offset(row, 0));
           }
         }
       }
@@ -896,7 +897,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
           } else {
             for (int pr = 0; pr < p.world; ++pr) {
               if (pr == p.rank) continue;
-              OutPiece<Out>::unpack(load16_any_nt(slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row, 0)), x);
+              OutPiece<Out>::unpack(load_peer(slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row, 0)), x);
 #pragma unroll
               for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
             }
@@ -924,11 +925,16 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
       }
     }
   };
+  auto reduce_with = [&](auto np_tag) INLINED {
+    // (The 32x32 tile is for small outputs: one way is enough.)
+    if (CFG::WK == 1 && p.stream_peers) reduce(np_tag, std::integral_constant<bool, CFG::WK == 1>{});
+    else reduce(np_tag, std::false_type{});
+  };
   switch (p.world - 1) {
-    case 1: reduce(std::integral_constant<int, 1>{}); break;
-    case 3: reduce(std::integral_constant<int, 3>{}); break;
-    case 7: reduce(std::integral_constant<int, 7>{}); break;
-    default: reduce(std::integral_constant<int, 0>{}); break;
+    case 1: reduce_with(std::integral_constant<int, 1>{}); break;
+    case 3: reduce_with(std::integral_constant<int, 3>{}); break;
+    case 7: reduce_with(std::integral_constant<int, 7>{}); break;
+    default: reduce(std::integral_constant<int, 0>{}, std::false_type{}); break;
   }
   PHASE_STAMP(7);
 }

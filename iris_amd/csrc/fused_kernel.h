@@ -61,6 +61,8 @@ struct FusedParams {
   int flag_bm, flag_bn;
   int epi;
   int acc_mode;
+  int whole_lines;   // rows of C and aux start and end with 128-byte lines (see store16_system_nt)
+  int stream_peers;  // the peers' tiles are read past the caches (peers_past_caches in iris_hip.hip)
   int clear_c;  // IRIS_HIP_CLEAR_C: the own slot's C ends up as if it had been zeroed before the launch
   int all_owners;
   int sum_peers;
@@ -340,7 +342,15 @@ __device__ __forceinline__ void store16_system(char* p, u32x4_t v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
 }
 
-// The same for data that the next instructions overwrite with VALU results (accumulator reads, say):
+// The same for rows that are whole lines, past the caches' keep policy as well: own tiles on their way to the peers do not push
+// everything else out of the last-level cache (bf16, eight ranks, six workspaces in turn: reduce-scatter 8192x4096x1376
+// 118.6 -> 104.9 us, two-shot 8192x4096x1376 126.6 -> 112.2; with one workspace, which the cache holds, 103.4 -> 104.4 and 107 ->
+// 111).  A line that two workgroups write in parts does better in the cache (2000x2896x1376 51.2 us, this way 53.8).
+__device__ __forceinline__ void store16_system_nt(char* p, u32x4_t v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(v) : "memory");
+}
+
+// store16_system for data that the next instructions overwrite with VALU results (accumulator reads, say):
 // a store of more than 8 bytes is still fetching its data registers for the last lanes when the next
 // instruction issues, and a VALU write to them in that slot reaches memory for those lanes.  The
 // compiler pads this hazard between instructions it can see; it cannot see into the asm statement, so
@@ -1223,7 +1233,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
           const u32x4_t v = *(const LDS_AS u32x4_t*)(LDS_AS char*)(smem + t_pass[ps & 1] + ps * RPP * CFG::TROW);
           if (gm < p.M && col_ok) {
             const long long eoff = ((long long)gm * p.s_cm + gn) * 2;
-            store16_system(p.aux + eoff, v);  // aux: read by the peers as soon as the flag is up
+            if (p.whole_lines) store16_system_nt(p.aux + eoff, v);
+            else store16_system(p.aux + eoff, v);  // aux: read by the peers as soon as the flag is up
             int owner = p.rank;
             if (by_owner) {
               owner = owner_of(p.epi, (gm / p.flag_bm) * ftn1 + gn / p.flag_bn, ftotal1, p.world, p.rank);
@@ -1281,17 +1292,20 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       for (int i = 0; i < kMaxCachedSlots - 1; ++i) pb[i] = (i < p.rank ? hb[i] : hb[i + 1]) + (aux_own - hb_own);
       const long long safe_off = ((long long)m0 * p.s_cm + n0) * 2;  // first element of the tile
 
-      // The peers' tiles are read once and C is written once, so both go past the caches' keep
-      // policy (non-temporal): they neither displace the operands nor - what costs more - make the
-      // last-level cache write back whatever dirty lines it holds to take them in (measured on the
-      // 4096 x 4096 x 1376 bf16 launch with seven peers, after a 256 MB buffer had been zeroed: phase 2
-      // 68 -> 39 us; with the peers' tiles already cached the two policies tie for the one-shot variant).
+      // The peers' tiles are read once and C is written once.  C, and the peers' tiles of launches that move more than
+      // the last-level cache takes in, go past the caches' keep policy (non-temporal): they neither displace the operands nor -
+      // what costs more - make that cache write back whatever dirty lines it holds (4096 x 4096 x 1376
+      // bf16 with seven peers, after a 256 MB buffer had been zeroed: phase 2 68 -> 39 us).  Smaller launches, and rows
+      // that are not whole lines, read the peers' tiles through the caches (peers_past_caches in iris_hip.hip has the figures).
       // Chunks are handed to the threads either over the whole kernel tile (RECT false: thread t
       // takes chunk t of every pass, ownership looked up per chunk) or over one rectangle of it,
       // rows [r0, r1) and `ncw` chunks from column c0, all of which `rect_owner` reduces (RECT true).
-      auto reduce_chunks = [&](auto np_tag, auto rect_tag, int r0, int r1, int c0, int ncw, int rect_owner) {
+      auto reduce_chunks = [&](auto np_tag, auto nt_tag, auto rect_tag, int r0, int r1, int c0, int ncw, int rect_owner) {
         constexpr int NP = decltype(np_tag)::value;  // peers with cached bases; -1: any number
         constexpr bool RECT = decltype(rect_tag)::value;
+        auto load_peer = [](unsigned long long at) {
+          return decltype(nt_tag)::value ? __builtin_nontemporal_load((const u32x4_t*)at) : *(const u32x4_t*)at;
+        };
         constexpr int NPV = NP > 0 ? NP : 1;
         const int npasses = RECT ? cdiv((r1 - r0) * ncw, NT) : PASSES;
         // One pass of the workgroup: the addresses of this thread's chunk, the peers' chunks requested, the
@@ -1326,7 +1340,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
           st.eoff = st.active ? ((long long)gm * p.s_cm + gc) * 2 : safe_off;
           if constexpr (NP > 0) {
 #pragma unroll
-            for (int i = 0; i < NP; ++i) st.pv[i] = __builtin_nontemporal_load((const u32x4_t*)(pb[i] + st.eoff));
+            for (int i = 0; i < NP; ++i) st.pv[i] = load_peer(pb[i] + st.eoff);
           }
           st.own = *(const LDS_AS u32x4_t*)(LDS_AS char*)(smem + lds_off);
         };
@@ -1354,7 +1368,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
             for (int i = 0; i < NP; ++i) add_peer(st.pv[i]);
           } else if constexpr (NP < 0) {
             for (int pr = 0; pr < p.world; ++pr)
-              if (pr != p.rank) add_peer(__builtin_nontemporal_load((const u32x4_t*)(in_slot(aux_own, pr) + st.eoff)));
+              if (pr != p.rank) add_peer(load_peer(in_slot(aux_own, pr) + st.eoff));
           }
           u32x4_t res;
 #pragma unroll
@@ -1417,11 +1431,11 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       // large enough to keep the workgroup busy, each owned one is streamed as a rectangle by all
       // threads, and a kernel tile without an owned flag tile issues nothing at all; with small flag
       // tiles the threads keep their places in the kernel tile and the stores are predicated.
-      auto reduce_tile = [&](auto np_tag) {
+      auto reduce_tile = [&](auto np_tag, auto nt_tag) {
         const int m1 = min(m0 + BM, p.M), n1 = min(n0 + BN, p.N);
         const bool by_rect = p.epi != EPI_ONE_SHOT && min(p.flag_bm, BM) * (min(p.flag_bn, BN) / 8) * 2 >= NT;
         if (!by_rect) {
-          reduce_chunks(np_tag, std::false_type{}, 0, 0, 0, 0, 0);
+          reduce_chunks(np_tag, nt_tag, std::false_type{}, 0, 0, 0, 0, 0);
           return;
         }
         for (int fr = m0 / p.flag_bm; fr * p.flag_bm < m1; ++fr)
@@ -1430,15 +1444,19 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
             if (!p.all_owners && owner != p.rank) continue;
             const int r0 = max(m0, fr * p.flag_bm), r1 = min(m1, (fr + 1) * p.flag_bm);
             const int c0 = max(n0, fc * p.flag_bn), c1 = min(n1, (fc + 1) * p.flag_bn);
-            reduce_chunks(np_tag, std::true_type{}, r0, r1, c0, (c1 - c0) / 8, owner);
+            reduce_chunks(np_tag, nt_tag, std::true_type{}, r0, r1, c0, (c1 - c0) / 8, owner);
           }
+      };
+      auto reduce_with = [&](auto np_tag) {
+        if (p.stream_peers) reduce_tile(np_tag, std::true_type{});
+        else reduce_tile(np_tag, std::false_type{});
       };
       switch (solo ? -2 : (p.world <= kMaxCachedSlots ? npeers : -1)) {
         case -2: break;  // C was written in phase 1
-        case 1: reduce_tile(std::integral_constant<int, 1>{}); break;
-        case 3: reduce_tile(std::integral_constant<int, 3>{}); break;
-        case 7: reduce_tile(std::integral_constant<int, 7>{}); break;
-        default: reduce_tile(std::integral_constant<int, -1>{}); break;
+        case 1: reduce_with(std::integral_constant<int, 1>{}); break;
+        case 3: reduce_with(std::integral_constant<int, 3>{}); break;
+        case 7: reduce_with(std::integral_constant<int, 7>{}); break;
+        default: reduce_tile(std::integral_constant<int, -1>{}, std::true_type{}); break;
       }
     }
     PHASE_STAMP(7);

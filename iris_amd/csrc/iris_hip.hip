@@ -263,6 +263,25 @@ bool decode_gather_ok(const FusedParams& p, int in_dtype) {
   return true;
 }
 
+// Whether the slot sum reads the peers' tiles past the caches' keep policy.  Up to 32 MiB of them are read through the
+// caches: the slots of such a launch, its neighbours' and their outputs fit the 256 MB last-level cache, which then serves
+// what the peers have just written, and lines that two tiles share are fetched once.  What does not fit would only push the rest
+// out of it, dirty lines first.  Eight ranks, us, past the caches -> through them, with two workspaces in turn (and with six): fp16 two-shot
+// 896x2880x512 (5 MB read) 18.9 -> 17.3 (20.2 -> 18.8), bf16 900x2896x512 23.5 -> 19.8 (23.6 -> 20.1), reduce-scatter
+// 4096x4096x1376 (29 MB) 66.8 -> 57.9 (70.0 -> 69.9), float32 two-shot 2048x2880x1024 of four ranks (18 MB) 107.7 -> 103.6;
+// one-shot 1024x2880x1376 (41 MB) 29.9 -> 28.6 (30.0 -> 32.3), 4096x4096x1376 (235 MB) 84.9 -> 95.5.
+bool peers_past_caches(const FusedParams& p, int out_dtype) {
+  const long long all = (long long)p.M * p.N * elem_size(out_dtype) * (p.world - 1);
+  const long long read = p.epi == EPI_ONE_SHOT || p.all_owners ? all : all / p.world;
+  return epi_has_flags(p.epi) && read > (32ll << 20);
+}
+
+// Whether every row of C and aux starts and ends with a 128-byte line.
+bool rows_of_whole_lines(const FusedParams& p, int out_dtype) {
+  const int es = elem_size(out_dtype);
+  return p.s_cn == 1 && ((p.s_cm * es) | ((long long)p.N * es)) % 128 == 0 && (((uintptr_t)p.aux | (uintptr_t)p.C) & 127) == 0;
+}
+
 // check_only: run every argument check and the kernel choice, launch nothing (0 = the launch would go out).
 int run_fused(FusedParams p, int in_dtype, int out_dtype, int path, void* stream, bool check_only = false) {
   g_last_error[0] = 0;
@@ -293,6 +312,8 @@ int run_fused(FusedParams p, int in_dtype, int out_dtype, int path, void* stream
   int rc = facts_for(device, &facts);
   if (rc) return rc;
   p.num_xcd = facts->xcc_count;
+  p.whole_lines = rows_of_whole_lines(p, out_dtype);
+  p.stream_peers = peers_past_caches(p, out_dtype);
   hipStream_t s = (hipStream_t)stream;
 
   // Tile choice (the tile list in fused_kernel.h has the measurements): the 256x256 tile from about half the
