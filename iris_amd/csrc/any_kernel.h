@@ -17,6 +17,7 @@
 // of a source.
 #pragma once
 
+#include "any_epilogue.h"
 #include "fused_kernel.h"
 
 constexpr int IN_F32 = 3;  // next to IN_BF16, IN_F16, IN_FP8
@@ -86,65 +87,6 @@ struct AnyCfg {
   static_assert(SMEM_BYTES * WG_PER_CU <= 160 * 1024, "LDS budget of a gfx950 CU");
   static_assert((BM * 8) % NT == 0 && (BN * 8) % NT == 0 && NT % CPR == 0, "whole pieces per thread");
 };
-
-typedef u32x4_t u32x4_any_t __attribute__((aligned(1)));  // 16 bytes at any address
-#define GLOBAL_AS __attribute__((address_space(1)))
-// For the lambdas that the kernel is made of.  They keep their arrays in the kernel's registers only where they are inlined,
-// which the compiler's cost limit did not allow where a piece has sixteen elements: e4m3 operands were worked on in
-// scratch memory (1999x2877x1371 as a plain GEMM 200 -> 31 us, 4095x4095x2047 223 -> 75, 200x1001x3001 56 -> 12.5).  On the
-// 256x256 tile (the 4095x4095x2047) 17 to 19 registers still do not fit and are spilled, 72 to 80 bytes a lane.
-#define INLINED __attribute__((always_inline))
-
-// (Addresses computed from heap bases are integers to the compiler: without the address space it emits flat
-// accesses, which also wait on, and are waited for with, the LDS counter.)
-__device__ __forceinline__ u32x4_t load16_any(const char* p) { return *(const GLOBAL_AS u32x4_any_t*)(GLOBAL_AS const char*)p; }
-__device__ __forceinline__ u32x4_t load16_any_nt(const char* p) {
-  return __builtin_nontemporal_load((const GLOBAL_AS u32x4_any_t*)(GLOBAL_AS const char*)p);
-}
-// Results: past the caches' keep policy when the rows are whole 16-byte pieces, through them otherwise, where the L2 puts
-// the pieces of a line together first (bf16 4096x4095x352 27.3 -> 25.0 us; the aligned 4096x4096x352 23.5 against 24.5).
-__device__ __forceinline__ void store16_result(char* p, u32x4_t v, bool aligned) {
-  if (aligned) __builtin_nontemporal_store(v, (GLOBAL_AS u32x4_t*)(GLOBAL_AS char*)p);
-  else *(GLOBAL_AS u32x4_any_t*)(GLOBAL_AS char*)p = v;
-}
-
-// One 16-byte piece of output elements as floats.
-template <class Out>
-struct OutPiece;
-template <class Out16>
-struct OutPiece16 {
-  static __device__ __forceinline__ void unpack(u32x4_t v, float (&f)[8]) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      f[2 * e] = Out16::to_float((unsigned short)(v[e] & 0xFFFF));
-      f[2 * e + 1] = Out16::to_float((unsigned short)(v[e] >> 16));
-    }
-  }
-  static __device__ __forceinline__ u32x4_t pack(const float (&f)[8]) {
-    return (u32x4_t){Out16::pack(f[0], f[1]), Out16::pack(f[2], f[3]), Out16::pack(f[4], f[5]), Out16::pack(f[6], f[7])};
-  }
-};
-template <> struct OutPiece<ElemBF16> : OutPiece16<OutBF16> {};
-template <> struct OutPiece<ElemF16> : OutPiece16<OutF16> {};
-template <>
-struct OutPiece<ElemF32> {
-  static __device__ __forceinline__ void unpack(u32x4_t v, float (&f)[4]) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) f[e] = __uint_as_float(v[e]);
-  }
-  static __device__ __forceinline__ u32x4_t pack(const float (&f)[4]) {
-    return (u32x4_t){__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
-  }
-};
-
-// Element stores that are written through to memory at system scope (see store16_system).
-template <class Out>
-__device__ __forceinline__ void store_element_system(char* p, const char* from) {
-  if constexpr (Out::size == 2)
-    __hip_atomic_store((unsigned short*)p, *(const LDS_AS unsigned short*)(LDS_AS const char*)from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  else
-    __hip_atomic_store((unsigned*)p, *(const LDS_AS unsigned*)(LDS_AS const char*)from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 
 template <class CFG>
 __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_any_kernel(const FusedParams p) {
@@ -685,258 +627,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
 
   PHASE_STAMP(3);
 
-  // ---- epilogue: pieces of OE consecutive columns, handed out row by row ---------------------------------------
-  constexpr int PPR = BN / OE;             // pieces per tile row
-  constexpr int RPP = NT / PPR;            // tile rows per pass of the workgroup
-  constexpr int PASSES = BM > RPP ? BM / RPP : 1;
-  static_assert(NT % PPR == 0 && (BM % RPP == 0 || BM < RPP), "epilogue pass shape");
-  const int m_end = min(m0 + BM, p.M);  // one past the tile's last row (threads may have no row in a 32x32 tile)
-  // A piece that would reach past the last column starts further left (both its threads then write the same
-  // values twice), as long as the tile has that many columns.
-  const int t_row = tid / PPR, tile_cols = min(BN, p.N - n0);
-  int t_col = tid % PPR * OE;
-  if (p.s_cn == 1 && t_col < tile_cols && t_col + OE > tile_cols && tile_cols >= OE) t_col = tile_cols - OE;
-  const int gn = n0 + t_col;
-  const int cols = min(p.N - gn, OE);           // columns of this thread's pieces that exist (may be <= 0)
-  const bool whole = cols == OE && p.s_cn == 1;  // moved as 16 bytes, else element by element
-  const int ftn = cdiv(p.N, p.flag_bn);
-  const int ftotal = cdiv(p.M, p.flag_bm) * ftn;
-  auto staged = [&](int row) INLINED { return smem + row * CFG::TROW + t_col * Out::size; };
-  auto staged_piece = [&](int row) INLINED { return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)staged(row); };
-  auto staged_element = [&](int row, int e) INLINED -> float {
-    if constexpr (Out::size == 4) {
-      return *(const LDS_AS float*)(LDS_AS char*)(staged(row) + e * 4);
-    } else {
-      const unsigned short b = *(const LDS_AS unsigned short*)(LDS_AS char*)(staged(row) + e * 2);
-      return Out::kFp32SumInReference ? f16_bits_to_float(b) : bf16_bits_to_float(b);
-    }
-  };
-  auto offset = [&](int row, int e) INLINED {  // bytes into C (or aux) of element e of this thread's piece
-    return ((long long)(m0 + row + p.row_offset) * p.s_cm + (long long)(gn + e) * p.s_cn) * Out::size;
-  };
-  auto owner_at = [&](int gm, int g) INLINED { return owner_of(p.epi, (gm / p.flag_bm) * ftn + g / p.flag_bn, ftotal, p.world, p.rank); };
-
-  if (p.epi == EPI_ATOMIC) {
-    if constexpr (Out::size == 4) {
-      for (int d = tid; d < BM * BN; d += NT) {
-        const int row = d / BN, col = d % BN;
-        if (m0 + row >= p.M || n0 + col >= p.N) continue;
-        const float v = *(const LDS_AS float*)(LDS_AS char*)(smem + row * CFG::TROW + col * 4);
-        const long long eoff = ((long long)(m0 + row) * p.s_cm + (long long)(n0 + col) * p.s_cn) * 4;
-        for (int pr = 0; pr < p.world; ++pr) {
-          if (p.clear_c && pr == p.rank) *(float*)(p.C + eoff) = 0.f + v;
-          else atomicAdd((float*)(slot_ptr(p.heap_bases, p.C, p.rank, pr) + eoff), v);
-        }
-      }
-    } else if (p.s_cn == 1) {
-      // Packed adds of aligned dwords, one per thread.  A row that starts in the middle of a dword is shifted by
-      // one element against them; the half of a dword that is not this tile's gets -0 added, which leaves
-      // every value of C as it is.  What lies next to C need not be a number (-0 makes a signalling NaN quiet): dwords
-      // that reach past the first or the last column are for the element of C alone.
-      using Out16 = typename std::conditional<Out::kFp32SumInReference, OutF16, OutBF16>::type;
-      constexpr int DPR = BN / 2 + 1;
-      for (int d = tid; d < BM * DPR; d += NT) {
-        const int row = d / DPR;
-        if (m0 + row >= p.M) continue;
-        char* const at = p.C + ((long long)(m0 + row) * p.s_cm + n0) * 2;
-        const int e = 2 * (d - row * DPR) - (int)(((unsigned long long)at >> 1) & 1);
-        const bool lo = e >= 0 && e < BN && n0 + e < p.N, hi = e + 1 < BN && n0 + e + 1 < p.N;
-        if (!lo && !hi) continue;
-        const bool inside = n0 + e >= 0 && n0 + e + 1 < p.N;
-        const char* const s = smem + row * CFG::TROW;
-        const unsigned w = (lo ? *(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2) : 0x8000u) |
-                           (hi ? (unsigned)*(const LDS_AS unsigned short*)(LDS_AS char*)(s + e * 2 + 2) : 0x8000u) << 16;
-        for (int pr = 0; pr < p.world; ++pr) {
-          if (p.clear_c && pr == p.rank) {
-            const unsigned z = added_to_zero(w);
-            if (lo) *(unsigned short*)(at + e * 2) = (unsigned short)z;
-            if (hi) *(unsigned short*)(at + e * 2 + 2) = (unsigned short)(z >> 16);
-          } else if (inside) {
-            atomic_add_packed<Out16>(slot_ptr(p.heap_bases, at, p.rank, pr) + e * 2, w);
-          }
-        }
-      }
-      // The elements of C in dwords that reach past it, a row and a rank per thread: each is a load and an exchange one behind
-      // the other (fp16 3693x5963x258, eight ranks: 581 us with the ranks in turn above, 530 us).
-      if (n0 == 0 || n0 + BN >= p.N) {
-        for (int i = tid; i < BM * 2 * p.world; i += NT) {
-          const int row = i % BM, last = i / BM & 1, pr = i / (2 * BM), e = last ? p.N - 1 - n0 : 0;
-          if (m0 + row >= p.M || e >= BN || (n0 > 0 && !last) || (p.clear_c && pr == p.rank)) continue;
-          char* const at = p.C + ((long long)(m0 + row) * p.s_cm + n0 + e) * 2;
-          if ((int)(((unsigned long long)at >> 1) & 1) == last) continue;  // inside: not the high half, not the low half
-          Out::atomic_add(slot_ptr(p.heap_bases, at, p.rank, pr),
-                          Out16::to_float(*(const LDS_AS unsigned short*)(LDS_AS char*)(smem + row * CFG::TROW + e * 2)));
-        }
-      }
-    } else {
-      for (int ps = 0; ps < PASSES; ++ps) {
-        const int row = ps * RPP + t_row;
-        if (m0 + row >= m_end) continue;
-        for (int e = 0; e < cols; ++e)
-          for (int pr = 0; pr < p.world; ++pr) {
-            if (p.clear_c && pr == p.rank) Out::store(p.C + offset(row, e), 0.f + staged_element(row, e));
-            else Out::atomic_add(slot_ptr(p.heap_bases, p.C, p.rank, pr) + offset(row, e), staged_element(row, e));
-          }
-      }
-    }
-    return;
-  }
-
-  const bool flags = epi_has_flags(p.epi);
-  const bool solo = flags && (!p.sum_peers || p.world == 1);  // no peer contributes: the sum is the own tile
-  // Stores of a result piece (or its elements) to wherever the operator wants it.
-  auto each_destination = [&](int gm, int g, auto&& store) INLINED {
-    if (p.epi == EPI_STORE) {
-      store(p.C);
-    } else if (p.epi == EPI_ALL_GATHER) {
-      for (int pr = 0; pr < p.world; ++pr) store(slot_ptr(p.heap_bases, p.C, p.rank, pr));
-    } else if (p.epi == EPI_ONE_SHOT) {
-      store(p.C);
-    } else {
-      const int owner = owner_at(gm, g);
-      if (!p.all_owners && owner != p.rank) return;
-      if (p.epi == EPI_TWO_SHOT) {
-        for (int pr = 0; pr < p.world; ++pr) store(slot_ptr(p.heap_bases, p.C, p.rank, pr));
-      } else {
-        store(slot_ptr(p.heap_bases, p.C, p.rank, p.all_owners ? owner : p.rank));
-      }
-    }
-  };
-  const bool aligned = (((unsigned long long)p.C | (unsigned long long)(p.s_cm * Out::size)) & 15) == 0 && p.N % OE == 0;
-  const bool owners = flags && p.epi != EPI_ONE_SHOT;
-  // A piece may be moved whole when all of it has one owner.
-  const bool piece_ok = whole && (!owners || gn / p.flag_bn == (gn + OE - 1) / p.flag_bn);
-
-#pragma unroll 2
-  for (int ps = 0; ps < PASSES; ++ps) {
-    const int row = ps * RPP + t_row, gm = m0 + row;
-    if (gm >= m_end) break;
-    if (flags) {
-      if (whole) {
-        store16_system_of_valu_data(p.aux + offset(row, 0), staged_piece(row));
-      } else {
-        for (int e = 0; e < cols; ++e) store_element_system<Out>(p.aux + offset(row, e), staged(row) + e * Out::size);
-      }
-      if (p.clear_c && owners) {  // other ranks' tiles: zeros
-        if (piece_ok) {
-          if (owner_at(gm, gn) != p.rank) store16_result(p.C + offset(row, 0), (u32x4_t){0u, 0u, 0u, 0u}, aligned);
-        } else {
-          for (int e = 0; e < cols; ++e)
-            if (owner_at(gm, gn + e) != p.rank) Out::store(p.C + offset(row, e), 0.f);
-        }
-      }
-      if (!solo) continue;
-    }
-    if (piece_ok) {
-      const u32x4_t v = staged_piece(row);
-      each_destination(gm, gn, [&](char* base) { store16_result(base + offset(row, 0), v, aligned); });
-    } else {
-      for (int e = 0; e < cols; ++e)
-        each_destination(gm, gn + e, [&](char* base) { Out::store(base + offset(row, e), staged_element(row, e)); });
-    }
-  }
-  PHASE_STAMP(4);
-  if (!flags) return;
-
-  // Publish and wait, as in the tiled kernel: aux is written through, so relaxed flag stores behind the
-  // acknowledgement are enough.
-  const bool up_already = solo ? true : probe_peer_flags<BM, BN, NT>(p, m0, n0, tid);
-  wait_vmcnt<0>();
-  __syncthreads();
-  PHASE_STAMP(5);
-  raise_flags<BM, BN, NT, true>(p, m0, n0, tid);
-  if (solo) return;
-  if (!up_already) wait_peer_flags<BM, BN, NT>(p, m0, n0, tid);
-  __syncthreads();
-  PHASE_STAMP(6);
-
-  // Slot sum in ascending rank order from the own (already rounded) value, in fp32 or by the reference's rule.
-  const bool ref_chain = (p.acc_mode == IRIS_HIP_ACC_REFERENCE) && !Out::kFp32SumInReference;
-  auto add = [&](float sum, float x) INLINED {
-    sum += x;
-    return ref_chain ? Out::round(sum) : sum;
-  };
-  auto reduce = [&](auto np_tag, auto nt_tag) INLINED {
-    auto load_peer = [](const char* at) INLINED { return decltype(nt_tag)::value ? load16_any_nt(at) : load16_any(at); };
-    constexpr int NP = decltype(np_tag)::value;  // peers, all of whose loads go out together; 0: any number
-    constexpr int NPV = NP > 0 ? NP : 1;
-    // Passes whose loads are in flight together: as many as the registers hold (the sums are staged and their
-    // accumulators free), every group of passes is a round trip to memory.
-    constexpr int kInFlight = CFG::NW == 8 ? 16 : 14;  // 16-byte pieces per thread; with more, fewer workgroups share a CU
-    constexpr int G = PASSES % 8 == 0 && 8 * NPV <= kInFlight ? 8 : PASSES % 4 == 0 && 4 * NPV <= kInFlight ? 4 : PASSES % 2 == 0 ? 2 : 1;
-    for (int pg = 0; pg < PASSES; pg += G) {
-      if (m0 + pg * RPP >= p.M) break;
-      bool act[G];
-      u32x4_t pv[G][NPV];
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int row = (pg + g) * RPP + t_row;
-        act[g] = m0 + row < m_end && cols > 0;
-        if (act[g] && owners && !p.all_owners && piece_ok) act[g] = owner_at(m0 + row, gn) == p.rank;
-        if constexpr (NP > 0) {
-          if (act[g] && piece_ok) {
-#pragma unroll
-            for (int i = 0; i < NP; ++i) pv[g][i] = load_peer(slot_ptr(p.heap_bases, p.aux, p.rank, i < p.rank ? i : i + 1) + offset(row, 0));
-          }
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int row = (pg + g) * RPP + t_row, gm = m0 + row;
-        if (!act[g]) continue;
-        if (piece_ok) {
-          float sum[OE], x[OE];
-          OutPiece<Out>::unpack(staged_piece(row), sum);
-          if constexpr (NP > 0) {
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-              OutPiece<Out>::unpack(pv[g][i], x);
-#pragma unroll
-              for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
-            }
-          } else {
-            for (int pr = 0; pr < p.world; ++pr) {
-              if (pr == p.rank) continue;
-              OutPiece<Out>::unpack(load_peer(slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row, 0)), x);
-#pragma unroll
-              for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
-            }
-          }
-          const u32x4_t v = OutPiece<Out>::pack(sum);
-          each_destination(gm, gn, [&](char* base) { store16_result(base + offset(row, 0), v, aligned); });
-        } else {
-          // Fewer columns than a piece, strided columns or several owners: all elements of a peer in one go.
-          float sum[OE];
-#pragma unroll
-          for (int e = 0; e < OE; ++e) sum[e] = e < cols ? staged_element(row, e) : 0.f;
-          for (int pr = 0; pr < p.world; ++pr) {
-            if (pr == p.rank) continue;
-            const char* const src = slot_ptr(p.heap_bases, p.aux, p.rank, pr);
-            float x[OE];
-#pragma unroll
-            for (int e = 0; e < OE; ++e) x[e] = e < cols ? Out::load(src + offset(row, e)) : 0.f;
-#pragma unroll
-            for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
-          }
-#pragma unroll
-          for (int e = 0; e < OE; ++e)
-            if (e < cols) each_destination(gm, gn + e, [&](char* base) { Out::store(base + offset(row, e), sum[e]); });
-        }
-      }
-    }
-  };
-  auto reduce_with = [&](auto np_tag) INLINED {
-    // (The 32x32 tile is for small outputs: one way is enough.)
-    if (CFG::WK == 1 && p.stream_peers) reduce(np_tag, std::integral_constant<bool, CFG::WK == 1>{});
-    else reduce(np_tag, std::false_type{});
-  };
-  switch (p.world - 1) {
-    case 1: reduce_with(std::integral_constant<int, 1>{}); break;
-    case 3: reduce_with(std::integral_constant<int, 3>{}); break;
-    case 7: reduce_with(std::integral_constant<int, 7>{}); break;
-    default: reduce(std::integral_constant<int, 0>{}, std::false_type{}); break;
-  }
-  PHASE_STAMP(7);
+  const LinearTile<CFG::TROW> tile{smem};
+  finish_any<Out, BM, BN, NT, CFG::NW == 8 ? 16 : 14, CFG::WK == 1>(p, tile, m0, n0, tid);
 }
 
 // ------------------------------------------------------------------------------------------------

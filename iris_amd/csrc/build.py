@@ -21,8 +21,8 @@ SOURCES = [os.path.join(HERE, f) for f in (
     "iris_hip_mfma_bf16.hip", "iris_hip_mfma_f16.hip", "iris_hip_mfma_fp8.hip", "iris_hip_any_bf16.hip",
     "iris_hip_any_f16.hip", "iris_hip_any_fp8.hip", "iris_hip_any_f32.hip", "iris_hip_decode_bf16.hip",
     "iris_hip_decode_f16.hip", "iris_hip_decode_fp8.hip", "iris_hip.hip", "iris_ccl.hip")]
-HEADERS = [os.path.join(HERE, h) for h in ("fused_kernel.h", "decode_kernel.h", "any_kernel.h", "layout.h", "device_util.h",
-                                           "host_common.h")] + [
+HEADERS = [os.path.join(HERE, h) for h in ("fused_kernel.h", "decode_kernel.h", "any_kernel.h", "any_epilogue.h", "fused_params.h",
+                                           "layout.h", "device_util.h", "host_common.h")] + [
     os.path.join(ROOT, "include", "iris_hip.h")]
 OUTPUT = os.path.join(os.path.dirname(HERE), "lib", "libiris_hip.so")
 # The Python module through which the operators call the library's entry points (host code only; it reads torch's
