@@ -32,6 +32,7 @@
 #ifndef IRIS_HIP_H
 #define IRIS_HIP_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
@@ -321,7 +322,19 @@ const char* iris_hip_last_kernel(void);
 /* 1 if launches on `stream` are being recorded into a graph, 0 if not (also when that cannot be found out). */
 int iris_hip_stream_capturing(void* stream);
 
-/* ABI version of this header.  6: IRIS_HIP_CLEAR_C (a version-5 library would take it for an accumulation rule it does not
+/*
+ * Device memory for the length of a launch.  Launches on operands that have to be laid out anew first (rows of 16- and 8-bit
+ * data that do not start on 16-byte boundaries) take it from the caller's allocator and give it back
+ * as soon as they are enqueued: memory that is given back may be used again by later work on the same stream only.
+ * allocate(bytes, stream) is called with the launch's device current and returns NULL when there is none; such launches, those
+ * of a stream under capture and all of them while no allocator is set (NULL, NULL) take a kernel that needs no memory.
+ * Set it before the first launch; both functions are called from whatever thread launches.
+ */
+typedef void* (*iris_hip_allocate_fn)(size_t bytes, void* stream);
+typedef void (*iris_hip_release_fn)(void* memory);
+void iris_hip_set_scratch_allocator(iris_hip_allocate_fn allocate, iris_hip_release_fn release);
+
+/* ABI version of this header.  7: iris_hip_set_scratch_allocator.  6: IRIS_HIP_CLEAR_C (a version-5 library would take it for an accumulation rule it does not
  * know, and leave C as it is). */
 int iris_hip_abi_version(void);
 

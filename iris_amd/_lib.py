@@ -13,7 +13,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIBRARY_PATH = os.environ.get("IRIS_HIP_LIBRARY") or os.path.join(_HERE, "lib", "libiris_hip.so")
 LAUNCHER_PATH = os.path.join(_HERE, "lib", "_launch.so")
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 # Enumerations of include/iris_hip.h
 BF16, FP16, FP32, FP8_E4M3 = 0, 1, 2, 3

@@ -1,5 +1,5 @@
 // The end of a tile whose output rows may start and end anywhere: from the tile in the output type, staged in LDS, to
-// aux, the flags, the slot sum and C.
+// aux, the flags, the slot sum and C.  fused_any_kernel always ends here, fused_mfma_kernel in its ANY_ROWS builds.
 #pragma once
 
 #include "fused_params.h"

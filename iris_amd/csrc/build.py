@@ -20,9 +20,10 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 SOURCES = [os.path.join(HERE, f) for f in (
     "iris_hip_mfma_bf16.hip", "iris_hip_mfma_f16.hip", "iris_hip_mfma_fp8.hip", "iris_hip_any_bf16.hip",
     "iris_hip_any_f16.hip", "iris_hip_any_fp8.hip", "iris_hip_any_f32.hip", "iris_hip_decode_bf16.hip",
-    "iris_hip_decode_f16.hip", "iris_hip_decode_fp8.hip", "iris_hip.hip", "iris_ccl.hip")]
-HEADERS = [os.path.join(HERE, h) for h in ("fused_kernel.h", "decode_kernel.h", "any_kernel.h", "any_epilogue.h", "fused_params.h",
-                                           "layout.h", "device_util.h", "host_common.h")] + [
+    "iris_hip_decode_f16.hip", "iris_hip_decode_fp8.hip", "iris_hip_rows_bf16.hip", "iris_hip_rows_f16.hip", "iris_hip_rows_fp8.hip",
+    "iris_hip.hip", "iris_ccl.hip")]
+HEADERS = [os.path.join(HERE, h) for h in ("fused_kernel.h", "decode_kernel.h", "any_kernel.h", "any_epilogue.h", "fused_params.h", "pack_kernel.h", "layout.h", "device_util.h",
+                                           "host_common.h")] + [
     os.path.join(ROOT, "include", "iris_hip.h")]
 OUTPUT = os.path.join(os.path.dirname(HERE), "lib", "libiris_hip.so")
 # The Python module through which the operators call the library's entry points (host code only; it reads torch's
@@ -69,11 +70,11 @@ def _build_launcher(verbose):
     from torch.utils.cpp_extension import include_paths, library_paths
 
     tmp = LAUNCHER_OUTPUT + ".tmp"
-    includes = [sysconfig.get_paths()["include"]] + include_paths()
-    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+    includes = [sysconfig.get_paths()["include"]] + include_paths() + [os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f'-DIRIS_LAUNCHER_TAG="{launcher_tag()}"', "-I" + os.path.join(ROOT, "include")]
          + [flag for path in includes for flag in ("-isystem", path)] + ["-o", tmp, LAUNCHER_SOURCE]
-         + ["-L" + path for path in library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"], verbose)
+         + ["-L" + path for path in library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"], verbose)
     os.replace(tmp, LAUNCHER_OUTPUT)
 
 

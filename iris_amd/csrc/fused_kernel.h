@@ -5,7 +5,7 @@
 // instantiates dispatch_mfma_in<IN> below, so that the build can compile them side by side.
 #pragma once
 
-#include "fused_params.h"
+#include "any_epilogue.h"
 
 // Stages of the slot-sum pipeline of the eight-wave tile (see reduce_chunks).
 #ifndef IRIS_HIP_EPILOGUE_DEPTH
@@ -211,6 +211,29 @@ __device__ __forceinline__ FusedParams pin_loader_arguments(const FusedParams& a
   return q;
 }
 
+// The staged tile of a configuration, for finish_any.  Swizzled rows keep the 16-byte chunks whole: a piece that starts inside one
+// (the last of a row that is not a whole number of pieces) is put together from two of them.
+template <class CFG>
+struct StagedTile {
+  char* base;
+  __device__ __forceinline__ char* at(int row, int byte) const { return base + CFG::stage_offset(row, byte); }
+  __device__ __forceinline__ u32x4_t piece(int row, int byte, int) const {
+    if constexpr (!CFG::STAGE_SWIZZLED) {
+      return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)at(row, byte);
+    } else {
+      const u32x4_t v = *(const LDS_AS u32x4_t*)(LDS_AS char*)at(row, byte & ~15);
+      if ((byte & 15) == 0) return v;
+      const u32x4_t w = *(const LDS_AS u32x4_t*)(LDS_AS char*)at(row, (byte & ~15) + 16);
+      const int shift = byte & 15;
+      const unsigned long long lo = v[0] | (unsigned long long)v[1] << 32, hi = v[2] | (unsigned long long)v[3] << 32;
+      const unsigned long long lo2 = w[0] | (unsigned long long)w[1] << 32, hi2 = w[2] | (unsigned long long)w[3] << 32;
+      const unsigned long long x0 = shift < 8 ? lo : hi, x1 = shift < 8 ? hi : lo2, x2 = shift < 8 ? lo2 : hi2;
+      const int bits = (shift & 7) * 8;
+      const unsigned long long y0 = bits ? x0 >> bits | x1 << (64 - bits) : x0, y1 = bits ? x1 >> bits | x2 << (64 - bits) : x1;
+      return (u32x4_t){(unsigned)y0, (unsigned)(y0 >> 32), (unsigned)y1, (unsigned)(y1 >> 32)};
+    }
+  }
+};
 
 // ------------------------------------------------------------------------------------------------
 // MFMA kernel
@@ -228,8 +251,12 @@ __device__ __forceinline__ FusedParams pin_loader_arguments(const FusedParams& a
 // their partial sums in ascending piece order and runs the ordinary epilogue.  Helpers are the XCD's
 // first workgroups and never wait, mains wait only for helpers - workgroups with lower indices, which
 // the hardware dispatches first - so the waits end whatever part of the grid is resident.
-template <class CFG, bool ONE_ROUND, bool STREAMK = false>
+//
+// ANY_ROWS: the rows of C and aux start and end anywhere (any_epilogue.h), N is not a whole number of 16-byte pieces; A and
+// B are whole pieces all the same, because they lie so or because pack_kernel has laid them out (pack_kernel.h).
+template <class CFG, bool ONE_ROUND, bool STREAMK = false, bool ANY_ROWS = false>
 __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kernel(const FusedParams p_in) {
+  static_assert(!ANY_ROWS || (ONE_ROUND && !STREAMK), "any rows: one workgroup per tile");
   static_assert(!STREAMK || (CFG::NW == 8 && !ONE_ROUND), "split tiles: eight-wave tile, looping build");
   using Out = typename OutOf<CFG::IN>::type;
   // LDS layouts of A (and of B given K-contiguous, whose rows are as long), and of row-major B
@@ -913,6 +940,12 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     __syncthreads();
     PHASE_STAMP(3);
 
+    if constexpr (ANY_ROWS) {
+      using Elem = typename std::conditional<CFG::IN == IN_F16, ElemF16, ElemBF16>::type;
+      finish_any<Elem, BM, BN, NT, CFG::NW == 8 ? 16 : 14, true>(p, StagedTile<CFG>{smem}, m0, n0, tid);
+      return;
+    } else {
+
     constexpr int CPR = BN / 8;            // 16-byte chunks per tile row
     constexpr int RPP = NT / CPR;          // tile rows covered by one pass of the workgroup
     constexpr int PASSES = BM / RPP;
@@ -1212,6 +1245,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
     wait_vmcnt<0>();
     PHASE_STAMP(8);
 #endif
+    }  // !ANY_ROWS
     // Staging shares LDS with the operand ring of the next tile: every wave must be done reading it.
     // A bare barrier - __syncthreads() would also wait for this tile's global stores to be
     // acknowledged (1-4 us), which nothing here depends on; they drain behind the next tile's
@@ -1224,19 +1258,19 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
 // ------------------------------------------------------------------------------------------------
 // Launch of the MFMA kernel
 // ------------------------------------------------------------------------------------------------
-template <class CFG, bool ONE_ROUND, bool STREAMK = false>
+template <class CFG, bool ONE_ROUND, bool STREAMK = false, bool ANY_ROWS = false>
 int launch_mfma_grid(const FusedParams& p, int device, int grid, hipStream_t stream) {
   // The dynamic-LDS limit is a per-device attribute of the kernel: set it once on every device used
   // (atomic flags: two host threads may both set it, which is harmless, but neither skips it).
   static std::atomic<bool> attr_set[64];
   if (device < 0 || device >= 64) return iris_host::fail("device index %d out of range", device);
   if (!attr_set[device].load(std::memory_order_acquire)) {
-    hipError_t e = hipFuncSetAttribute((const void*)fused_mfma_kernel<CFG, ONE_ROUND, STREAMK>,
+    hipError_t e = hipFuncSetAttribute((const void*)fused_mfma_kernel<CFG, ONE_ROUND, STREAMK, ANY_ROWS>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, CFG::SMEM_BYTES);
     if (e != hipSuccess) return (int)e;
     attr_set[device].store(true, std::memory_order_release);
   }
-  hipLaunchKernelGGL((fused_mfma_kernel<CFG, ONE_ROUND, STREAMK>), dim3(grid), dim3(CFG::NT), CFG::SMEM_BYTES, stream, p);
+  hipLaunchKernelGGL((fused_mfma_kernel<CFG, ONE_ROUND, STREAMK, ANY_ROWS>), dim3(grid), dim3(CFG::NT), CFG::SMEM_BYTES, stream, p);
   return (int)hipGetLastError();
 }
 
@@ -1356,10 +1390,9 @@ inline int tile_cols(int kind) { return kind == TILE_BIG ? 256 : kind == TILE_DE
 template <int IN>
 int dispatch_decode(FusedParams& p, bool bkc, int device, int cu, hipStream_t s);
 
-template <int IN>
-int dispatch_mfma_in(FusedParams& p, int kind, bool bkc, int device, int cu, hipStream_t s) {
+// The tiles of a launch and their order.
+inline void plan_tiles(FusedParams& p, int kind, int cu) {
   const int bm = tile_rows(kind), bn = tile_cols(kind);
-  if (kind == TILE_DECODE) return dispatch_decode<IN>(p, bkc, device, cu, s);
   p.tiles_m = cdiv(p.M, bm);
   p.tiles_n = cdiv(p.N, bn);
   // Group height: tile-rows walked together so that the tiles an XCD works on at one time - its whole
@@ -1436,6 +1469,13 @@ int dispatch_mfma_in(FusedParams& p, int kind, bool bkc, int device, int cu, hip
     p.group_m_spans = g;
   }
   p.group_m = g;
+}
+
+template <int IN>
+int dispatch_mfma_in(FusedParams& p, int kind, bool bkc, int device, int cu, hipStream_t s) {
+  if (kind == TILE_DECODE) return dispatch_decode<IN>(p, bkc, device, cu, s);
+  plan_tiles(p, kind, cu);
+  const int bm = tile_rows(kind), bn = tile_cols(kind);
   static const char* names[3] = {"bf16", "f16", "fp8"};
   char name[96];
   snprintf(name, sizeof(name), "mfma_%s_%dx%dx%d_%s", names[IN], bm, bn, tile_bk(kind, IN), bkc ? "nt" : "nn");
@@ -1450,5 +1490,30 @@ int dispatch_mfma_in(FusedParams& p, int kind, bool bkc, int device, int cu, hip
       return bkc ? launch_mfma<Skinny64Tile<IN, true>>(p, device, cu, s, name) : launch_mfma<Skinny64Tile<IN, false>>(p, device, cu, s, name);
     default:
       return bkc ? launch_mfma<SkinnyTile<IN, true>>(p, device, cu, s, name) : launch_mfma<SkinnyTile<IN, false>>(p, device, cu, s, name);
+  }
+}
+
+// ANY_ROWS builds, in translation units of their own (iris_hip_rows_<type>.hip): one workgroup per tile.
+template <class CFG>
+int launch_mfma_rows(const FusedParams& p, int device, hipStream_t s, const char* name) {
+  iris_host::set_last_kernel(name);
+  return launch_mfma_grid<CFG, true, false, true>(p, device, cdiv(p.tiles_m * p.tiles_n, p.num_xcd) * p.num_xcd, s);
+}
+
+template <int IN>
+int dispatch_mfma_rows(FusedParams& p, int kind, bool bkc, int device, int cu, hipStream_t s) {
+  plan_tiles(p, kind, cu);
+  static const char* names[3] = {"bf16", "f16", "fp8"};
+  char name[96];
+  snprintf(name, sizeof(name), "mfma_%s_%dx%dx%d_%s_rows", names[IN], tile_rows(kind), tile_cols(kind), tile_bk(kind, IN), bkc ? "nt" : "nn");
+  switch (kind) {
+    case TILE_BIG:
+      return bkc ? launch_mfma_rows<BigTile<IN, true>>(p, device, s, name) : launch_mfma_rows<BigTile<IN, false>>(p, device, s, name);
+    case TILE_SMALL:
+      return bkc ? launch_mfma_rows<SmallTile<IN, true>>(p, device, s, name) : launch_mfma_rows<SmallTile<IN, false>>(p, device, s, name);
+    case TILE_SMALL2:
+      return bkc ? launch_mfma_rows<Small2Tile<IN, true>>(p, device, s, name) : launch_mfma_rows<Small2Tile<IN, false>>(p, device, s, name);
+    default:
+      return bkc ? launch_mfma_rows<Skinny64Tile<IN, true>>(p, device, s, name) : launch_mfma_rows<Skinny64Tile<IN, false>>(p, device, s, name);
   }
 }

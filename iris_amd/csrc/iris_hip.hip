@@ -14,7 +14,8 @@
 //    unit-stride rows (see mfma_ineligible()).
 //  * fused_any_kernel (any_kernel.h, compiled in the iris_hip_any_<type>.hip translation units) - any alignment,
 //    stride, size and element type, operands through registers: everything the first does not take (fp32
-//    data, odd strides, sizes that are not multiples of 8 elements).
+//    data, odd strides, sizes that are not multiples of 8 elements) - unless it is large enough that the first is
+//    ahead behind one pass that lays the operands out anew (pack_kernel.h, iris_hip_rows_<type>.hip; worth_packing below).
 //
 // The flag-less operators (all_gather_matmul, matmul_all_gather, the atomic all-reduce) store or add
 // the tile directly.  The others end in the same epilogue protocol, which follows the reference kernels
@@ -39,6 +40,7 @@
 
 #include "any_kernel.h"
 #include "fused_kernel.h"
+#include "pack_kernel.h"
 
 // ------------------------------------------------------------------------------------------------
 // Host side
@@ -49,6 +51,26 @@ thread_local char g_last_error[512] = "";
 thread_local char g_last_kernel[128] = "";
 
 using iris_host::fail;  // defined below, shared with the other translation units
+
+// Device memory for the length of a launch, from the caller's allocator (iris_hip_set_scratch_allocator).
+struct ScratchAllocator {
+  std::atomic<iris_hip_allocate_fn> allocate{nullptr};
+  std::atomic<iris_hip_release_fn> release{nullptr};
+  // NULL: there is none, none is left, or the stream is being captured (what a graph holds has to outlive the call).
+  void* take(size_t bytes, hipStream_t stream) const {
+    const iris_hip_allocate_fn f = allocate.load(std::memory_order_acquire);
+    if (!f) return nullptr;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    return f(bytes, (void*)stream);
+  }
+  void give_back(void* memory) const {
+    if (memory) release.load(std::memory_order_acquire)(memory);
+  }
+};
 
 struct DeviceFacts {
   int cu_count = 0;
@@ -143,6 +165,10 @@ bool generic_supported(int in_dtype, int out_dtype) {
 extern template int dispatch_mfma_in<IN_BF16>(FusedParams&, int, bool, int, int, hipStream_t);
 extern template int dispatch_mfma_in<IN_F16>(FusedParams&, int, bool, int, int, hipStream_t);
 extern template int dispatch_mfma_in<IN_FP8>(FusedParams&, int, bool, int, int, hipStream_t);
+// Instantiated in iris_hip_rows_<type>.hip.
+extern template int dispatch_mfma_rows<IN_BF16>(FusedParams&, int, bool, int, int, hipStream_t);
+extern template int dispatch_mfma_rows<IN_F16>(FusedParams&, int, bool, int, int, hipStream_t);
+extern template int dispatch_mfma_rows<IN_FP8>(FusedParams&, int, bool, int, int, hipStream_t);
 // Instantiated in iris_hip_any_<type>.hip.
 extern template int dispatch_any<IN_BF16, ElemBF16>(const FusedParams&, int, int, hipStream_t, const char*);
 extern template int dispatch_any<IN_BF16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
@@ -282,6 +308,156 @@ bool rows_of_whole_lines(const FusedParams& p, int out_dtype) {
   return p.s_cn == 1 && ((p.s_cm * es) | ((long long)p.N * es)) % 128 == 0 && (((uintptr_t)p.aux | (uintptr_t)p.C) & 127) == 0;
 }
 
+// ------------------------------------------------------------------------------------------------
+// 16- and 8-bit operands whose rows start anywhere, on the direct-to-LDS kernel (pack_kernel.h)
+// ------------------------------------------------------------------------------------------------
+ScratchAllocator g_scratch_allocator;
+
+struct PackPlan {
+  FusedParams p;      // the launch on the packed operands
+  PackParams pack;
+  size_t bytes;       // of both packed operands
+  int kind;
+};
+
+// What a launch that the MFMA kernel cannot take as it is would look like with A and B laid out anew where they have to be.
+// False: it cannot be brought to that kernel this way.
+bool plan_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, PackPlan& plan) {
+  if (in_dtype == IRIS_HIP_FP32 || out_dtype != (in_dtype == IRIS_HIP_FP16 ? IRIS_HIP_FP16 : IRIS_HIP_BF16)) return false;
+  if (p.s_ak != 1 || (p.s_bn != 1 && p.s_bk != 1) || p.s_cn != 1) return false;
+  const int es = elem_size(in_dtype), ce = 16 / es;
+  const bool bkc = p.s_bn != 1;
+  const int sources = p.gather == GATHER_K ? p.world : 1;
+  auto whole = [&](long long n) { return (n + ce - 1) / ce * ce; };
+
+  const long long big_tiles = (long long)cdiv(p.M, 256) * cdiv(p.N, 256), tiles128 = (long long)cdiv(p.M, 128) * cdiv(p.N, 128);
+  plan.kind = TILE_SMALL;
+  if (big_tiles * 100 >= (long long)cu * 53 && p.M > 64) plan.kind = TILE_BIG;
+  else if ((long long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 2ll * cu) plan.kind = TILE_SKINNY64;
+  else if (tiles128 > cu) plan.kind = TILE_SMALL2;
+
+  FusedParams& q = plan.p;
+  q = p;
+  memset(&plan.pack, 0, sizeof(plan.pack));
+  plan.pack.heap_bases = p.heap_bases;
+  plan.pack.rank = p.rank;
+  const bool pack_a = !aligned16(p.A) || (p.s_am * es) % 16 || p.K_local % ce || (p.gather == GATHER_M && p.M_local % tile_rows(plan.kind));
+  // (with several sources A's runs are padded one by one, and B's K has to follow)
+  const bool pack_b = !aligned16(p.B) || ((bkc ? p.s_bn : p.s_bk) * es) % 16 || (bkc ? p.K_local : p.N) % ce || (sources > 1 && p.K_local % ce);
+  const long long k_run = whole(p.K_local), k_all = sources * k_run;
+  long long bytes_a = 0, bytes_b = 0;
+  if (pack_a) {
+    PackJob& j = plan.pack.job[0];
+    j.src = p.A;
+    j.src_row = p.s_am * es;
+    j.rows = p.M;
+    j.segments = sources;
+    j.run = p.K_local;
+    j.run_pieces = (int)(k_run / ce);
+    j.slots_of_rows = p.gather == GATHER_M ? p.M_local : 0;
+    j.slots_of_segments = p.gather == GATHER_K;
+    bytes_a = (long long)p.M * k_all * es;
+    q.s_am = k_all;
+    q.gather = GATHER_NONE;
+    q.M_local = p.M;
+    q.K = q.K_local = sources > 1 ? (int)k_all : p.K;
+  }
+  if (pack_b) {
+    PackJob& j = plan.pack.job[1];
+    j.src = p.B;
+    if (bkc) {
+      j.src_row = p.s_bn * es;
+      j.src_segment = (long long)p.K_local * es;
+      j.rows = p.N;
+      j.segments = sources;
+      j.run = p.K_local;
+      j.run_pieces = (int)(k_run / ce);
+      q.s_bn = k_all;
+      bytes_b = (long long)p.N * k_all * es;
+    } else {
+      const long long n_run = whole(p.N);
+      j.src_row = p.s_bk * es;
+      j.rows = sources > 1 ? (int)k_all : p.K;
+      j.segments = 1;
+      j.run = p.N;
+      j.run_pieces = (int)(n_run / ce);
+      if (sources > 1) {
+        j.row_period = (int)k_run;
+        j.row_run = p.K_local;
+      }
+      q.s_bk = n_run;
+      bytes_b = j.rows * n_run * es;
+    }
+  }
+  if (bytes_a >= (1ll << 31) || bytes_b >= (1ll << 31)) return false;  // (also what the kernel's tile offsets reach)
+  const int bm = tile_rows(plan.kind), bn = tile_cols(plan.kind);
+  const long long a_span = (long long)bm * q.s_am * es + (long long)q.K * es;
+  const long long b_span = bkc ? (long long)bn * q.s_bn * es + (long long)q.K * es : (long long)q.K * q.s_bk * es + (long long)bn * es;
+  if (a_span >= (1ll << 31) || b_span >= (1ll << 31)) return false;
+  plan.pack.job[1].dst = (char*)((bytes_a + 255) / 256 * 256);  // offsets until the memory is there
+  plan.bytes = (size_t)((bytes_a + 255) / 256 * 256 + bytes_b);
+  if (plan.bytes > (1ull << 30)) return false;  // as much memory as a launch may ask for
+  const int per_block = kPackThreads * kPackPieces;
+  plan.pack.blocks[0] = (int)((bytes_a / 16 + per_block - 1) / per_block);
+  plan.pack.blocks[1] = (int)((bytes_b / 16 + per_block - 1) / per_block);
+  return true;
+}
+
+// Whether that is expected to take less time than the any-shape kernel, in us.  Both are modelled as a K loop, every CU as busy as the
+// busiest one, at the rates (TFLOP/s) that 190 plain products showed (M 130 to 16000, N 300 to 8001, K 331 to 8001, bf16,
+// two sets of operands in turn); packing moves its bytes at 5.2 TB/s and costs a launch.  What it gives and where it
+// does not: 4000x2877x2501 125.4 -> 72.1 us, 2000x1501x8001 133.7 -> 84.3, 1000x701x8001 65.5 -> 44.8, e4m3 4000x4095x1371
+// 55.5 -> 38.5; 4000x4095x331 25.6 -> 28.0, 500x4095x5001 54.0 -> 53.0, 16000x300x5001 127 -> 159, the last three left where they
+// were.  Two 128x128 tiles per CU have to win more when the peers' tiles are read behind them: the 64x128 tiles of the
+// any-shape kernel, three to a CU, hide each other's round trips (one-shot, eight ranks, fp16 1999x2877x2501 85.7 -> 88.5).
+bool worth_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, const PackPlan& plan) {
+  const bool fp8 = in_dtype == IRIS_HIP_FP8_E4M3;
+  float any = 0.f;
+  choose_any_tile(p.M, p.N, cu, false, false, &any);
+  const float products = 2e-6f * cu * p.K;
+  const float results = (float)p.M * p.N * elem_size(out_dtype) * 2e-7f;  // C, either way
+  const int bm = tile_rows(plan.kind), bn = tile_cols(plan.kind);
+  const long long tiles = (long long)cdiv(p.M, bm) * cdiv(p.N, bn);
+  const float rate = (plan.kind == TILE_BIG ? 1400.f : plan.kind == TILE_SMALL ? 1220.f : plan.kind == TILE_SMALL2 ? 964.f : tiles > cu ? 671.f : 560.f) * (fp8 ? 1.9f : 1.f);
+  const float there = (float)bm * bn * ((tiles + cu - 1) / cu) / rate;
+  const float packing = (plan.bytes ? 4.5f + plan.bytes * 2 / 5.2e6f : 0.f) + (plan.kind == TILE_SKINNY64 ? 4.f : 3.f);
+  const float margin = plan.kind == TILE_SMALL2 && epi_has_flags(p.epi) && p.sum_peers && p.world > 1 ? 0.85f : 0.92f;
+  return packing + products * there + results < margin * (4.f + products * any * (fp8 ? 0.7f : 1.f) + results);
+}
+
+// Launches p on packed operands.  Returns 0 or an error, or -1 with nothing done where it is not to be: the any-shape kernel takes it.
+int run_packed(const FusedParams& p, int in_dtype, int out_dtype, int device, int cu, hipStream_t s) {
+  PackPlan plan;
+  if (p.no_workspace_alloc || !plan_packing(p, in_dtype, out_dtype, cu, plan) || !worth_packing(p, in_dtype, out_dtype, cu, plan)) return -1;
+  void* memory = nullptr;
+  if (plan.bytes) {
+    memory = g_scratch_allocator.take(plan.bytes, s);
+    if (!memory) return -1;
+    PackParams& pack = plan.pack;
+    pack.job[0].dst = (char*)memory;
+    pack.job[1].dst = (char*)memory + (size_t)pack.job[1].dst;
+    if (pack.blocks[0]) plan.p.A = pack.job[0].dst;
+    if (pack.blocks[1]) plan.p.B = pack.job[1].dst;
+    const dim3 grid(pack.blocks[0] + pack.blocks[1]);
+    if (elem_size(in_dtype) == 2) hipLaunchKernelGGL((pack_kernel<2>), grid, dim3(kPackThreads), 0, s, pack);
+    else hipLaunchKernelGGL((pack_kernel<1>), grid, dim3(kPackThreads), 0, s, pack);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      g_scratch_allocator.give_back(memory);
+      return (int)e;
+    }
+  }
+  const bool bkc = p.s_bn != 1;
+  int rc = 0;
+  switch (in_dtype) {
+    case IRIS_HIP_BF16: rc = dispatch_mfma_rows<IN_BF16>(plan.p, plan.kind, bkc, device, cu, s); break;
+    case IRIS_HIP_FP16: rc = dispatch_mfma_rows<IN_F16>(plan.p, plan.kind, bkc, device, cu, s); break;
+    default: rc = dispatch_mfma_rows<IN_FP8>(plan.p, plan.kind, bkc, device, cu, s);
+  }
+  g_scratch_allocator.give_back(memory);
+  return rc;
+}
+
 // check_only: run every argument check and the kernel choice, launch nothing (0 = the launch would go out).
 int run_fused(FusedParams p, int in_dtype, int out_dtype, int path, void* stream, bool check_only = false) {
   g_last_error[0] = 0;
@@ -350,7 +526,12 @@ int run_fused(FusedParams p, int in_dtype, int out_dtype, int path, void* stream
   if (path == IRIS_HIP_PATH_MFMA && why) return fail("MFMA kernel not applicable: %s", why);
   if (path == IRIS_HIP_PATH_GENERIC || why) {
     if (!generic_supported(in_dtype, out_dtype)) return fail("unsupported element types in=%d out=%d", in_dtype, out_dtype);
-    return check_only ? 0 : dispatch_generic(p, in_dtype, out_dtype, device, facts->cu_count, s);
+    if (check_only) return 0;
+    if (path == IRIS_HIP_PATH_AUTO) {
+      rc = run_packed(p, in_dtype, out_dtype, device, facts->cu_count, s);
+      if (rc >= 0) return rc;
+    }
+    return dispatch_generic(p, in_dtype, out_dtype, device, facts->cu_count, s);
   }
   if (check_only) return 0;
 
@@ -705,6 +886,11 @@ void iris_hip_set_split_tiles(int32_t mode) { iris_host::set_split_tile_mode(mod
 
 const char* iris_hip_last_error(void) { return g_last_error; }
 const char* iris_hip_last_kernel(void) { return g_last_kernel; }
+void iris_hip_set_scratch_allocator(iris_hip_allocate_fn allocate, iris_hip_release_fn release) {
+  g_scratch_allocator.release.store(release, std::memory_order_release);
+  g_scratch_allocator.allocate.store(release ? allocate : nullptr, std::memory_order_release);
+}
+
 int iris_hip_stream_capturing(void* stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess) {
@@ -714,6 +900,6 @@ int iris_hip_stream_capturing(void* stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-int iris_hip_abi_version(void) { return 6; }
+int iris_hip_abi_version(void) { return 7; }
 
 }  // extern "C"

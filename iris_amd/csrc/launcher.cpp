@@ -13,6 +13,7 @@
 //                  a launch that went out.
 //
 //   load(path)     dlopen the library (once) and resolve the entry points; raises OSError
+#include <c10/hip/HIPCachingAllocator.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -75,6 +76,22 @@ int (*fn_stream_capturing)(void*) = nullptr;
   PyObject* py_##name(PyObject*, PyObject* const* args, Py_ssize_t n) { return call(fn_##name, #name, args, n); }
 ENTRY_POINTS(DEFINE)
 
+// Memory for the length of a launch comes from torch's caching allocator, which hands a block on to later work of the same
+// stream only.
+void* allocate_scratch(size_t bytes, void* stream) noexcept {
+  try {
+    return c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, (hipStream_t)stream);
+  } catch (...) {
+    return nullptr;
+  }
+}
+void release_scratch(void* memory) noexcept {
+  try {
+    c10::hip::HIPCachingAllocator::raw_delete(memory);
+  } catch (...) {
+  }
+}
+
 PyObject* load(PyObject*, PyObject* path_object) {
   const char* path = PyUnicode_AsUTF8(path_object);
   if (!path) return nullptr;
@@ -86,6 +103,8 @@ PyObject* load(PyObject*, PyObject* path_object) {
   ENTRY_POINTS(RESOLVE)
   fn_stream_capturing = (decltype(fn_stream_capturing))dlsym(lib, "iris_hip_stream_capturing");
   if (!fn_stream_capturing) return PyErr_Format(PyExc_OSError, "%s has no iris_hip_stream_capturing", path);
+  const auto set_allocator = (decltype(&::iris_hip_set_scratch_allocator))dlsym(lib, "iris_hip_set_scratch_allocator");
+  if (set_allocator) set_allocator(allocate_scratch, release_scratch);
   Py_RETURN_NONE;
 }
 
