@@ -646,12 +646,7 @@ int launch_any(FusedParams p, int device, int cu_count, hipStream_t stream, cons
   p.tiles_n = cdiv(p.N, CFG::BN);
   const long long total = (long long)p.tiles_m * p.tiles_n;
   if (total > (1ll << 30)) return iris_host::fail("output of %d x %d has too many tiles", p.M, p.N);
-  // Close to square groups of the tiles an XCD works on at one time, as in dispatch_mfma_in.
-  const int resident = cu_count / p.num_xcd * CFG::WG_PER_CU, span = cdiv((int)total, p.num_xcd);
-  const int at_once = span < resident ? span : resident;
-  int g = 1;
-  while (g * g * 2 <= at_once && g * 2 <= p.tiles_m) g *= 2;
-  p.group_m = g;
+  p.group_m = any_group_m(p.tiles_m, p.tiles_n, p.num_xcd, cu_count / p.num_xcd * CFG::WG_PER_CU);
   const int grid = cdiv((int)total, p.num_xcd) * p.num_xcd;
   char name[96];
   snprintf(name, sizeof(name), "generic_%s_%dx%d_%s", types, CFG::BM, CFG::BN, CFG::BKC ? "nt" : "nn");

@@ -1308,17 +1308,9 @@ template <class CFG>
 int launch_mfma(const FusedParams& p, int device, int cu_count, hipStream_t stream, const char* name) {
   const int total = p.tiles_m * p.tiles_n;
   const int cap = cu_count * CFG::WG_PER_CU;
-  // A multiple of the XCD count keeps the XCD mapping exact.  Rounded up when the tiles fit in one
-  // round (the surplus workgroups find no tile and leave), so that no tile waits for a second round.
-  int grid = total < cap ? total : cap;
-  if (grid % p.num_xcd) {
-    const int up = grid + p.num_xcd - grid % p.num_xcd;
-    grid = up <= cap ? up : grid - grid % p.num_xcd;
-  }
-  if (grid < 1) grid = 1;
+  const int grid = resident_grid(total, cap, p.num_xcd);
   iris_host::set_last_kernel(name);
-  const bool uneven_tiles = p.epi == EPI_TWO_SHOT || (p.epi == EPI_REDUCE_SCATTER && !p.all_owners);
-  const bool per_tile_launch = uneven_tiles && p.world > 1 && p.sum_peers && total > grid;
+  const bool per_tile_launch = total > grid && workgroup_per_tile(p.epi, p.world, p.sum_peers, p.all_owners);
   if constexpr (CFG::NW == 8) {
     FusedParams q = p;
     const int sk_grid = per_tile_launch ? 0 : split_tile_grid<CFG>(q, total, cu_count);
@@ -1338,13 +1330,7 @@ int launch_mfma(const FusedParams& p, int device, int cu_count, hipStream_t stre
     }
   }
   if (total <= grid) return launch_mfma_grid<CFG, true>(p, device, grid, stream);
-  // More tiles than workgroups that fit at once: normally the resident workgroups loop over the tiles.
-  // The two-shot all-reduce does better with one workgroup per tile, handed out by the hardware as CUs
-  // free up (measured at W = 8: 16384x4096x1376 322 -> 273 us, 8192x8192x2752 461 -> 417 us,
-  // 8192x8192x8192 1059 -> 1009 us); the one-shot variant does worse that way (+3-7 %), launches
-  // without peers do not care.  The same goes for a reduce-scatter whose rank owns one block of
-  // rows: the few tiles that carry the slot sum take half as long again as the others, and a fixed
-  // tile-to-workgroup assignment gives some workgroups two of them.
+  // More tiles than workgroups that fit at once: the resident workgroups loop over the tiles, or get one each in turn.
   if (per_tile_launch) {
     int per_tile = total;
     if (per_tile % p.num_xcd) per_tile += p.num_xcd - per_tile % p.num_xcd;
@@ -1390,71 +1376,24 @@ inline int tile_cols(int kind) { return kind == TILE_BIG ? 256 : kind == TILE_DE
 template <int IN>
 int dispatch_decode(FusedParams& p, bool bkc, int device, int cu, hipStream_t s);
 
+inline TileLaunch tile_launch(const FusedParams& p, int kind, int cu) {
+  const int two_per_cu = !(kind == TILE_BIG || kind == TILE_SMALL);
+  return {p.M, p.N, tile_rows(kind), tile_cols(kind), p.num_xcd, (cu / p.num_xcd) * (1 + two_per_cu), two_per_cu,
+          p.epi, p.world, p.rank, p.sum_peers, p.all_owners, p.flag_bm, p.flag_bn};
+}
+
 // The tiles of a launch and their order.
 inline void plan_tiles(FusedParams& p, int kind, int cu) {
-  const int bm = tile_rows(kind), bn = tile_cols(kind);
-  p.tiles_m = cdiv(p.M, bm);
-  p.tiles_n = cdiv(p.N, bn);
-  // Group height: tile-rows walked together so that the tiles an XCD works on at one time - its whole
-  // span, or one round of it when the span is longer than its resident workgroups - are close to a
-  // square (fewest operand panels per L2).
-  const int span = cdiv(p.tiles_m * p.tiles_n, p.num_xcd);
-  const int resident = (cu / p.num_xcd) * (kind == TILE_BIG || kind == TILE_SMALL ? 1 : 2);
-  const bool rounds = span > resident;
-  const int at_once = rounds ? resident : span;
-  int g = 1;
-  while (g * g * 2 <= at_once && g * 2 <= p.tiles_m) g *= 2;
-  // Two-shot launches of several rounds (one workgroup per tile, handed out in this order) do better with
-  // groups of at most four rows (eight ranks, fp16: 16384x3584x8192 1006 -> 977 us, 8192x8192x2752 441 -> 428).
-  if (rounds && p.sum_peers && p.world > 1 && p.epi == EPI_TWO_SHOT) g = g < 4 ? g : 4;
-  // A reduce-scatter rank sums the slots only for its own band of rows.  With XCD spans that are
-  // close to square that band falls to one or two XCDs, whose CUs then carry all the slow tiles;
-  // taller groups spread it over more XCDs at the price of more operand panels per L2
-  // (8192 x 4096 x 1376, 8 ranks, seven peers, on one box: 131 us at the default height 8, 114 at
-  // 16, 119 at 32; fetched by the L2s: 207, 290 and 443 MB).
-  if (p.epi == EPI_REDUCE_SCATTER && !p.all_owners && p.sum_peers && p.world > 1)
-    g = g * 2 < p.tiles_m ? g * 2 : p.tiles_m;
-  p.interleave = 0;
-  p.tile_rotate = 0;
-  // Launches whose epilogue streams whole tiles from or to every rank - the one-shot all-reduce with peers
-  // spends half its time reading the peers' tiles, matmul_all_gather and the atomic variant write every
-  // tile into all slots - want the workgroups that run together to touch long pieces of the same rows
-  // (DRAM pages stay open): flat groups of two rows - more for narrow outputs, so that g x tiles_n stays
-  // near 32 (64 with two workgroups per CU) and an L2 still sees as few operand panels as with a square
-  // span.  When the launch fills at least three quarters of the chip the grouped order is also dealt out
-  // workgroup by workgroup instead of in one span per XCD: XCD x then holds the tiles at positions x modulo
-  // the XCD count, 1/g of the rows and g/8 of the columns of one band of rows that the whole chip works on.
-  // Measured, eight ranks, one box, square spans -> this rule; one-shot: fp8 16384x8192x1024 568 -> 496 us
-  // (520 with flat spans), bf16 8192x4096x1376 216 -> 194, 4096x4096x1376 98.0 -> 96.8, 2048x8192x1376
-  // 108 -> 99, 2048x4096x1376 (128x128 tiles) 64.6 -> 60.4, 256x4096x4096 (64x64 tiles, chip half full:
-  // spans) 39.3 -> 32.2; atomic fp16 8192x4096x1376 566 -> 520; matmul_all_gather fp16 2048x3584x8192
-  // 175 -> 168, 512x4096x1376 22.9 -> 21.4.  Dealt out with one-row groups or spans of eight rows are the
-  // outliers (+9 % on 1536x6144x2048), and a chip that is little more than half full does better with spans
-  // (3072x3072x1024: 67.9 against 70.6).  Two-shot launches lose 3-5 % when dealt out; launches that
-  // neither read nor write other ranks' tiles do not care.
-  const bool streams_tiles = p.world > 1 && ((p.epi == EPI_ONE_SHOT && p.sum_peers) || p.epi == EPI_ALL_GATHER || p.epi == EPI_ATOMIC);
-  if (streams_tiles) {
-    const int two_per_cu = !(kind == TILE_BIG || kind == TILE_SMALL);
-    g = 2;
-    while (g < 8 && g * 2 * p.tiles_n <= (two_per_cu ? 64 : 32)) g *= 2;
-    while (g > p.tiles_m && g > 1) g /= 2;
-    p.interleave = (long long)p.tiles_m * p.tiles_n * 4 >= (long long)resident * p.num_xcd * 3;
-  }
-  p.group_m_spans = g;
-  // The reduce-scatter with peers is dealt out as well (its launches hand one workgroup per tile to the
-  // hardware in this order), starting with the band of rows this rank sums: those tiles take half as long
-  // again as the others, so they go first and spread over every XCD (8192x4096x1376, eight ranks, rank 0:
-  // 111.8 -> 106.6 us against spans of sixteen rows).
+  const TileOrder o = tile_order(tile_launch(p, kind, cu));
+  p.tiles_m = o.tiles_m;
+  p.tiles_n = o.tiles_n;
+  p.interleave = o.interleave;
+  p.tile_rotate = o.tile_rotate;
+  p.group_m_spans = o.group_m_spans;
+  int g = o.group_m;
   const bool rs_band = p.epi == EPI_REDUCE_SCATTER && !p.all_owners && p.sum_peers && p.world > 1;
-  if (rs_band) {
-    p.interleave = 1;
-    g = p.tiles_m >= 2 ? 2 : 1;
-    const int ftn = cdiv(p.N, p.flag_bn), ftotal = cdiv(p.M, p.flag_bm) * ftn;
-    const int band_row = (p.rank * (ftotal / p.world)) / ftn * p.flag_bm / bm;  // first tile row of the rank's band
-    p.tile_rotate = band_row / g * g * p.tiles_n;
-  }
   static const int forced_order = [] {
-    const char* e = getenv("IRIS_HIP_TILE_ORDER");  // "spans" or "dealt": a tuning aid
+    const char* e = getenv("IRIS_HIP_TILE_ORDER");  // "spans" or "dealt": a tuning aid, the same on all ranks
     return !e ? -1 : (e[0] == 'd' ? 1 : 0);
   }();
   if (forced_order >= 0) p.interleave = forced_order;

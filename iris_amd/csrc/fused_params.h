@@ -30,10 +30,6 @@ typedef __attribute__((ext_vector_type(4))) short i16x4_t;
 typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
 
-enum { EPI_STORE = 0, EPI_ONE_SHOT = 1, EPI_TWO_SHOT = 2, EPI_REDUCE_SCATTER = 3, EPI_ALL_GATHER = 4, EPI_ATOMIC = 5 };
-
-// Epilogues that publish aux + flags and then reduce over the slots.
-__host__ __device__ inline bool epi_has_flags(int epi) { return epi == EPI_ONE_SHOT || epi == EPI_TWO_SHOT || epi == EPI_REDUCE_SCATTER; }
 enum { GATHER_NONE = 0, GATHER_K = 1, GATHER_M = 2 };
 
 struct FusedParams {
@@ -63,7 +59,7 @@ struct FusedParams {
   int tiles_m, tiles_n, group_m, num_xcd;
   // Tile order: 0 gives every XCD one contiguous span of the grouped order (tiles that share operand
   // panels share an L2), 1 deals the grouped order out workgroup by workgroup (the chip works on one
-  // contiguous band of rows at a time; launches that stream the peers' tiles, see dispatch_mfma_in).
+  // contiguous band of rows at a time; launches that stream the peers' tiles, see tile_order in layout.h).
   int interleave;
   int tile_rotate;  // with interleave: the workgroups start this many positions into the grouped order (and wrap)
   int group_m_spans;  // host only: the group height to use if the launch falls back to spans (split tiles)

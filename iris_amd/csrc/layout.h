@@ -244,6 +244,162 @@ IRIS_HD int macro_tiles_over_flag_tile(int fm, int fn, int FM, int FN, int KM, i
 }
 
 // ---------------------------------------------------------------------------------------------
+// Order of a launch's tiles, and what it has to guarantee.
+//
+// Epilogues with flags publish their tile and then wait in place for the peers' flags: a waiting workgroup keeps its CU.  A
+// launch with more tiles than workgroups that run at one time therefore needs an order that lets the ranks finish together.
+//   - The same order on every rank does: the first unfinished tile of that order is running, and published, on all of them.
+//   - A rank whose waiting workgroups leave others room to run (publishes_alone) publishes everything whatever the
+//     others do.  It may take any order, and no order of its own can hold up anybody else.
+// tests/host_sim/layout_sim.cpp replays the launches of all ranks, with what fits at one time, until they end.
+// ---------------------------------------------------------------------------------------------
+enum { EPI_STORE = 0, EPI_ONE_SHOT = 1, EPI_TWO_SHOT = 2, EPI_REDUCE_SCATTER = 3, EPI_ALL_GATHER = 4, EPI_ATOMIC = 5 };
+
+// Epilogues that publish aux + flags and then reduce over the slots.
+IRIS_HD bool epi_has_flags(int epi) { return epi == EPI_ONE_SHOT || epi == EPI_TWO_SHOT || epi == EPI_REDUCE_SCATTER; }
+
+struct TileLaunch {
+  int M, N, tile_m, tile_n;
+  int num_xcd;
+  int resident;    // workgroups that run at one time on an XCD
+  int two_per_cu;  // ... two of them on a CU
+  int epi, world, rank;
+  int sum_peers;   // 0: the peers' tiles are neither waited for nor read
+  int all_owners;  // reduce-scatter: this rank sums the tiles of every owner
+  int flag_bm, flag_bn;
+};
+
+struct TileOrder {
+  int tiles_m, tiles_n;
+  int group_m, group_m_spans;  // group height; the one to use if the launch falls back to spans (split tiles)
+  int interleave, tile_rotate;  // see FusedParams
+};
+
+// This rank's band of a reduce-scatter as rows [first, last] of kernel tiles; false when it owns no flag tile.
+IRIS_HD bool band_tile_rows(const TileLaunch& t, int& first, int& last) {
+  const int ftn = cdiv(t.N, t.flag_bn), ftotal = cdiv(t.M, t.flag_bm) * ftn, per = ftotal / t.world;
+  const int lo = t.rank * per, hi = t.rank == t.world - 1 ? ftotal : lo + per;
+  if (lo >= hi) return false;
+  const long end = (long)((hi - 1) / ftn + 1) * t.flag_bm;
+  first = (int)((long)(lo / ftn) * t.flag_bm / t.tile_m);
+  last = (int)(((end < t.M ? end : t.M) - 1) / t.tile_m);
+  return true;
+}
+
+// Whether the workgroups of a launch on this rank that wait for peers leave room for the others to run and publish.  The order
+// is the one of tile_order with a reduce-scatter's tiles dealt out, in groups of `group_m` rows.
+IRIS_HD bool publishes_alone(const TileLaunch& t, int group_m) {
+  if (!epi_has_flags(t.epi) || !t.sum_peers || t.world == 1) return true;
+  const int tiles_m = cdiv(t.M, t.tile_m), tiles_n = cdiv(t.N, t.tile_n);
+  if (cdiv(tiles_m * tiles_n, t.num_xcd) <= t.resident) return true;
+  if (t.epi != EPI_REDUCE_SCATTER || t.all_owners) return false;
+  int first, last;
+  if (!band_tile_rows(t, first, last)) return true;
+  // The groups that hold the band (its tiles may be every second one of a group's), at most half of what runs at one time:
+  // CUs may be busy with other launches.
+  first = first / group_m * group_m;
+  last = last / group_m * group_m + group_m - 1;
+  if (last >= tiles_m) last = tiles_m - 1;
+  return cdiv((last - first + 1) * tiles_n, t.num_xcd) * 2 <= t.resident;
+}
+
+IRIS_HD TileOrder tile_order(const TileLaunch& t) {
+  TileOrder o;
+  o.tiles_m = cdiv(t.M, t.tile_m);
+  o.tiles_n = cdiv(t.N, t.tile_n);
+  // Group height: tile-rows walked together so that the tiles an XCD works on at one time - its whole
+  // span, or one round of it when the span is longer than its resident workgroups - are close to a
+  // square (fewest operand panels per L2).
+  const int span = cdiv(o.tiles_m * o.tiles_n, t.num_xcd);
+  const bool rounds = span > t.resident, peers = t.sum_peers && t.world > 1;
+  const int at_once = rounds ? t.resident : span;
+  int g = 1;
+  while (g * g * 2 <= at_once && g * 2 <= o.tiles_m) g *= 2;
+  // Two-shot launches of several rounds (one workgroup per tile, handed out in this order) do better with
+  // groups of at most four rows (eight ranks, fp16: 16384x3584x8192 1006 -> 977 us, 8192x8192x2752 441 -> 428).
+  if (rounds && peers && t.epi == EPI_TWO_SHOT) g = g < 4 ? g : 4;
+  // A reduce-scatter rank sums the slots only for its own band of rows.  With XCD spans that are
+  // close to square that band falls to one or two XCDs, whose CUs then carry all the slow tiles;
+  // taller groups spread it over more XCDs at the price of more operand panels per L2
+  // (8192 x 4096 x 1376, 8 ranks, seven peers, on one box: 131 us at the default height 8, 114 at
+  // 16, 119 at 32; fetched by the L2s: 207, 290 and 443 MB).
+  const bool rs_band = t.epi == EPI_REDUCE_SCATTER && !t.all_owners && peers;
+  if (rs_band) g = g * 2 < o.tiles_m ? g * 2 : o.tiles_m;
+  o.interleave = 0;
+  o.tile_rotate = 0;
+  // Launches whose epilogue streams whole tiles from or to every rank - the one-shot all-reduce with peers
+  // spends half its time reading the peers' tiles, matmul_all_gather and the atomic variant write every
+  // tile into all slots - want the workgroups that run together to touch long pieces of the same rows
+  // (DRAM pages stay open): flat groups of two rows - more for narrow outputs, so that g x tiles_n stays
+  // near 32 (64 with two workgroups per CU) and an L2 still sees as few operand panels as with a square
+  // span.  When the launch fills at least three quarters of the chip the grouped order is also dealt out
+  // workgroup by workgroup instead of in one span per XCD: XCD x then holds the tiles at positions x modulo
+  // the XCD count, 1/g of the rows and g/8 of the columns of one band of rows that the whole chip works on.
+  // Measured, eight ranks, one box, square spans -> this rule; one-shot: fp8 16384x8192x1024 568 -> 496 us
+  // (520 with flat spans), bf16 8192x4096x1376 216 -> 194, 4096x4096x1376 98.0 -> 96.8, 2048x8192x1376
+  // 108 -> 99, 2048x4096x1376 (128x128 tiles) 64.6 -> 60.4, 256x4096x4096 (64x64 tiles, chip half full:
+  // spans) 39.3 -> 32.2; atomic fp16 8192x4096x1376 566 -> 520; matmul_all_gather fp16 2048x3584x8192
+  // 175 -> 168, 512x4096x1376 22.9 -> 21.4.  Dealt out with one-row groups or spans of eight rows are the
+  // outliers (+9 % on 1536x6144x2048), and a chip that is little more than half full does better with spans
+  // (3072x3072x1024: 67.9 against 70.6).  Two-shot launches lose 3-5 % when dealt out; launches that
+  // neither read nor write other ranks' tiles do not care.
+  const bool streams_tiles = t.world > 1 && ((t.epi == EPI_ONE_SHOT && t.sum_peers) || t.epi == EPI_ALL_GATHER || t.epi == EPI_ATOMIC);
+  if (streams_tiles) {
+    g = 2;
+    while (g < 8 && g * 2 * o.tiles_n <= (t.two_per_cu ? 64 : 32)) g *= 2;
+    while (g > o.tiles_m && g > 1) g /= 2;
+    o.interleave = (long long)o.tiles_m * o.tiles_n * 4 >= (long long)t.resident * t.num_xcd * 3;
+  }
+  o.group_m_spans = g;
+  // The reduce-scatter with peers is dealt out as well (its launches hand one workgroup per tile to the
+  // hardware in this order), starting with the band of rows this rank sums: those tiles take half as long
+  // again as the others, so they go first and spread over every XCD (8192x4096x1376, eight ranks, rank 0:
+  // 111.8 -> 106.6 us against spans of sixteen rows).  A band that would fill more than half of the chip with workgroups
+  // that wait - for tiles that the other ranks only reach behind theirs - has to keep its place in the common order (last of
+  // eight ranks, own band first -> common order, us: 16384x8192x512, bands of 256 tiles, 228 -> 244; of two ranks 8192x8192x1024
+  // 156 -> 159, 8192x4096x1376 97 -> 97).
+  if (rs_band) {
+    o.interleave = 1;
+    g = o.tiles_m >= 2 ? 2 : 1;
+    int first = 0, last = 0;
+    if (band_tile_rows(t, first, last) && publishes_alone(t, g)) o.tile_rotate = first / g * g * o.tiles_n;
+  }
+  o.group_m = g;
+  return o;
+}
+
+// Workgroups of a launch whose tiles are walked by the resident workgroups: as many as run at one time (`cap`), or the
+// tiles if these are fewer.  A multiple of the XCD count keeps the XCD mapping exact.  Rounded up when the tiles fit in one
+// round (the surplus workgroups find no tile and leave), so that no tile waits for a second round.
+IRIS_HD int resident_grid(int total, int cap, int num_xcd) {
+  int grid = total < cap ? total : cap;
+  if (grid % num_xcd) {
+    const int up = grid + num_xcd - grid % num_xcd;
+    grid = up <= cap ? up : grid - grid % num_xcd;
+  }
+  return grid < 1 ? 1 : grid;
+}
+
+// Whether a launch of several rounds has one workgroup per tile, handed out by the hardware as CUs free up.  The two-shot
+// all-reduce does better that way (measured at W = 8: 16384x4096x1376 322 -> 273 us, 8192x8192x2752 461 -> 417 us,
+// 8192x8192x8192 1059 -> 1009 us); the one-shot variant does worse (+3-7 %), launches
+// without peers do not care.  The same goes for a reduce-scatter whose rank owns one block of
+// rows: the few tiles that carry the slot sum take half as long again as the others, and a fixed
+// tile-to-workgroup assignment gives some workgroups two of them.
+IRIS_HD bool workgroup_per_tile(int epi, int world, int sum_peers, int all_owners) {
+  return world > 1 && sum_peers && (epi == EPI_TWO_SHOT || (epi == EPI_REDUCE_SCATTER && !all_owners));
+}
+
+// Group height of the any-shape kernel's spans (one workgroup per tile, xcd_tile_index): close to square groups of the tiles an XCD
+// works on at one time, the same on every rank.
+IRIS_HD int any_group_m(int tiles_m, int tiles_n, int num_xcd, int resident) {
+  const int span = cdiv(tiles_m * tiles_n, num_xcd), at_once = span < resident ? span : resident;
+  int g = 1;
+  while (g * g * 2 <= at_once && g * 2 <= tiles_m) g *= 2;
+  return g;
+}
+
+// ---------------------------------------------------------------------------------------------
 // Tail policy of the 256x256 tile: how the tiles of a partly filled last round are split along K.
 //
 // An XCD's `wgs` workgroups meet `left` (< wgs) tiles in the last round.  When at most half of them

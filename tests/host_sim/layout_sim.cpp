@@ -5,6 +5,7 @@
 // counts are exact.  The transpose-read semantics used here (within each 16-lane group, output lane i
 // element e comes from input lane 4e + i/4, element i%4 for 16-bit data; input lane 2e + i/8, byte
 // i%8 for 8-bit data) were measured on an MI355X.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -452,6 +453,143 @@ void check_row_rects() {
       }
 }
 
+// ---- ranks that wait for each other ------------------------------------------------------------------
+// One rank's launch: the tiles of every workgroup in turn, and the flag tiles that a tile publishes and waits for.
+struct RankLaunch {
+  TileLaunch t;
+  std::vector<std::vector<int>> chain;  // kernel tiles (row * tiles_n + column) of workgroup b
+  int resident;                         // workgroups that run at one time on an XCD
+};
+
+RankLaunch make_launch(const TileLaunch& t, const TileOrder& o, bool one_each, int xcds_of_order) {
+  RankLaunch l;
+  l.t = t;
+  l.resident = t.resident;
+  const int total = o.tiles_m * o.tiles_n;
+  const int grid = one_each ? cdiv(total, t.num_xcd) * t.num_xcd : resident_grid(total, t.resident * t.num_xcd, t.num_xcd);
+  l.chain.resize(grid);
+  for (int wg = 0; wg < grid; ++wg)
+    for (int it = 0; it == 0 || !one_each; ++it) {
+      int idx = xcd_tile_index(wg, grid, it, total, xcds_of_order);
+      if (idx < 0) break;
+      idx = (idx + o.tile_rotate) % total;
+      int tm, tn;
+      grouped_tile(idx, o.tiles_m, o.tiles_n, o.group_m, tm, tn);
+      l.chain[wg].push_back(tm * o.tiles_n + tn);
+    }
+  return l;
+}
+
+// fused_mfma_kernel as launch_mfma launches it.
+RankLaunch tiled_launch(const TileLaunch& t) {
+  const TileOrder o = tile_order(t);
+  const bool rounds = o.tiles_m * o.tiles_n > resident_grid(o.tiles_m * o.tiles_n, t.resident * t.num_xcd, t.num_xcd);
+  return make_launch(t, o, rounds && workgroup_per_tile(t.epi, t.world, t.sum_peers, t.all_owners), o.interleave ? 1 : t.num_xcd);
+}
+
+// How many workgroups of all ranks are left when nobody can go on.  Workgroup b runs on XCD b % num_xcd, in order, as
+// soon as one in front of it has left (`in_order`: and not before all workgroups below b have started).
+int replay(const std::vector<RankLaunch>& ranks, bool in_order) {
+  struct State {
+    std::vector<int> at, needed, published;  // tile of its chain a workgroup is at; per flag tile: kernel tiles over it, those done
+    std::vector<char> told;
+    std::vector<int> next, running;          // per XCD
+    std::vector<int> live;                   // workgroups that run
+    int started = 0;
+  };
+  std::vector<State> st(ranks.size());
+  int left = 0;
+  const TileLaunch& t0 = ranks[0].t;
+  const int ftm = cdiv(t0.M, t0.flag_bm), ftn = cdiv(t0.N, t0.flag_bn);
+  for (size_t r = 0; r < ranks.size(); ++r) {
+    const RankLaunch& l = ranks[r];
+    st[r].at.assign(l.chain.size(), 0);
+    st[r].told.assign(l.chain.size(), 0);
+    st[r].next.resize(l.t.num_xcd);
+    for (int x = 0; x < l.t.num_xcd; ++x) st[r].next[x] = x;
+    st[r].running.assign(l.t.num_xcd, 0);
+    st[r].published.assign(ftm * ftn, 0);
+    for (int f = 0; f < ftm * ftn; ++f)
+      st[r].needed.push_back(macro_tiles_over_flag_tile(f / ftn, f % ftn, l.t.flag_bm, l.t.flag_bn, l.t.tile_m, l.t.tile_n, l.t.M, l.t.N));
+    left += (int)l.chain.size();
+  }
+  for (bool moved = true; moved;) {
+    moved = false;
+    for (size_t r = 0; r < ranks.size(); ++r) {
+      const RankLaunch& l = ranks[r];
+      State& s = st[r];
+      const TileLaunch& t = l.t;
+      const int tiles_n = cdiv(t.N, t.tile_n), nwg = (int)l.chain.size();
+      for (bool any = true; any;) {
+        any = false;
+        for (int x = 0; x < t.num_xcd; ++x)
+          while (s.next[x] < nwg && s.running[x] < l.resident && (!in_order || s.next[x] == s.started)) {
+            s.live.push_back(s.next[x]);
+            s.next[x] += t.num_xcd;
+            ++s.running[x];
+            ++s.started;
+            any = moved = true;
+          }
+      }
+      std::vector<int> still;
+      for (int wg : s.live) {
+        bool waits = false;
+        while (!waits && s.at[wg] < (int)l.chain[wg].size()) {
+          const int tile = l.chain[wg][s.at[wg]], m0 = tile / tiles_n * t.tile_m, n0 = tile % tiles_n * t.tile_n;
+          const int m1 = std::min(m0 + t.tile_m, t.M), n1 = std::min(n0 + t.tile_n, t.N);
+          for (int fm = m0 / t.flag_bm; fm <= (m1 - 1) / t.flag_bm; ++fm)
+            for (int fn = n0 / t.flag_bn; fn <= (n1 - 1) / t.flag_bn; ++fn) {
+              const int f = fm * ftn + fn;
+              if (!s.told[wg]) ++s.published[f], moved = true;
+              const int owner = t.epi == EPI_TWO_SHOT ? owner_interleaved(f, t.world) : t.epi == EPI_REDUCE_SCATTER ? owner_contiguous(f, ftm * ftn, t.world) : t.rank;
+              if (owner != t.rank && !t.all_owners) continue;
+              for (size_t peer = 0; peer < ranks.size(); ++peer) waits |= peer != r && st[peer].published[f] < st[peer].needed[f];
+            }
+          s.told[wg] = 1;
+          if (waits) break;
+          s.told[wg] = 0;
+          ++s.at[wg];
+          moved = true;
+        }
+        if (waits) {
+          still.push_back(wg);
+        } else {
+          --s.running[wg % t.num_xcd];
+          --left;
+        }
+      }
+      s.live = still;
+    }
+  }
+  return left;
+}
+
+TileLaunch launch_of(int epi, int M, int N, int tile_m, int tile_n, int two_per_cu, int world, int rank, int flag_bm, int flag_bn) {
+  return {M, N, tile_m, tile_n, 8, 32 * (1 + two_per_cu), two_per_cu, epi, world, rank, 1, 0, flag_bm, flag_bn};
+}
+
+// Launches of several rounds end on every rank, whatever they wait for.
+void check_ranks_finish() {
+  struct Case { int epi, M, N, tile_m, tile_n, two_per_cu, world, flag_bm, flag_bn; };
+  for (Case c : {Case{EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 2, 256, 64}, Case{EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 4, 256, 64},
+                 Case{EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 8, 256, 64}, Case{EPI_REDUCE_SCATTER, 8001, 4095, 256, 256, 0, 2, 256, 64},
+                 Case{EPI_REDUCE_SCATTER, 8192, 4097, 256, 256, 0, 2, 256, 64}, Case{EPI_REDUCE_SCATTER, 16383, 4093, 256, 256, 0, 4, 256, 64},
+                 Case{EPI_REDUCE_SCATTER, 16383, 8191, 256, 256, 0, 8, 128, 64}, Case{EPI_REDUCE_SCATTER, 16384, 8192, 256, 256, 0, 2, 96, 80},
+                 Case{EPI_REDUCE_SCATTER, 8192, 1024, 128, 128, 1, 2, 64, 64}, Case{EPI_REDUCE_SCATTER, 16384, 256, 128, 128, 1, 3, 128, 64},
+                 Case{EPI_REDUCE_SCATTER, 16384, 2048, 256, 256, 0, 8, 8192, 64}, Case{EPI_REDUCE_SCATTER, 8192, 8192, 256, 256, 0, 8, 4096, 4096},
+                 Case{EPI_ONE_SHOT, 16384, 8192, 256, 256, 0, 8, 256, 64}, Case{EPI_ONE_SHOT, 8191, 4097, 256, 256, 0, 2, 96, 80},
+                 Case{EPI_TWO_SHOT, 16384, 4096, 256, 256, 0, 8, 256, 64}, Case{EPI_TWO_SHOT, 8191, 4097, 256, 256, 0, 2, 96, 80}})
+    for (bool in_order : {false, true}) {
+      std::vector<RankLaunch> ranks;
+      for (int r = 0; r < c.world; ++r) ranks.push_back(tiled_launch(launch_of(c.epi, c.M, c.N, c.tile_m, c.tile_n, c.two_per_cu, c.world, r, c.flag_bm, c.flag_bn)));
+      const int left = replay(ranks, in_order);
+      CHECK(left == 0, "%d workgroups wait for ever: epilogue %d of %d ranks, %dx%d, tiles %dx%d, flag tiles %dx%d", left, c.epi, c.world, c.M, c.N, c.tile_m, c.tile_n, c.flag_bm, c.flag_bn);
+    }
+  // A rank starts with its own band of rows while that leaves half of the chip to the others.
+  CHECK(tile_order(launch_of(EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 8, 3, 256, 64)).tile_rotate == 12 * 16, "reduce-scatter of eight ranks starts with its band");
+  CHECK(tile_order(launch_of(EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 2, 1, 256, 64)).tile_rotate == 0, "reduce-scatter of two ranks: the same order on both");
+}
+
 // ---- vote of a workgroup in a loop with one barrier per step -----------------------------------------
 // A wave meets the first reason to leave in step `seen`.  Reads behind the barrier of step s may come as early as right
 // behind it or as late as right in front of the next one, when votes written in step s + 1 are there too: both have to
@@ -506,6 +644,7 @@ int main() {
   check_split_plan();
   check_row_rects();
   check_vote();
+  check_ranks_finish();
   if (failures) { printf("%d check(s) failed\n", failures); return 1; }
   printf("layout_sim: all checks passed\n");
   return 0;
