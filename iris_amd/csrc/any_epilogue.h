@@ -272,10 +272,12 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
     sum += x;
     return ref_chain ? Out::round(sum) : sum;
   };
+  // Both ways to read the peers' tiles differ in nothing but the loads.  (32x32 tiles are for outputs of at most 5.2 MB, of which
+  // seven peers' are 37 MB: the line of peers_past_caches, and one way is enough.)
+  const bool stream = LARGE && p.stream_peers;
   // The pieces of the tile are handed out row by row (RECT false: each thread keeps its column, what another rank reduces is
   // left out), or those of one rectangle of it, rows [r0, r1) and columns [c0, c1) of the tile, all with one owner (RECT true).
-  auto reduce = [&](auto np_tag, auto nt_tag, auto rect_tag, int r0, int r1, int c0, int c1) INLINED {
-    auto load_peer = [](const char* at) INLINED { return decltype(nt_tag)::value ? load16_any_nt(at) : load16_any(at); };
+  auto reduce = [&](auto np_tag, auto rect_tag, int r0, int r1, int c0, int c1) INLINED {
     constexpr int NP = decltype(np_tag)::value;  // peers, all of whose loads go out together; 0: any number
     constexpr bool RECT = decltype(rect_tag)::value;
     constexpr int NPV = NP > 0 ? NP : 1;
@@ -304,8 +306,18 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
         }
         if constexpr (NP > 0) {
           if (act[g] && (RECT || piece_ok)) {
+            auto at = [&](int i) INLINED {
+              return (LARGE ? p.aux + (i < p.rank ? to_slot[i] : to_slot[i + 1]) : slot_ptr(p.heap_bases, p.aux, p.rank, i < p.rank ? i : i + 1)) + offset(row[g], col[g]);
+            };
+            if (stream) {
+              KEEP_BRANCHES_APART();
 #pragma unroll
-            for (int i = 0; i < NP; ++i) pv[g][i] = load_peer((LARGE ? p.aux + (i < p.rank ? to_slot[i] : to_slot[i + 1]) : slot_ptr(p.heap_bases, p.aux, p.rank, i < p.rank ? i : i + 1)) + offset(row[g], col[g]));
+              for (int i = 0; i < NP; ++i) pv[g][i] = load16_any_nt(at(i));
+              KEEP_BRANCHES_APART();
+            } else {
+#pragma unroll
+              for (int i = 0; i < NP; ++i) pv[g][i] = load16_any(at(i));
+            }
           }
         }
       }
@@ -326,7 +338,16 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
           } else {
             for (int pr = 0; pr < p.world; ++pr) {
               if (pr == p.rank) continue;
-              OutPiece<Out>::unpack(load_peer(slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row[g], col[g])), x);
+              const char* const at = slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row[g], col[g]);
+              u32x4_t v;
+              if (p.stream_peers) {
+                KEEP_BRANCHES_APART();
+                v = load16_any_nt(at);
+                KEEP_BRANCHES_APART();
+              } else {
+                v = load16_any(at);
+              }
+              OutPiece<Out>::unpack(v, x);
 #pragma unroll
               for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
             }
@@ -368,11 +389,11 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
   // Variants with owners: a thread that keeps its column has nothing to do in most rows, so flag tiles that keep half of the
   // threads busy are streamed one after the other by all of them (two-shot, eight ranks, bf16 1999x2877x1371 59.8 -> 50.7 us,
   // 4000x2877x2501 160 -> 143; float32 2048x2880x1024 of four ranks 102.8 -> 100.5).
-  auto reduce_tile = [&](auto np_tag, auto nt_tag) INLINED {
+  auto reduce_tile = [&](auto np_tag) INLINED {
     const int n1 = min(n0 + BN, p.N);
     const bool by_rect = LARGE && owners && p.s_cn == 1 && p.flag_bn >= OE && (long long)min(p.flag_bm, BM) * (min(p.flag_bn, BN) / OE) * 2 >= NT;
     if (!by_rect) {
-      reduce(np_tag, nt_tag, std::false_type{}, 0, 0, 0, 0);
+      reduce(np_tag, std::false_type{}, 0, 0, 0, 0);
       return;
     }
     if constexpr (LARGE)
@@ -381,19 +402,15 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
         if (!p.all_owners && owner_of(p.epi, fr * ftn + fc, ftotal, p.world, p.rank) != p.rank) continue;
         const int r0 = max(m0, fr * p.flag_bm) - m0, r1 = min(m_end, (fr + 1) * p.flag_bm) - m0;
         const int c0 = max(n0, fc * p.flag_bn) - n0, c1 = min(n1, (fc + 1) * p.flag_bn) - n0;
-        if (c1 - c0 >= OE) reduce(np_tag, nt_tag, std::true_type{}, r0, r1, c0, c1);
+        if (c1 - c0 >= OE) reduce(np_tag, std::true_type{}, r0, r1, c0, c1);
         else reduce_sliver(r0, r1, c0, c1);
       }
   };
-  auto reduce_with = [&](auto np_tag) INLINED {
-    if (LARGE && p.stream_peers) reduce_tile(np_tag, std::integral_constant<bool, LARGE>{});
-    else reduce_tile(np_tag, std::false_type{});
-  };
   switch (p.world - 1) {
-    case 1: reduce_with(std::integral_constant<int, 1>{}); break;
-    case 3: reduce_with(std::integral_constant<int, 3>{}); break;
-    case 7: reduce_with(std::integral_constant<int, 7>{}); break;
-    default: reduce_tile(std::integral_constant<int, 0>{}, std::false_type{}); break;
+    case 1: reduce_tile(std::integral_constant<int, 1>{}); break;
+    case 3: reduce_tile(std::integral_constant<int, 3>{}); break;
+    case 7: reduce_tile(std::integral_constant<int, 7>{}); break;
+    default: reduce_tile(std::integral_constant<int, 0>{}); break;
   }
   PHASE_STAMP(7);
 }

@@ -1076,8 +1076,8 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
       // The peers' tiles are read once and C is written once.  C, and the peers' tiles of launches that move more than
       // the last-level cache takes in, go past the caches' keep policy (non-temporal): they neither displace the operands nor -
       // what costs more - make that cache write back whatever dirty lines it holds (4096 x 4096 x 1376
-      // bf16 with seven peers, after a 256 MB buffer had been zeroed: phase 2 68 -> 39 us).  Smaller launches, and rows
-      // that are not whole lines, read the peers' tiles through the caches (peers_past_caches in iris_hip.hip has the figures).
+      // bf16 with seven peers, after a 256 MB buffer had been zeroed: phase 2 68 -> 39 us).  Smaller launches read the peers' tiles
+      // through the caches (peers_past_caches in iris_hip.hip has the line and the figures).
       // Chunks are handed to the threads either over the whole kernel tile (RECT false: thread t
       // takes chunk t of every pass, ownership looked up per chunk) or over one rectangle of it,
       // rows [r0, r1) and `ncw` chunks from column c0, all of which `rect_owner` reduces (RECT true).
@@ -1237,7 +1237,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WAVES_PER_SIMD) fused_mfma_kerne
         case 1: reduce_with(std::integral_constant<int, 1>{}); break;
         case 3: reduce_with(std::integral_constant<int, 3>{}); break;
         case 7: reduce_with(std::integral_constant<int, 7>{}); break;
-        default: reduce_tile(std::integral_constant<int, -1>{}, std::true_type{}); break;
+        default: reduce_with(std::integral_constant<int, -1>{}); break;
       }
     }
     PHASE_STAMP(7);

@@ -254,6 +254,10 @@ __device__ __forceinline__ u32x4_t load16_any_nt(const char* p) {
   return __builtin_nontemporal_load((const GLOBAL_AS u32x4_any_t*)(GLOBAL_AS const char*)p);
 }
 
+// Around the loads on one side of a branch: the compiler takes loads that both sides make for one, and drops the cache policy that
+// only one of them has.
+#define KEEP_BRANCHES_APART() asm volatile("" ::: "memory")
+
 constexpr int kMaxCachedSlots = 8;  // heap bases kept in registers; larger worlds re-load them
 
 // A 64-bit value that is the same in every lane, moved to scalar registers.
