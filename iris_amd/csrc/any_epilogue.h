@@ -220,6 +220,7 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
   };
   const bool aligned = (((unsigned long long)p.C | (unsigned long long)(p.s_cm * Out::size)) & 15) == 0 && p.N % OE == 0;
   const bool owners = flags && p.epi != EPI_ONE_SHOT;
+  const bool rects_aligned = rect_pieces_aligned(aligned, p.flag_bn, OE);
   // A piece may be moved whole when all of it has one owner.
   const bool piece_ok = whole && (!owners || gn / p.flag_bn == (gn + OE - 1) / p.flag_bn);
 
@@ -296,7 +297,7 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
         if constexpr (RECT) {
           const unsigned i = (unsigned)((pg + g) * NT + tid), r = i / (unsigned)per_row;
           row[g] = r0 + (int)r;
-          col[g] = min(c0 + (int)(i - r * per_row) * OE, c1 - OE);
+          col[g] = rect_piece_col(c0, c1, (int)(i - r * per_row), OE);
           act[g] = row[g] < r1;
         } else {
           row[g] = (pg + g) * RPP + t_row;
@@ -353,7 +354,7 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
             }
           }
           const u32x4_t v = OutPiece<Out>::pack(sum);
-          each_destination(gm, n0 + col[g], [&](char* base) { store16_result(base + offset(row[g], col[g]), v, aligned); });
+          each_destination(gm, n0 + col[g], [&](char* base) { store16_result(base + offset(row[g], col[g]), v, RECT ? rects_aligned : aligned); });
         } else {
           // Fewer columns than a piece, strided columns or several owners: all elements of a peer in one go.
           float sum[OE];

@@ -233,6 +233,12 @@ IRIS_HD int owner_contiguous(int t, int total, int world) {
   return o < world - 1 ? o : world - 1;
 }
 
+// A flag tile's columns [c0, c1) of a tile in pieces of `oe` elements, the last one from as far left as it takes: the column of
+// piece i, and whether all such pieces of a launch start on 16-byte boundaries when its rows do (tiles always do, flag tiles
+// start at multiples of flag_bn).
+IRIS_HD int rect_piece_col(int c0, int c1, int i, int oe) { return c0 + i * oe < c1 - oe ? c0 + i * oe : c1 - oe; }
+IRIS_HD bool rect_pieces_aligned(bool rows_aligned, int flag_bn, int oe) { return rows_aligned && flag_bn % oe == 0; }
+
 // How many kernel macro-tiles (KM x KN) overlap flag tile (fm, fn) of size (FM x FN) in an
 // M x N matrix.  A flag is raised by the last of them to finish.
 IRIS_HD int macro_tiles_over_flag_tile(int fm, int fn, int FM, int FN, int KM, int KN, int M, int N) {

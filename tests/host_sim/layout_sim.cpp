@@ -350,6 +350,28 @@ void check_flag_counts() {
     }
 }
 
+// Flag tiles summed as rectangles: their pieces cover the columns, stay inside, and start on 16-byte boundaries of rows that do
+// wherever the rule says so.
+void check_rect_pieces() {
+  for (int oe : {4, 8})
+    for (int bn : {64, 128, 256})
+      for (int N : {bn, 2 * bn + oe, 5 * bn - oe})
+        for (int flag_bn = oe; flag_bn <= 300; ++flag_bn)
+          for (int n0 = 0; n0 < N; n0 += bn)
+            for (int n1 = std::min(n0 + bn, N), fc = n0 / flag_bn; fc * flag_bn < n1; ++fc) {
+              const int c0 = std::max(n0, fc * flag_bn) - n0, c1 = std::min(n1, (fc + 1) * flag_bn) - n0;
+              if (c1 - c0 < oe) continue;
+              int covered = c0;
+              for (int i = 0; i < cdiv(c1 - c0, oe); ++i) {
+                const int col = rect_piece_col(c0, c1, i, oe);
+                CHECK(col >= c0 && col <= covered && col + oe <= c1, "piece %d of columns [%d, %d) at %d", i, c0, c1, col);
+                CHECK(!rect_pieces_aligned(true, flag_bn, oe) || (n0 + col) % oe == 0, "flag tiles of %d columns, pieces of %d: one at column %d", flag_bn, oe, n0 + col);
+                covered = col + oe;
+              }
+              CHECK(covered == c1, "pieces end at %d of [%d, %d)", covered, c0, c1);
+            }
+}
+
 // The rule that keeps launches away from the 32x32 kernel when its 32-bit offsets would not reach.
 void check_decode_offsets() {
   CHECK(decode_offsets_fit(32, 1024, 1024, 1, 32, 8192, 8192), "decode shape 32 x 8192 x 1024 fp8");
@@ -640,6 +662,7 @@ int main() {
   check_tile_orders();
   check_dealt_order();
   check_flag_counts();
+  check_rect_pieces();
   check_decode_offsets();
   check_split_plan();
   check_row_rects();

@@ -1,4 +1,5 @@
-"""The end of tiles whose rows start anywhere: numbers of ranks with and without a loop of their own.  Operands are small integers
+"""The end of tiles whose rows start anywhere: flag tiles that end inside a piece of rows that are aligned, numbers of
+ranks with and without a loop of their own.  Operands are small integers
 and the outputs are compared bit for bit with the CPU oracle."""
 
 import pytest
@@ -51,6 +52,12 @@ def _run(dtype, op, W, M, N, K, bm, bn, strided=False):
     for r in range(W) if op == "two_shot" else [rank]:
         assert_bits_equal(got[r], exp["C"][r], f"{name}, slot {r}")
     return name
+
+
+@pytest.mark.parametrize("op", ["two_shot", "reduce_scatter"])
+@pytest.mark.parametrize("dtype,N,bn", [(torch.bfloat16, 2824, 100), (torch.float32, 2820, 70), (torch.float16, 2816, 12), (torch.bfloat16, 2824, 104)])
+def test_flag_tiles_that_end_inside_a_piece_of_aligned_rows(op, dtype, N, bn):
+    _run(dtype, op, 8, 1000, N, 24, 64, bn)
 
 
 # Both ways to read the peers' tiles, from other numbers of ranks than 2, 4 and 8 (the line lies at 32 MiB read).
