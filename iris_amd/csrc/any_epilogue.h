@@ -61,7 +61,7 @@ template <int TROW>
 struct LinearTile {  // rows of TROW bytes
   char* base;
   __device__ __forceinline__ char* at(int row, int byte) const { return base + row * TROW + byte; }
-  __device__ __forceinline__ u32x4_t piece(int row, int byte, int) const { return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)at(row, byte); }
+  __device__ __forceinline__ u32x4_t piece(int row, int byte) const { return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)at(row, byte); }
 };
 
 // IN_FLIGHT: 16-byte pieces of the peers per thread that are loaded together; with more, fewer workgroups share a CU.  LARGE: with
@@ -89,7 +89,7 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
   const bool whole = cols == OE && p.s_cn == 1;  // moved as 16 bytes, else element by element
   const int ftn = cdiv(p.N, p.flag_bn);
   const int ftotal = cdiv(p.M, p.flag_bm) * ftn;
-  auto staged_piece = [&](int row, int col) INLINED { return tile.piece(row, col * Out::size, Out::size); };
+  auto staged_piece = [&](int row, int col) INLINED { return tile.piece(row, col * Out::size); };
   auto staged_element = [&](int row, int col) INLINED -> float {
     if constexpr (Out::size == 4) {
       return *(const LDS_AS float*)(LDS_AS char*)tile.at(row, col * 4);
@@ -220,37 +220,88 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
   };
   const bool aligned = (((unsigned long long)p.C | (unsigned long long)(p.s_cm * Out::size)) & 15) == 0 && p.N % OE == 0;
   const bool owners = flags && p.epi != EPI_ONE_SHOT;
-  const bool rects_aligned = rect_pieces_aligned(aligned, p.flag_bn, OE);
   // A piece may be moved whole when all of it has one owner.
   const bool piece_ok = whole && (!owners || gn / p.flag_bn == (gn + OE - 1) / p.flag_bn);
 
+  // Elements that no piece takes, in one place of the code.  Those of the last columns - fewer than a piece, or a piece that was moved to
+  // the left over the edge of a flag tile - are dealt to all threads: with one thread per row the 7 columns that N = 3207
+  // leaves for the last 128x128 tiles took longer than the rest of a bf16 product 691x3207x849, and the owners of the elements of the moved
+  // pieces 30 to 40 us of a two-shot sum 1124x7618x1965.  Strided columns and flag tiles that are no whole pieces stay with the thread that has them.
+  const int tail = p.s_cn != 1 ? 0 : tile_cols < OE ? tile_cols : owners && tile_cols % OE && p.flag_bn % OE == 0 && (n0 + tile_cols - OE) / p.flag_bn != (n0 + tile_cols - 1) / p.flag_bn ? OE : 0;
+  auto each_element = [&](auto&& f) INLINED {
+    if (!tail && (piece_ok || cols <= 0)) return;
+    const int per_row = tail ? tail : cols, first = tail ? tile_cols - tail : t_col;
+    const int row_step = tail ? NT / tail : 0, col_step = tail ? NT % tail : 1, next_row = tail ? 1 : RPP;
+    int row = tail ? tid / tail : t_row, col = tail ? tid % tail : 0;
+#pragma unroll 1
+    while (row < m_end - m0) {
+      f(row, first + col);
+      row += row_step;
+      col += col_step;
+      if (col >= per_row) {
+        col -= per_row;
+        row += next_row;
+      }
+    }
+  };
 #pragma unroll 2
   for (int ps = 0; ps < PASSES; ++ps) {
     const int row = ps * RPP + t_row, gm = m0 + row;
     if (gm >= m_end) break;
     if (flags) {
-      if (whole) {
-        store16_system_of_valu_data(p.aux + offset(row, t_col), staged_piece(row, t_col));
-      } else {
-        for (int e = 0; e < cols; ++e) store_element_system<Out>(p.aux + offset(row, t_col + e), tile.at(row, (t_col + e) * Out::size));
-      }
-      if (p.clear_c && owners) {  // other ranks' tiles: zeros
-        if (piece_ok) {
-          if (owner_at(gm, gn) != p.rank) store16_result(p.C + offset(row, t_col), (u32x4_t){0u, 0u, 0u, 0u}, aligned);
-        } else {
-          for (int e = 0; e < cols; ++e)
-            if (owner_at(gm, gn + e) != p.rank) Out::store(p.C + offset(row, t_col + e), 0.f);
-        }
-      }
+      if (whole) store16_system_of_valu_data(p.aux + offset(row, t_col), staged_piece(row, t_col));
+      if (p.clear_c && owners && piece_ok && owner_at(gm, gn) != p.rank)  // other ranks' tiles: zeros
+        store16_result(p.C + offset(row, t_col), (u32x4_t){0u, 0u, 0u, 0u}, aligned);
       if (!solo) continue;
     }
     if (piece_ok) {
       const u32x4_t v = staged_piece(row, t_col);
       each_destination(gm, gn, [&](char* base) { store16_result(base + offset(row, t_col), v, aligned); });
-    } else {
-      for (int e = 0; e < cols; ++e)
-        each_destination(gm, gn + e, [&](char* base) { Out::store(base + offset(row, t_col + e), staged_element(row, t_col + e)); });
     }
+  }
+  // A thread's own elements where little is to be done with them: all of a row at one time (two-shot of two ranks, bf16
+  // 4000x2877x200, flag tiles of 70 columns, 88.9 -> 55.8 us).  64x64 and 32x32 tiles go without: launches of 10 us were 1 to 2 % slower for
+  // the longer code.
+  constexpr bool OWN_ROWS = LARGE && BM * BN > 64 * 64;
+  auto my_elements = [&](auto&& f) INLINED {
+    if (piece_ok || cols <= 0) return;
+#pragma unroll 1
+    for (int row = t_row; row < m_end - m0; row += RPP) {
+#pragma unroll
+      for (int e = 0; e < OE; ++e)
+        if (e < cols) f(row, t_col + e);
+    }
+  };
+  if (OWN_ROWS && !tail && p.epi == EPI_STORE) {
+    my_elements([&](int row, int col) INLINED { Out::store(p.C + offset(row, col), staged_element(row, col)); });
+  } else if (OWN_ROWS && !tail && flags && !solo) {
+    if (p.s_cn != 1) my_elements([&](int row, int col) INLINED { store_element_system<Out>(p.aux + offset(row, col), tile.at(row, col * Out::size)); });
+    if (p.clear_c && owners && !piece_ok && cols > 0) {
+      const int split = (gn + cols - 1) / p.flag_bn * p.flag_bn - gn;  // columns left of the last flag tile
+#pragma unroll 1
+      for (int row = t_row; row < m_end - m0; row += RPP) {
+        const int left = owner_at(m0 + row, gn), right = owner_at(m0 + row, gn + cols - 1);
+        if (p.flag_bn >= OE) {
+#pragma unroll
+          for (int e = 0; e < OE; ++e)
+            if (e < cols && (e < split ? left : right) != p.rank) Out::store(p.C + offset(row, t_col + e), 0.f);
+        } else {
+#pragma unroll 1
+          for (int e = 0; e < cols; ++e)
+            if (owner_at(m0 + row, gn + e) != p.rank) Out::store(p.C + offset(row, t_col + e), 0.f);
+        }
+      }
+    }
+  } else if (!flags || solo || (p.clear_c && owners) || tile_cols < OE || p.s_cn != 1) {  // (else there is nothing to do for them)
+    each_element([&](int row, int col) INLINED {
+      const int gm = m0 + row, g = n0 + col;
+      if (flags) {
+        if (tile_cols < OE || p.s_cn != 1) store_element_system<Out>(p.aux + offset(row, col), tile.at(row, col * Out::size));
+        if (p.clear_c && owners && owner_at(gm, g) != p.rank) Out::store(p.C + offset(row, col), 0.f);
+        if (!solo) return;
+      }
+      each_destination(gm, g, [&](char* base) { Out::store(base + offset(row, col), staged_element(row, col)); });
+    });
   }
   PHASE_STAMP(4);
   if (!flags) return;
@@ -302,11 +353,11 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
         } else {
           row[g] = (pg + g) * RPP + t_row;
           col[g] = t_col;
-          act[g] = m0 + row[g] < m_end && cols > 0;
-          if (act[g] && owners && !p.all_owners && piece_ok) act[g] = owner_at(m0 + row[g], gn) == p.rank;
+          act[g] = m0 + row[g] < m_end && piece_ok;
+          if (act[g] && owners && !p.all_owners) act[g] = owner_at(m0 + row[g], gn) == p.rank;
         }
         if constexpr (NP > 0) {
-          if (act[g] && (RECT || piece_ok)) {
+          if (act[g]) {
             auto at = [&](int i) INLINED {
               return (LARGE ? p.aux + (i < p.rank ? to_slot[i] : to_slot[i + 1]) : slot_ptr(p.heap_bases, p.aux, p.rank, i < p.rank ? i : i + 1)) + offset(row[g], col[g]);
             };
@@ -326,92 +377,119 @@ __device__ __forceinline__ void finish_any(const FusedParams& p, const Tile& til
       for (int g = 0; g < G; ++g) {
         if (!act[g]) continue;
         const int gm = m0 + row[g];
-        if (RECT || piece_ok) {
-          float sum[OE], x[OE];
-          OutPiece<Out>::unpack(staged_piece(row[g], col[g]), sum);
-          if constexpr (NP > 0) {
+        float sum[OE], x[OE];
+        OutPiece<Out>::unpack(staged_piece(row[g], col[g]), sum);
+        if constexpr (NP > 0) {
 #pragma unroll
-            for (int i = 0; i < NP; ++i) {
-              OutPiece<Out>::unpack(pv[g][i], x);
-#pragma unroll
-              for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
-            }
-          } else {
-            for (int pr = 0; pr < p.world; ++pr) {
-              if (pr == p.rank) continue;
-              const char* const at = slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row[g], col[g]);
-              u32x4_t v;
-              if (p.stream_peers) {
-                KEEP_BRANCHES_APART();
-                v = load16_any_nt(at);
-                KEEP_BRANCHES_APART();
-              } else {
-                v = load16_any(at);
-              }
-              OutPiece<Out>::unpack(v, x);
-#pragma unroll
-              for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
-            }
-          }
-          const u32x4_t v = OutPiece<Out>::pack(sum);
-          each_destination(gm, n0 + col[g], [&](char* base) { store16_result(base + offset(row[g], col[g]), v, RECT ? rects_aligned : aligned); });
-        } else {
-          // Fewer columns than a piece, strided columns or several owners: all elements of a peer in one go.
-          float sum[OE];
-#pragma unroll
-          for (int e = 0; e < OE; ++e) sum[e] = e < cols ? staged_element(row[g], t_col + e) : 0.f;
-          for (int pr = 0; pr < p.world; ++pr) {
-            if (pr == p.rank) continue;
-            const char* const src = slot_ptr(p.heap_bases, p.aux, p.rank, pr);
-            float x[OE];
-#pragma unroll
-            for (int e = 0; e < OE; ++e) x[e] = e < cols ? Out::load(src + offset(row[g], t_col + e)) : 0.f;
+          for (int i = 0; i < NP; ++i) {
+            OutPiece<Out>::unpack(pv[g][i], x);
 #pragma unroll
             for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
           }
+        } else {
+          for (int pr = 0; pr < p.world; ++pr) {
+            if (pr == p.rank) continue;
+            const char* const at = slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row[g], col[g]);
+            u32x4_t v;
+            if (p.stream_peers) {
+              KEEP_BRANCHES_APART();
+              v = load16_any_nt(at);
+              KEEP_BRANCHES_APART();
+            } else {
+              v = load16_any(at);
+            }
+            OutPiece<Out>::unpack(v, x);
 #pragma unroll
-          for (int e = 0; e < OE; ++e)
-            if (e < cols) each_destination(gm, gn + e, [&](char* base) { Out::store(base + offset(row[g], t_col + e), sum[e]); });
+            for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
+          }
         }
+        const u32x4_t v = OutPiece<Out>::pack(sum);
+        each_destination(gm, n0 + col[g], [&](char* base) { store16_result(base + offset(row[g], col[g]), v, RECT ? rect_pieces_aligned(aligned, p.flag_bn, OE) : aligned); });
       }
     }
   };
-  // What a flag tile has in this tile when that is narrower than a piece.
+  // Fewer columns than a piece, strided columns or several owners: all elements of a peer in one go.
+  auto reduce_elements = [&](int row) INLINED {
+    float sum[OE];
+#pragma unroll
+    for (int e = 0; e < OE; ++e) sum[e] = e < cols ? staged_element(row, t_col + e) : 0.f;
+    for (int pr = 0; pr < p.world; ++pr) {
+      if (pr == p.rank) continue;
+      const char* const src = slot_ptr(p.heap_bases, p.aux, p.rank, pr);
+      float x[OE];
+#pragma unroll
+      for (int e = 0; e < OE; ++e) x[e] = e < cols ? Out::load(src + offset(row, t_col + e)) : 0.f;
+#pragma unroll
+      for (int e = 0; e < OE; ++e) sum[e] = add(sum[e], x[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < OE; ++e)
+      if (e < cols) each_destination(m0 + row, gn + e, [&](char* base) { Out::store(base + offset(row, t_col + e), sum[e]); });
+  };
+  // What a flag tile has in this tile, or the tile itself, when that is narrower than a piece: an element per thread, all peers of it in one go.
   auto reduce_sliver = [&](int r0, int r1, int c0, int c1) INLINED {
     const int wide = c1 - c0;
+#pragma unroll 1
     for (int i = tid; i < (r1 - r0) * wide; i += NT) {
       const int row = r0 + i / wide, col = c0 + i % wide;
-      float sum = staged_element(row, col);
-      for (int pr = 0; pr < p.world; ++pr)
-        if (pr != p.rank) sum = add(sum, Out::load(slot_ptr(p.heap_bases, p.aux, p.rank, pr) + offset(row, col)));
+      if (owners && !p.all_owners && owner_at(m0 + row, n0 + col) != p.rank) continue;
+      const char* const own = p.aux + offset(row, col);
+      float sum = staged_element(row, col), x[kMaxCachedSlots];
+#pragma unroll
+      for (int r = 0; r < kMaxCachedSlots; ++r)  // (slots that there are not: the own one)
+        x[r] = Out::load(LARGE ? own + (r < p.world ? to_slot[r] : 0) : slot_ptr(p.heap_bases, own, p.rank, r < p.world ? r : p.rank));
+#pragma unroll
+      for (int r = 0; r < kMaxCachedSlots; ++r)
+        if (r < p.world && r != p.rank) sum = add(sum, x[r]);
+      for (int r = kMaxCachedSlots; r < p.world; ++r)
+        if (r != p.rank) sum = add(sum, Out::load(slot_ptr(p.heap_bases, own, p.rank, r)));
       each_destination(m0 + row, n0 + col, [&](char* base) { Out::store(base + offset(row, col), sum); });
     }
   };
   // Variants with owners: a thread that keeps its column has nothing to do in most rows, so flag tiles that keep half of the
   // threads busy are streamed one after the other by all of them (two-shot, eight ranks, bf16 1999x2877x1371 59.8 -> 50.7 us,
   // 4000x2877x2501 160 -> 143; float32 2048x2880x1024 of four ranks 102.8 -> 100.5).
-  auto reduce_tile = [&](auto np_tag) INLINED {
+  const bool by_rect = LARGE && owners && p.s_cn == 1 && p.flag_bn >= OE && (long long)min(p.flag_bm, BM) * (min(p.flag_bn, BN) / OE) * 2 >= NT;
+  auto each_owned = [&](auto&& f) INLINED {
     const int n1 = min(n0 + BN, p.N);
-    const bool by_rect = LARGE && owners && p.s_cn == 1 && p.flag_bn >= OE && (long long)min(p.flag_bm, BM) * (min(p.flag_bn, BN) / OE) * 2 >= NT;
-    if (!by_rect) {
-      reduce(np_tag, std::false_type{}, 0, 0, 0, 0);
-      return;
-    }
-    if constexpr (LARGE)
     for (int fr = m0 / p.flag_bm; fr * p.flag_bm < m_end; ++fr)
       for (int fc = n0 / p.flag_bn; fc * p.flag_bn < n1; ++fc) {
         if (!p.all_owners && owner_of(p.epi, fr * ftn + fc, ftotal, p.world, p.rank) != p.rank) continue;
-        const int r0 = max(m0, fr * p.flag_bm) - m0, r1 = min(m_end, (fr + 1) * p.flag_bm) - m0;
-        const int c0 = max(n0, fc * p.flag_bn) - n0, c1 = min(n1, (fc + 1) * p.flag_bn) - n0;
-        if (c1 - c0 >= OE) reduce(np_tag, std::true_type{}, r0, r1, c0, c1);
-        else reduce_sliver(r0, r1, c0, c1);
+        f(max(m0, fr * p.flag_bm) - m0, min(m_end, (fr + 1) * p.flag_bm) - m0, max(n0, fc * p.flag_bn) - n0, min(n1, (fc + 1) * p.flag_bn) - n0);
       }
   };
+  auto reduce_pieces = [&](auto np_tag) INLINED {
+    if (!by_rect) {
+      reduce(np_tag, std::false_type{}, 0, 0, 0, 0);
+    } else {
+      if constexpr (LARGE)
+        each_owned([&](int r0, int r1, int c0, int c1) INLINED {
+          if (c1 - c0 >= OE) reduce(np_tag, std::true_type{}, r0, r1, c0, c1);
+        });
+    }
+  };
+  if (tile_cols < OE && p.s_cn == 1) {
+    reduce_sliver(0, m_end - m0, 0, tile_cols);
+    return;
+  }
+  if (by_rect) {
+    // Only the first and the last flag tile of a row can be that narrow here.
+    const int first = p.flag_bn - n0 % p.flag_bn, last = (n0 + tile_cols - 1) % p.flag_bn + 1;
+    if (LARGE && min(first, last) < OE)
+      each_owned([&](int r0, int r1, int c0, int c1) INLINED {
+        if (c1 - c0 < OE) reduce_sliver(r0, r1, c0, c1);
+      });
+  } else if (tail) {
+    reduce_sliver(0, m_end - m0, tile_cols - tail, tile_cols);
+  } else if (!piece_ok && cols > 0) {
+#pragma unroll 1
+    for (int row = t_row; row < m_end - m0; row += RPP) reduce_elements(row);
+  }
   switch (p.world - 1) {
-    case 1: reduce_tile(std::integral_constant<int, 1>{}); break;
-    case 3: reduce_tile(std::integral_constant<int, 3>{}); break;
-    case 7: reduce_tile(std::integral_constant<int, 7>{}); break;
-    default: reduce_tile(std::integral_constant<int, 0>{}); break;
+    case 1: reduce_pieces(std::integral_constant<int, 1>{}); break;
+    case 3: reduce_pieces(std::integral_constant<int, 3>{}); break;
+    case 7: reduce_pieces(std::integral_constant<int, 7>{}); break;
+    default: reduce_pieces(std::integral_constant<int, 0>{}); break;
   }
   PHASE_STAMP(7);
 }

@@ -217,7 +217,7 @@ template <class CFG>
 struct StagedTile {
   char* base;
   __device__ __forceinline__ char* at(int row, int byte) const { return base + CFG::stage_offset(row, byte); }
-  __device__ __forceinline__ u32x4_t piece(int row, int byte, int) const {
+  __device__ __forceinline__ u32x4_t piece(int row, int byte) const {
     if constexpr (!CFG::STAGE_SWIZZLED) {
       return *(const LDS_AS u32x4_any_t*)(LDS_AS char*)at(row, byte);
     } else {
