@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(CFG::NT, CFG::WG_PER_CU * CFG::NW / 4) fused_a
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wk = wave / (CFG::WM * CFG::WN), wm = wave / CFG::WN % CFG::WM, wn = wave % CFG::WN;
 
-  const int tidx = xcd_tile_index(blockIdx.x, gridDim.x, 0, p.tiles_m * p.tiles_n, p.num_xcd);
+  const int tidx = xcd_tile_index(blockIdx.x, gridDim.x, 0, p.tiles_m * p.tiles_n, p.interleave ? 1 : p.num_xcd);
   if (tidx < 0) return;
 #ifdef IRIS_HIP_PHASE_STAMPS
   constexpr int it = 0;  // PHASE_STAMP records the first tile of a workgroup; there is only one here
@@ -646,7 +646,8 @@ int launch_any(FusedParams p, int device, int cu_count, hipStream_t stream, cons
   p.tiles_n = cdiv(p.N, CFG::BN);
   const long long total = (long long)p.tiles_m * p.tiles_n;
   if (total > (1ll << 30)) return iris_host::fail("output of %d x %d has too many tiles", p.M, p.N);
-  p.group_m = any_group_m(p.tiles_m, p.tiles_n, p.num_xcd, cu_count / p.num_xcd * CFG::WG_PER_CU);
+  // (A launch that takes the place of one on packed operands comes with that one's order.)
+  if (p.group_m == 0) p.group_m = any_group_m(p.tiles_m, p.tiles_n, p.num_xcd, cu_count / p.num_xcd * CFG::WG_PER_CU);
   const int grid = cdiv((int)total, p.num_xcd) * p.num_xcd;
   char name[96];
   snprintf(name, sizeof(name), "generic_%s_%dx%d_%s", types, CFG::BM, CFG::BN, CFG::BKC ? "nt" : "nn");
@@ -694,9 +695,9 @@ inline int choose_any_tile(int M, int N, int cu, bool f32_in, bool f32_out, floa
 }
 
 template <int IN, class Out, bool BKC>
-int dispatch_any_layout(const FusedParams& p, int device, int cu, hipStream_t s, const char* types) {
+int dispatch_any_layout(const FusedParams& p, int device, int cu, hipStream_t s, const char* types, int tile) {
   constexpr bool F32_IN = AnyIn<IN>::ES == 4, F32_OUT = Out::size == 4;
-  switch (choose_any_tile(p.M, p.N, cu, F32_IN, F32_OUT)) {
+  switch (tile >= 0 ? tile : choose_any_tile(p.M, p.N, cu, F32_IN, F32_OUT)) {
     case 0:  // (a staged 256x256 tile of float32 would not fit the LDS)
       if constexpr (!F32_OUT) return launch_any<AnyCfg<IN, Out, 256, 256, 2, 4, 1, BKC>>(p, device, cu, s, types);
       break;
@@ -707,9 +708,9 @@ int dispatch_any_layout(const FusedParams& p, int device, int cu, hipStream_t s,
   return launch_any<AnyCfg<IN, Out, 128, 128, 2, F32_IN ? 4 : 2, 1, BKC>>(p, device, cu, s, types);
 }
 
-// The layout of B in LDS follows its unit stride: [k][n] when N is contiguous, else [n][k].
+// The layout of B in LDS follows its unit stride: [k][n] when N is contiguous, else [n][k].  tile: index into kAnyTiles, or -1 for the choice.
 template <int IN, class Out>
-int dispatch_any(const FusedParams& p, int device, int cu, hipStream_t s, const char* types) {
-  return p.s_bn == 1 ? dispatch_any_layout<IN, Out, false>(p, device, cu, s, types)
-                     : dispatch_any_layout<IN, Out, true>(p, device, cu, s, types);
+int dispatch_any(const FusedParams& p, int device, int cu, hipStream_t s, const char* types, int tile) {
+  return p.s_bn == 1 ? dispatch_any_layout<IN, Out, false>(p, device, cu, s, types, tile)
+                     : dispatch_any_layout<IN, Out, true>(p, device, cu, s, types, tile);
 }

@@ -1432,7 +1432,7 @@ int dispatch_mfma_in(FusedParams& p, int kind, bool bkc, int device, int cu, hip
   }
 }
 
-// ANY_ROWS builds, in translation units of their own (iris_hip_rows_<type>.hip): one workgroup per tile.
+// ANY_ROWS builds, in translation units of their own (iris_hip_rows_<type>.hip): one workgroup per tile, in the order of plan_tiles.
 template <class CFG>
 int launch_mfma_rows(const FusedParams& p, int device, hipStream_t s, const char* name) {
   iris_host::set_last_kernel(name);
@@ -1440,8 +1440,7 @@ int launch_mfma_rows(const FusedParams& p, int device, hipStream_t s, const char
 }
 
 template <int IN>
-int dispatch_mfma_rows(FusedParams& p, int kind, bool bkc, int device, int cu, hipStream_t s) {
-  plan_tiles(p, kind, cu);
+int dispatch_mfma_rows(const FusedParams& p, int kind, bool bkc, int device, hipStream_t s) {
   static const char* names[3] = {"bf16", "f16", "fp8"};
   char name[96];
   snprintf(name, sizeof(name), "mfma_%s_%dx%dx%d_%s_rows", names[IN], tile_rows(kind), tile_cols(kind), tile_bk(kind, IN), bkc ? "nt" : "nn");

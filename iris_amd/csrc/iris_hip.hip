@@ -166,31 +166,31 @@ extern template int dispatch_mfma_in<IN_BF16>(FusedParams&, int, bool, int, int,
 extern template int dispatch_mfma_in<IN_F16>(FusedParams&, int, bool, int, int, hipStream_t);
 extern template int dispatch_mfma_in<IN_FP8>(FusedParams&, int, bool, int, int, hipStream_t);
 // Instantiated in iris_hip_rows_<type>.hip.
-extern template int dispatch_mfma_rows<IN_BF16>(FusedParams&, int, bool, int, int, hipStream_t);
-extern template int dispatch_mfma_rows<IN_F16>(FusedParams&, int, bool, int, int, hipStream_t);
-extern template int dispatch_mfma_rows<IN_FP8>(FusedParams&, int, bool, int, int, hipStream_t);
+extern template int dispatch_mfma_rows<IN_BF16>(const FusedParams&, int, bool, int, hipStream_t);
+extern template int dispatch_mfma_rows<IN_F16>(const FusedParams&, int, bool, int, hipStream_t);
+extern template int dispatch_mfma_rows<IN_FP8>(const FusedParams&, int, bool, int, hipStream_t);
 // Instantiated in iris_hip_any_<type>.hip.
-extern template int dispatch_any<IN_BF16, ElemBF16>(const FusedParams&, int, int, hipStream_t, const char*);
-extern template int dispatch_any<IN_BF16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
-extern template int dispatch_any<IN_F16, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*);
-extern template int dispatch_any<IN_F16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
-extern template int dispatch_any<IN_F32, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
-extern template int dispatch_any<IN_FP8, ElemBF16>(const FusedParams&, int, int, hipStream_t, const char*);
-extern template int dispatch_any<IN_FP8, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*);
+extern template int dispatch_any<IN_BF16, ElemBF16>(const FusedParams&, int, int, hipStream_t, const char*, int);
+extern template int dispatch_any<IN_BF16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*, int);
+extern template int dispatch_any<IN_F16, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*, int);
+extern template int dispatch_any<IN_F16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*, int);
+extern template int dispatch_any<IN_F32, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*, int);
+extern template int dispatch_any<IN_FP8, ElemBF16>(const FusedParams&, int, int, hipStream_t, const char*, int);
+extern template int dispatch_any<IN_FP8, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*, int);
 
 namespace {
 
-int dispatch_generic(const FusedParams& p, int in_dtype, int out_dtype, int device, int cu, hipStream_t s) {
+int dispatch_generic(const FusedParams& p, int in_dtype, int out_dtype, int device, int cu, hipStream_t s, int tile = -1) {
   const bool out_f32 = out_dtype == IRIS_HIP_FP32;
   switch (in_dtype) {
     case IRIS_HIP_BF16:
-      return out_f32 ? dispatch_any<IN_BF16, ElemF32>(p, device, cu, s, "bf16_f32") : dispatch_any<IN_BF16, ElemBF16>(p, device, cu, s, "bf16");
+      return out_f32 ? dispatch_any<IN_BF16, ElemF32>(p, device, cu, s, "bf16_f32", tile) : dispatch_any<IN_BF16, ElemBF16>(p, device, cu, s, "bf16", tile);
     case IRIS_HIP_FP16:
-      return out_f32 ? dispatch_any<IN_F16, ElemF32>(p, device, cu, s, "f16_f32") : dispatch_any<IN_F16, ElemF16>(p, device, cu, s, "f16");
-    case IRIS_HIP_FP32: return dispatch_any<IN_F32, ElemF32>(p, device, cu, s, "f32");
+      return out_f32 ? dispatch_any<IN_F16, ElemF32>(p, device, cu, s, "f16_f32", tile) : dispatch_any<IN_F16, ElemF16>(p, device, cu, s, "f16", tile);
+    case IRIS_HIP_FP32: return dispatch_any<IN_F32, ElemF32>(p, device, cu, s, "f32", tile);
     default:
-      return out_dtype == IRIS_HIP_BF16 ? dispatch_any<IN_FP8, ElemBF16>(p, device, cu, s, "fp8_bf16")
-                                        : dispatch_any<IN_FP8, ElemF16>(p, device, cu, s, "fp8_f16");
+      return out_dtype == IRIS_HIP_BF16 ? dispatch_any<IN_FP8, ElemBF16>(p, device, cu, s, "fp8_bf16", tile)
+                                        : dispatch_any<IN_FP8, ElemF16>(p, device, cu, s, "fp8_f16", tile);
   }
 }
 
@@ -425,14 +425,24 @@ bool worth_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, co
   return packing + products * there + results < margin * (4.f + products * any * (fp8 ? 0.7f : 1.f) + results);
 }
 
-// Launches p on packed operands.  Returns 0 or an error, or -1 with nothing done where it is not to be: the any-shape kernel takes it.
+// Launches p on packed operands, or, without memory for them, on the any-shape kernel.  Returns 0 or an error, or -1 with
+// nothing done where the latter is to be launched as always.
 int run_packed(const FusedParams& p, int in_dtype, int out_dtype, int device, int cu, hipStream_t s) {
   PackPlan plan;
-  if (p.no_workspace_alloc || !plan_packing(p, in_dtype, out_dtype, cu, plan) || !worth_packing(p, in_dtype, out_dtype, cu, plan)) return -1;
+  if (!plan_packing(p, in_dtype, out_dtype, cu, plan) || !worth_packing(p, in_dtype, out_dtype, cu, plan)) return -1;
+  plan_tiles(plan.p, plan.kind, cu);
   void* memory = nullptr;
   if (plan.bytes) {
-    memory = g_scratch_allocator.take(plan.bytes, s);
-    if (!memory) return -1;
+    memory = p.no_workspace_alloc ? nullptr : g_scratch_allocator.take(plan.bytes, s);
+    if (!memory) {
+      // Other ranks may have got theirs.  Where they could wait for tiles that this one never reaches, it takes the same tiles in the
+      // same order (layout.h; replayed in tests/host_sim/layout_sim.cpp).
+      if (publishes_alone(tile_launch(plan.p, plan.kind, cu), plan.p.group_m) && (p.epi != EPI_REDUCE_SCATTER || plan.p.interleave)) return -1;
+      FusedParams q = p;
+      q.group_m = plan.p.group_m;
+      q.interleave = plan.p.interleave;
+      return dispatch_generic(q, in_dtype, out_dtype, device, cu, s, plan.kind == TILE_BIG ? 0 : plan.kind == TILE_SKINNY64 ? 3 : 1);
+    }
     PackParams& pack = plan.pack;
     pack.job[0].dst = (char*)memory;
     pack.job[1].dst = (char*)memory + (size_t)pack.job[1].dst;
@@ -450,9 +460,9 @@ int run_packed(const FusedParams& p, int in_dtype, int out_dtype, int device, in
   const bool bkc = p.s_bn != 1;
   int rc = 0;
   switch (in_dtype) {
-    case IRIS_HIP_BF16: rc = dispatch_mfma_rows<IN_BF16>(plan.p, plan.kind, bkc, device, cu, s); break;
-    case IRIS_HIP_FP16: rc = dispatch_mfma_rows<IN_F16>(plan.p, plan.kind, bkc, device, cu, s); break;
-    default: rc = dispatch_mfma_rows<IN_FP8>(plan.p, plan.kind, bkc, device, cu, s);
+    case IRIS_HIP_BF16: rc = dispatch_mfma_rows<IN_BF16>(plan.p, plan.kind, bkc, device, s); break;
+    case IRIS_HIP_FP16: rc = dispatch_mfma_rows<IN_F16>(plan.p, plan.kind, bkc, device, s); break;
+    default: rc = dispatch_mfma_rows<IN_FP8>(plan.p, plan.kind, bkc, device, s);
   }
   g_scratch_allocator.give_back(memory);
   return rc;

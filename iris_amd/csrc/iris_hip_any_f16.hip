@@ -1,5 +1,5 @@
 // The any-shape kernel for f16 inputs (see any_kernel.h).
 #include "any_kernel.h"
 
-template int dispatch_any<IN_F16, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*);
-template int dispatch_any<IN_F16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*);
+template int dispatch_any<IN_F16, ElemF16>(const FusedParams&, int, int, hipStream_t, const char*, int);
+template int dispatch_any<IN_F16, ElemF32>(const FusedParams&, int, int, hipStream_t, const char*, int);

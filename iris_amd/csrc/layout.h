@@ -257,6 +257,8 @@ IRIS_HD int macro_tiles_over_flag_tile(int fm, int fn, int FM, int FN, int KM, i
 //   - The same order on every rank does: the first unfinished tile of that order is running, and published, on all of them.
 //   - A rank whose waiting workgroups leave others room to run (publishes_alone) publishes everything whatever the
 //     others do.  It may take any order, and no order of its own can hold up anybody else.
+// What only one rank knows - whether it got memory, whether its stream is captured - may choose the kernel of such a rank, and for
+// the others only between kernels that take the same tiles in the same order (run_packed in iris_hip.hip).
 // tests/host_sim/layout_sim.cpp replays the launches of all ranks, with what fits at one time, until they end.
 // ---------------------------------------------------------------------------------------------
 enum { EPI_STORE = 0, EPI_ONE_SHOT = 1, EPI_TWO_SHOT = 2, EPI_REDUCE_SCATTER = 3, EPI_ALL_GATHER = 4, EPI_ATOMIC = 5 };

@@ -509,6 +509,20 @@ RankLaunch tiled_launch(const TileLaunch& t) {
   return make_launch(t, o, rounds && workgroup_per_tile(t.epi, t.world, t.sum_peers, t.all_owners), o.interleave ? 1 : t.num_xcd);
 }
 
+// The same tiles on packed operands (launch_mfma_rows), or the any-shape kernel in their place: as always, with a tile and an
+// order of its own, or with the tiles and the order of the packed launch.
+RankLaunch packed_launch(const TileLaunch& t, bool has_memory, int any_m, int any_n, int any_resident) {
+  const TileOrder o = tile_order(t);
+  if (has_memory || !publishes_alone(t, o.group_m)) return make_launch(t, o, true, o.interleave ? 1 : t.num_xcd);
+  TileLaunch a = t;
+  a.tile_m = any_m;
+  a.tile_n = any_n;
+  a.resident = any_resident;
+  TileOrder own = {cdiv(a.M, any_m), cdiv(a.N, any_n), 0, 0, 0, 0};
+  own.group_m = any_group_m(own.tiles_m, own.tiles_n, a.num_xcd, a.resident);
+  return make_launch(a, own, true, a.num_xcd);
+}
+
 // How many workgroups of all ranks are left when nobody can go on.  Workgroup b runs on XCD b % num_xcd, in order, as
 // soon as one in front of it has left (`in_order`: and not before all workgroups below b have started).
 int replay(const std::vector<RankLaunch>& ranks, bool in_order) {
@@ -606,6 +620,20 @@ void check_ranks_finish() {
       for (int r = 0; r < c.world; ++r) ranks.push_back(tiled_launch(launch_of(c.epi, c.M, c.N, c.tile_m, c.tile_n, c.two_per_cu, c.world, r, c.flag_bm, c.flag_bn)));
       const int left = replay(ranks, in_order);
       CHECK(left == 0, "%d workgroups wait for ever: epilogue %d of %d ranks, %dx%d, tiles %dx%d, flag tiles %dx%d", left, c.epi, c.world, c.M, c.N, c.tile_m, c.tile_n, c.flag_bm, c.flag_bn);
+    }
+  // Some ranks multiply packed operands, the others had no memory for them.
+  struct Tile { int m, n, resident; };
+  for (Tile any : {Tile{256, 256, 32}, Tile{128, 128, 64}, Tile{64, 128, 64}, Tile{64, 64, 64}})
+  for (Case c : {Case{EPI_TWO_SHOT, 16001, 4097, 256, 256, 0, 2, 256, 64}, Case{EPI_ONE_SHOT, 16001, 4097, 256, 256, 0, 3, 256, 64},
+                 Case{EPI_ONE_SHOT, 4001, 2877, 256, 256, 0, 8, 256, 64}, Case{EPI_TWO_SHOT, 1999, 2877, 128, 128, 1, 4, 128, 64},
+                 Case{EPI_REDUCE_SCATTER, 8001, 4095, 256, 256, 0, 2, 256, 64}, Case{EPI_REDUCE_SCATTER, 8001, 4095, 256, 256, 0, 4, 256, 64},
+                 Case{EPI_REDUCE_SCATTER, 16383, 8191, 256, 256, 0, 8, 128, 64}, Case{EPI_REDUCE_SCATTER, 4001, 2877, 256, 256, 0, 8, 256, 64}})
+    for (int memory = 0; memory < 1 << c.world; memory += c.world > 4 ? 37 : 1) {
+      std::vector<RankLaunch> ranks;
+      for (int r = 0; r < c.world; ++r)
+        ranks.push_back(packed_launch(launch_of(c.epi, c.M, c.N, c.tile_m, c.tile_n, c.two_per_cu, c.world, r, c.flag_bm, c.flag_bn), memory >> r & 1, any.m, any.n, any.resident));
+      const int left = replay(ranks, false);
+      CHECK(left == 0, "%d workgroups wait for ever: epilogue %d of %d ranks, %dx%d, tiles %dx%d, packed on ranks %x, else %dx%d", left, c.epi, c.world, c.M, c.N, c.tile_m, c.tile_n, memory, any.m, any.n);
     }
   // A rank starts with its own band of rows while that leaves half of the chip to the others.
   CHECK(tile_order(launch_of(EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 8, 3, 256, 64)).tile_rotate == 12 * 16, "reduce-scatter of eight ranks starts with its band");
