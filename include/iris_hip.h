@@ -327,7 +327,8 @@ int iris_hip_stream_capturing(void* stream);
  * data that do not start on 16-byte boundaries) take it from the caller's allocator and give it back
  * as soon as they are enqueued: memory that is given back may be used again by later work on the same stream only.
  * allocate(bytes, stream) is called with the launch's device current and returns NULL when there is none; such launches, those
- * of a stream under capture and all of them while no allocator is set (NULL, NULL) take a kernel that needs no memory.
+ * of a stream under capture and all of them while no allocator is set (NULL, NULL) take a kernel that needs no memory and
+ * gives the same results, bit for bit.
  * Set it before the first launch; both functions are called from whatever thread launches.
  */
 typedef void* (*iris_hip_allocate_fn)(size_t bytes, void* stream);

@@ -413,7 +413,8 @@ bool plan_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, Pac
 bool worth_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, const PackPlan& plan) {
   const bool fp8 = in_dtype == IRIS_HIP_FP8_E4M3;
   float any = 0.f;
-  choose_any_tile(p.M, p.N, cu, false, false, &any);
+  // The 32x32 tile splits K over its waves: the sums would no longer be those of a launch that gets no memory.
+  if (choose_any_tile(p.M, p.N, cu, false, false, &any) == 4) return false;
   const float products = 2e-6f * cu * p.K;
   const float results = (float)p.M * p.N * elem_size(out_dtype) * 2e-7f;  // C, either way
   const int bm = tile_rows(plan.kind), bn = tile_cols(plan.kind);
