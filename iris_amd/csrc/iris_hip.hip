@@ -334,7 +334,7 @@ bool plan_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, Pac
   plan.kind = TILE_SMALL;
   if (big_tiles * 100 >= (long long)cu * 53 && p.M > 64) plan.kind = TILE_BIG;
   else if ((long long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 2ll * cu) plan.kind = TILE_SKINNY64;
-  else if (tiles128 > cu) plan.kind = TILE_SMALL2;
+  else if (tiles128 > cu && p.gather == GATHER_K) plan.kind = TILE_SMALL2;
 
   FusedParams& q = plan.p;
   q = p;
@@ -410,15 +410,36 @@ bool plan_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, Pac
 // 55.5 -> 38.5; 4000x4095x331 25.6 -> 28.0, 500x4095x5001 54.0 -> 53.0, 16000x300x5001 127 -> 159, the last three left where they
 // were.  Two 128x128 tiles per CU have to win more when the peers' tiles are read behind them: the 64x128 tiles of the
 // any-shape kernel, three to a CU, hide each other's round trips (one-shot, eight ranks, fp16 1999x2877x2501 85.7 -> 88.5).
+//
+// The model alone packed 2733 of 10000 launches of every operator (2, 4, 8 ranks and plain products, 16- and 8-bit, both layouts of
+// B, M 1 to 12000, N 64 to 8192, K 200 to 9000, both ways timed in turn): 705 were slower for it, up to 1.9 times.  By tile, time
+// packed : any-shape kernel, and how many were more than 3 % slower:
+//   256x256               0.82, 55 of 758
+//   128x128, one per CU   0.86, 66 of 472 from K = 2400 on; 0.96 at 2000 to 2500, 1.02 at 1600 to 2000, 1.15 at 800 to 1200
+//   128x128, more tiles   1.04, two to a CU or one behind the other, but where the any-shape kernel has three nearly full rounds of
+//                         64x128 tiles against two here and K is long: 0.93 (1999x2877x4003, bf16 93.6 -> 87.9 us, B transposed
+//                         100.6 -> 97.9, e4m3 64.3 -> 58.6)
+//   64x64, one per CU     0.83, 17 of 430; with more tiles 1.04, 154 of 297
+//   instead of 32x32      1.03, 48 of 103 (e4m3 3x120x8685 18.7 -> 23.4 us); that tile also splits K over its waves, and the sums would not be
+//                         those of a launch that gets no memory
+// Operands gathered along K gain with every tile (0.54 to 0.82): the any-shape kernel pads the share of every slot to whole steps.
+// Slot sums of other numbers of ranks than 2, 4 and 8 read the peers one behind the other, which one workgroup per CU does not
+// hide (one-shot of three ranks, bf16 6000x2877x640 112 -> 138 us).
 bool worth_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, const PackPlan& plan) {
   const bool fp8 = in_dtype == IRIS_HIP_FP8_E4M3;
   float any = 0.f;
-  // The 32x32 tile splits K over its waves: the sums would no longer be those of a launch that gets no memory.
-  if (choose_any_tile(p.M, p.N, cu, false, false, &any) == 4) return false;
+  const int any_tile = choose_any_tile(p.M, p.N, cu, false, false, &any);
+  if (any_tile == 4) return false;
+  if (epi_has_flags(p.epi) && p.sum_peers && p.world != 1 && p.world != 2 && p.world != 4 && p.world != 8) return false;
   const float products = 2e-6f * cu * p.K;
   const float results = (float)p.M * p.N * elem_size(out_dtype) * 2e-7f;  // C, either way
   const int bm = tile_rows(plan.kind), bn = tile_cols(plan.kind);
   const long long tiles = (long long)cdiv(p.M, bm) * cdiv(p.N, bn);
+  if (p.gather != GATHER_K && plan.kind != TILE_BIG) {
+    if (plan.kind == TILE_SMALL && p.K < (tiles > cu ? 4000 : 2400)) return false;
+    const long long tiles_64x128 = (long long)cdiv(p.M, 64) * cdiv(p.N, 128);
+    if (tiles > cu && !(plan.kind == TILE_SMALL && any_tile == 2 && tiles_64x128 * 3 > 8ll * cu && tiles_64x128 <= 3ll * cu)) return false;
+  }
   const float rate = (plan.kind == TILE_BIG ? 1400.f : plan.kind == TILE_SMALL ? 1220.f : plan.kind == TILE_SMALL2 ? 964.f : tiles > cu ? 671.f : 560.f) * (fp8 ? 1.9f : 1.f);
   const float there = (float)bm * bn * ((tiles + cu - 1) / cu) / rate;
   const float packing = (plan.bytes ? 4.5f + plan.bytes * 2 / 5.2e6f : 0.f) + (plan.kind == TILE_SKINNY64 ? 4.f : 3.f);
