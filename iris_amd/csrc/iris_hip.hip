@@ -313,6 +313,12 @@ bool rows_of_whole_lines(const FusedParams& p, int out_dtype) {
 // ------------------------------------------------------------------------------------------------
 ScratchAllocator g_scratch_allocator;
 
+// The sizes that choose among the tiled kernels (run_fused, plan_packing): enough 256x256 tiles; at most two 64x64 tiles per CU; more
+// 128x128 tiles than CUs.
+bool fills_big_tiles(const FusedParams& p, int cu) { return (long long)cdiv(p.M, 256) * cdiv(p.N, 256) * 100 >= (long long)cu * 53; }
+bool fits_64x64_tiles(const FusedParams& p, int cu) { return (long long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 2ll * cu; }
+bool needs_two_128x128_tiles(const FusedParams& p, int cu) { return (long long)cdiv(p.M, 128) * cdiv(p.N, 128) > cu; }
+
 struct PackPlan {
   FusedParams p;      // the launch on the packed operands
   PackParams pack;
@@ -330,11 +336,10 @@ bool plan_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, Pac
   const int sources = p.gather == GATHER_K ? p.world : 1;
   auto whole = [&](long long n) { return (n + ce - 1) / ce * ce; };
 
-  const long long big_tiles = (long long)cdiv(p.M, 256) * cdiv(p.N, 256), tiles128 = (long long)cdiv(p.M, 128) * cdiv(p.N, 128);
   plan.kind = TILE_SMALL;
-  if (big_tiles * 100 >= (long long)cu * 53 && p.M > 64) plan.kind = TILE_BIG;
-  else if ((long long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 2ll * cu) plan.kind = TILE_SKINNY64;
-  else if (tiles128 > cu && p.gather == GATHER_K) plan.kind = TILE_SMALL2;
+  if (fills_big_tiles(p, cu) && p.M > 64) plan.kind = TILE_BIG;
+  else if (fits_64x64_tiles(p, cu)) plan.kind = TILE_SKINNY64;
+  else if (needs_two_128x128_tiles(p, cu) && p.gather == GATHER_K) plan.kind = TILE_SMALL2;
 
   FusedParams& q = plan.p;
   q = p;
@@ -529,16 +534,15 @@ int run_fused(FusedParams p, int in_dtype, int out_dtype, int path, void* stream
   // has at most 64 rows; the latency-oriented 32x32 kernel (decode_kernel.h) for at most two such tiles per CU;
   // 64x64 tiles for at most two of those per CU; 64x128 tiles for at most 64 rows, and for at most two such
   // tiles per CU when K is short; else 128x128 - two workgroups per CU when there are more such tiles than CUs.
-  const long long big_tiles = (long long)cdiv(p.M, 256) * cdiv(p.N, 256);
   const bool rows64_ok = !(p.gather == GATHER_M && p.M_local % 64);
   int kind = TILE_SMALL;
-  if (big_tiles * 100 >= (long long)facts->cu_count * 53 && !(p.M <= 64 && rows64_ok)) kind = TILE_BIG;
+  if (fills_big_tiles(p, facts->cu_count) && !(p.M <= 64 && rows64_ok)) kind = TILE_BIG;
   else if (decode_sized(p, facts->cu_count, in_dtype) && decode_gather_ok(p, in_dtype) && p.world <= 8) kind = TILE_DECODE;
-  else if ((long long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 2ll * facts->cu_count && rows64_ok) kind = TILE_SKINNY64;
+  else if (fits_64x64_tiles(p, facts->cu_count) && rows64_ok) kind = TILE_SKINNY64;
   else if (rows64_ok && (p.M <= 64 || ((long long)cdiv(p.M, 64) * cdiv(p.N, 128) <= 2ll * facts->cu_count &&
                                        (long long)p.K * elem_size(in_dtype) <= 2048)))
     kind = TILE_SKINNY;
-  else if ((long long)cdiv(p.M, 128) * cdiv(p.N, 128) > facts->cu_count) kind = TILE_SMALL2;
+  else if (needs_two_128x128_tiles(p, facts->cu_count)) kind = TILE_SMALL2;
   // IRIS_HIP_TILE = big | small | small2 | skinny | skinny64 overrides the choice among the tiled kernels (a tuning
   // aid; results do not depend on the tile shape beyond the order of the fp32 sums over K).
   static const int forced_tile = [] {

@@ -4,7 +4,7 @@
 // The any-shape kernel fetches such rows through registers, every tile again: 16-byte loads that straddle lines, LDS writes
 // and a barrier chain per K step.  With more than a few tiles to a row or column of the output one pass over the
 // operands costs less than that (which launches: worth_packing in iris_hip.hip).  It is bound by memory: one 16-byte load and
-// one 16-byte store per piece, four of each in flight per thread.
+// one 16-byte store per piece, two of each in flight per thread.
 #pragma once
 
 #include "fused_params.h"
