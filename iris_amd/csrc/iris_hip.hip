@@ -339,7 +339,7 @@ bool plan_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, Pac
   plan.kind = TILE_SMALL;
   if (fills_big_tiles(p, cu) && p.M > 64) plan.kind = TILE_BIG;
   else if (fits_64x64_tiles(p, cu)) plan.kind = TILE_SKINNY64;
-  else if (needs_two_128x128_tiles(p, cu) && p.gather == GATHER_K) plan.kind = TILE_SMALL2;
+  else if (needs_two_128x128_tiles(p, cu) && sources > 1) plan.kind = TILE_SMALL2;
 
   FusedParams& q = plan.p;
   q = p;
@@ -440,7 +440,7 @@ bool worth_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, co
   const float results = (float)p.M * p.N * elem_size(out_dtype) * 2e-7f;  // C, either way
   const int bm = tile_rows(plan.kind), bn = tile_cols(plan.kind);
   const long long tiles = (long long)cdiv(p.M, bm) * cdiv(p.N, bn);
-  if (p.gather != GATHER_K && plan.kind != TILE_BIG) {
+  if ((p.gather != GATHER_K || p.world == 1) && plan.kind != TILE_BIG) {
     if (plan.kind == TILE_SMALL && p.K < (tiles > cu ? 4000 : 2400)) return false;
     const long long tiles_64x128 = (long long)cdiv(p.M, 64) * cdiv(p.N, 128);
     if (tiles > cu && !(plan.kind == TILE_SMALL && any_tile == 2 && tiles_64x128 * 3 > 8ll * cu && tiles_64x128 <= 3ll * cu)) return false;

@@ -102,3 +102,24 @@ def test_tiles_that_split_k_stay_on_the_any_shape_kernel():
     dA, dB, out = heap_tensor(ctx, randn_cpu((M, K), 1, torch.float16)), heap_tensor(ctx, randn_cpu((K, N), 2, torch.float16)), ctx.zeros((2 * M, N), dtype=torch.float16)
     ops.matmul_all_gather(ctx, out, dA, dB, config=cfg)
     assert _lib.last_kernel() == "generic_f16_32x32_nn", _lib.last_kernel()
+
+
+# What packing costs more than it gives: a short K on 128x128 tiles, more 128x128 or 64x64 tiles than CUs, sums of three ranks; and the
+# other side of each line.
+@pytest.mark.parametrize("op,W,M,N,K,packed", [
+    ("plain", 1, 1001, 2877, 2301, False), ("plain", 1, 1001, 2877, 2501, True), ("plain", 1, 1999, 2877, 3501, False),
+    ("plain", 1, 1999, 2877, 4003, True), ("plain", 1, 2999, 2877, 4003, True), ("plain", 1, 1501, 2877, 4003, False),
+    ("plain", 1, 501, 2301, 5001, False), ("plain", 1, 501, 1501, 5001, True), ("one_shot", 3, 4003, 2877, 1003, False), ("one_shot", 2, 4003, 2877, 1003, True)])
+def test_where_operands_are_laid_out_anew(op, W, M, N, K, packed):
+    dtype = torch.bfloat16
+    ctx = iris.iris(1 << 28, num_ranks=W, rank=W - 1)
+    dA, dB, out = ctx.zeros((M, K), dtype=dtype), ctx.zeros((K, N), dtype=dtype), ctx.zeros((M, N), dtype=dtype)
+    cfg = iris.FusedConfig(block_size_m=64, block_size_n=64, block_size_k=1, all_reduce_variant="one_shot")
+    if op == "plain":
+        ops.all_gather_matmul(ctx, out, dA, dB, config=cfg)
+    else:
+        ws = ops.matmul_all_reduce_preamble(ctx, out, dA, dB, config=cfg)
+        stage_peers(ctx, ws, [torch.zeros((M, N), dtype=dtype) for _ in range(W)])
+        ops.matmul_all_reduce(ctx, out, dA, dB, config=cfg, workspace=ws)
+    assert _lib.last_kernel().endswith("_rows") == packed, _lib.last_kernel()
+    assert not out.any()
