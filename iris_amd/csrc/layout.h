@@ -303,12 +303,13 @@ IRIS_HD bool publishes_alone(const TileLaunch& t, int group_m) {
   if (t.epi != EPI_REDUCE_SCATTER || t.all_owners) return false;
   int first, last;
   if (!band_tile_rows(t, first, last)) return true;
-  // The groups that hold the band (its tiles may be every second one of a group's), at most half of what runs at one time:
-  // CUs may be busy with other launches.
+  // The groups that hold the band (its tiles may be every second one of a group's), at most five eighths of what runs at one time:
+  // CUs may be busy with other launches.  (At a half the last of four ranks no longer starts with its band of 140 tiles: bf16
+  // 3128x7162x1270, 256 CUs, 112 -> 143 us.)
   first = first / group_m * group_m;
   last = last / group_m * group_m + group_m - 1;
   if (last >= tiles_m) last = tiles_m - 1;
-  return cdiv((last - first + 1) * tiles_n, t.num_xcd) * 2 <= t.resident;
+  return cdiv((last - first + 1) * tiles_n, t.num_xcd) * 8 <= t.resident * 5;
 }
 
 IRIS_HD TileOrder tile_order(const TileLaunch& t) {
@@ -362,7 +363,7 @@ IRIS_HD TileOrder tile_order(const TileLaunch& t) {
   // The reduce-scatter with peers is dealt out as well (its launches hand one workgroup per tile to the
   // hardware in this order), starting with the band of rows this rank sums: those tiles take half as long
   // again as the others, so they go first and spread over every XCD (8192x4096x1376, eight ranks, rank 0:
-  // 111.8 -> 106.6 us against spans of sixteen rows).  A band that would fill more than half of the chip with workgroups
+  // 111.8 -> 106.6 us against spans of sixteen rows).  A band that would fill more than five eighths of the chip with workgroups
   // that wait - for tiles that the other ranks only reach behind theirs - has to keep its place in the common order (last of
   // eight ranks, own band first -> common order, us: 16384x8192x512, bands of 256 tiles, 228 -> 244; of two ranks 8192x8192x1024
   // 156 -> 159, 8192x4096x1376 97 -> 97).

@@ -612,6 +612,7 @@ void check_ranks_finish() {
                  Case{EPI_REDUCE_SCATTER, 8192, 4097, 256, 256, 0, 2, 256, 64}, Case{EPI_REDUCE_SCATTER, 16383, 4093, 256, 256, 0, 4, 256, 64},
                  Case{EPI_REDUCE_SCATTER, 16383, 8191, 256, 256, 0, 8, 128, 64}, Case{EPI_REDUCE_SCATTER, 16384, 8192, 256, 256, 0, 2, 96, 80},
                  Case{EPI_REDUCE_SCATTER, 8192, 1024, 128, 128, 1, 2, 64, 64}, Case{EPI_REDUCE_SCATTER, 16384, 256, 128, 128, 1, 3, 128, 64},
+                 Case{EPI_REDUCE_SCATTER, 3128, 7162, 256, 256, 0, 4, 256, 64},
                  Case{EPI_REDUCE_SCATTER, 16384, 2048, 256, 256, 0, 8, 8192, 64}, Case{EPI_REDUCE_SCATTER, 8192, 8192, 256, 256, 0, 8, 4096, 4096},
                  Case{EPI_ONE_SHOT, 16384, 8192, 256, 256, 0, 8, 256, 64}, Case{EPI_ONE_SHOT, 8191, 4097, 256, 256, 0, 2, 96, 80},
                  Case{EPI_TWO_SHOT, 16384, 4096, 256, 256, 0, 8, 256, 64}, Case{EPI_TWO_SHOT, 8191, 4097, 256, 256, 0, 2, 96, 80}})
@@ -635,9 +636,10 @@ void check_ranks_finish() {
       const int left = replay(ranks, false);
       CHECK(left == 0, "%d workgroups wait for ever: epilogue %d of %d ranks, %dx%d, tiles %dx%d, packed on ranks %x, else %dx%d", left, c.epi, c.world, c.M, c.N, c.tile_m, c.tile_n, memory, any.m, any.n);
     }
-  // A rank starts with its own band of rows while that leaves half of the chip to the others.
+  // A rank starts with its own band of rows while that leaves room for the others.
   CHECK(tile_order(launch_of(EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 8, 3, 256, 64)).tile_rotate == 12 * 16, "reduce-scatter of eight ranks starts with its band");
   CHECK(tile_order(launch_of(EPI_REDUCE_SCATTER, 8192, 4096, 256, 256, 0, 2, 1, 256, 64)).tile_rotate == 0, "reduce-scatter of two ranks: the same order on both");
+  CHECK(tile_order(launch_of(EPI_REDUCE_SCATTER, 3128, 7162, 256, 256, 0, 4, 3, 256, 64)).tile_rotate == 8 * 28, "the last of four ranks starts with its 140 tiles");
 }
 
 // ---- vote of a workgroup in a loop with one barrier per step -----------------------------------------
