@@ -78,7 +78,9 @@ struct FusedParams {
   int no_workspace_alloc;  // host only: the caller must not trigger an allocation (split tiles need one)
   // (Behind the arguments of the small kernel, which is 1 % slower with anything in between.)
   int whole_lines;   // rows of C and aux start and end with 128-byte lines (see store16_system_nt)
-  int stream_peers;  // the peers' tiles are read past the caches (peers_past_caches in iris_hip.hip)
+  // The peers' tiles are read past the caches (peers_past_caches in iris_hip.hip).  The tiled kernel with other numbers of ranks than 2,
+  // 4 and 8 always does, the any-shape kernel's 32x32 tile does only with such.
+  int stream_peers;
 #ifdef IRIS_HIP_PHASE_STAMPS
   unsigned long long* stamps;  // diagnostic build: rows of 16 time stamps (see PHASE_STAMP)
   long long stamp_rows;        // rows the buffer holds; rows beyond it are not written
@@ -231,7 +233,9 @@ __device__ __forceinline__ void store16_system(char* p, u32x4_t v) {
 // The same for rows that are whole lines, past the caches' keep policy as well: own tiles on their way to the peers do not push
 // everything else out of the last-level cache (bf16, eight ranks, six workspaces in turn: reduce-scatter 8192x4096x1376
 // 118.6 -> 104.9 us, two-shot 8192x4096x1376 126.6 -> 112.2; with one workspace, which the cache holds, 103.4 -> 104.4 and 107 ->
-// 111).  A line that two workgroups write in parts does better in the cache (2000x2896x1376 51.2 us, this way 53.8).
+// 111).  It is done at every size: launches whose slots the cache holds lose 0 to 2 % by it with one or two workspaces in turn and gain 4
+// to 20 % with six (two-shot 2048x4096x512 31.2 -> 26.1 us, 4096x4096x1376 of four ranks 66.5 -> 61.0, reduce-scatter 2048x4096x1376
+// 42.9 -> 38.8).  A line that two workgroups write in parts does better in the cache (2000x2896x1376 51.2 us, this way 53.8).
 __device__ __forceinline__ void store16_system_nt(char* p, u32x4_t v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(p), "v"(v) : "memory");
 }
