@@ -23,7 +23,8 @@
  *   - Return value: 0 on success, otherwise a hipError_t value.  Argument errors return
  *     hipErrorInvalidValue (1); iris_hip_last_error() then describes the problem.
  *   - The library calls hipMalloc only for the split-tile workspace described at iris_hip_set_split_tiles
- *     (iris_hip_matmul_all_reduce_noalloc never does).  It keeps between calls: device facts (CU count, XCD count, LDS
+ *     (iris_hip_matmul_all_reduce_noalloc never does); an allocator set with iris_hip_set_scratch_allocator may. The library
+ *     keeps between calls: that allocator's two functions, device facts (CU count, XCD count, LDS
  *     size) cached per device under a mutex, a once-per-device "attribute set" flag per kernel build
  *     (atomic), the last error and last kernel name per host thread, the contents of context tensors
  *     registered with iris_hip_register_context (under a mutex), and one static device array that

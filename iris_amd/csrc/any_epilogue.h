@@ -7,7 +7,7 @@
 // For the lambdas that the kernel is made of.  They keep their arrays in the kernel's registers only where they are inlined,
 // which the compiler's cost limit did not allow where a piece has sixteen elements: e4m3 operands were worked on in
 // scratch memory (1999x2877x1371 as a plain GEMM 200 -> 31 us, 4095x4095x2047 223 -> 75, 200x1001x3001 56 -> 12.5).  On the
-// 256x256 tile (the 4095x4095x2047) 17 to 19 registers still do not fit and are spilled, 72 to 80 bytes a lane.
+// 256x256 tile (the 4095x4095x2047) 19 to 25 registers still do not fit and are spilled, 80 to 88 bytes a lane.
 #define INLINED __attribute__((always_inline))
 
 // Results: past the caches' keep policy when the rows are whole 16-byte pieces, through them otherwise, where the L2 puts
