@@ -415,8 +415,7 @@ bool plan_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, Pac
 // two sets of operands in turn); packing moves its bytes at 5.2 TB/s and costs a launch.  What it gives and where it
 // does not: 4000x2877x2501 125.4 -> 72.1 us, 2000x1501x8001 133.7 -> 84.3, 1000x701x8001 65.5 -> 44.8, e4m3 4000x4095x1371
 // 55.5 -> 38.5; 4000x4095x331 25.6 -> 28.0, 500x4095x5001 54.0 -> 53.0, 16000x300x5001 127 -> 159, the last three left where they
-// were.  Two 128x128 tiles per CU have to win more when the peers' tiles are read behind them: the 64x128 tiles of the
-// any-shape kernel, three to a CU, hide each other's round trips (one-shot, eight ranks, fp16 1999x2877x2501 85.7 -> 88.5).
+// were.
 //
 // The model alone packed 2733 of 10000 launches of every operator (2, 4, 8 ranks and plain products, 16- and 8-bit, both layouts of
 // B, M 1 to 12000, N 64 to 8192, K 200 to 9000, both ways timed in turn): 705 were slower for it, up to 1.9 times.  By tile, time
@@ -450,8 +449,7 @@ bool worth_packing(const FusedParams& p, int in_dtype, int out_dtype, int cu, co
   const float rate = (plan.kind == TILE_BIG ? 1400.f : plan.kind == TILE_SMALL ? 1220.f : plan.kind == TILE_SMALL2 ? 964.f : tiles > cu ? 671.f : 560.f) * (fp8 ? 1.9f : 1.f);
   const float there = (float)bm * bn * ((tiles + cu - 1) / cu) / rate;
   const float packing = (plan.bytes ? 4.5f + plan.bytes * 2 / 5.2e6f : 0.f) + (plan.kind == TILE_SKINNY64 ? 4.f : 3.f);
-  const float margin = plan.kind == TILE_SMALL2 && epi_has_flags(p.epi) && p.sum_peers && p.world > 1 ? 0.85f : 0.92f;
-  return packing + products * there + results < margin * (4.f + products * any * (fp8 ? 0.7f : 1.f) + results);
+  return packing + products * there + results < 0.92f * (4.f + products * any * (fp8 ? 0.7f : 1.f) + results);
 }
 
 // Launches p on packed operands, or, without memory for them, on the any-shape kernel.  Returns 0 or an error, or -1 with
